@@ -371,6 +371,7 @@ int grouped(int fmt, const uint16_t* act, size_t act_stride, const DgppMoeSegmen
   a.k = k;
   a.rows_per_block = rows_per_block > 0 ? rows_per_block : INT_MAX;
   a.group_rows = max_stage_rows(k);
+  a.max_rows = max_rows;
   a.act_rows = act_rows;
   a.gate_up = out_up ? 2 : (gate_up_limit != nullptr ? 1 : 0);
   a.limit = gate_up_limit ? *gate_up_limit : 0.f;

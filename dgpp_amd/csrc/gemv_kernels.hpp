@@ -7,6 +7,8 @@
 // :999-1059 and :2149-2195 (grouped kernels).
 #pragma once
 
+#include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "../../include/dgpp_amd.h"
@@ -902,6 +904,7 @@ struct GroupedArgs {
   int n, k;
   int rows_per_block;  // segment rows per z block
   int group_rows;      // activation rows staged per pass (<= kMaxActRows)
+  int max_rows;        // no segment has more
   const int32_t* act_rows;  // matrix-core form only, nullable: activation row of each segment row
   int once;                 // every segment fits one pass over its expert (nontemporal loads)
   int gate_up;              // matrix-core form only, `which` unused, bf16 out: 1 = gate and up rows + SwiGLU in one
@@ -958,6 +961,7 @@ __global__ __launch_bounds__(kBlockThreads, kMinWavesPerSimd) void grouped_gemv_
 }  // namespace dgpp_amd
 
 #include "gemv_mfma_kernels.hpp"
+#include "gemv_tiled.hpp"
 
 namespace dgpp_amd {
 
@@ -1096,8 +1100,76 @@ inline bool use_mfma_core() { return tune_get(kTuneCore) == 2; }
 // `ws` (nullable) holds parts * m * n floats: the K parts then run in separate blocks and a second
 // launch folds them (same bits); worth it only when the unsplit grid leaves the chip under-filled.
 
+// The tiled form (gemv_tiled.hpp) reads activation rows in whole 16-byte vectors.
+template <class Args>
+inline bool tiled_rows_aligned(const Args& a) {
+  if ((reinterpret_cast<uintptr_t>(a.act) & 15u) != 0) return false;
+  if (a.a4_scales == nullptr) return (a.act_stride & 7u) == 0;
+  return (a.act_stride & 15u) == 0 && ((reinterpret_cast<uintptr_t>(a.a4_scales) | a.a4_scale_stride) & 1u) == 0;
+}
+// Bench / test switch 15: 1 never, 2 always (where it can); 16: passes of a segment side by side.
+inline bool dense_takes_tiled(const DenseArgs& a) {
+  const int knob = tune_get(kTuneTiled);
+  if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return false;
+  if (knob == 2) return true;
+  return a.m > 64;
+}
+inline bool grouped_takes_tiled(const GroupedArgs& a, int max_rows) {
+  const int knob = tune_get(kTuneTiled);
+  if (knob == 1 || a.rows_per_block != INT_MAX || !tiled_rows_aligned(a)) return false;
+  if (knob == 2) return true;
+  return max_rows > 128;
+}
+
+template <int FMT>
+hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
+  const MGeom g = mgeom<FMT>(a.k);
+  const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows, passes = (a.m + kTiledCols - 1) / kTiledCols;
+  const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
+  hipError_t err = hipSuccess;
+  auto go = [&](auto kern) {
+    err = ensure_lds(kern, kTiledLds);
+    if (err == hipSuccess) hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), kTiledLds, stream, a, g, row_tiles, passes);
+  };
+  if constexpr (FMT == kFmtNvfp4) {
+    if (a.a4_scales != nullptr) {
+      go(tiled_dense_kernel<FMT, true>);
+      return err != hipSuccess ? err : hipGetLastError();
+    }
+  }
+  go(tiled_dense_kernel<FMT, false>);
+  return err != hipSuccess ? err : hipGetLastError();
+}
+
+template <int FMT>
+hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, hipStream_t stream) {
+  const MGeom g = mgeom<FMT>(a.k);
+  const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
+  const int row_tiles = (a.n + block_rows - 1) / block_rows;
+  const unsigned gx = static_cast<unsigned>((n_segs + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(row_tiles);
+  // passes of a segment that run side by side: all of them where the segments are few, else some
+  const unsigned all = static_cast<unsigned>((max_rows + kTiledCols - 1) / kTiledCols);
+  const unsigned want = tune_get(kTuneTiledPasses) > 0 ? static_cast<unsigned>(tune_get(kTuneTiledPasses)) : std::max(1u, 8192u / gx);
+  const dim3 grid(gx, std::min(all, want));
+  hipError_t err = hipSuccess;
+  auto go = [&](auto kern) {
+    err = ensure_lds(kern, kTiledLds);
+    if (err == hipSuccess) hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), kTiledLds, stream, a, g, n_segs, row_tiles);
+  };
+  if constexpr (FMT == kFmtNvfp4) {
+    if (a.a4_scales != nullptr) {
+      go(tiled_grouped_kernel<FMT, false, true>);
+      return err != hipSuccess ? err : hipGetLastError();
+    }
+  }
+  if (a.gate_up != 0) go(tiled_grouped_kernel<FMT, true, false>);
+  else go(tiled_grouped_kernel<FMT, false, false>);
+  return err != hipSuccess ? err : hipGetLastError();
+}
+
 template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
+  if (dense_takes_tiled(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const unsigned gx = static_cast<unsigned>((a.n + 63) / 64), gy = static_cast<unsigned>((a.m + kTileCols - 1) / kTileCols);
   const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
@@ -1179,6 +1251,7 @@ hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, f
 
 template <int FMT>
 hipError_t launch_grouped_mfma(const GroupedArgs& a, int n_segs, int z_ext, hipStream_t stream) {
+  if (grouped_takes_tiled(a, a.max_rows)) return launch_grouped_tiled<FMT>(a, n_segs, a.max_rows, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const dim3 grid(static_cast<unsigned>((a.n + 63) / 64), static_cast<unsigned>(n_segs), static_cast<unsigned>(z_ext));
   hipError_t err = hipSuccess;

@@ -263,6 +263,7 @@ int grouped_w4a4(const uint8_t* codes, const uint8_t* scales, const float* gs, c
   a.k = k;
   a.rows_per_block = INT_MAX;
   a.group_rows = kMaxActRows;
+  a.max_rows = max_rows;
   a.act_rows = act_rows;
   a.gate_up = 0;
   a.limit = 0.f;
