@@ -11,6 +11,7 @@
 
 #include "../../include/dgpp_amd.h"
 #include "capi_errors.hpp"
+#include "gemv_core.hpp"
 #include "numerics.hpp"
 
 namespace dgpp_amd {
@@ -265,6 +266,196 @@ hipError_t launch_gemm_waves(const uint8_t* a, const uint8_t* as, const uint8_t*
   return launch_gemm_mt<Out, 4, WAVES>(a, as, w, ws, out, m, n, k, stride, s);
 }
 
+// ---- GEMM, many activation rows --------------------------------------------------------------------
+//
+// A block of 2 x 2 wavefronts owns TN = 32 WN rows of W and TM = 32 WM rows of A, a wavefront WN x WM 16 x 16 tiles of
+// them. The form above has every 16 rows of W pull all of A's k range through the L2 (m * k * n / 16 bytes); here an
+// operand byte in LDS serves TN or TM rows. A step's (TN + TM) x 128 bytes go through registers, DEPTH steps ahead of their
+// use, into one of two LDS stages in the layout above, the rows' four scale bytes beside them; one barrier per step.
+//
+// The chain of an output element is the other form's bit for bit: the steps s = c, c + CHAINS, ... accumulate one after
+// the other, and the CHAINS sums are added in order of c - the steps are only visited in that order here.
+template <int WN, int WM>
+struct TileStage {
+  static constexpr int kTN = 32 * WN, kTM = 32 * WM, kRows = kTN + kTM;
+  u32x4 unit[kRows * 8];
+  uint32_t scale[kRows];
+};
+
+template <typename Out, int WN, int WM, int DEPTH, int CHAINS>
+__global__ __launch_bounds__(256, 2) void mxfp8_gemm_tiled_kernel(
+    const uint8_t* __restrict__ a, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ w,
+    const uint8_t* __restrict__ w_scales, Out* __restrict__ out, int m, int n, int k, size_t out_stride, int row_tiles,
+    int passes) {
+  using Stage = TileStage<WN, WM>;
+  constexpr int kTN = Stage::kTN, kTM = Stage::kTM, kLoads = Stage::kRows / 32;
+  __shared__ Stage stages[2];
+  // Consecutive workgroups go to the eight XCDs in turn: an XCD keeps the column passes of a row tile to itself, so
+  // that its L2 reads the tile's weights once.
+  const int lin = static_cast<int>(blockIdx.x), idx = lin / 8;
+  const int row_tile = idx / passes * 8 + lin % 8;
+  if (row_tile >= row_tiles) return;
+  const int n0 = row_tile * kTN, m0 = idx % passes * kTM;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int wn = (wave & 1) * WN * 16, wm = kTN + (wave >> 1) * WM * 16;   // first rows of the stage that the wave reads
+  const int kblocks = k >> 5, steps = (kblocks + 3) >> 2;
+  const int piece = threadIdx.x & 7;
+  const uint8_t* src[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = i * 32 + static_cast<int>(threadIdx.x >> 3);
+    src[i] = i * 32 < kTN ? w + static_cast<size_t>(min(n0 + row, n - 1)) * k
+                          : a + static_cast<size_t>(min(m0 + row - kTN, m - 1)) * k;
+  }
+  static_assert(Stage::kRows <= 256, "a thread carries the scales of one row");
+  const int srow = min(static_cast<int>(threadIdx.x), Stage::kRows - 1);   // the threads past it write the last row's again
+  const uint8_t* ssrc = srow < kTN ? w_scales + static_cast<size_t>(min(n0 + srow, n - 1)) * kblocks
+                                   : a_scales + static_cast<size_t>(min(m0 + srow - kTN, m - 1)) * kblocks;
+
+  // No branch around a load: only then does the compiler count the loads in flight and wait for the oldest step alone.
+  // Past k a lane reads the start of its row (W's become zeros in commit(), which is enough: A's and the scales that
+  // meet them are the row's own, NaN only where the sums are). A row's four scale bytes are one unaligned word; where
+  // the last step has two, it is the row's last word, turned so that they come first.
+  struct __attribute__((packed, aligned(1))) Word { uint32_t v; };
+  u32x4 t[DEPTH][kLoads];
+  uint32_t sc[DEPTH];
+  auto load = [&](int s, u32x4 (&to)[kLoads], uint32_t& scale) {
+    const int at = s * 128 + piece * 16, from = at < k ? at : 0;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) to[i] = *reinterpret_cast<const u32x4*>(src[i] + from);
+    scale = reinterpret_cast<const Word*>(ssrc + min(s * 4, kblocks - 4))->v;
+  };
+  auto commit = [&](int s, Stage& st, const u32x4 (&from)[kLoads], uint32_t scale) {
+    const bool inside = s * 128 + piece * 16 < k;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      u32x4 v = from[i];
+      if (i * 32 < kTN) v = inside ? v : u32x4{0u, 0u, 0u, 0u};
+      st.unit[region_unit(i * 32 + static_cast<int>(threadIdx.x >> 3), piece)] = v;
+    }
+    st.scale[srow] = __builtin_amdgcn_alignbit(scale, scale, s * 4 + 4 > kblocks ? 16 : 0);
+  };
+
+  v4f acc[WN][WM], sum[WN][WM];
+#pragma unroll
+  for (int i = 0; i < WN; ++i)
+#pragma unroll
+    for (int j = 0; j < WM; ++j) acc[i][j] = sum[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  // The order of the steps: s, s + CHAINS, ... of chain c, then chain c + 1 (c < CHAINS: every step once). `ahead` is
+  // DEPTH steps before `at`.
+  struct Walk {
+    int s, c;
+    __device__ __forceinline__ bool last_of_chain(int steps) const { return s + CHAINS >= steps; }
+    __device__ __forceinline__ void next(int steps) { s = last_of_chain(steps) ? ++c : s + CHAINS; }
+  };
+  const int chains = min(CHAINS, steps);
+  Walk at = {0, 0}, ahead = {0, 0};
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    load(min(ahead.s, steps - 1), t[d], sc[d]);   // past the last step: that step again, unused
+    ahead.next(steps);
+  }
+  int buf = 0;
+  for (;;) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      Stage& st = stages[buf];
+      buf ^= 1;
+      commit(at.s, st, t[d], sc[d]);
+      load(min(ahead.s, steps - 1), t[d], sc[d]);
+      ahead.next(steps);
+      __syncthreads();   // the stage is whole; its readers of two steps before passed the barrier of the step between
+      const uint8_t* sb = reinterpret_cast<const uint8_t*>(st.scale);
+      v8i wv[WN];
+      int ws[WN];
+#pragma unroll
+      for (int i = 0; i < WN; ++i) {
+        const int row = wn + i * 16 + r;
+        wv[i] = as_operand(st.unit[region_unit(row, g)], st.unit[region_unit(row, 4 + g)]);
+        ws[i] = sb[row * 4 + g];
+      }
+#pragma unroll
+      for (int j = 0; j < WM; ++j) {
+        const int row = wm + j * 16 + r;
+        const v8i av = as_operand(st.unit[region_unit(row, g)], st.unit[region_unit(row, 4 + g)]);
+        const int as = sb[row * 4 + g];
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wv[i], av, acc[i][j], 0, 0, 0, ws[i], 0, as);
+      }
+      if (at.last_of_chain(steps)) {
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+#pragma unroll
+          for (int j = 0; j < WM; ++j) {
+            sum[i][j] = at.c == 0 ? acc[i][j] : sum[i][j] + acc[i][j];
+            acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+      at.next(steps);
+      if (at.c >= chains) goto summed;   // not a break: a loop condition would join here with fewer loads in flight
+    }
+  }
+summed:
+  if (chains < CHAINS) {   // the other form's empty partial sums: -0 becomes +0
+#pragma unroll
+    for (int i = 0; i < WN; ++i)
+#pragma unroll
+      for (int j = 0; j < WM; ++j) sum[i][j] = sum[i][j] + acc[i][j];
+  }
+
+#pragma unroll
+  for (int j = 0; j < WM; ++j) {
+    const int a_row = m0 + wm - kTN + j * 16 + r;
+    if (a_row >= m) continue;
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+      const int col = n0 + wn + i * 16 + g * 4;
+      Out* dst = out + static_cast<size_t>(a_row) * out_stride + col;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < n) put<Out>(dst + e, sum[i][j][e]);
+    }
+  }
+}
+
+template <typename Out, int WN, int WM, int DEPTH>
+hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* ws, Out* out, int m, int n,
+                             int k, size_t stride, hipStream_t stream) {
+  constexpr int tn = 32 * WN, tm = 32 * WM;
+  const int row_tiles = (n + tn - 1) / tn, passes = (m + tm - 1) / tm;
+  const dim3 grid(static_cast<unsigned>((row_tiles + 7) / 8 * 8) * static_cast<unsigned>(passes));
+  if (k >= 16 * 128)
+    hipLaunchKernelGGL((mxfp8_gemm_tiled_kernel<Out, WN, WM, DEPTH, 16>), grid, dim3(256), 0, stream, a, as, w, ws, out, m, n, k, stride, row_tiles, passes);
+  else
+    hipLaunchKernelGGL((mxfp8_gemm_tiled_kernel<Out, WN, WM, DEPTH, 4>), grid, dim3(256), 0, stream, a, as, w, ws, out, m, n, k, stride, row_tiles, passes);
+  return hipGetLastError();
+}
+
+// Which form takes an m x n x k product: 0 the 16-row one, 1 - 3 tiles of 32 x 64, 64 x 64 and 64 x 128 (W x A rows).
+// Measured (us, 16-row form -> the form taken): n = 4096, k = 6144: m = 65 26.2 -> 25.1, 128 33.0 -> 26.4, 300 75 -> 41,
+// 1024 244 -> 62; n = 6144, k = 4096: m = 65 28.4 -> 21.9, 300 78 -> 31, 1024 246 -> 74. A tiled step takes about 0.6 us
+// however few blocks there are (LDS round trip, barrier, operand reads, matrix core in turn), so the 16-row form
+// stays where it has no more work than one round of its blocks (of 64 A rows) on every CU: n = 1536, k = 2048, m = 128
+// 6.9 against 10.7; below k = 2048, whose chains are short, up to 1.75 rounds: n = 4096, k = 1024, m = 100 6.1 against
+// 6.8, m = 128 7.4 against 6.9. Up to 64 rows it
+// reads W once and stays until 64 x 64 tiles fill the chip too: n = 6144, m = 48 16.8 against 21.9, n = 17408 52.8
+// against 42.4. Among the tiles: the smallest while they are no more than the CUs (n = 4096, m = 128: 26.4 against
+// 31.7), the largest once there are two for every CU and little of the last one is padding (m = 1024: 62 against 76).
+int tiles_for(int m, int n, int k) {
+  if (k < 128) return 0;   // the tiles read whole words of scales
+  const int knob = tune_get(kTuneTiled);   // bench / test switch: 1 never tiled, 2 - 4 the three tiles
+  if (knob >= 1 && knob <= 4) return knob - 1;
+  constexpr int64_t kCus = 256;
+  auto blocks = [&](int tn, int tm) { return static_cast<int64_t>((n + tn - 1) / tn) * ((m + tm - 1) / tm); };
+  if (m <= 32 || (m <= 64 && blocks(64, 64) <= kCus)) return 0;
+  if (m > 64 && blocks(16, 16) <= (k < 2048 ? 7 * kCus : 4 * kCus)) return 0;
+  if (m > 512 && blocks(64, 128) >= 2 * kCus) return 3;
+  return blocks(32, 64) <= kCus ? 1 : 2;
+}
+
 // src/kernels/mxfp8_gemm.cu:217-243.
 template <typename Out>
 int gemm(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* ws, Out* out, int m, int n, int k,
@@ -283,6 +474,12 @@ int gemm(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* w
   // Waves per block from k alone (an output element's chain must not depend on m or n): sixteen once every
   // wave has a step of its own.
   hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (tiles_for(m, n, k)) {
+    case 1: return report_hip(launch_gemm_tiled<Out, 1, 2, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 2: return report_hip(launch_gemm_tiled<Out, 2, 2, 2>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 3: return report_hip(launch_gemm_tiled<Out, 2, 4, 2>(a, as, w, ws, out, m, n, k, stride, s), who);
+    default: break;
+  }
   const hipError_t err = k >= 16 * 128 ? launch_gemm_waves<Out, 16>(a, as, w, ws, out, m, n, k, stride, s)
                                        : launch_gemm_waves<Out, 4>(a, as, w, ws, out, m, n, k, stride, s);
   return report_hip(err, who);

@@ -1,0 +1,37 @@
+"""The MXFP8 GEMM's form for many activation rows against its 16-row form, bit for bit: both add the same steps of the
+same chains in the same order, and the 16-row form is held to the oracle in test_gpu_mxfp8.py. Sizes at the edges of the
+tiles of 32, 64 and 128 rows, k of a part of a step, of fewer steps than chains and of several steps a chain, scale
+rows that are whole words and not, and a scale pointer that is no word's. Bench switch 15 pins the form."""
+import numpy as np
+import pytest
+
+import mxfp8_data as md
+from dgpp_amd import _lib, launch as L
+from gpu_util import dev, dev_empty, host, sync
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 64), (65, 63, 128), (64, 64, 192), (129, 130, 1088), (200, 128, 2048), (128, 257, 6144),
+                                   (333, 200, 2112)])
+def test_tiled_is_bitwise_the_16_row_form(gpu, m, n, k):
+    a, a_s, w, w_s = md.gemm_case(m, n, k, 3)
+    a_d, as_d, w_d, ws_d = dev(a), dev(a_s), dev(w), dev(w_s)
+    shifted = dev(np.concatenate([np.zeros(1, np.uint8), a_s.reshape(-1)]))
+    out, outh = dev_empty((m, n + 7), np.float32), dev_empty((m, n + 4), np.uint16)
+    want = None
+    for form in (1, 2, 3, 4, 0):
+        for scales in (as_d, shifted[1:]):
+            out.fill_(-1)
+            outh.fill_(0x55)
+            _lib.load().dgpp_tune_set(15, form)
+            try:
+                L.launch_mxfp8_gemm_f32(a_d, scales, w_d, ws_d, out, m, n, k, None, n + 7)
+                L.launch_mxfp8_gemm_bf16(a_d, scales, w_d, ws_d, outh, m, n, k, None, n + 4)
+            finally:
+                _lib.load().dgpp_tune_set(15, 0)
+            sync()
+            got = host(out).view(np.uint32).copy(), host(outh).copy()
+            want = want or got
+            for x, y in zip(want, got):
+                assert np.array_equal(x, y), (form, m, n, k)
