@@ -1114,11 +1114,17 @@ inline bool dense_takes_tiled(const DenseArgs& a) {
   if (knob == 2) return true;
   return a.m > 64;
 }
-inline bool grouped_takes_tiled(const GroupedArgs& a, int max_rows) {
+// The tiled form's pass costs the same for a few rows as for 32, the 16-row form's grows with every 16: the line lies
+// where a segment has 8 to 18 rows on average (16-row form -> tiled, us, one layer: MXFP4, 256 experts, top 8, 9 rows
+// 746 -> 636; NVFP4, 288 experts, 8 rows 491 -> 497; block FP8, 256 experts, top 4, 8 rows 477 -> 519, 12 rows 635 ->
+// 575; 128 experts, top 8, 12 rows 223 -> 263, 19 rows 310 -> 296; W4A4, 9 rows 778 -> 941, 16 rows 1158 -> 1058). The
+// launcher knows max_rows, a prompt's tokens, of which a segment gets top_k / n_segs: 4 to 10 of them.
+template <int FMT>
+inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs, int max_rows) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || a.rows_per_block != INT_MAX || !tiled_rows_aligned(a)) return false;
   if (knob == 2) return true;
-  return max_rows > 128;
+  return max_rows > 128 && 2ll * max_rows >= (FmtTraits<FMT>::kIsFp4 ? 4ll : 5ll) * n_segs;
 }
 
 template <int FMT>
@@ -1126,19 +1132,17 @@ hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
   const MGeom g = mgeom<FMT>(a.k);
   const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows, passes = (a.m + kTiledCols - 1) / kTiledCols;
   const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
-  hipError_t err = hipSuccess;
   auto go = [&](auto kern) {
-    err = ensure_lds(kern, kTiledLds);
-    if (err == hipSuccess) hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), kTiledLds, stream, a, g, row_tiles, passes);
+    hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), 0, stream, a, g, row_tiles, passes);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {
       go(tiled_dense_kernel<FMT, true>);
-      return err != hipSuccess ? err : hipGetLastError();
+      return hipGetLastError();
     }
   }
   go(tiled_dense_kernel<FMT, false>);
-  return err != hipSuccess ? err : hipGetLastError();
+  return hipGetLastError();
 }
 
 template <int FMT>
@@ -1151,20 +1155,18 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
   const unsigned all = static_cast<unsigned>((max_rows + kTiledCols - 1) / kTiledCols);
   const unsigned want = tune_get(kTuneTiledPasses) > 0 ? static_cast<unsigned>(tune_get(kTuneTiledPasses)) : std::max(1u, 8192u / gx);
   const dim3 grid(gx, std::min(all, want));
-  hipError_t err = hipSuccess;
   auto go = [&](auto kern) {
-    err = ensure_lds(kern, kTiledLds);
-    if (err == hipSuccess) hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), kTiledLds, stream, a, g, n_segs, row_tiles);
+    hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), 0, stream, a, g, n_segs, row_tiles);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {
       go(tiled_grouped_kernel<FMT, false, true>);
-      return err != hipSuccess ? err : hipGetLastError();
+      return hipGetLastError();
     }
   }
   if (a.gate_up != 0) go(tiled_grouped_kernel<FMT, true, false>);
   else go(tiled_grouped_kernel<FMT, false, false>);
-  return err != hipSuccess ? err : hipGetLastError();
+  return hipGetLastError();
 }
 
 template <int FMT>
@@ -1251,7 +1253,7 @@ hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, f
 
 template <int FMT>
 hipError_t launch_grouped_mfma(const GroupedArgs& a, int n_segs, int z_ext, hipStream_t stream) {
-  if (grouped_takes_tiled(a, a.max_rows)) return launch_grouped_tiled<FMT>(a, n_segs, a.max_rows, stream);
+  if (grouped_takes_tiled<FMT>(a, n_segs, a.max_rows)) return launch_grouped_tiled<FMT>(a, n_segs, a.max_rows, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const dim3 grid(static_cast<unsigned>((a.n + 63) / 64), static_cast<unsigned>(n_segs), static_cast<unsigned>(z_ext));
   hipError_t err = hipSuccess;

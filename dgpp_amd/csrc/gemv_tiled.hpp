@@ -10,9 +10,10 @@
 // the MFMAs.
 //
 // Tile. k advances by 128 elements: the weights go from memory straight to the operand layout in registers (nothing
-// of them is shared between wavefronts), the block's activation rows through registers into one of two LDS stages of
+// of them is shared between wavefronts), the block's activation rows into one of two LDS stages of
 // [row][16 units of 16 bytes], unit u of row r at u ^ (r % 16) - both the row-major writes and the operand reads are
-// conflict-free. Loads of a tile are issued one tile ahead of its use; one barrier per tile. 64 KB of LDS and up to
+// conflict-free (BF16 rows go from memory to LDS without passing registers, which the sums need). Loads of a tile are
+// issued one tile ahead of its use; one barrier per tile. 64 KB of LDS and up to
 // 256 registers: two blocks per CU, one computing while the other waits.
 //
 // Arithmetic. The sums of a (weight row, activation row) pair are those of the 16-row form: the same elements in the
@@ -27,7 +28,6 @@ constexpr int kTileK = 128;                       // elements of k per tile
 constexpr int kTiledCols = 128;                   // activation rows per pass
 constexpr int kTiledRows = 128;                   // weight rows of a block (gate + up: 64 of each)
 constexpr int kTiledStage = kTiledCols * 16;      // 16-byte units of one stage
-constexpr size_t kTiledLds = 2 * kTiledStage * sizeof(uint4);
 
 // The two row groups of a wavefront: two groups of one matrix, or one of gate and one of up.
 struct TiledRows {
@@ -45,7 +45,7 @@ struct TiledPass {
   static constexpr int kActRegs = A4 ? kCodeLoads : kUnits;
 
   struct Regs {          // one tile on its way
-    uint4 act[kActRegs];
+    uint4 act[A4 ? kCodeLoads : 1];
     uint32_t act_s[A4 ? kCodeLoads : 1];
     uint4 w[2][kSteps];
     uint32_t s[2][kSteps];
@@ -91,13 +91,27 @@ struct TiledPass {
           r.act_s[i] = *reinterpret_cast<const uint16_t*>(act_scales + act_srow[i] + tile * 8 + piece * 2);
         }
       }
+    }
+  }
+
+  // A tile's BF16 rows, from memory straight to their places in a stage: a wavefront's lanes fill 64 units in a row (four
+  // rows' places), so it is the lane that reads the unit which belongs there. Waited for by the next __syncthreads().
+  __device__ __forceinline__ void stage_rows(int tile, uint4* __restrict__ stage) const {
+    const int u = (threadIdx.x & 15) ^ (threadIdx.x >> 4);   // row % 16 is threadIdx.x / 16 for each of the rows
+    const int place = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWave;
+    if ((tile + 1) * kTileK <= k) {
+#pragma unroll
+      for (int i = 0; i < kUnits; ++i)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) uint32_t*)(uintptr_t)(act + (static_cast<size_t>(act_off[i]) + tile * 16 + u) * 16),
+            (__attribute__((address_space(3))) uint32_t*)(stage + place + i * 256), 16, 0, 0);
     } else {
-      const int u = threadIdx.x & 15;
 #pragma unroll
       for (int i = 0; i < kUnits; ++i) {
-        r.act[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (full || tile * kTileK + u * 8 < k)
-          r.act[i] = *reinterpret_cast<const uint4*>(act + (static_cast<size_t>(act_off[i]) + tile * 16 + u) * 16);
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (tile * kTileK + u * 8 < k)
+          v = *reinterpret_cast<const uint4*>(act + (static_cast<size_t>(act_off[i]) + tile * 16 + u) * 16);
+        stage[threadIdx.x + i * 256] = v;
       }
     }
   }
@@ -117,13 +131,6 @@ struct TiledPass {
 #pragma unroll
           for (int j = 0; j < 4; ++j) stage[row * 16 + ((piece * 4 + j) ^ (row & 15))] = __builtin_bit_cast(uint4, f[j].v);
         }
-      }
-    } else {
-      const int u = threadIdx.x & 15;
-#pragma unroll
-      for (int i = 0; i < kUnits; ++i) {
-        const int row = (threadIdx.x >> 4) + i * 16;
-        stage[row * 16 + (u ^ (row & 15))] = r.act[i];
       }
     }
   }
@@ -179,7 +186,7 @@ struct TiledPass {
   // Rows from mt on repeat row mt - 1; their sums are not stored. Every thread of the block must call.
   __device__ __forceinline__ void run(const TiledRows& rows, int n, int k_, const uint8_t* act_, size_t act_stride_bytes,
                                       const int32_t* act_rows, int act_row0, int mt, const A4Src& a4, const MGeom& g,
-                                      uint4* __restrict__ lds, f32x4_t (&sum)[2][CT]) {
+                                      uint4* __restrict__ lds0, uint4* __restrict__ lds1, f32x4_t (&sum)[2][CT]) {
     const int lane = threadIdx.x & (kWave - 1);
     k = k_;
     chunks = k / MTraits<FMT>::kLoadElems;
@@ -207,37 +214,58 @@ struct TiledPass {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int t = 0; t < CT; ++t) sum[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t acc[2][CT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < CT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     Regs pre;
     load(0, pre);
-    int buf = 0;
-    for (int t0 = 0; t0 < tiles; t0 += part_tiles) {
-      const int t1 = min(tiles, t0 + part_tiles);
-      f32x4_t acc[2][CT];
+    if constexpr (!A4) stage_rows(0, lds0);
+    auto step = [&](int t, uint4* __restrict__ cur, uint4* __restrict__ other) {
+      if constexpr (A4) commit(cur, pre);
+      else __syncthreads();   // `cur` is whole, and its wavefronts are done with `other`
+      uint4 w[2][kSteps];
+      uint32_t sc[2][kSteps];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int t = 0; t < CT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      for (int t = t0; t < t1; ++t) {
-        uint4* stage = lds + buf * kTiledStage;
-        buf ^= 1;
-        commit(stage, pre);
-        uint4 w[2][kSteps];
-        uint32_t sc[2][kSteps];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int s = 0; s < kSteps; ++s) {
-            w[i][s] = pre.w[i][s];
-            sc[i][s] = pre.s[i][s];
-          }
-        if (t + 1 < tiles) load(t + 1, pre);
-        __syncthreads();   // the stage is whole; its readers of two tiles before passed the barrier of the tile between
-        multiply(stage, w, sc, acc);
+        for (int s = 0; s < kSteps; ++s) {
+          w[i][s] = pre.w[i][s];
+          sc[i][s] = pre.s[i][s];
+        }
+      if (t + 1 < tiles) {
+        load(t + 1, pre);
+        if constexpr (!A4) stage_rows(t + 1, other);
       }
+      if constexpr (A4) __syncthreads();   // the stage is whole; its readers of two tiles before passed the barrier of the tile between
+      multiply(cur, w, sc, acc);
+    };
+    int part_end = min(tiles, part_tiles);
+    auto ends = [&](int done) {
+      if (done != part_end) return false;
+      const bool first = part_end <= part_tiles;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int t = 0; t < CT; ++t) sum[i][t] = t0 == 0 ? acc[i][t] : sum[i][t] + acc[i][t];
+        for (int t = 0; t < CT; ++t) {
+          sum[i][t] = first ? acc[i][t] : sum[i][t] + acc[i][t];
+          acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      part_end = min(tiles, part_end + part_tiles);
+      return done == tiles;
+    };
+    if constexpr (A4) {
+#pragma unroll 1
+      for (int t = 0;;) {
+        step(t, t & 1 ? lds1 : lds0, nullptr);
+        if (ends(++t)) break;
+      }
+    } else for (int t = 0;;) {   // the stages by name: the compiler then knows that a read of one need not wait for loads to the other
+      step(t, lds0, lds1);
+      if (ends(++t)) break;
+      step(t, lds1, lds0);
+      if (ends(++t)) break;
     }
     __syncthreads();   // the stages are free for the next pass
   }
@@ -284,10 +312,11 @@ struct TiledOut {
 template <int FMT, bool GU, bool A4, int CT>
 __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
-                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds) {
+                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds0,
+                                           uint4* __restrict__ lds1) {
   TiledPass<FMT, A4, CT> pass;
   f32x4_t sum[2][CT];
-  pass.run(rows, n, k, act, act_stride_bytes, act_rows, act_row0, mt, a4, g, lds, sum);
+  pass.run(rows, n, k, act, act_stride_bytes, act_rows, act_row0, mt, a4, g, lds0, lds1, sum);
   const int lane = threadIdx.x & (kWave - 1);
   const bool vec = ((reinterpret_cast<uintptr_t>(o.out) | (GU ? reinterpret_cast<uintptr_t>(o.out_up) : 0)) & 15u) == 0 &&
                    (o.out_stride & 3u) == 0;
@@ -334,13 +363,14 @@ __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&
 template <int FMT, bool GU, bool A4>
 __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
-                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds) {
+                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds0,
+                                           uint4* __restrict__ lds1) {
   if (mt > 64)
-    tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds);
+    tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
   else if (mt > 32)
-    tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds);
+    tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
   else
-    tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds);
+    tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
 }
 
 // Blocks of one segment share its activation rows and blocks of one row tile its weights: consecutive workgroups go to
@@ -352,7 +382,7 @@ constexpr int kXcds = 8;
 // grid.y-th pass of 128 rows).
 template <int FMT, bool GU, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, int n_segs, int row_tiles) {
-  extern __shared__ uint4 lds[];
+  __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
   const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
   const int si = idx / row_tiles * kXcds + lin % kXcds, tile = idx % row_tiles;
   if (si >= n_segs) return;
@@ -377,14 +407,14 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(Grouped
     const int first = seg.row0 + c0;
     tiled_rows<FMT, GU, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
                             a.act_rows ? a.act_rows + first : nullptr, first, static_cast<size_t>(first),
-                            min(kTiledCols, seg.rows - c0), src, g, o, lds);
+                            min(kTiledCols, seg.rows - c0), src, g, o, lds0, lds1);
   }
 }
 
 // grid.x = kXcds * ceil(row tiles / kXcds) * column passes.
 template <int FMT, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs a, MGeom g, int row_tiles, int passes) {
-  extern __shared__ uint4 lds[];
+  __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
   const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
   const int tile = idx / passes * kXcds + lin % kXcds, c0 = idx % passes * kTiledCols;
   if (tile >= row_tiles) return;
@@ -402,7 +432,7 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
   src.scale_stride = a.a4_scale_stride;
   const TiledOut o = {a.out, nullptr, a.out_stride, a.out_f32, 0, 0.f, a.a4_gs};
   tiled_rows<FMT, false, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
-                             nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, lds);
+                             nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, lds0, lds1);
 }
 
 }  // namespace dgpp_amd
