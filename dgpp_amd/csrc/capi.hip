@@ -432,6 +432,7 @@ void dgpp_tune_set(int key, int value) {
 #endif
 }
 int dgpp_tune_get(int key) { return tune_get(key); }
+int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k) { return dense_fills_tiles(fmt, m, n, k) ? 1 : 0; }
 
 int dgpp_moe_config_validate(const DgppMoeConfig* c) {
   // src/models/glm/moe.hpp:119-133

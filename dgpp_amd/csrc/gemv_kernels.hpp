@@ -1064,10 +1064,27 @@ inline int max_stage_rows(int k) {
   return static_cast<int>(fit < 1 ? 1 : (fit > kMaxActRows ? kMaxActRows : fit));
 }
 
+// Blocks of the 16-row dense form: 64 weight rows x 16 activation rows each.
+inline size_t dense_mfma_tiles(int m, int n) {
+  return static_cast<size_t>((n + 63) / 64) * static_cast<size_t>((m + 15) / 16);
+}
 // Whether the dense matrix-core launch runs its K parts in separate blocks through a workspace when it is given one
 // that is large enough (launch_dense_mfma's rule): more than one part, and row tiles that leave the chip under-filled.
-inline bool dense_mfma_would_split(int parts, int m, int n) {
-  return parts > 1 && static_cast<size_t>((n + 63) / 64) * static_cast<size_t>((m + 15) / 16) < 1024;
+inline bool dense_mfma_would_split(int parts, int m, int n) { return parts > 1 && dense_mfma_tiles(m, n) < 1024; }
+
+// Whether a dense product has work enough for the 128 x 128 tiles (gemv_tiled.hpp). Their blocks walk all of k, so a
+// launch takes the same time until they are more than the chip holds (k = 4096: 50 to 66 us), while the 16-row form has
+// eight times the blocks, runs the K parts side by side where even those are few, and holds 1024 blocks (four to a CU)
+// in one round. The line is the end of that round. Measured, 16-row form -> tiles, us, k = 4096: n = 512, m = 100 14 ->
+// 54 (block FP8), 15 -> 50 (NVFP4); n = 4096, m = 100 29 -> 55 and 28 -> 54; at 1024 blocks (n = 4096, m = 256) 42 ->
+// 56, 45 -> 54, MXFP4 41 -> 52, MXFP8 56 -> 66, NVFP4 activations 53 -> 56; at 1080 to 1100 blocks 57 to 67 -> 56
+// (block FP8), 81 to 90 -> 62 to 68 (MXFP8), the others between; n = 12288, m = 1000 412 -> 126 and 415 -> 122. A short
+// walk does not pay for its ramp as soon: below 1024 elements of k, and below 2048 for block FP8, the line lies at a
+// round and a quarter (k = 1024, block FP8: 1080 to 1224 blocks 18 to 22 -> 18 to 21, up to 11 % slower, 1288 to 1296
+// 18 to 23 -> 18 to 20). Above the line no launch is one that splits its K parts over a workspace.
+inline bool dense_fills_tiles(int fmt, int m, int n, int k) {
+  const size_t line = k < (fmt == kFmtFp8F32 ? 2048 : 1024) ? 1280 : 1024;
+  return m > 64 && dense_mfma_tiles(m, n) > line;
 }
 
 // Row groups per block of the dense matrix-core launch that runs the four parts of K side by side inside a block
@@ -1079,7 +1096,7 @@ constexpr size_t kTeamsMaxTilesHalf = 320;
 inline int dense_mfma_team_row_groups(int parts, int m, int n, bool plain) {
   const int knob = tune_get(kTuneTeams);
   if (!plain || parts != 4 || knob == 1) return 0;
-  const size_t tiles = static_cast<size_t>((n + 63) / 64) * static_cast<size_t>((m + 15) / 16);
+  const size_t tiles = dense_mfma_tiles(m, n);
   if (knob == 2 || tiles <= kTeamsMaxTiles) return 4;
   if ((knob == 3 || tiles <= kTeamsMaxTilesHalf) && m <= 8) return 2;
   return 0;
@@ -1108,11 +1125,12 @@ inline bool tiled_rows_aligned(const Args& a) {
   return (a.act_stride & 15u) == 0 && ((reinterpret_cast<uintptr_t>(a.a4_scales) | a.a4_scale_stride) & 1u) == 0;
 }
 // Bench / test switch 15: 1 never, 2 always (where it can); 16: passes of a segment side by side.
+template <int FMT>
 inline bool dense_takes_tiled(const DenseArgs& a) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return false;
   if (knob == 2) return true;
-  return a.m > 64;
+  return dense_fills_tiles(FMT, a.m, a.n, a.k);
 }
 // The tiled form's pass costs the same for a few rows as for 32, the 16-row form's grows with every 16: the line lies
 // where a segment has 8 to 18 rows on average (16-row form -> tiled, us, one layer: MXFP4, 256 experts, top 8, 9 rows
@@ -1171,7 +1189,7 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
 
 template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
-  if (dense_takes_tiled(a)) return launch_dense_tiled<FMT>(a, stream);
+  if (dense_takes_tiled<FMT>(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const unsigned gx = static_cast<unsigned>((a.n + 63) / 64), gy = static_cast<unsigned>((a.m + kTileCols - 1) / kTileCols);
   const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);

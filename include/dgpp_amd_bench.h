@@ -49,6 +49,11 @@ int dgpp_tune_get(int key);
  * runs its measured default, whatever any component of the process calls. */
 int dgpp_tune_enabled(void);
 
+/* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):
+ * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a
+ * workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
+int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k);
+
 /* Measurement aid with no counterpart in the reference: a plain streaming copy of `bytes`
  * (a multiple of 16; both pointers 16-byte aligned) on `stream`. A profiler's HBM byte counters
  * are calibrated against it: it reads `bytes` and writes `bytes`, nothing else. */
