@@ -13,6 +13,7 @@
 #include "../../include/dgpp_amd_bench.h"
 #include "capi_errors.hpp"
 #include "gemv_kernels.hpp"
+#include "moe_grouped.hpp"
 #include "moe_misc.hpp"
 
 using namespace dgpp_amd;
@@ -350,10 +351,11 @@ SlotArgs slot_args(const uint16_t* x, size_t x_stride, const int32_t* ids, const
   return a;
 }
 
-int grouped(int fmt, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, int max_rows,
+int grouped(int fmt, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, const SegmentRows& rows,
             int rows_per_block, const DgppMoeExpertView* views, int which, void* out, int out_f32, size_t out_stride,
             int n, int k, void* stream, const char* who, bool mma = false, const int32_t* act_rows = nullptr,
             const float* gate_up_limit = nullptr, void* out_up = nullptr) {
+  const int max_rows = rows.max_rows;
   if (max_rows <= 0) return fail_arg(std::string(who) + ": max_rows must be positive");
   if (which < 0 || which > 2) return fail_arg(std::string(who) + ": which must be 0, 1 or 2");
   const unsigned z_ext = rows_per_block > 0 ? static_cast<unsigned>((max_rows + rows_per_block - 1) / rows_per_block) : 1u;
@@ -372,6 +374,7 @@ int grouped(int fmt, const uint16_t* act, size_t act_stride, const DgppMoeSegmen
   a.rows_per_block = rows_per_block > 0 ? rows_per_block : INT_MAX;
   a.group_rows = max_stage_rows(k);
   a.max_rows = max_rows;
+  a.long_segs = rows.long_segs;
   a.act_rows = act_rows;
   a.gate_up = out_up ? 2 : (gate_up_limit != nullptr ? 1 : 0);
   a.limit = gate_up_limit ? *gate_up_limit : 0.f;
@@ -432,6 +435,19 @@ void dgpp_tune_set(int key, int value) {
 #endif
 }
 int dgpp_tune_get(int key) { return tune_get(key); }
+int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place) {
+  if (n_segs <= 0 || long_segs < 0 || long_segs > n_segs || row_tiles <= 0 || max_rows <= 0) return 0;
+  const TiledDeal d = tiled_deal(n_segs, long_segs, row_tiles, max_rows, 0);
+  const int blocks = static_cast<int>(d.blocks());
+  if (block >= 0 && block < blocks && place) {
+    const TiledPlace at = tiled_place(d, block);
+    place[0] = at.seg;
+    place[1] = at.tile;
+    place[2] = at.slot;
+    place[3] = at.slots;
+  }
+  return blocks;
+}
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k) { return dense_fills_tiles(fmt, m, n, k) ? 1 : 0; }
 
 int dgpp_moe_config_validate(const DgppMoeConfig* c) {
@@ -1430,7 +1446,7 @@ int dgpp_launch_dense_mma_fp4_f32(const uint16_t* act, size_t act_stride, const 
   return dense_mma_fp4(act, act_stride, w, out, 1, m, n, k, stream);
 }
 
-static int grouped_mma_fp8(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, int max_rows,
+static int grouped_mma_fp8(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, const SegmentRows& rows,
                            int rows_per_block, const DgppMoeExpertView* views, int which, void* out, int out_f32,
                            size_t out_stride, int n, int k, void* stream, const int32_t* act_rows,
                            const float* gate_up_limit = nullptr) {
@@ -1438,23 +1454,23 @@ static int grouped_mma_fp8(const uint16_t* act, size_t act_stride, const DgppMoe
   if (n_segs <= 0 || n <= 0) return DGPP_OK;
   if (!act || !segs || !views || !out) return fail_arg(std::string(who) + ": null pointer");
   if (k <= 0 || k % 16 != 0) return fail_arg(std::string(who) + ": k must be a positive multiple of 16");
-  return grouped(kFmtFp8F32, act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, out_f32,
+  return grouped(kFmtFp8F32, act, act_stride, segs, n_segs, rows, rows_per_block, views, which, out, out_f32,
                  out_stride, n, k, stream, who, true, act_rows, gate_up_limit);
 }
 int dgpp_launch_moe_grouped_mma_bf16(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
                                      int max_rows, int rows_per_block, const DgppMoeExpertView* views, int which,
                                      uint16_t* out, size_t out_stride, int n, int k, void* stream,
                                      const int32_t* act_rows) {
-  return grouped_mma_fp8(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, 0, out_stride, n, k,
+  return grouped_mma_fp8(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, which, out, 0, out_stride, n, k,
                          stream, act_rows);
 }
 int dgpp_launch_moe_grouped_mma_f32(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
                                     int max_rows, int rows_per_block, const DgppMoeExpertView* views, int which, float* out,
                                     size_t out_stride, int n, int k, void* stream, const int32_t* act_rows) {
-  return grouped_mma_fp8(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, 1, out_stride, n, k,
+  return grouped_mma_fp8(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, which, out, 1, out_stride, n, k,
                          stream, act_rows);
 }
-static int grouped_mma_fp4(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, int max_rows,
+static int grouped_mma_fp4(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs, const SegmentRows& rows,
                            int rows_per_block, const DgppMoeExpertView* views, int which, void* out, int out_f32,
                            size_t out_stride, int n, int k, void* stream, const int32_t* act_rows, int fp4_group,
                            const float* gate_up_limit = nullptr, void* out_up = nullptr) {
@@ -1463,15 +1479,26 @@ static int grouped_mma_fp4(const uint16_t* act, size_t act_stride, const DgppMoe
   if (!act || !segs || !views || !out) return fail_arg(std::string(who) + ": null pointer");
   if (fp4_group != 16 && fp4_group != 32) return fail_arg(std::string(who) + ": the fp4 scale group must be 16 or 32");
   if (k <= 0 || k % 32 != 0) return fail_arg(std::string(who) + ": k must be a positive multiple of 32");
-  return grouped(fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4, act, act_stride, segs, n_segs, max_rows, rows_per_block, views,
+  return grouped(fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4, act, act_stride, segs, n_segs, rows, rows_per_block, views,
                  which, out, out_f32, out_stride, n, k, stream, who, true, act_rows, gate_up_limit, out_up);
 }
+}  // extern "C"
+int dgpp_amd::grouped_mma(int fp4_group, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
+                          const SegmentRows& rows, const DgppMoeExpertView* views, int which, void* out, int out_f32,
+                          size_t out_stride, int n, int k, void* stream, const int32_t* act_rows, const float* gate_up_limit) {
+  if (fp4_group == 0)
+    return grouped_mma_fp8(act, act_stride, segs, n_segs, rows, 0, views, which, out, out_f32, out_stride, n, k, stream,
+                           act_rows, gate_up_limit);
+  return grouped_mma_fp4(act, act_stride, segs, n_segs, rows, 0, views, which, out, out_f32, out_stride, n, k, stream, act_rows,
+                         fp4_group, gate_up_limit);
+}
+extern "C" {
 /* src/kernels/glm_moe.cu:4809-4823: one segment read from the device, the grouped kernel's chain. */
 int dgpp_launch_dense_mma_fp4_prod_bf16(const uint16_t* act, size_t act_stride, const DgppMoeSegment* seg,
                                         const DgppMoeExpertView* views, int which, uint16_t* out, int m, int n, int k,
                                         void* stream, int fp4_group) {
   if (m <= 0 || n <= 0) return DGPP_OK;
-  return grouped_mma_fp4(act, act_stride, seg, 1, m, 0, views, which, out, 0, static_cast<size_t>(n), n, k, stream, nullptr,
+  return grouped_mma_fp4(act, act_stride, seg, 1, {m}, 0, views, which, out, 0, static_cast<size_t>(n), n, k, stream, nullptr,
                          fp4_group);
 }
 /* src/kernels/dense_fp4_decode.cu:297-308: the small dense NVFP4 shard form. The shape rule is the reference's (one
@@ -1495,14 +1522,14 @@ int dgpp_launch_dense_mma_fp4_gate_up_bf16(const uint16_t* act, size_t act_strid
                                            int k, void* stream, int fp4_group) {
   if (m <= 0 || n <= 0) return DGPP_OK;
   if (!up) return fail_arg("dense mma fp4 gate_up: null pointer");
-  return grouped_mma_fp4(act, act_stride, seg, 1, m, 0, views, 0, gate, 0, static_cast<size_t>(n), n, k, stream, nullptr,
+  return grouped_mma_fp4(act, act_stride, seg, 1, {m}, 0, views, 0, gate, 0, static_cast<size_t>(n), n, k, stream, nullptr,
                          fp4_group, nullptr, up);
 }
 int dgpp_launch_moe_grouped_mma_gate_up_swiglu(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs,
                                                int n_segs, int max_rows, int rows_per_block, const DgppMoeExpertView* views,
                                                uint16_t* out, size_t out_stride, int n, int k, float limit, void* stream,
                                                const int32_t* act_rows) {
-  return grouped_mma_fp8(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, 0, out, 0, out_stride, n, k, stream,
+  return grouped_mma_fp8(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, 0, out, 0, out_stride, n, k, stream,
                          act_rows, &limit);
 }
 int dgpp_launch_moe_grouped_mma_gate_up_swiglu_fp4(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs,
@@ -1510,7 +1537,7 @@ int dgpp_launch_moe_grouped_mma_gate_up_swiglu_fp4(const uint16_t* act, size_t a
                                                    const DgppMoeExpertView* views, uint16_t* out, size_t out_stride, int n,
                                                    int k, float limit, void* stream, const int32_t* act_rows,
                                                    int fp4_group) {
-  return grouped_mma_fp4(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, 0, out, 0, out_stride, n, k, stream,
+  return grouped_mma_fp4(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, 0, out, 0, out_stride, n, k, stream,
                          act_rows, fp4_group, &limit);
 }
 int dgpp_launch_moe_grouped_mma_fp4_bf16(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
@@ -1518,7 +1545,7 @@ int dgpp_launch_moe_grouped_mma_fp4_bf16(const uint16_t* act, size_t act_stride,
                                          uint16_t* out, size_t out_stride, int n, int k, void* stream,
                                          const int32_t* act_rows, int fp4_group, int tile_rows) {
   (void)tile_rows;   // the reference's activation ring depth; one 16-row tile per weight pass here
-  return grouped_mma_fp4(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, 0, out_stride, n, k,
+  return grouped_mma_fp4(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, which, out, 0, out_stride, n, k,
                          stream, act_rows, fp4_group);
 }
 int dgpp_launch_moe_grouped_mma_fp4_f32(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
@@ -1526,7 +1553,7 @@ int dgpp_launch_moe_grouped_mma_fp4_f32(const uint16_t* act, size_t act_stride, 
                                         float* out, size_t out_stride, int n, int k, void* stream, const int32_t* act_rows,
                                         int fp4_group, int tile_rows) {
   (void)tile_rows;
-  return grouped_mma_fp4(act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, 1, out_stride, n, k,
+  return grouped_mma_fp4(act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, which, out, 1, out_stride, n, k,
                          stream, act_rows, fp4_group);
 }
 
@@ -1539,7 +1566,7 @@ static int grouped_fp8(const uint16_t* act, size_t act_stride, const DgppMoeSegm
   if (!act || !segs || !views || !out) return fail_arg(std::string(who) + ": null pointer");
   if (k <= 0 || k % 16 != 0) return fail_arg(std::string(who) + ": k must be a positive multiple of 16");
   if (stage_bytes(1, k) > kMaxLdsBytes) return fail_arg(std::string(who) + ": k exceeds the smem budget");
-  return grouped(kFmtFp8F32, act, act_stride, segs, n_segs, max_rows, rows_per_block, views, which, out, out_f32,
+  return grouped(kFmtFp8F32, act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views, which, out, out_f32,
                  out_stride, n, k, stream, who);
 }
 int dgpp_launch_moe_grouped_gemv_bf16(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
@@ -1563,7 +1590,7 @@ static int grouped_fp4(const uint16_t* act, size_t act_stride, const DgppMoeSegm
   if (fp4_group != 16 && fp4_group != 32) return fail_arg(std::string(who) + ": the fp4 scale group must be 16 or 32");
   if (!fp4_k_supported(k) || !fp4_k_compiled(k, fp4_group))
     return fail_arg(std::string(who) + ": k must be a multiple of 32 in the fp4 core's compiled set");
-  return grouped(fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4, act, act_stride, segs, n_segs, max_rows, rows_per_block, views,
+  return grouped(fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4, act, act_stride, segs, n_segs, {max_rows}, rows_per_block, views,
                  which, out, out_f32, out_stride, n, k, stream, who);
 }
 int dgpp_launch_moe_grouped_gemv_fp4_bf16(const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs,

@@ -905,6 +905,7 @@ struct GroupedArgs {
   int rows_per_block;  // segment rows per z block
   int group_rows;      // activation rows staged per pass (<= kMaxActRows)
   int max_rows;        // no segment has more
+  int long_segs = 0;   // so many segments at the table's end are known to have that many
   const int32_t* act_rows;  // matrix-core form only, nullable: activation row of each segment row
   int once;                 // every segment fits one pass over its expert (nontemporal loads)
   int gate_up;              // matrix-core form only, `which` unused, bf16 out: 1 = gate and up rows + SwiGLU in one
@@ -1168,13 +1169,9 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
   const MGeom g = mgeom<FMT>(a.k);
   const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
   const int row_tiles = (a.n + block_rows - 1) / block_rows;
-  const unsigned gx = static_cast<unsigned>((n_segs + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(row_tiles);
-  // passes of a segment that run side by side: all of them where the segments are few, else some
-  const unsigned all = static_cast<unsigned>((max_rows + kTiledCols - 1) / kTiledCols);
-  const unsigned want = tune_get(kTuneTiledPasses) > 0 ? static_cast<unsigned>(tune_get(kTuneTiledPasses)) : std::max(1u, 8192u / gx);
-  const dim3 grid(gx, std::min(all, want));
+  const TiledDeal deal = tiled_deal(n_segs, a.long_segs, row_tiles, max_rows, tune_get(kTuneTiledPasses));
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), 0, stream, a, g, n_segs, row_tiles);
+    hipLaunchKernelGGL(kern, dim3(deal.blocks()), dim3(kBlockThreads), 0, stream, a, g, deal);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {

@@ -373,21 +373,73 @@ __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&
     tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
 }
 
-// Blocks of one segment share its activation rows and blocks of one row tile its weights: consecutive workgroups go to
-// the eight XCDs in turn, so the linear index is dealt such that an XCD (its own L2) keeps a segment's row tiles, or a
-// row tile's column passes, to itself.
+// Consecutive workgroups go to the eight XCDs in turn. Blocks of one segment share its activation rows and blocks of one
+// row tile its weights, so the linear index is dealt such that an XCD (its own L2) keeps a segment's row tiles, or a row
+// tile's column passes, to itself.
 constexpr int kXcds = 8;
 
-// grid.x = kXcds * ceil(n_segs / kXcds) * row tiles, grid.y = passes in flight per segment (a block takes every
-// grid.y-th pass of 128 rows).
+// The grouped launch's blocks. A table's segments go to the XCDs whole, one each in turn. Fewer segments than XCDs - a
+// shared expert's, a dense product's by views - and those which the caller knows to be as long as the prompt (a shared
+// expert behind the table's) go over all XCDs instead, an eighth of their (row tile, pass) pairs to each, and first, so
+// that a long one is no tail: dealt whole, one segment had 32 of the 256 CUs. Measured, us, whole -> spread: one segment,
+// block FP8 gate + up, 129 x 17408 x 5120 721 -> 205 (the 16-row form 378), 4096 x 512 x 4096 393 -> 89; NVFP4 product
+// 1024 x 2048 x 6144 238 -> 95; whole layers with a shared expert: MXFP4, 256 experts and one in
+// the table, 2048 tokens 2167 -> 1312; block FP8, 36 experts, 2048 tokens 739 -> 477. Spreading the up to
+// seven segments by which a table misses a multiple of eight as well was slower: their blocks stand for the longest
+// possible segment, and most have no pass (36 segments, 2048 tokens 176 -> 213).
+struct TiledDeal {
+  int whole;          // segments that go to an XCD whole
+  int slots;          // blocks that share the passes of one of them and a row tile
+  int spread;         // the others, behind them in the table
+  int spread_slots;
+  int spread_per_xcd; // blocks
+  int row_tiles;
+  __host__ __device__ unsigned whole_blocks() const {   // of one slot
+    return static_cast<unsigned>((whole + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(row_tiles);
+  }
+  __host__ __device__ unsigned blocks() const {
+    return static_cast<unsigned>(spread_per_xcd) * kXcds + whole_blocks() * static_cast<unsigned>(slots);
+  }
+};
+// max_rows: no segment has more; long_segs: so many at the table's end have that many. tuned > 0: slots (bench switch 16).
+inline TiledDeal tiled_deal(int n_segs, int long_segs, int row_tiles, int max_rows, int tuned) {
+  const int passes = (max_rows + kTiledCols - 1) / kTiledCols;
+  auto side_by_side = [&](int64_t blocks) {   // all passes where the blocks of one slot are few, else some
+    const int64_t want = tuned > 0 ? tuned : 8192 / blocks;
+    return static_cast<int>(want < 1 ? 1 : (want < passes ? want : passes));
+  };
+  TiledDeal d;
+  d.row_tiles = row_tiles;
+  d.spread = n_segs < kXcds ? n_segs : long_segs;
+  d.whole = n_segs - d.spread;
+  d.slots = d.whole ? side_by_side(d.whole_blocks()) : 0;
+  d.spread_slots = d.spread ? side_by_side(static_cast<int64_t>(d.spread) * row_tiles) : 0;
+  d.spread_per_xcd = (d.spread * row_tiles * d.spread_slots + kXcds - 1) / kXcds;
+  return d;
+}
+struct TiledPlace {
+  int seg, tile, slot, slots;   // the block takes passes slot, slot + slots, ... of the segment; seg -1: none
+};
+__host__ __device__ __forceinline__ TiledPlace tiled_place(const TiledDeal& d, int block) {
+  const int xcd = block % kXcds, first_whole = d.spread_per_xcd * kXcds;
+  if (block < first_whole) {
+    const int of_seg = d.row_tiles * d.spread_slots, item = xcd * d.spread_per_xcd + block / kXcds;
+    if (item >= d.spread * of_seg) return {-1, 0, 0, 1};
+    return {d.whole + item / of_seg, item % of_seg / d.spread_slots, item % d.spread_slots, d.spread_slots};
+  }
+  const int of_slot = static_cast<int>(d.whole_blocks()), at = block - first_whole;
+  const int idx = at % of_slot / kXcds, seg = idx / d.row_tiles * kXcds + xcd;
+  if (seg >= d.whole) return {-1, 0, 0, 1};
+  return {seg, idx % d.row_tiles, at / of_slot, d.slots};
+}
+
 template <int FMT, bool GU, bool A4>
-__global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, int n_segs, int row_tiles) {
+__global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, TiledDeal deal) {
   __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
-  const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
-  const int si = idx / row_tiles * kXcds + lin % kXcds, tile = idx % row_tiles;
-  if (si >= n_segs) return;
-  const DgppMoeSegment seg = a.segs[si];
-  const int first_pass = static_cast<int>(blockIdx.y) * kTiledCols;
+  const TiledPlace at = tiled_place(deal, static_cast<int>(blockIdx.x));
+  if (at.seg < 0) return;
+  const DgppMoeSegment seg = a.segs[at.seg];
+  const int first_pass = at.slot * kTiledCols, tile = at.tile;
   if (first_pass >= seg.rows) return;
   const int wave = threadIdx.x >> 6;
   TiledRows rows;
@@ -403,7 +455,7 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(Grouped
   src.scales = a.a4_scales;
   src.scale_stride = a.a4_scale_stride;
   const TiledOut o = {a.out, a.out_up, a.out_stride, a.out_f32, a.gate_up, a.limit, a.a4_gs};
-  for (int c0 = first_pass; c0 < seg.rows; c0 += static_cast<int>(gridDim.y) * kTiledCols) {
+  for (int c0 = first_pass; c0 < seg.rows; c0 += at.slots * kTiledCols) {
     const int first = seg.row0 + c0;
     tiled_rows<FMT, GU, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
                             a.act_rows ? a.act_rows + first : nullptr, first, static_cast<size_t>(first),

@@ -1,0 +1,22 @@
+// The grouped matrix-core launches for callers that know more of the segments than their largest size: the layer driver,
+// which made the table. Arguments and results as the dgpp_launch_moe_grouped_mma_* and _w4a4_* entry points.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include "../../include/dgpp_amd.h"
+
+namespace dgpp_amd {
+
+struct SegmentRows {
+  int max_rows;       // no segment has more
+  int long_segs = 0;  // so many segments at the table's end have exactly that many (a shared expert's)
+};
+
+// fp4_group: 0 block FP8, 16 NVFP4, 32 MXFP4. gate_up_limit: null, or gate + up + SwiGLU (`which` 0).
+int grouped_mma(int fp4_group, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
+                const SegmentRows& rows, const DgppMoeExpertView* views, int which, void* out, int out_f32, size_t out_stride,
+                int n, int k, void* stream, const int32_t* act_rows, const float* gate_up_limit);
+
+}  // namespace dgpp_amd

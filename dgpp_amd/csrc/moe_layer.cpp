@@ -8,6 +8,7 @@
 
 #include "../../include/dgpp_amd_bench.h"
 #include "../../include/dgpp_amd_layer.h"
+#include "moe_grouped.hpp"
 
 namespace dgpp {
 namespace {
@@ -548,25 +549,20 @@ void GlmMoeLayer::prefill_chain(const uint16_t* x, size_t x_stride, const int32_
   const size_t stride = with_shared ? static_cast<size_t>(max_inter_) : static_cast<size_t>(I);
   const int n_segs = in_table ? E + 1 : E;
   launch_moe_segment(ids, tokens, K, E, d_rows_, d_slot_row_, d_segs_, stream);
-  const int max_rows = tokens;
+  const dgpp_amd::SegmentRows table{tokens, in_table ? 1 : 0}, shared{tokens, 1};
+  const int group = fp8 ? 0 : fp4_group_;
+  const float limit = cfg_.swiglu_limit;
   // gate + up + SwiGLU in one launch (the bits of the two grouped launches and the elementwise kernel)
-  if (fp8)
-    launch_moe_grouped_mma_gate_up_swiglu(x, x_stride, d_segs_, n_segs, max_rows, 0, d_views_, d_slot_act_, stride, I, H,
-                                          cfg_.swiglu_limit, stream, d_rows_);
-  else
-    launch_moe_grouped_mma_gate_up_swiglu_fp4(x, x_stride, d_segs_, n_segs, max_rows, 0, d_views_, d_slot_act_, stride, I, H,
-                                              cfg_.swiglu_limit, stream, d_rows_, fp4_group_);
+  detail::check(dgpp_amd::grouped_mma(group, x, x_stride, d_segs_, n_segs, table, d_views_, 0, d_slot_act_, 0, stride, I, H, stream,
+                                      d_rows_, &limit));
   if (with_shared && !in_table)   // a block-FP8 shared expert of its own width
-    launch_moe_grouped_mma_gate_up_swiglu(x, x_stride, d_segs_ + E, 1, max_rows, 0, d_sh_views_, d_slot_act_, stride,
-                                          w_.shared_inter, H, cfg_.swiglu_limit, stream, d_rows_);
-  if (fp8)
-    launch_moe_grouped_mma_f32(d_slot_act_, stride, d_segs_, n_segs, max_rows, 0, d_views_, 2, d_slot_down_, H, H, I, stream);
-  else
-    launch_moe_grouped_mma_fp4_f32(d_slot_act_, stride, d_segs_, n_segs, max_rows, 0, d_views_, 2, d_slot_down_, H, H, I, stream,
-                                   nullptr, fp4_group_);
+    detail::check(dgpp_amd::grouped_mma(0, x, x_stride, d_segs_ + E, 1, shared, d_sh_views_, 0, d_slot_act_, 0, stride,
+                                        w_.shared_inter, H, stream, d_rows_, &limit));
+  detail::check(dgpp_amd::grouped_mma(group, d_slot_act_, stride, d_segs_, n_segs, table, d_views_, 2, d_slot_down_, 1, H, H, I,
+                                      stream, nullptr, nullptr));
   if (with_shared && !in_table)
-    launch_moe_grouped_mma_f32(d_slot_act_, stride, d_segs_ + E, 1, max_rows, 0, d_sh_views_, 2, d_slot_down_, H, H,
-                               w_.shared_inter, stream);
+    detail::check(dgpp_amd::grouped_mma(0, d_slot_act_, stride, d_segs_ + E, 1, shared, d_sh_views_, 2, d_slot_down_, 1, H, H,
+                                        w_.shared_inter, stream, nullptr, nullptr));
   if (!accumulate) return;
   const int shared_row0 = with_shared ? tk : -1;
   if (out_f32)

@@ -53,6 +53,10 @@ int dgpp_tune_enabled(void);
  * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a
  * workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k);
+/* What a block of the grouped launch's 128-row form works on (the last long_segs of the table's segments are known to
+ * have max_rows rows): place[0 .. 3] = segment
+ * (-1: nothing), row tile, first pass and step of its passes of 128 rows. Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */
+int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place);
 
 /* Measurement aid with no counterpart in the reference: a plain streaming copy of `bytes`
  * (a multiple of 16; both pointers 16-byte aligned) on `stream`. A profiler's HBM byte counters

@@ -1,4 +1,5 @@
 """Which form the matrix-core launchers take, checked on the host: the rules are arithmetic on sizes."""
+import numpy as np
 import pytest
 
 from dgpp_amd import _lib
@@ -30,3 +31,38 @@ def test_dense_tiles_never_take_a_launch_that_splits_over_a_workspace(fmt):
         for m in (17, 64, 65, 80, 129, 256, 257, 1024, 2000):
             if -(-n // 64) * -(-m // 16) < 1024:
                 assert not any(takes_tiles(fmt, m, n, k) for k in (512, 2048, 4096, 17408)), (m, n)
+
+
+def tiled_blocks(n_segs, long_segs, row_tiles, max_rows):
+    """(segment, row tile, first pass, step) of each block of a grouped launch; block b runs on XCD b % 8."""
+    place = np.zeros(4, np.int32)
+    count = _lib.load().dgpp_bench_tiled_place(n_segs, long_segs, row_tiles, max_rows, -1, place.ctypes.data)
+    out = []
+    for b in range(count):
+        _lib.load().dgpp_bench_tiled_place(n_segs, long_segs, row_tiles, max_rows, b, place.ctypes.data)
+        out.append(tuple(int(v) for v in place))
+    return out
+
+
+@pytest.mark.parametrize("n_segs,long_segs,row_tiles,max_rows",
+                         [(1, 0, 1, 129), (1, 1, 8, 4096), (1, 1, 12, 777), (1, 0, 136, 256), (3, 0, 5, 300), (8, 0, 4, 1000),
+                          (9, 1, 16, 2048), (8, 1, 16, 640), (100, 0, 7, 129), (257, 1, 16, 4096), (31, 0, 33, 640)])
+def test_tiled_grouped_blocks_cover_every_pass_once_and_spread_long_segments(n_segs, long_segs, row_tiles, max_rows):
+    passes = -(-max_rows // 128)
+    spread_from = 0 if n_segs < 8 else n_segs - long_segs
+    seen, work = {}, [0] * 8
+    for b, (seg, tile, slot, step) in enumerate(tiled_blocks(n_segs, long_segs, row_tiles, max_rows)):
+        if seg < 0:
+            continue
+        assert 0 <= seg < n_segs and 0 <= tile < row_tiles and 0 <= slot < step
+        for p in range(slot, passes, step):
+            assert (seg, tile, p) not in seen
+            seen[seg, tile, p] = b % 8
+        if seg >= spread_from:
+            work[b % 8] += 1
+    assert len(seen) == n_segs * row_tiles * passes
+    # a shared expert's segment, above all one that is alone in its launch, occupies all XCDs alike
+    assert max(work) <= -(-sum(work) // 8)
+    # the others stay on one XCD each, with their activation rows
+    for seg in range(spread_from):
+        assert {x for (s, _, _), x in seen.items() if s == seg} == {seg % 8}
