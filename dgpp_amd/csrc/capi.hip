@@ -374,6 +374,7 @@ int grouped(int fmt, const uint16_t* act, size_t act_stride, const DgppMoeSegmen
   a.rows_per_block = rows_per_block > 0 ? rows_per_block : INT_MAX;
   a.group_rows = max_stage_rows(k);
   a.max_rows = max_rows;
+  a.total_rows = rows.total_rows;
   a.long_segs = rows.long_segs;
   a.act_rows = act_rows;
   a.gate_up = out_up ? 2 : (gate_up_limit != nullptr ? 1 : 0);
@@ -435,6 +436,10 @@ void dgpp_tune_set(int key, int value) {
 #endif
 }
 int dgpp_tune_get(int key) { return tune_get(key); }
+int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_segs, int k, int max_rows, int total_rows,
+                                   int long_segs) {
+  return grouped_fills_tiles(fmt, act_nvfp4 != 0, gate_up != 0, n_segs, k, max_rows, total_rows, long_segs) ? 1 : 0;
+}
 int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place) {
   if (n_segs <= 0 || long_segs < 0 || long_segs > n_segs || row_tiles <= 0 || max_rows <= 0) return 0;
   const TiledDeal d = tiled_deal(n_segs, long_segs, row_tiles, max_rows, 0);

@@ -905,6 +905,7 @@ struct GroupedArgs {
   int rows_per_block;  // segment rows per z block
   int group_rows;      // activation rows staged per pass (<= kMaxActRows)
   int max_rows;        // no segment has more
+  int64_t total_rows = 0;   // of all segments, 0: not known
   int long_segs = 0;   // so many segments at the table's end are known to have that many
   const int32_t* act_rows;  // matrix-core form only, nullable: activation row of each segment row
   int once;                 // every segment fits one pass over its expert (nontemporal loads)
@@ -1088,6 +1089,37 @@ inline bool dense_fills_tiles(int fmt, int m, int n, int k) {
   return m > 64 && dense_mfma_tiles(m, n) > line;
 }
 
+// Whether a grouped launch takes the tiles of up to 128 activation rows (gemv_tiled.hpp): by the rows of a segment on
+// average. A pass of the tiles costs the same for a few rows as for 32, the 16-row form grows with every 16. A block of
+// the tiles spends its start on a pass that a short k does not repay, so the line rises as k falls; gate + up in one launch
+// walks twice the weights per start, and the 16-row form holds half as many of them: its line is lower. Measured, time of the
+// tiles over the 16-row form's, 128 and 288 segments, n = 384 to 7168, at rows per segment:
+//   block FP8   plain  k = 384 48: 0.98 to 1.25, 96: 0.83 to 0.96; 768 32: 0.98 to 1.11, 40: 0.92 to 1.01; 2048 16: 1.07 to
+//               1.18, 24: 0.93 to 0.96; 4096 12: 1.04 to 1.15, 16: 0.94 to 0.99
+//               gate + up  k = 768 16: 0.83 to 1.09, 20: 0.75 to 0.97; 4096 10: 0.92 to 1.11, 14: 0.82 to 0.94
+//   NVFP4       plain  k = 512 20: 1.04 to 1.29, 28: 0.87 to 1.08; 1024 16: 0.94 to 1.15, 20: 0.84 to 1.03; 4096 12: 0.98 to 1.09
+//               gate + up  k = 512 to 6144 7: 0.83 to 1.12, 10: 0.74 to 0.99
+//   MXFP4       plain  k = 512 20: 0.93 to 1.13, 28: 0.81 to 0.97; 1024 12: 1.00 to 1.17, 16: 0.84 to 0.99; gate + up 6: 0.76 to
+//               1.05, 8: 0.62 to 0.96
+//   NVFP4 activations  plain  k = 512 16: 1.04 to 1.11; 2048 12: 1.12 to 1.15, 15: 0.97 to 1.00; 6144 12: 0.98 to 1.02
+// A line by max_rows alone (2 tokens a segment, 2.5 for block FP8) had sent down projections there that took 1.1 to 1.8
+// times as long as before. Fewer segments than XCDs, and a table with a segment as long as the prompt (long_segs, a shared
+// expert's), always take the tiles: the 16-row form walks the long one as a tail (256 experts and one, 130 tokens 831 us
+// against 582, 777 tokens 3271 against 783; 103 and one, 130 tokens 1256 against 775; one alone, 129 rows, 0.34 to 0.61 of
+// it). total_rows 0: the caller did not say; a table's segments are then taken to have six of max_rows between them
+// (of the four to ten experts that a token goes to).
+inline bool grouped_fills_tiles(int fmt, bool a4, bool gate_up, int n_segs, int k, int max_rows, int64_t total_rows, int long_segs) {
+  if (max_rows <= kTiledCols) return false;
+  if (n_segs < kXcds || long_segs > 0) return true;
+  const int64_t rows = total_rows > 0 ? total_rows : int64_t{6} * max_rows;
+  int64_t least, start;   // the line: least + start / k rows per segment
+  if (a4) least = 12, start = 4096;
+  else if (fmt == kFmtNvfp4) least = gate_up ? 9 : 11, start = gate_up ? 0 : 8192;
+  else if (fmt == kFmtMxfp4) least = gate_up ? 7 : 9, start = gate_up ? 0 : 8192;
+  else least = gate_up ? 11 : 12, start = gate_up ? 6144 : 20480;
+  return rows * k >= n_segs * (least * k + start);
+}
+
 // Row groups per block of the dense matrix-core launch that runs the four parts of K side by side inside a block
 // (0: the row-tile form). Four up to one round of the chip's 256 CUs - one such block fills a CU, and 272 tiles, two
 // rounds with the second nearly empty, measured slower than the row-tile form; two (blocks half the size, two to a CU)
@@ -1133,17 +1165,12 @@ inline bool dense_takes_tiled(const DenseArgs& a) {
   if (knob == 2) return true;
   return dense_fills_tiles(FMT, a.m, a.n, a.k);
 }
-// The tiled form's pass costs the same for a few rows as for 32, the 16-row form's grows with every 16: the line lies
-// where a segment has 8 to 18 rows on average (16-row form -> tiled, us, one layer: MXFP4, 256 experts, top 8, 9 rows
-// 746 -> 636; NVFP4, 288 experts, 8 rows 491 -> 497; block FP8, 256 experts, top 4, 8 rows 477 -> 519, 12 rows 635 ->
-// 575; 128 experts, top 8, 12 rows 223 -> 263, 19 rows 310 -> 296; W4A4, 9 rows 778 -> 941, 16 rows 1158 -> 1058). The
-// launcher knows max_rows, a prompt's tokens, of which a segment gets top_k / n_segs: 4 to 10 of them.
 template <int FMT>
-inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs, int max_rows) {
+inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || a.rows_per_block != INT_MAX || !tiled_rows_aligned(a)) return false;
   if (knob == 2) return true;
-  return max_rows > 128 && 2ll * max_rows >= (FmtTraits<FMT>::kIsFp4 ? 4ll : 5ll) * n_segs;
+  return grouped_fills_tiles(FMT, a.a4_scales != nullptr, a.gate_up != 0, n_segs, a.k, a.max_rows, a.total_rows, a.long_segs);
 }
 
 template <int FMT>
@@ -1268,7 +1295,7 @@ hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, f
 
 template <int FMT>
 hipError_t launch_grouped_mfma(const GroupedArgs& a, int n_segs, int z_ext, hipStream_t stream) {
-  if (grouped_takes_tiled<FMT>(a, n_segs, a.max_rows)) return launch_grouped_tiled<FMT>(a, n_segs, a.max_rows, stream);
+  if (grouped_takes_tiled<FMT>(a, n_segs)) return launch_grouped_tiled<FMT>(a, n_segs, a.max_rows, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const dim3 grid(static_cast<unsigned>((a.n + 63) / 64), static_cast<unsigned>(n_segs), static_cast<unsigned>(z_ext));
   hipError_t err = hipSuccess;

@@ -549,7 +549,7 @@ void GlmMoeLayer::prefill_chain(const uint16_t* x, size_t x_stride, const int32_
   const size_t stride = with_shared ? static_cast<size_t>(max_inter_) : static_cast<size_t>(I);
   const int n_segs = in_table ? E + 1 : E;
   launch_moe_segment(ids, tokens, K, E, d_rows_, d_slot_row_, d_segs_, stream);
-  const dgpp_amd::SegmentRows table{tokens, in_table ? 1 : 0}, shared{tokens, 1};
+  const dgpp_amd::SegmentRows table{tokens, tk + (in_table ? tokens : 0), in_table ? 1 : 0}, shared{tokens, tokens, 1};
   const int group = fp8 ? 0 : fp4_group_;
   const float limit = cfg_.swiglu_limit;
   // gate + up + SwiGLU in one launch (the bits of the two grouped launches and the elementwise kernel)
@@ -633,10 +633,13 @@ void GlmMoeLayer::enqueue_prefill_routed_w4a4(const uint16_t* x, size_t x_stride
   }
   launch_moe_segment(ids, tokens, K, E, d_rows_, d_slot_row_, d_segs_, stream);
   launch_quantize_rows_nvfp4(x, x_stride, tokens, H, d_q_codes_, d_q_scales_, d_q_gs_, stream, 0.f, act_scales_dev);
-  launch_moe_grouped_w4a4_bf16(d_q_codes_, d_q_scales_, d_q_gs_, d_rows_, d_segs_, E, tokens, d_views_, 0, d_gate_, I, I, H,
-                               stream);
-  launch_moe_grouped_w4a4_bf16(d_q_codes_, d_q_scales_, d_q_gs_, d_rows_, d_segs_, E, tokens, d_views_, 1, d_up_, I, I, H,
-                               stream);
+  const dgpp_amd::SegmentRows table{tokens, tk};
+  auto grouped = [&](const int32_t* rows, int which, void* out, int f32, int n, int k) {
+    detail::check(dgpp_amd::grouped_w4a4(d_q_codes_, d_q_scales_, d_q_gs_, rows, d_segs_, E, table, d_views_, which, out, f32,
+                                         static_cast<size_t>(n), n, k, stream));
+  };
+  grouped(d_rows_, 0, d_gate_, 0, I, H);
+  grouped(d_rows_, 1, d_up_, 0, I, H);
   launch_swiglu_quantize_rows_nvfp4(d_gate_, d_up_, I, tk, I, cfg_.swiglu_limit, d_q_codes_, d_q_scales_, d_q_gs_, stream, 0.f,
                                     act_scales_dev ? act_scales_dev + 1 : nullptr);
   if (seg_shared) {
@@ -656,8 +659,7 @@ void GlmMoeLayer::enqueue_prefill_routed_w4a4(const uint16_t* x, size_t x_stride
       launch_moe_grouped_mma_f32(d_slot_act_, stride, d_segs_ + E, 1, tokens, 0, table, 2, d_slot_down_, H, H, SI, stream);
   }
   if (f32_down || seg_shared) {   // the shared rows are fp32: so are the routed ones (src/models/glm/moe_layer.cpp:1121)
-    launch_moe_grouped_w4a4_f32(d_q_codes_, d_q_scales_, d_q_gs_, nullptr, d_segs_, E, tokens, d_views_, 2, d_slot_down_, H, H,
-                                I, stream);
+    grouped(nullptr, 2, d_slot_down_, 1, H, I);
     const int shared_row0 = seg_shared ? tk : -1;
     if (acc)
       launch_moe_accum_ordered_f32(acc, d_slot_down_, H, d_slot_row_, ids, weights, shared_row0, tokens, K, H, stream);
@@ -665,8 +667,7 @@ void GlmMoeLayer::enqueue_prefill_routed_w4a4(const uint16_t* x, size_t x_stride
       launch_moe_accum_ordered(rounded, d_slot_down_, H, d_slot_row_, ids, weights, shared_row0, tokens, K, H, stream);
   } else {
     uint16_t* down = reinterpret_cast<uint16_t*>(d_slot_down_);
-    launch_moe_grouped_w4a4_bf16(d_q_codes_, d_q_scales_, d_q_gs_, nullptr, d_segs_, E, tokens, d_views_, 2, down, H, H, I,
-                                 stream);
+    grouped(nullptr, 2, down, 0, H, I);
     if (acc)
       launch_moe_accum_ordered_f32_bf16down(acc, down, H, d_slot_row_, ids, weights, tokens, K, H, stream);
     else

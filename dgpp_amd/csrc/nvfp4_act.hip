@@ -21,6 +21,7 @@
 #include "../../include/dgpp_amd.h"
 #include "capi_errors.hpp"
 #include "gemv_kernels.hpp"
+#include "moe_grouped.hpp"
 #include "numerics.hpp"
 #include "swiglu.hpp"
 
@@ -237,10 +238,12 @@ int quantize(const uint16_t* x, const uint16_t* up, size_t stride, int rows, int
   return report_hip(err, who);
 }
 
+}  // namespace
 int grouped_w4a4(const uint8_t* codes, const uint8_t* scales, const float* gs, const int32_t* act_rows,
-                 const DgppMoeSegment* segs, int n_segs, int max_rows, const DgppMoeExpertView* views, int which, void* out,
-                 int out_f32, size_t out_stride, int n, int k, void* stream) {
+                 const DgppMoeSegment* segs, int n_segs, const SegmentRows& rows, const DgppMoeExpertView* views, int which,
+                 void* out, int out_f32, size_t out_stride, int n, int k, void* stream) {
   const char* who = "moe w4a4";
+  const int max_rows = rows.max_rows;
   if (n_segs <= 0 || n <= 0) return DGPP_OK;
   if (k <= 0 || k % 64 != 0) return report_invalid(std::string(who) + ": k must be a multiple of 64");
   if (max_rows <= 0) return report_invalid(std::string(who) + ": max_rows");
@@ -264,6 +267,8 @@ int grouped_w4a4(const uint8_t* codes, const uint8_t* scales, const float* gs, c
   a.rows_per_block = INT_MAX;
   a.group_rows = kMaxActRows;
   a.max_rows = max_rows;
+  a.total_rows = rows.total_rows;
+  a.long_segs = rows.long_segs;
   a.act_rows = act_rows;
   a.gate_up = 0;
   a.limit = 0.f;
@@ -274,6 +279,8 @@ int grouped_w4a4(const uint8_t* codes, const uint8_t* scales, const float* gs, c
   a.a4_gs = gs;
   return report_hip(launch_grouped_mma(kFmtNvfp4, a, n_segs, static_cast<int>(z_ext), static_cast<hipStream_t>(stream)), who);
 }
+
+namespace {
 
 int dense_w4a4(const uint8_t* a_codes, const uint8_t* a_scales, size_t a_scale_stride, const float* a_gs,
                const uint8_t* w_codes, const uint8_t* w_scales, const float* w_global, void* out, int out_f32, size_t out_stride,
@@ -369,13 +376,13 @@ int dgpp_launch_swiglu_quantize_rows_nvfp4(const uint16_t* gate, const uint16_t*
 int dgpp_launch_moe_grouped_w4a4_bf16(const uint8_t* codes, const uint8_t* scales, const float* gs, const int32_t* act_rows,
                                       const DgppMoeSegment* segs, int n_segs, int max_rows, const DgppMoeExpertView* views,
                                       int which, uint16_t* out, size_t out_stride, int n, int k, void* stream) {
-  return grouped_w4a4(codes, scales, gs, act_rows, segs, n_segs, max_rows, views, which, out, 0, out_stride, n, k, stream);
+  return grouped_w4a4(codes, scales, gs, act_rows, segs, n_segs, {max_rows}, views, which, out, 0, out_stride, n, k, stream);
 }
 
 int dgpp_launch_moe_grouped_w4a4_f32(const uint8_t* codes, const uint8_t* scales, const float* gs, const int32_t* act_rows,
                                      const DgppMoeSegment* segs, int n_segs, int max_rows, const DgppMoeExpertView* views,
                                      int which, float* out, size_t out_stride, int n, int k, void* stream) {
-  return grouped_w4a4(codes, scales, gs, act_rows, segs, n_segs, max_rows, views, which, out, 1, out_stride, n, k, stream);
+  return grouped_w4a4(codes, scales, gs, act_rows, segs, n_segs, {max_rows}, views, which, out, 1, out_stride, n, k, stream);
 }
 
 int dgpp_dense_w4a4_supported(int k) { return k > 0 && k % 128 == 0; }

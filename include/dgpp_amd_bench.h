@@ -53,6 +53,11 @@ int dgpp_tune_enabled(void);
  * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a
  * workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k);
+/* Likewise for a grouped matrix-core launch over n_segs segments (act_nvfp4: NVFP4 activations; gate_up: gate and up in one
+ * launch) of max_rows rows at most and total_rows together (0: the caller does not know), of which the last long_segs
+ * have max_rows: 1 = tiles of up to 128 activation rows, 0 = the 16-row form. */
+int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_segs, int k, int max_rows, int total_rows,
+                                   int long_segs);
 /* What a block of the grouped launch's 128-row form works on (the last long_segs of the table's segments are known to
  * have max_rows rows): place[0 .. 3] = segment
  * (-1: nothing), row tile, first pass and step of its passes of 128 rows. Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */

@@ -33,6 +33,32 @@ def test_dense_tiles_never_take_a_launch_that_splits_over_a_workspace(fmt):
                 assert not any(takes_tiles(fmt, m, n, k) for k in (512, 2048, 4096, 17408)), (m, n)
 
 
+@pytest.mark.parametrize("fmt,a4,gate_up,k,below,above", [
+    (FP8, 0, 0, 384, 48, 96), (FP8, 0, 0, 768, 32, 40), (FP8, 0, 0, 2048, 16, 24), (FP8, 0, 0, 4096, 12, 20),
+    (FP8, 0, 1, 768, 16, 20), (FP8, 0, 1, 4096, 10, 14), (NVFP4, 0, 0, 512, 20, 28), (NVFP4, 0, 0, 1024, 16, 20),
+    (NVFP4, 0, 1, 2048, 7, 10), (MXFP4, 0, 0, 512, 20, 28), (MXFP4, 0, 0, 1024, 12, 20), (MXFP4, 0, 1, 4096, 6, 8),
+    (NVFP4, 1, 0, 512, 16, 24), (NVFP4, 1, 0, 2048, 12, 15), (NVFP4, 1, 0, 6144, 9, 16)])
+@pytest.mark.parametrize("segs", [128, 288])
+def test_grouped_tiles_by_rows_per_segment(fmt, a4, gate_up, k, below, above, segs):
+    """The tiles are slower at `below` rows per segment and faster at `above` (measured), whatever the tokens among which
+    they are shared out."""
+    def takes(rows, tokens, long_segs=0):
+        return _lib.load().dgpp_bench_grouped_takes_tiles(fmt, a4, gate_up, segs, k, tokens, rows * segs, long_segs)
+    for top_k in (4, 10):
+        assert not takes(below, max(129, below * segs // top_k))
+        assert takes(above, max(129, above * segs // top_k))
+        assert not takes(above, 128)
+        assert takes(below, 129, 1)   # a shared expert's segment behind the others
+
+
+def test_grouped_tiles_without_the_rows_known():
+    takes = _lib.load().dgpp_bench_grouped_takes_tiles
+    assert takes(NVFP4, 0, 0, 1, 128, 129, 0, 0) and not takes(NVFP4, 0, 0, 1, 128, 128, 0, 0)   # one segment: a dense product
+    # NVFP4 activations, four experts a token, 9 rows a segment: measured 1.1 to 1.4 times slower in the tiles
+    assert not takes(NVFP4, 1, 0, 256, 6144, 512, 0, 0)
+    assert takes(NVFP4, 1, 0, 256, 6144, 1024, 0, 0)
+
+
 def tiled_blocks(n_segs, long_segs, row_tiles, max_rows):
     """(segment, row tile, first pass, step) of each block of a grouped launch; block b runs on XCD b % 8."""
     place = np.zeros(4, np.int32)
