@@ -69,9 +69,14 @@ namespace dgpp_amd {
 // switch once). A build with -DDGPP_NO_TUNE compiles them out: every switch reads 0 and dgpp_tune_set does nothing.
 #ifdef DGPP_NO_TUNE
 int tune_get(int) { return 0; }
+void note_tiled_launch() {}
 #else
 static std::atomic<int> g_tune[kTuneCount];
 int tune_get(int key) { return key >= 0 && key < kTuneCount ? g_tune[key].load(std::memory_order_relaxed) : 0; }
+static std::atomic<int> g_tiled_launches;
+void note_tiled_launch() {
+  if (dgpp_tune_enabled()) g_tiled_launches.fetch_add(1, std::memory_order_relaxed);
+}
 #endif
 
 hipError_t ensure_lds_impl(const void* kernel, size_t bytes) {
@@ -436,6 +441,13 @@ void dgpp_tune_set(int key, int value) {
 #endif
 }
 int dgpp_tune_get(int key) { return tune_get(key); }
+int dgpp_bench_tiled_launches(void) {
+#ifdef DGPP_NO_TUNE
+  return 0;
+#else
+  return g_tiled_launches.load(std::memory_order_relaxed);
+#endif
+}
 int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_segs, int k, int max_rows, int total_rows,
                                    int long_segs) {
   return grouped_fills_tiles(fmt, act_nvfp4 != 0, gate_up != 0, n_segs, k, max_rows, total_rows, long_segs) ? 1 : 0;

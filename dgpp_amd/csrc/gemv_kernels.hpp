@@ -1175,6 +1175,7 @@ inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
 
 template <int FMT>
 hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
+  note_tiled_launch();
   const MGeom g = mgeom<FMT>(a.k);
   const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows, passes = (a.m + kTiledCols - 1) / kTiledCols;
   const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
@@ -1193,6 +1194,7 @@ hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
 
 template <int FMT>
 hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, hipStream_t stream) {
+  note_tiled_launch();
   const MGeom g = mgeom<FMT>(a.k);
   const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
   const int row_tiles = (a.n + block_rows - 1) / block_rows;

@@ -38,8 +38,13 @@ extern "C" {
  * the layer driver take the one-launch chain for small routed-only decode batches (default: the driver runs the
  * launches; the chain measured slower); key 13: row steps per wavefront of the chain's down part (0 = automatic);
  * key 14: the fused gate + up matrix-core grouped launch: 1 = every wavefront walks both matrices in turn, 2 = the block's
- * wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most 2048 blocks). Outputs do not
- * depend on keys 1 - 4 and 6 - 14; keys 0 and
+ * wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most 2048 blocks);
+ * key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row form, 2 = tiles
+ * of 128 activation rows wherever the rows are 16-byte aligned (0 = automatic: dgpp_bench_dense_takes_tiles,
+ * dgpp_bench_grouped_takes_tiles). The MXFP8 GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x
+ * activation rows; 0 = automatic); key 16: blocks that share the passes of a segment and a row tile in the grouped tiles
+ * (0 = automatic). Outputs do not
+ * depend on keys 1 - 4 and 6 - 16; keys 0 and
  * 5 change the fp32 summation order (every GEMV launcher follows them alike, so the launchers stay
  * bitwise twins of each other). */
 void dgpp_tune_set(int key, int value);
@@ -48,6 +53,9 @@ int dgpp_tune_get(int key);
  * call of dgpp_tune_set / dgpp_tune_enabled (read once). Without it dgpp_tune_set stores nothing and every launcher
  * runs its measured default, whatever any component of the process calls. */
 int dgpp_tune_enabled(void);
+
+/* How many launches took a form of key 15's tiles so far, counted in a process that enabled the switches. */
+int dgpp_bench_tiled_launches(void);
 
 /* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):
  * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a

@@ -35,3 +35,34 @@ def test_tiled_is_bitwise_the_16_row_form(gpu, m, n, k):
             want = want or got
             for x, y in zip(want, got):
                 assert np.array_equal(x, y), (form, m, n, k)
+
+
+@pytest.mark.parametrize("k", [192, 1088, 2112])
+def test_non_finite_codes_and_scales_reach_the_same_outputs(gpu, k):
+    """NaN codes and scales in the first, an inner and the last block of some rows of either operand; k is no multiple of a
+    step, so the lanes past it read bytes that are their row's own."""
+    m, n = 70, 66
+    a, a_s, w, w_s = md.gemm_case(m, n, k, 4)
+    a[2, 0], a[30, k - 1], w[7, k // 2], w[65, 0] = 0x7F, 0xFF, 0x7F, 0xFF
+    a_s[11, 0] = a_s[69, -1] = w_s[20, -1] = w_s[33, 1] = 0xFF
+    nan_rows, nan_cols = [2, 11, 30, 69], [7, 20, 33, 65]
+    ops = [dev(v) for v in (a, a_s, w, w_s)]
+    out = dev_empty((m, n), np.float32)
+    want = None
+    for form in (1, 2, 3, 4):
+        out.fill_(-1)
+        before = _lib.load().dgpp_bench_tiled_launches()
+        _lib.load().dgpp_tune_set(15, form)
+        try:
+            L.launch_mxfp8_gemm_f32(*ops, out, m, n, k)
+        finally:
+            _lib.load().dgpp_tune_set(15, 0)
+        sync()
+        assert _lib.load().dgpp_bench_tiled_launches() - before == (form > 1)
+        got = host(out).copy()
+        want = got if want is None else want
+        nan = np.isnan(got)
+        expected = np.zeros((m, n), bool)
+        expected[nan_rows], expected[:, nan_cols] = True, True
+        assert np.array_equal(nan, expected), form
+        assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32)), form

@@ -9,28 +9,32 @@ import moe_data
 from dgpp_amd import _lib, hostgen as hg, launch as L
 from gpu_util import DeviceMoe, dev, dev_empty, fp4_matrix, host, sync
 from test_gpu_dense_gemv import make_fp4
+from test_gpu_moe_layer import make_layer
 
 pytestmark = pytest.mark.gpu
 
 
-def both(run, *outs):
-    """The outputs of run() under the 16-row form and under the tiled one."""
+def both(run, *outs, tiled=1):
+    """The outputs of run() under the 16-row form and under the tiled one, in `tiled` launches of it (0: the rows are not
+    aligned and the 16-row form stays)."""
     got = []
     for form in (1, 2):
         for o in outs:
             o.fill_(-1 if o.dtype.is_floating_point else 0x55)
         _lib.load().dgpp_tune_set(15, form)
+        before = _lib.load().dgpp_bench_tiled_launches()
         try:
             run()
         finally:
             _lib.load().dgpp_tune_set(15, 0)
         sync()
+        assert _lib.load().dgpp_bench_tiled_launches() - before == (tiled if form == 2 else 0)
         got.append([host(o).copy() for o in outs])
     return got
 
 
-def same(run, what, *outs):
-    want, got = both(run, *outs)
+def same(run, what, *outs, tiled=1):
+    want, got = both(run, *outs, tiled=tiled)
     for a, b in zip(want, got):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), what
 
@@ -58,13 +62,13 @@ def test_dense_tiled_is_bitwise_the_16_row_form(gpu, kind, m, n, k):
     if kind == "mxfp8":
         payload, scales = hg.encode_mxfp8(hg.bf16_to_f32(wf))
         p_d, s_d = dev(payload), dev(scales)
-        same(lambda: L.launch_mma_gemv_fp8e8m0_bf16(act_d, k, p_d, s_d, out, m, n, k, n + 4, 0, 5), kind, out)
+        same(lambda: L.launch_mma_gemv_fp8e8m0_bf16(act_d, k, p_d, s_d, out, m, n, k, n + 4, 0, 5), kind, out, tiled=m > 1)
         return
     rs, cs = (7, 7) if kind == "fp8" else (5, 6)
     payload, _ = hg.encode_fp8_blocks(wf, 128, 128)
     scales = rng.uniform(0.5, 2.0, ((n + (1 << rs) - 1) >> rs, (k + (1 << cs) - 1) >> cs)).astype(np.float32) * 1e-3
     p_d, s_d = dev(payload), dev(scales)
-    same(lambda: L.launch_mma_gemv_fp8_bf16(act_d, k, p_d, s_d, out, m, n, k, n + 4, rs, cs), kind, out)
+    same(lambda: L.launch_mma_gemv_fp8_bf16(act_d, k, p_d, s_d, out, m, n, k, n + 4, rs, cs), kind, out, tiled=m > 1)   # a row keeps to the vector core
 
 
 @pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8"])
@@ -103,7 +107,8 @@ def test_grouped_tiled_is_bitwise_the_16_row_form(gpu, kind, H, I):
     same(lambda: plain_f(slot, I, segs, E, most, 0, d.views, 2, down_odd, H + 1, H, I, None, None, *more), "odd stride", down_odd)
     # rows that are no whole 16-byte vectors keep the 16-row form
     odd = dev(hg.normal_bf16(0x79, (total, I + 2)))
-    same(lambda: plain_f(odd, I + 2, segs, E, most, 0, d.views, 2, down, H, H, I, None, None, *more), "unaligned rows", down)
+    same(lambda: plain_f(odd, I + 2, segs, E, most, 0, d.views, 2, down, H, H, I, None, None, *more), "unaligned rows", down,
+         tiled=0)
     if kind == "nvfp4":
         codes, gs = dev_empty((T, H // 2), np.uint8), dev_empty((T,), np.float32)
         scales = dev_empty((T, _lib.load().dgpp_nvfp4_act_scale_stride(H)), np.uint8)
@@ -114,3 +119,115 @@ def test_grouped_tiled_is_bitwise_the_16_row_form(gpu, kind, H, I):
         s2 = dev_empty((total, _lib.load().dgpp_nvfp4_act_scale_stride(I)), np.uint8)
         L.launch_quantize_rows_nvfp4(slot, I, total, I, c2, s2, g2)
         same(lambda: L.launch_moe_grouped_w4a4_f32(c2, s2, g2, None, segs, E, most, d.views, 2, down, H, H, I), "w4a4 down", down)
+
+
+@pytest.mark.parametrize("kind,group", [("nvfp4", 16), ("mxfp4", 32)])
+@pytest.mark.parametrize("m,n,k", [(129, 100, 1152), (300, 257, 2304), (64, 64, 576)])
+def test_gate_and_up_apart_of_one_segment(gpu, kind, group, m, n, k):
+    """The form that stores gate and up unmerged (the dense product by views), a lone segment spread over the XCDs."""
+    k = {1152: 1024, 2304: 2048, 576: 640}[k] if kind == "nvfp4" else k
+    p = moe_data.make_problem(2, k, 288, 1, 4, kind, 17 + m, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    x = dev(hg.normal_bf16(0x9C0 + k, (m, k)))
+    seg = dev(np.array([[0, m, 1]], np.int32))
+    gate, up = dev_empty((m, n), np.uint16), dev_empty((m, n), np.uint16)
+    same(lambda: L.launch_dense_mma_fp4_gate_up_bf16(x, k, seg, d.views, gate, up, m, n, k, None, group), kind, gate, up)
+    same(lambda: L.launch_dense_mma_fp4_prod_bf16(x, k, seg, d.views, 1, up, m, n, k, None, group), "prod", up)
+
+
+def w4a4_rows(x, rows, k):
+    codes, gs = dev_empty((rows, k // 2), np.uint8), dev_empty((rows,), np.float32)
+    scales = dev_empty((rows, _lib.load().dgpp_nvfp4_act_scale_stride(k)), np.uint8)
+    L.launch_quantize_rows_nvfp4(x, k, rows, k, codes, scales, gs)
+    return codes, scales, gs
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 130, 128), (129, 257, 1152), (300, 100, 4224), (33, 64, 2304)])
+def test_dense_nvfp4_activations_tiled_is_bitwise_the_16_row_form(gpu, m, n, k):
+    """k of one tile, of tiles that the parts do not divide, and of a last part that is empty (33 tiles, 12 to a part)."""
+    act, payload, scales, glob = make_fp4(m, n, k, 0xA40 + k, 16)
+    codes, a_s, gs = w4a4_rows(dev(act), m, k)
+    p_d, s_d, g_d = dev(payload), dev(scales), dev(glob)
+    out = dev_empty((m, n + 5), np.uint16)
+    same(lambda: L.launch_dense_w4a4_bf16(codes, a_s, a_s.shape[1], gs, p_d, s_d, g_d, out, n + 5, m, n, k), "dense w4a4", out)
+
+
+@pytest.mark.parametrize("H,I", [(192, 320), (64, 1088)])
+def test_grouped_nvfp4_activations_tiled_with_a_part_of_a_k_tile(gpu, H, I):
+    rows = [1, 0, 33, 130, 64, 17, 65, 32, 300]
+    E, total = len(rows), sum(rows)
+    p = moe_data.make_problem(E, H, I, 2, 8, "nvfp4", 71, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    starts = np.concatenate([[0], np.cumsum(rows)[:-1]])
+    segs = dev(np.array([[starts[i], rows[i], (i * 4) % E] for i in range(E)], np.int32))
+    for which, n, k in ((0, I, H), (2, H, I)):
+        codes, scales, gs = w4a4_rows(dev(hg.normal_bf16(0xB60 + k, (total, k))), total, k)
+        out, outf = dev_empty((total, n + 4), np.uint16), dev_empty((total, n), np.float32)
+        same(lambda: L.launch_moe_grouped_w4a4_bf16(codes, scales, gs, None, segs, E, 300, d.views, which, out, n + 4, n, k), "bf16", out)
+        same(lambda: L.launch_moe_grouped_w4a4_f32(codes, scales, gs, None, segs, E, 300, d.views, which, outf, n, n, k), "f32", outf)
+
+
+def same_with_nan(run, what, *outs):
+    """As same(); a NaN stands for any NaN, and some of the values are."""
+    want, got = both(run, *outs)
+    for a, b in zip(want, got):
+        v = [o if o.dtype == np.float32 else hg.bf16_to_f32(o.view(np.uint16)) for o in (a, b)]
+        nan = np.isnan(v[0])
+        assert nan.any() and not nan.all(), what
+        assert np.array_equal(nan, np.isnan(v[1])) and np.array_equal(v[0][~nan], v[1][~nan]), what
+
+
+@pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "mxfp8", "w4a4"])
+def test_non_finite_values_reach_the_same_outputs(gpu, kind):
+    """Infinite and NaN activations in the first, an inner and the last element of a row, NaN scales and (FP8) codes of some
+    weight rows, with a part of a k tile where the format has one."""
+    m, n = 130, 140
+    k = {"nvfp4": 1024, "mxfp4": 1152, "fp8": 1104, "mxfp8": 1120, "w4a4": 1152}[kind]
+    rng = np.random.default_rng(5)
+    act = hg.normal_bf16(0xC10, (m, k))
+    if kind != "w4a4":
+        act[3, 0], act[40, k - 1], act[77, k // 2], act[129, 0] = 0x7F80, 0x7FC0, 0xFF80, 0x7FC0
+    act_d = dev(act)
+    if kind in ("nvfp4", "mxfp4", "w4a4"):
+        _, payload, scales, glob = make_fp4(1, n, k, 0xC20, 32 if kind == "mxfp4" else 16)
+        scales[5, 0] = scales[139, -1] = 0xFF if kind == "mxfp4" else 0x7F
+        p_d, s_d, g_d = dev(payload), dev(scales), dev(glob) if glob is not None else None
+        if kind == "w4a4":
+            codes, a_s, gs = w4a4_rows(act_d, m, k)
+            a_s[9, 1] = 0x7F
+            gs[64] = float("inf")
+            out = dev_empty((m, n), np.uint16)
+            same_with_nan(lambda: L.launch_dense_w4a4_bf16(codes, a_s, a_s.shape[1], gs, p_d, s_d, g_d, out, n, m, n, k), kind, out)
+            return
+        w = fp4_matrix(p_d, s_d, g_d, n, k, 32 if kind == "mxfp4" else 16)
+        outf = dev_empty((m, n), np.float32)
+        same_with_nan(lambda: L.launch_mma_gemv_fp4_f32(act_d, k, w, outf, m, n, k, n), kind, outf)
+        return
+    wf = hg.f32_to_bf16(hg.normal_f32(0xC30, (n, k), 0.02))
+    out = dev_empty((m, n), np.uint16)
+    if kind == "mxfp8":
+        payload, scales = hg.encode_mxfp8(hg.bf16_to_f32(wf))
+        payload[6, k - 1], payload[100, 0], scales[8, -1] = 0x7F, 0xFF, 0xFF
+        p_d, s_d = dev(payload), dev(scales)
+        same_with_nan(lambda: L.launch_mma_gemv_fp8e8m0_bf16(act_d, k, p_d, s_d, out, m, n, k, n, 0, 5), kind, out)
+        return
+    payload, _ = hg.encode_fp8_blocks(wf, 128, 128)
+    payload[6, k - 1], payload[100, 0] = 0x7F, 0xFF
+    scales = rng.uniform(0.5, 2.0, ((n + 127) >> 7, (k + 127) >> 7)).astype(np.float32) * 1e-3
+    scales[1, -1] = np.inf
+    p_d, s_d = dev(payload), dev(scales)
+    same_with_nan(lambda: L.launch_mma_gemv_fp8_bf16(act_d, k, p_d, s_d, out, m, n, k, n, 7, 7), kind, out)
+
+
+@pytest.mark.parametrize("kind,shared,launches", [("nvfp4", "nvfp4", 2), ("mxfp4", "mxfp4", 2), ("nvfp4", "fp8", 4), ("fp8", "fp8", 4),
+                                                  ("fp8", None, 2)])
+@pytest.mark.parametrize("E,T", [(17, 300), (6, 140)])
+def test_a_layer_with_a_shared_expert_is_bitwise_its_16_row_form(gpu, kind, shared, launches, E, T):
+    """A shared expert's segment, as long as the prompt, behind the routed ones or in launches of its own: its blocks go
+    over all XCDs, a table of fewer segments than XCDs likewise."""
+    p = moe_data.make_problem(E, 512, 256, 3, T, kind, 55 + E, shared_kind=shared, shared_I=256 if shared else None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    layer = make_layer(p, d, L.ROUTER_SOFTMAX_TOPK, 1.0, T)
+    out = dev_empty((T, 512), np.uint16)
+    same(lambda: layer.enqueue_prefill(d.x, 512, out, T), kind, out, tiled=launches)
+    layer.close()
