@@ -2,19 +2,25 @@
 // activation rows, so a weight is fetched and decoded once per 128 activation rows instead of once per 16
 // (gemv_mfma_kernels.hpp). Included by gemv_kernels.hpp after the argument structs.
 //
-// What bounds it. With 16 rows per pass a prompt of T tokens decodes every weight T / 16 times and gathers the
-// activations again for every 64 weight rows: the vector ALU and the gathers, not the matrix core, were the time.
-// Here a wavefront owns two row groups (16 weight rows each) and CT column tiles: per 32 elements of k it decodes two
-// operands and runs 2 CT MFMAs on them, and reads CT operands from LDS - at CT = 8 the LDS reads (128 bytes per
-// cycle and CU) and the MFMAs take the same time, which is the bound that is left; the weights' decode hides behind
-// the MFMAs.
+// With 16 rows per pass a prompt of T tokens decodes every weight T / 16 times and gathers the activations again for
+// every 64 weight rows: the vector ALU and the gathers, not the matrix core, were the time. Here a wavefront owns two row
+// groups (16 weight rows each) and CT column tiles: per 32 elements of k it decodes two operands and runs 2 CT MFMAs on
+// them, and reads CT operands from LDS.
+//
+// What bounds it: the latency of a tile, with two wavefronts per SIMD to cover it. Counters (busy share of the chip's
+// cycles, share of a wavefront's life): block FP8 1000 x 12288 x 6144 MFMA 33 %, vector ALU 42 %, LDS 17 %, waiting for
+// data or a barrier 29 %, for an issue slot 33 %; MXFP4 prompt of 2048 tokens, gate + up MFMA 18 %, vector ALU 21 %, LDS
+// 18 %, waiting 42 % and 33 %; NVFP4 activations, 16 rows a segment MFMA 13 %, waiting 61 %: 64-byte pieces of 16
+// weight rows, one tile ahead. A pass of up to 32 rows pays for the registers and the LDS of one of 128. The grouped
+// kernels spill around a pass, not in the walk over k (16 to 81 registers, MXFP4 gate + up 4): a short k pays most.
 //
 // Tile. k advances by 128 elements: the weights go from memory straight to the operand layout in registers (nothing
 // of them is shared between wavefronts), the block's activation rows into one of two LDS stages of
-// [row][16 units of 16 bytes], unit u of row r at u ^ (r % 16) - both the row-major writes and the operand reads are
-// conflict-free (BF16 rows go from memory to LDS without passing registers, which the sums need). Loads of a tile are
-// issued one tile ahead of its use; one barrier per tile. 64 KB of LDS and up to
-// 256 registers: two blocks per CU, one computing while the other waits.
+// [row][16 units of 16 bytes], unit u of row r at u ^ (r % 16). The row-major writes and the FP8 operand reads (two
+// units per lane and step) are conflict-free; of the FP4 reads (four units) the quarters meet in pairs, and half of their
+// LDS cycles are conflicts. BF16 rows go from memory to LDS without passing registers, which the sums need. Loads of a
+// tile are issued one tile ahead of its use; one barrier per tile. 64 KB of LDS and up to 256 registers: two blocks per
+// CU, one computing while the other waits.
 //
 // Arithmetic. The sums of a (weight row, activation row) pair are those of the 16-row form: the same elements in the
 // same MFMAs, K parts on their own, added in ascending order. A call's bits do not depend on which form takes it.
