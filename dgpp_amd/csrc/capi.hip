@@ -207,7 +207,7 @@ bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool
 }
 int dense_rows(int fmt, const uint16_t* act, size_t act_stride, const MatRef& mat, const float* global, void* out,
                size_t out_stride, int out_f32, int m, int n, int k, hipStream_t stream, const char* who, int from_rows,
-               void* ws = nullptr, size_t ws_bytes = 0) {
+               void* ws = nullptr, size_t ws_bytes = 0, bool beside = false) {
   const int core = tune_get(kTuneCore);   // bench switch: 1 pins the vector core, 2 the matrix core
   if (core != 1 && (core == 2 || dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, from_rows))) {
     if ((m + kTileCols - 1) / kTileCols > 65535) return fail_arg(std::string(who) + ": grid dimension overflow");
@@ -223,6 +223,7 @@ int dense_rows(int fmt, const uint16_t* act, size_t act_stride, const MatRef& ma
     a.n = n;
     a.k = k;
     a.once = m <= kTileCols;
+    a.beside = beside;
     return finish(launch_dense_mma(fmt, a, static_cast<float*>(ws), ws_bytes, stream), who);
   }
   const int max_rows = max_stage_rows(k);
@@ -275,7 +276,7 @@ int fp4_gemv(const uint16_t* act, size_t act_stride, const DgppFp4Matrix* w, voi
 int scale_gemm(const uint16_t* act, size_t act_stride, const uint8_t* payload, const void* scales, int e8m0, void* out,
                int out_f32, int m, int n, int k, void* stream, size_t out_stride, int rs, int cs, int last_row_only,
                int compact_row, bool grid_form, const char* who, int mma_from_rows = 0, void* ws = nullptr,
-               size_t ws_bytes = 0) {
+               size_t ws_bytes = 0, bool beside = false) {
   if (m <= 0 || n <= 0) return DGPP_OK;
   if (!act || !payload || !scales || !out) return fail_arg(std::string(who) + ": null pointer");
   if (grid_form) {
@@ -306,7 +307,7 @@ int scale_gemm(const uint16_t* act, size_t act_stride, const uint8_t* payload, c
     return fail_arg(std::string(who) + ": k must be a multiple of 16 with a 16-byte aligned payload");
   const int mma_from = mma_from_rows > 0 ? mma_from_rows : 0;   // the caller's own boundary can only add matrix-core cases
   return dense_rows(e8m0 ? kFmtFp8E8M0 : kFmtFp8F32, act, act_stride, fp8_mat(payload, scales, rs, cs), nullptr, o,
-                    out_stride, out_f32, m, n, k, as_stream(stream), who, mma_from, ws, ws_bytes);
+                    out_stride, out_f32, m, n, k, as_stream(stream), who, mma_from, ws, ws_bytes, beside);
 }
 
 // src/kernels/glm_moe.cu:1683-1703 (check_slot_args) and :2197-2228 (check_fp4_slot_args).
@@ -1688,6 +1689,13 @@ int dgpp_launch_scale_gemm_grid_e8m0_f32(const uint16_t* act, size_t act_row_str
                     cs, 0, -1, true, "scale_gemm_grid_e8m0", 0, ws, ws_bytes);
 }
 
+}  // extern "C"
+int dgpp_amd::scale_gemm_mxfp8(const uint16_t* act, size_t act_stride, const uint8_t* payload, const uint8_t* scales, void* out,
+                               int out_f32, int m, int n, int k, void* stream, void* ws, size_t ws_bytes, bool beside) {
+  return scale_gemm(act, act_stride, payload, scales, 1, out, out_f32, m, n, k, stream, static_cast<size_t>(n), 0, 5, 0, -1, true,
+                    "scale_gemm_grid_e8m0", 0, ws, ws_bytes, beside);
+}
+extern "C" {
 int dgpp_launch_scale_gemv_multi_bf16(const DgppFp8GemvProblem* problems, int n_problems, const uint16_t* act,
                                       size_t act_row_stride_elems, int rows, int k, void* stream) {
   // src/kernels/scale_gemm.cu:625-672: each problem's output is bitwise the single launcher's.

@@ -67,7 +67,7 @@ struct RowGeom {
 };
 // Bench A/B switches (host side, process-wide; 0 = the default behaviour). Set through
 // dgpp_tune_set; launchers read them when they pick a geometry or a kernel form.
-enum : int { kTunePreferP = 0, kTuneSlotRun = 1, kTuneSlotSteps = 2, kTuneSplitStage = 3, kTuneCore = 5, kTuneSelectAlone = 7, kTuneXcdGroup = 8, kTuneRouterTile = 10, kTuneTeams = 11, kTuneChain = 12, kTuneChainDownSteps = 13, kTuneGateUpWalks = 14, kTuneTiled = 15, kTuneTiledPasses = 16, kTuneCount = 17 };
+enum : int { kTunePreferP = 0, kTuneSlotRun = 1, kTuneSlotSteps = 2, kTuneSplitStage = 3, kTuneCore = 5, kTuneSelectAlone = 7, kTuneXcdGroup = 8, kTuneRouterTile = 10, kTuneTeams = 11, kTuneChain = 12, kTuneChainDownSteps = 13, kTuneGateUpWalks = 14, kTuneTiled = 15, kTuneTiledPasses = 16, kTuneSharedBeside = 17, kTuneCount = 18 };
 int tune_get(int key);
 void note_tiled_launch();   // counted for the tests while the switches are enabled
 

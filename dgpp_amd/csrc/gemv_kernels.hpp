@@ -71,6 +71,7 @@ struct DenseArgs {
   const uint8_t* a4_scales = nullptr;
   size_t a4_scale_stride = 0;
   const float* a4_gs = nullptr;
+  bool beside = false;      // other work fills the chip meanwhile: the form that does the least, not the one that ends first
 };
 
 template <int FMT, int MAXR, int NB, bool NT>
@@ -1163,7 +1164,7 @@ inline bool dense_takes_tiled(const DenseArgs& a) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return false;
   if (knob == 2) return true;
-  return dense_fills_tiles(FMT, a.m, a.n, a.k);
+  return a.beside ? a.m > 64 : dense_fills_tiles(FMT, a.m, a.n, a.k);
 }
 template <int FMT>
 inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {

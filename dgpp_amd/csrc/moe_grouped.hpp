@@ -1,5 +1,5 @@
-// The grouped matrix-core launches for callers that know more of the segments than their largest size: the layer driver,
-// which made the table. Arguments and results as the dgpp_launch_moe_grouped_mma_* and _w4a4_* entry points.
+// The matrix-core launches for the layer driver, which knows more than their entry points take: of the segments, whose table it
+// made, and of what runs beside a launch. Arguments and results as the dgpp_launch_moe_grouped_mma_* and _w4a4_* entry points.
 #pragma once
 
 #include <stddef.h>
@@ -22,5 +22,9 @@ int grouped_mma(int fp4_group, const uint16_t* act, size_t act_stride, const Dgp
 int grouped_w4a4(const uint8_t* codes, const uint8_t* scales, const float* gs, const int32_t* act_rows,
                  const DgppMoeSegment* segs, int n_segs, const SegmentRows& rows, const DgppMoeExpertView* views, int which,
                  void* out, int out_f32, size_t out_stride, int n, int k, void* stream);
+
+// A projection with MXFP8 weights (one scale byte per 32 values). beside: other work fills the chip meanwhile.
+int scale_gemm_mxfp8(const uint16_t* act, size_t act_stride, const uint8_t* payload, const uint8_t* scales, void* out, int out_f32,
+                     int m, int n, int k, void* stream, void* ws, size_t ws_bytes, bool beside);
 
 }  // namespace dgpp_amd

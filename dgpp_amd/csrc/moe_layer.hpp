@@ -84,6 +84,7 @@ class GlmMoeLayer {
   void release();
   void check_tokens(int tokens) const;
   bool needs_order(int tokens) const;
+  bool shared_beside_takes_tiles(int tokens) const;
   void dense_shared_chain(const uint16_t* x, size_t x_stride, int tokens, hipStream_t stream);
   void prefill_chain(const uint16_t* x, size_t x_stride, const int32_t* ids, const float* weights, uint16_t* out_bf16,
                      float* out_f32, int tokens, hipStream_t stream, bool with_shared, bool accumulate = true);

@@ -43,8 +43,9 @@ extern "C" {
  * of 128 activation rows wherever the rows are 16-byte aligned (0 = automatic: dgpp_bench_dense_takes_tiles,
  * dgpp_bench_grouped_takes_tiles). The MXFP8 GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x
  * activation rows; 0 = automatic); key 16: blocks that share the passes of a segment and a row tile in the grouped tiles
- * (0 = automatic). Outputs do not
- * depend on keys 1 - 4 and 6 - 16; keys 0 and
+ * (0 = automatic); key 17: the MXFP8 shared expert's projections of more than 64 rows on the layer driver's second stream: 1 =
+ * the form that is faster alone, 2 = the tiles (0 = automatic). Outputs do not
+ * depend on keys 1 - 4 and 6 - 17; keys 0 and
  * 5 change the fp32 summation order (every GEMV launcher follows them alike, so the launchers stay
  * bitwise twins of each other). */
 void dgpp_tune_set(int key, int value);

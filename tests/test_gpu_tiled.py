@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import moe_data
-from dgpp_amd import _lib, hostgen as hg, launch as L
+from dgpp_amd import _lib, hostgen as hg, launch as L, moe_layer as ML
 from gpu_util import DeviceMoe, dev, dev_empty, fp4_matrix, host, sync
 from test_gpu_dense_gemv import make_fp4
 from test_gpu_moe_layer import make_layer
@@ -230,4 +230,31 @@ def test_a_layer_with_a_shared_expert_is_bitwise_its_16_row_form(gpu, kind, shar
     layer = make_layer(p, d, L.ROUTER_SOFTMAX_TOPK, 1.0, T)
     out = dev_empty((T, 512), np.uint16)
     same(lambda: layer.enqueue_prefill(d.x, 512, out, T), kind, out, tiled=launches)
+    layer.close()
+
+
+@pytest.mark.parametrize("T", [70, 200])
+def test_a_layer_with_an_mxfp8_shared_expert_does_not_depend_on_its_projections_form(gpu, T):
+    """The projections beside the routed chain, in the form that is faster alone and in the tiles (bench switch 17)."""
+    p = moe_data.make_problem(24, 512, 256, 3, T, "nvfp4", 77, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    mats = [hg.encode_mxfp8(hg.normal_f32(0xD00 + i, (n, k), 0.05)) for i, (n, k) in enumerate(((384, 512), (384, 512), (512, 384)))]
+    pay, scales = [dev(m[0]) for m in mats], [dev(m[1]) for m in mats]
+    cfg = L.make_config(512, 256, 24, 3, n_shared_experts=1, routed_scaling_factor=1.0, swiglu_limit=7.0, router_mode=L.ROUTER_SOFTMAX_TOPK)
+    views = list((L.MoeExpertView * (d.views.numel() // 96)).from_buffer_copy(bytes(host(d.views))))
+    layer = ML.MoeLayer(cfg, ML.EXPERTS_NVFP4, views, T, shared_inter=384, sh_payload=pay, sh_scales_e8m0=scales, router_gate=dev(p.router_gate))
+    out, got = dev_empty((T, 512), np.uint16), []
+    for form in (1, 2, 0):
+        out.fill_(0x55)
+        before = _lib.load().dgpp_bench_tiled_launches()
+        _lib.load().dgpp_tune_set(17, form)
+        try:
+            layer.enqueue_prefill(d.x, 512, out, T)
+        finally:
+            _lib.load().dgpp_tune_set(17, 0)
+        sync()
+        tiled = _lib.load().dgpp_bench_tiled_launches() - before
+        got.append((host(out).copy(), tiled))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][0], got[2][0])
+    assert got[1][1] - got[0][1] == 3 and got[2][1] == got[1 if T == 200 else 0][1]
     layer.close()
