@@ -456,9 +456,9 @@ int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_se
 int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place) {
   if (n_segs <= 0 || long_segs < 0 || long_segs > n_segs || row_tiles <= 0 || max_rows <= 0) return 0;
   const TiledDeal d = tiled_deal(n_segs, long_segs, row_tiles, max_rows, 0);
-  const int blocks = static_cast<int>(d.blocks());
+  const int gx = static_cast<int>(d.grid_x()), blocks = gx * static_cast<int>(d.grid_y());
   if (block >= 0 && block < blocks && place) {
-    const TiledPlace at = tiled_place(d, block);
+    const TiledPlace at = tiled_place(d, block % gx, block / gx);
     place[0] = at.seg;
     place[1] = at.tile;
     place[2] = at.slot;

@@ -1201,7 +1201,7 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
   const int row_tiles = (a.n + block_rows - 1) / block_rows;
   const TiledDeal deal = tiled_deal(n_segs, a.long_segs, row_tiles, max_rows, tune_get(kTuneTiledPasses));
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(deal.blocks()), dim3(kBlockThreads), 0, stream, a, g, deal);
+    hipLaunchKernelGGL(kern, dim3(deal.grid_x(), deal.grid_y()), dim3(kBlockThreads), 0, stream, a, g, deal);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {

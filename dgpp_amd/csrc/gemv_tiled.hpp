@@ -407,12 +407,13 @@ struct TiledDeal {
   int spread_slots;
   int spread_per_xcd; // blocks
   int row_tiles;
-  __host__ __device__ unsigned whole_blocks() const {   // of one slot
+  unsigned whole_blocks() const {   // of one slot
     return static_cast<unsigned>((whole + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(row_tiles);
   }
-  __host__ __device__ unsigned blocks() const {
-    return static_cast<unsigned>(spread_per_xcd) * kXcds + whole_blocks() * static_cast<unsigned>(slots);
-  }
+  // The grid: x the spread segments' blocks, then a slot's of the whole ones; y the slots. (One index for all would cost every
+  // block, those without a pass too, another division: 1 us of a launch.)
+  unsigned grid_x() const { return static_cast<unsigned>(spread_per_xcd) * kXcds + whole_blocks(); }
+  unsigned grid_y() const { return static_cast<unsigned>(slots > 1 ? slots : 1); }
 };
 // max_rows: no segment has more; long_segs: so many at the table's end have that many. tuned > 0: slots (bench switch 16).
 inline TiledDeal tiled_deal(int n_segs, int long_segs, int row_tiles, int max_rows, int tuned) {
@@ -433,23 +434,23 @@ inline TiledDeal tiled_deal(int n_segs, int long_segs, int row_tiles, int max_ro
 struct TiledPlace {
   int seg, tile, slot, slots;   // the block takes passes slot, slot + slots, ... of the segment; seg -1: none
 };
-__host__ __device__ __forceinline__ TiledPlace tiled_place(const TiledDeal& d, int block) {
-  const int xcd = block % kXcds, first_whole = d.spread_per_xcd * kXcds;
-  if (block < first_whole) {
-    const int of_seg = d.row_tiles * d.spread_slots, item = xcd * d.spread_per_xcd + block / kXcds;
-    if (item >= d.spread * of_seg) return {-1, 0, 0, 1};
+__host__ __device__ __forceinline__ TiledPlace tiled_place(const TiledDeal& d, int x, int y) {
+  const int xcd = x & (kXcds - 1), idx = (x >> 3) - d.spread_per_xcd;
+  if (idx < 0) {
+    const int of_seg = d.row_tiles * d.spread_slots, item = xcd * d.spread_per_xcd + (x >> 3);
+    if (y > 0 || item >= d.spread * of_seg) return {-1, 0, 0, 1};
     return {d.whole + item / of_seg, item % of_seg / d.spread_slots, item % d.spread_slots, d.spread_slots};
   }
-  const int of_slot = static_cast<int>(d.whole_blocks()), at = block - first_whole;
-  const int idx = at % of_slot / kXcds, seg = idx / d.row_tiles * kXcds + xcd;
+  const int seg = idx / d.row_tiles * kXcds + xcd;
   if (seg >= d.whole) return {-1, 0, 0, 1};
-  return {seg, idx % d.row_tiles, at / of_slot, d.slots};
+  return {seg, idx % d.row_tiles, y, d.slots};
 }
+static_assert(kXcds == 8, "the shifts above");
 
 template <int FMT, bool GU, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, TiledDeal deal) {
   __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
-  const TiledPlace at = tiled_place(deal, static_cast<int>(blockIdx.x));
+  const TiledPlace at = tiled_place(deal, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y));
   if (at.seg < 0) return;
   const DgppMoeSegment seg = a.segs[at.seg];
   const int first_pass = at.slot * kTiledCols, tile = at.tile;
