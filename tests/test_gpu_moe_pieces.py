@@ -31,6 +31,13 @@ def test_segment_bit_exact(gpu, T, K, E):
         assert np.array_equal(host(segs_d), segs)
 
 
+@pytest.mark.parametrize("T,K,E", [(255, 1, 3), (257, 1, 1), (513, 1, 4), (1365, 3, 130), (4096, 1, 2), (4097, 1, 5),
+                                   (2731, 3, 3), (9001, 2, 1024), (4096, 8, 288)])
+def test_segment_over_several_wavefronts_bit_exact(gpu, T, K, E):
+    """Around one wavefront's run of 256 ids, sixteen wavefronts' and their eight reads of 64 each; experts without rows."""
+    test_segment_bit_exact(gpu, T, K, E)
+
+
 def test_segment_argument_errors(gpu):
     d = dev(np.zeros(64, np.int32))
     for bad in [dict(top_k=17), dict(top_k=0), dict(n_experts=1025), dict(n_experts=0)]:
