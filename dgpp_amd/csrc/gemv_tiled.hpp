@@ -7,33 +7,39 @@
 // groups (16 weight rows each) and CT column tiles: per 32 elements of k it decodes two operands and runs 2 CT MFMAs on
 // them, and reads CT operands from LDS.
 //
-// What bounds it: the latency of a tile, with two wavefronts per SIMD to cover it. Counters (busy share of the chip's
-// cycles, share of a wavefront's life): block FP8 1000 x 12288 x 6144 MFMA 33 %, vector ALU 42 %, LDS 17 %, waiting for
-// data or a barrier 29 %, for an issue slot 33 %; MXFP4 prompt of 2048 tokens, gate + up MFMA 18 %, vector ALU 21 %, LDS
-// 18 %, waiting 42 % and 33 %; NVFP4 activations, 16 rows a segment MFMA 13 %, waiting 61 %: 64-byte pieces of 16
-// weight rows, one tile ahead. A pass of up to 32 rows pays for the registers and the LDS of one of 128. The grouped
-// kernels spill around a pass, not in the walk over k (16 to 81 registers, MXFP4 gate + up 4): a short k pays most.
+// Tile. k advances by one step of a row group, 128 elements (FP4) or 64 (FP8). Weights are of one wavefront and go to its
+// registers, three tiles ahead of their use, two for the widest pass with NVFP4 activations; the block's activation rows
+// go into a ring of LDS stages, three tiles ahead as well (BF16: from memory to LDS without passing registers) where four
+// stages leave room for two blocks per CU, one tile ahead for FP4's widest pass. One barrier per tile, which waits for
+// those of a wavefront's loads that the tile needs and no others: waiting for all of them, the form before this one had
+// one tile on its way and took the latency of a load per tile.
 //
-// Tile. k advances by 128 elements: the weights go from memory straight to the operand layout in registers (nothing
-// of them is shared between wavefronts), the block's activation rows into one of two LDS stages of
-// [row][16 units of 16 bytes], unit u of row r at u ^ (r % 16). The row-major writes and the FP8 operand reads (two
-// units per lane and step) are conflict-free; of the FP4 reads (four units) the quarters meet in pairs, and half of their
-// LDS cycles are conflicts. BF16 rows go from memory to LDS without passing registers, which the sums need. Loads of a
-// tile are issued one tile ahead of its use; one barrier per tile. 64 KB of LDS and up to 256 registers: two blocks per
-// CU, one computing while the other waits.
+// Lanes. The matrix core wants 16 rows in 16 adjacent lanes, the memory pipe adjacent lanes in one row. Weights are
+// therefore asked for row by row (four lanes to the 64 bytes of a row's tile), the FP4 scales of four tiles at once, and
+// both pass through a region of LDS of the wavefront's own. The places in the stages and in that region are turned such
+// that sixteen lanes that read together meet no bank twice (SQ_LDS_BANK_CONFLICT 0; before, half of the LDS cycles for FP4).
+// Measured, us, uniform segments, lanes in the matrix core's order -> row by row: MXFP4 gate + up, 256 x 2 x 1024 x 4096, 16
+// rows 323 -> 271, 64 388 -> 351, 128 538 -> 550; NVFP4 activations, 256 x 2048 x 6144, 16 rows 557 -> 439.
+//
+// What bounds it: at 128 rows a pass the matrix core and the LDS together (a read feeds two MFMAs; dense block FP8
+// 1000 x 12288 x 6144 MFMA 42 % busy with a quarter of the places empty in the last round); at 16 rows the memory pipe,
+// 4.2 TB/s for FP4 and 4.9 for FP8, with two blocks per CU.
+// From the form before (a tile ahead, waiting for all): block FP8 gate + up, 128 x 2 x 768 x 2048, 777 tokens 193 -> 141 us,
+// down 146 -> 80; MXFP4, 2048 tokens 744 -> 582 and 445 -> 339; NVFP4, 288 experts, 4096 x 512, 4096 tokens 706 -> 549 and
+// 566 -> 401; NVFP4 activations, 512 tokens 708 -> 482; dense block FP8 1000 x 12288 x 6144 190 -> 166.
 //
 // Arithmetic. The sums of a (weight row, activation row) pair are those of the 16-row form: the same elements in the
 // same MFMAs, K parts on their own, added in ascending order. A call's bits do not depend on which form takes it.
 #pragma once
 
+#include <type_traits>
+
 #include "gemv_mfma_kernels.hpp"
 
 namespace dgpp_amd {
 
-constexpr int kTileK = 128;                       // elements of k per tile
-constexpr int kTiledCols = 128;                   // activation rows per pass
+constexpr int kTiledCols = 128;                   // activation rows of the widest pass
 constexpr int kTiledRows = 128;                   // weight rows of a block (gate + up: 64 of each)
-constexpr int kTiledStage = kTiledCols * 16;      // 16-byte units of one stage
 
 // The two row groups of a wavefront: two groups of one matrix, or one of gate and one of up.
 struct TiledRows {
@@ -41,150 +47,293 @@ struct TiledRows {
   int row0[2];
 };
 
-template <int FMT, bool A4, int CT>
+// All but the newest N of this wavefront's loads have arrived (a load to LDS with them), then the block's barrier. The
+// stage that is read next is whole when every wavefront has waited for its own loads to it.
+template <int N>
+__device__ __forceinline__ void tiled_barrier() {
+  __builtin_amdgcn_sched_barrier(0);   // nothing of the next tile comes forward: it would wait for loads of that tile here
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// RING: the LDS stages that the activation rows' tiles take in turn.
+template <int FMT, bool A4, int CT, int RING>
 struct TiledPass {
   static constexpr int kSub = MTraits<FMT>::kSub;
-  static constexpr int kSteps = kTileK / MTraits<FMT>::kStepElems;   // steps of a row group per tile: 1 (FP4) or 2 (FP8)
+  static constexpr int kTileElems = MTraits<FMT>::kStepElems;        // elements of k of a tile: 128 (FP4) or 64 (FP8)
+  static constexpr int kUnits = kTileElems / 8;                      // 16-byte units of a staged row
   static constexpr int kCols = CT * kTileCols;
-  static constexpr int kUnits = kCols * 16 / kBlockThreads;          // units of a stage per thread (BF16 rows)
+  static constexpr int kRowLoads = kCols * kUnits / kBlockThreads;   // loads to LDS per thread and tile (BF16 rows)
   static constexpr int kCodeLoads = (kCols * 4 + kBlockThreads - 1) / kBlockThreads;   // 32-code loads per thread (A4)
-  static constexpr int kActRegs = A4 ? kCodeLoads : kUnits;
+  static constexpr int kActRegs = A4 ? kCodeLoads : kRowLoads;
+  static_assert(A4 ? RING == 2 : RING == 2 || RING == 4, "tiles and stages are named in turns of four");
+  static_assert(kRowLoads >= 1 && kRowLoads * kBlockThreads == kCols * kUnits, "whole loads");
 
   struct Regs {          // one tile on its way
+    uint4 w[2];
+    uint32_t s[2];
     uint4 act[A4 ? kCodeLoads : 1];
     uint32_t act_s[A4 ? kCodeLoads : 1];
-    uint4 w[2][kSteps];
-    uint32_t s[2][kSteps];
+  };
+
+  // Weights are asked for row by row - lane l takes 16 bytes of row l / 4 - and pass through LDS of the wavefront's own into
+  // the layout of the matrix core, lane (r, q) quarter q of row r; FP4 scales come for a turn of four tiles at once, a
+  // tile's to a lane, the same way.
+  static constexpr bool kFp4 = FmtTraits<FMT>::kIsFp4;
+  static constexpr int kTileScale = FMT == kFmtNvfp4 ? 8 : 4;   // FP4: bytes of a row's scales of a tile
+  using ScaleWord = std::conditional_t<FMT == kFmtNvfp4, uint2, uint32_t>;
+  struct Exchange {
+    uint4 w[2][64];
+    ScaleWord s[kFp4 ? 2 : 1][kFp4 ? 64 : 1];
   };
 
   const uint8_t* payload[2];
-  uint32_t off[2];
-  ScaleLane sl[2];
+  const uint8_t* scales[2];
+  uint32_t off[2], soff[2];      // bytes: this lane's piece of the row it loads, of the first tile; the scales it loads
+  uint32_t scale_bytes;          // FP4: of the matrix
+  uint32_t row_at[2];            // rows that this lane multiplies
   int cs[2];
-  const uint8_t* act;            // bytes
+  const uint8_t* act;            // bytes; without a row list the pass's first row
   const uint8_t* act_scales;
-  uint32_t act_off[kActRegs];    // 16-byte units from `act`
+  size_t act_off[kActRegs];      // bytes from `act`: the row, and of the row this thread's unit of the first tile
   size_t act_srow[A4 ? kCodeLoads : 1];
-  int k, chunks;
+  int k, chunks, tid;
 
-  __device__ __forceinline__ void load(int tile, Regs& r) const {
-    const int q = (threadIdx.x & (kWave - 1)) >> 4;
-    const bool full = (tile + 1) * kTileK <= k;
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-#pragma unroll
-      for (int s = 0; s < kSteps; ++s) {
-        const int c = (tile * kSteps + s) * 4 + q;
-        typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-        const __attribute__((address_space(1))) u32x4_t* src =
-            (const __attribute__((address_space(1))) u32x4_t*)(uintptr_t)(payload[g] + off[g] + static_cast<uint32_t>(c) * 16u);
-        r.w[g][s] = make_uint4(0u, 0u, 0u, 0u);
-        if (full || c < chunks) {
-          const u32x4_t v = *src;
-          r.w[g][s] = make_uint4(v.x, v.y, v.z, v.w);
-        }
-        r.s[g][s] = load_scale<FMT>(sl[g], tile * kSteps + s, chunks, cs[g]);
-      }
+  // The place of sub-operand j of quarter q in row r of a stage: FP4 quarters at 0, 12, 4 and 8, FP8 ones side by side, the
+  // row's number folded in. (A read instruction takes sixteen lanes at a time: eight rows of one quarter, the other eight
+  // of the next. With the quarters in memory's order those met in pairs for FP4: half of the LDS cycles.)
+  __device__ static __forceinline__ int fold(int r) { return kSub == 4 ? r & 15 : (r >> 1) & 7; }
+  __device__ static __forceinline__ int place(int q, int j, int r) {
+    return (kSub == 4 ? ((q >> 1) ^ ((q & 1) * 3)) * 4 + j : j * 4 + q) ^ fold(r);
+  }
+  __device__ static __forceinline__ int unit_at(int p, int r) {   // the unit of row r that belongs at place p
+    const int at = p ^ fold(r), x = at >> 2;
+    return kSub == 4 ? (((x & 1) * 2) ^ ((x >> 1) * 3)) * 4 + (at & 3) : (at & 3) * 2 + x;
+  }
+
+  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+  template <class T>
+  __device__ static __forceinline__ T global_at(const uint8_t* base, uint32_t byte) {
+    return *(const __attribute__((address_space(1))) T*)(uintptr_t)(base + byte);
+  }
+  // The loads of the walk are buffer loads: the tile's offset is a scalar, a buffer of no bytes is one that reads nothing,
+  // and the compiler counts those to LDS among the others (after a global_load_lds it waits for every load).
+  __device__ static __forceinline__ const uint8_t* uniform(const void* p) {
+    const uint64_t v = reinterpret_cast<uintptr_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+    return reinterpret_cast<const uint8_t*>(static_cast<uintptr_t>(static_cast<uint64_t>(hi) << 32 | lo));
+  }
+  __device__ static __forceinline__ __amdgpu_buffer_rsrc_t buffer(const uint8_t* base, bool live) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, live ? 0xfffffff0u : 0u, 0x00027000);
+  }
+
+  // Block-FP8 scales come in whole words and are taken out of them where they are used: a byte that is carried over a loop as
+  // it was loaded gets its upper bits cleared, and waited for, at the loop's end.
+  __device__ __forceinline__ uint32_t fp8_scale_byte(int g, int tile) const {   // of a block-FP8 piece, from scales[g]
+    const uint32_t col = (static_cast<uint32_t>(tile) * 64u + (static_cast<uint32_t>(tid & 63) >> 4) * 16u) >> cs[g];
+    return soff[g] + col * (FMT == kFmtFp8F32 ? 4u : 1u);
+  }
+  __device__ __forceinline__ uint32_t fp8_scale_word(int g, int tile, bool live) const {
+    uint32_t at = fp8_scale_byte(g, tile);
+    const uint8_t* base = scales[g];
+    if constexpr (FMT == kFmtFp8E8M0) {   // the aligned word that holds the byte
+      const uint32_t low = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(base) & 3u);
+      at = (at + low) & ~3u;
+      base -= low;
     }
-    if constexpr (A4) {
-      const int piece = threadIdx.x & 3;
+    return __builtin_amdgcn_raw_buffer_load_b32(buffer(base, live), at, 0, 0);
+  }
+  __device__ __forceinline__ uint32_t fp8_scale_shift(int g, int tile) const {
+    if constexpr (FMT == kFmtFp8E8M0)
+      return ((fp8_scale_byte(g, tile) + static_cast<uint32_t>(reinterpret_cast<uintptr_t>(scales[g]))) & 3u) * 8u;
+    else return 0u;
+  }
+  __device__ __forceinline__ uint32_t scale_of(int g, int tile, uint32_t word) const {   // ChunkRegs::s
+    if constexpr (FMT == kFmtFp8E8M0) return (word >> fp8_scale_shift(g, tile)) & 0xffu;
+    else return word;
+  }
+
+  // The FP4 scales of the turn that starts at `tile`: this lane's tile of it. Past the matrix's end zeros come, and where a
+  // turn passes the end of k what follows; nobody uses either.
+  __device__ __forceinline__ void load_scales(int tile, ScaleWord (&to)[2]) const {
+    if constexpr (kFp4) {
 #pragma unroll
-      for (int i = 0; i < kCodeLoads; ++i) {
-        r.act[i] = make_uint4(0u, 0u, 0u, 0u);
-        r.act_s[i] = 0u;
-        if (full || tile * kTileK + piece * 32 < k) {
-          r.act[i] = *reinterpret_cast<const uint4*>(act + static_cast<size_t>(act_off[i]) * 16 + tile * 64 + piece * 16);
-          r.act_s[i] = *reinterpret_cast<const uint16_t*>(act_scales + act_srow[i] + tile * 8 + piece * 2);
+      for (int g = 0; g < 2; ++g) {
+        const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(scales[g]), 0, scale_bytes, 0x00027000);
+        if constexpr (FMT == kFmtNvfp4) {
+          typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+          const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(b, soff[g], tile * kTileScale, 0);
+          to[g] = make_uint2(v.x, v.y);
+        } else {
+          to[g] = __builtin_amdgcn_raw_buffer_load_b32(b, soff[g], tile * kTileScale, 0);
         }
       }
     }
   }
-
-  // A tile's BF16 rows, from memory straight to their places in a stage: a wavefront's lanes fill 64 units in a row (four
-  // rows' places), so it is the lane that reads the unit which belongs there. Waited for by the next __syncthreads().
-  __device__ __forceinline__ void stage_rows(int tile, uint4* __restrict__ stage) const {
-    const int u = (threadIdx.x & 15) ^ (threadIdx.x >> 4);   // row % 16 is threadIdx.x / 16 for each of the rows
-    const int place = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWave;
-    if ((tile + 1) * kTileK <= k) {
+  // Lane l writes the 16 bytes that it loaded to place l of a group's region; which piece of row l / 4 that is, is turned by
+  // the row.
+  __device__ static __forceinline__ int turned(int r) { return (0x1320 >> ((r >> 2) & 3) * 4) & 3; }
+  __device__ __forceinline__ void put_scales(Exchange& x, const ScaleWord (&from)[2]) const {
+    if constexpr (kFp4) {
 #pragma unroll
-      for (int i = 0; i < kUnits; ++i)
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) uint32_t*)(uintptr_t)(act + (static_cast<size_t>(act_off[i]) + tile * 16 + u) * 16),
-            (__attribute__((address_space(3))) uint32_t*)(stage + place + i * 256), 16, 0, 0);
-    } else {
+      for (int g = 0; g < 2; ++g) x.s[g][tid & 63] = from[g];
+    }
+  }
+  // A tile's weights, from as they were loaded to as they are multiplied, and its FP4 scales (`at`: which tile of its turn).
+  __device__ __forceinline__ void exchange(Exchange& x, int at, Regs& r) const {
+    const int lane = tid & 63, row = lane & 15, q = lane >> 4;
 #pragma unroll
-      for (int i = 0; i < kUnits; ++i) {
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (tile * kTileK + u * 8 < k)
-          v = *reinterpret_cast<const uint4*>(act + (static_cast<size_t>(act_off[i]) + tile * 16 + u) * 16);
-        stage[threadIdx.x + i * 256] = v;
+    for (int g = 0; g < 2; ++g) x.w[g][lane] = r.w[g];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) r.w[g] = x.w[g][row * 4 + (q ^ turned(row))];
+    if constexpr (kFp4) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const uint8_t* p = reinterpret_cast<const uint8_t*>(x.s[g]) + (row * 4 + at) * kTileScale;
+        if constexpr (FMT == kFmtNvfp4) r.s[g] = *reinterpret_cast<const uint16_t*>(p + q * 2);
+        else r.s[g] = p[q];
       }
+    }
+  }
+
+  // A whole tile's weights and NVFP4 rows into registers, its BF16 rows to a stage. No branch around the loads: the waits
+  // count them. Past the last whole tile they read nothing, and nobody uses it.
+  __device__ __forceinline__ void load(int tile, int full, Regs& r) const {
+    const bool live = tile < full;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(buffer(payload[g], live), off[g], tile * 64, 0);
+      r.w[g] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    if constexpr (!kFp4) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) r.s[g] = fp8_scale_word(g, tile, live);
+    }
+    if constexpr (A4) {
+#pragma unroll
+      for (int i = 0; i < kCodeLoads; ++i) {
+        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(buffer(act, live), static_cast<uint32_t>(act_off[i]), tile * 64, 0);
+        r.act[i] = make_uint4(v.x, v.y, v.z, v.w);
+        r.act_s[i] = __builtin_amdgcn_raw_buffer_load_b32(buffer(act_scales, live), static_cast<uint32_t>(act_srow[i]), tile * 8, 0);
+      }
+    }
+  }
+  // The BF16 rows go from memory to LDS without passing registers: a wavefront's lanes fill 64 places in a row, so it is
+  // the lane that reads the unit which belongs there.
+  __device__ __forceinline__ void stage_rows(int tile, int full, uint4* __restrict__ stage) const {
+    const int first = __builtin_amdgcn_readfirstlane(tid >> 6) * kWave;
+#pragma unroll
+    for (int i = 0; i < kRowLoads; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer(act, tile < full), (__attribute__((address_space(3))) void*)(stage + first + i * kBlockThreads),
+                                               16, static_cast<uint32_t>(act_off[i]), tile * kUnits * 16, 0, 0);
+  }
+
+  // The part of a tile past the last whole one (k is no multiple of it): zeros past the end of the rows.
+  __device__ __forceinline__ void load_rest(int tile, Regs& r) const {
+    const int q = (tid & (kWave - 1)) >> 4;
+    const bool inside = tile * 4 + q < chunks;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      r.w[g] = make_uint4(0u, 0u, 0u, 0u);
+      r.s[g] = 0u;
+      if (inside) {
+        const u32x4_t v = global_at<u32x4_t>(payload[g] + static_cast<size_t>(tile) * 64, row_at[g] * static_cast<uint32_t>(kFp4 ? k / 2 : k) + q * 16u);
+        r.w[g] = make_uint4(v.x, v.y, v.z, v.w);
+        const uint32_t at = row_at[g] * static_cast<uint32_t>(k / (FMT == kFmtNvfp4 ? 16 : 32)) + static_cast<uint32_t>(tile) * kTileScale;
+        if constexpr (FMT == kFmtFp8F32) r.s[g] = fp8_scale_word(g, tile, true);
+        else if constexpr (FMT == kFmtNvfp4) r.s[g] = global_at<uint16_t>(scales[g], at + q * 2);
+        else if constexpr (FMT == kFmtMxfp4) r.s[g] = global_at<uint8_t>(scales[g], at + q);
+        else r.s[g] = static_cast<uint32_t>(global_at<uint8_t>(scales[g], fp8_scale_byte(g, tile))) << fp8_scale_shift(g, tile);
+      }
+    }
+    if constexpr (A4) {
+      const int piece = tid & 3;
+#pragma unroll
+      for (int i = 0; i < kCodeLoads; ++i) {
+        r.act[i] = make_uint4(0u, 0u, 0u, 0u);
+        r.act_s[i] = 0u;
+        if (tile * kTileElems + piece * 32 < k) {
+          r.act[i] = *reinterpret_cast<const uint4*>(act + act_off[i] + tile * 64);
+          r.act_s[i] = static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(act_scales + act_srow[i] + tile * 8 + (piece & 1) * 2)) << (piece & 1) * 16;
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void stage_rest(int tile, uint4* __restrict__ stage) const {
+    const int u = unit_at(tid % kUnits, tid / kUnits);
+#pragma unroll
+    for (int i = 0; i < kRowLoads; ++i) {
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (tile * kTileElems + u * 8 < k)
+        v = *reinterpret_cast<const uint4*>(act + act_off[i] + tile * kUnits * 16);
+      stage[tid + i * kBlockThreads] = v;
     }
   }
 
   __device__ __forceinline__ void commit(uint4* __restrict__ stage, const Regs& r) const {
     if constexpr (A4) {
-      const int piece = threadIdx.x & 3;
+      const int piece = tid & 3;
 #pragma unroll
       for (int i = 0; i < kCodeLoads; ++i) {
-        const int row = (threadIdx.x >> 2) + i * (kBlockThreads / 4);
+        const int row = (tid >> 2) + i * (kBlockThreads / 4);
         if (kCols * 4 >= kBlockThreads || row < kCols) {
           ChunkRegs ch;
           ch.w = r.act[i];
-          ch.s = r.act_s[i];
+          ch.s = r.act_s[i] >> (piece & 1) * 16;
           FragH f[4];
           decode_frags_nvfp4_f16(ch, f);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) stage[row * 16 + ((piece * 4 + j) ^ (row & 15))] = __builtin_bit_cast(uint4, f[j].v);
+          for (int j = 0; j < 4; ++j) stage[row * kUnits + place(piece, j, row)] = __builtin_bit_cast(uint4, f[j].v);
         }
       }
     }
   }
 
-  __device__ __forceinline__ void multiply(const uint4* __restrict__ stage, const uint4 (&w)[2][kSteps],
-                                           const uint32_t (&sc)[2][kSteps], f32x4_t (&acc)[2][CT]) const {
-    const int lane = threadIdx.x & (kWave - 1), c = lane & 15, q = lane >> 4;
+  // The products of a tile. The operands from LDS are asked for kAhead products early, in an order that the compiler is held
+  // to: left alone it reads one, waits for it and uses it, with one other wavefront on the SIMD to cover the wait.
+  static constexpr int kAhead = CT < 4 ? CT * 2 : 4;
+  template <class Middle>
+  __device__ __forceinline__ void multiply(int tile, const uint4* __restrict__ stage, const Regs& r, f32x4_t (&acc)[2][CT], Middle middle) const {
+    const int lane = tid & (kWave - 1), c = lane & 15, q = lane >> 4;
+    using F = std::conditional_t<A4, FragH, Frag>;
+    F f[2][kSub];
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
+    for (int g = 0; g < 2; ++g) {
+      ChunkRegs ch;
+      ch.w = r.w[g];
+      ch.s = scale_of(g, tile, r.s[g]);
+      if constexpr (A4) decode_frags_nvfp4_f16(ch, f[g]);
+      else decode_frags<FMT>(ch, f[g]);
+    }
+    const uint4* at[kSub];
+#pragma unroll
+    for (int j = 0; j < kSub; ++j) at[j] = stage + c * kUnits + place(q, j, c);
+    constexpr int kReads = kSub * CT;
+    uint4 b[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) b[i] = at[i / CT][i % CT * kTileCols * kUnits];
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) {
+      const int j = i / CT, t = i % CT, n = i + kAhead;
+      if (i == kReads / 2) middle();
       if constexpr (A4) {
-        FragH f[2][kSub];
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          ChunkRegs ch;
-          ch.w = w[g][s];
-          ch.s = sc[g][s];
-          decode_frags_nvfp4_f16(ch, f[g]);
-        }
-#pragma unroll
-        for (int j = 0; j < kSub; ++j) {
-          const uint4* at = stage + c * 16 + (((s * 4 + q) * kSub + j) ^ c);
-#pragma unroll
-          for (int t = 0; t < CT; ++t) {
-            const uint4 b = at[t * 256];
-            acc[0][t] = mfma_f16(f[0][j], b, acc[0][t]);
-            acc[1][t] = mfma_f16(f[1][j], b, acc[1][t]);
-          }
-        }
+        acc[0][t] = mfma_f16(f[0][j], b[i % kAhead], acc[0][t]);
+        acc[1][t] = mfma_f16(f[1][j], b[i % kAhead], acc[1][t]);
       } else {
-        Frag f[2][kSub];
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          ChunkRegs ch;
-          ch.w = w[g][s];
-          ch.s = sc[g][s];
-          decode_frags<FMT>(ch, f[g]);
-        }
-#pragma unroll
-        for (int j = 0; j < kSub; ++j) {
-          const uint4* at = stage + c * 16 + (((s * 4 + q) * kSub + j) ^ c);
-#pragma unroll
-          for (int t = 0; t < CT; ++t) {
-            const uint4 b = at[t * 256];
-            acc[0][t] = mfma_bf16(f[0][j], b, acc[0][t]);
-            acc[1][t] = mfma_bf16(f[1][j], b, acc[1][t]);
-          }
-        }
+        acc[0][t] = mfma_bf16(f[0][j], b[i % kAhead], acc[0][t]);
+        acc[1][t] = mfma_bf16(f[1][j], b[i % kAhead], acc[1][t]);
       }
+      if (n < kReads) b[i % kAhead] = at[n / CT][n % CT * kTileCols * kUnits];
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);   // reads from LDS
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) {
+      if (i == kReads / 2) {
+        __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);    // the middle's writes to LDS and reads from it
+        __builtin_amdgcn_sched_group_barrier(0x100, kFp4 ? 4 : 2, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);      // products
+      if (i + kAhead < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   }
 
@@ -192,61 +341,52 @@ struct TiledPass {
   // Rows from mt on repeat row mt - 1; their sums are not stored. Every thread of the block must call.
   __device__ __forceinline__ void run(const TiledRows& rows, int n, int k_, const uint8_t* act_, size_t act_stride_bytes,
                                       const int32_t* act_rows, int act_row0, int mt, const A4Src& a4, const MGeom& g,
-                                      uint4* __restrict__ lds0, uint4* __restrict__ lds1, f32x4_t (&sum)[2][CT]) {
-    const int lane = threadIdx.x & (kWave - 1);
+                                      uint4* __restrict__ s0, uint4* __restrict__ s1, uint4* __restrict__ s2,
+                                      uint4* __restrict__ s3, Exchange& __restrict__ x, f32x4_t (&sum)[2][CT]) {
+    // A loop over passes would otherwise keep what every width computes from the thread's number in registers around all of them.
+    tid = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & (kWave - 1), q = lane >> 4;
     k = k_;
     chunks = k / MTraits<FMT>::kLoadElems;
-    act = act_;
-    act_scales = a4.scales;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int r = min(rows.row0[i] + (lane & 15), n - 1);   // rows past the end redo the last row
-      payload[i] = rows.mat[i].payload;
-      off[i] = static_cast<uint32_t>(r) * static_cast<uint32_t>(FmtTraits<FMT>::kIsFp4 ? k / 2 : k);
-      sl[i] = scale_lane<FMT>(rows.mat[i], rows.row0[i], n, k);
+      payload[i] = uniform(rows.mat[i].payload);
+      scales[i] = uniform(rows.mat[i].scales);
       cs[i] = rows.mat[i].cs;
+      // rows past the end redo the last row
+      const uint32_t r = static_cast<uint32_t>(min(rows.row0[i] + (lane >> 2), n - 1));
+      row_at[i] = static_cast<uint32_t>(min(rows.row0[i] + (lane & 15), n - 1));
+      off[i] = r * static_cast<uint32_t>(kFp4 ? k / 2 : k) + static_cast<uint32_t>((lane & 3) ^ turned(lane >> 2)) * 16u;
+      if constexpr (kFp4) soff[i] = r * static_cast<uint32_t>(k / (FMT == kFmtNvfp4 ? 16 : 32)) + static_cast<uint32_t>(lane & 3) * kTileScale;
+      else soff[i] = (row_at[i] >> rows.mat[i].rs) * ((static_cast<uint32_t>(k) + (1u << cs[i]) - 1) >> cs[i]) * (FMT == kFmtFp8F32 ? 4u : 1u);
     }
+    scale_bytes = static_cast<uint32_t>(n) * static_cast<uint32_t>(k / (FMT == kFmtNvfp4 ? 16 : 32));
+    act = uniform(act_ + (act_rows ? 0 : static_cast<size_t>(act_row0) * act_stride_bytes));
+    if constexpr (A4) act_scales = uniform(a4.scales + (act_rows ? 0 : static_cast<size_t>(act_row0) * a4.scale_stride));
 #pragma unroll
     for (int i = 0; i < kActRegs; ++i) {
-      const int c = min(A4 ? static_cast<int>(threadIdx.x >> 2) + i * (kBlockThreads / 4) : static_cast<int>(threadIdx.x >> 4) + i * 16,
-                        mt - 1);
-      const size_t row = act_rows ? static_cast<size_t>(act_rows[c]) : static_cast<size_t>(act_row0 + c);
-      act_off[i] = static_cast<uint32_t>(row * act_stride_bytes >> 4);
-      if constexpr (A4) act_srow[i] = row * a4.scale_stride;
+      const int c = min(A4 ? (tid >> 2) + i * (kBlockThreads / 4) : tid / kUnits + i * (kBlockThreads / kUnits), mt - 1);
+      const size_t row = static_cast<size_t>(act_rows ? act_rows[c] : c);
+      if constexpr (A4) {
+        act_off[i] = row * act_stride_bytes + (tid & 3) * 16;
+        act_srow[i] = row * a4.scale_stride + (tid & 2) * 2;
+      } else {
+        act_off[i] = row * act_stride_bytes + unit_at(tid % kUnits, tid / kUnits) * 16;   // rows 256 / kUnits apart fold alike
+      }
     }
-    const int tiles = (g.steps + kSteps - 1) / kSteps;
-    const int part_tiles = g.part_steps / kSteps;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int t = 0; t < CT; ++t) sum[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // A buffer load reaches 4 GB: a pass with a row that ends beyond takes the way of the last part of k all along.
+    bool far = false;
+    for (int c = lane; c < mt; c += kWave) {
+      const size_t row = static_cast<size_t>(act_rows ? act_rows[c] : c);
+      far = far || row * act_stride_bytes + static_cast<size_t>(k) * 2 > 0xfffffff0u || (A4 && row * a4.scale_stride + k > 0xfffffff0u);
+    }
+    const int full = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(far) != 0 ? 0 : k / kTileElems), part_tiles = g.part_steps;
     f32x4_t acc[2][CT];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int t = 0; t < CT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    Regs pre;
-    load(0, pre);
-    if constexpr (!A4) stage_rows(0, lds0);
-    auto step = [&](int t, uint4* __restrict__ cur, uint4* __restrict__ other) {
-      if constexpr (A4) commit(cur, pre);
-      else __syncthreads();   // `cur` is whole, and its wavefronts are done with `other`
-      uint4 w[2][kSteps];
-      uint32_t sc[2][kSteps];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-          w[i][s] = pre.w[i][s];
-          sc[i][s] = pre.s[i][s];
-        }
-      if (t + 1 < tiles) {
-        load(t + 1, pre);
-        if constexpr (!A4) stage_rows(t + 1, other);
-      }
-      if constexpr (A4) __syncthreads();   // the stage is whole; its readers of two tiles before passed the barrier of the tile between
-      multiply(cur, w, sc, acc);
-    };
+      for (int t = 0; t < CT; ++t) acc[i][t] = sum[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto add_part = [&](bool first) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
@@ -256,31 +396,94 @@ struct TiledPass {
           acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
     };
-    if constexpr (A4) {
-      // Codes pass registers, so a stage is chosen by parity; the parts in a loop of their own keep 6 registers more free
-      // than the flat loop below (256 experts, 6144 x 2048, 12 / 16 / 60 rows a segment: 2358 -> 2097, 2393 -> 2136, 3364
-      // -> 3178 us a layer).
-      for (int t0 = 0; t0 < tiles; t0 += part_tiles) {
-        const int t1 = min(tiles, t0 + part_tiles);
-        for (int t = t0; t < t1; ++t) step(t, t & 1 ? lds1 : lds0, nullptr);
-        add_part(t0 == 0);
+    Regs r0, r1, r2, r3;
+    ScaleWord sraw[2];
+    constexpr int kDeep = A4 && CT == 8 ? 2 : 3;   // tiles of weights on their way; a third of the widest with codes would spill
+    // One tile: its stage is whole and the one that is filled next is free after the barrier. Of a wavefront's loads
+    // those may still be on their way then that are younger than its loads to the stage: the weights (and block-FP8 scales)
+    // that followed those, and what the RING - 2 steps between asked for. (The FP4 scales of a turn are not counted: where
+    // they are among them, up to two fewer may be left.)
+    constexpr int kTileLoads = kFp4 ? 2 : 4;
+    constexpr int kYounger = kTileLoads + (RING - 2) * (kRowLoads + kTileLoads);
+    auto step = [&](int t, auto at, const uint4* __restrict__ cur, uint4* __restrict__ next, const Regs& now, Regs& coming, Regs& far) {
+      constexpr int kAt = decltype(at)::value;   // in its turn
+      if constexpr (A4) {
+        tiled_barrier<63>();
+      } else {
+        tiled_barrier<kYounger>();
+        stage_rows(t + RING - 1, full, next);
+        asm volatile("" ::: "memory");   // the weights are asked for after the rows: kYounger
       }
-    } else {
-      int part_end = min(tiles, part_tiles);
-      auto ends = [&](int done) {
-        if (done != part_end) return false;
-        add_part(part_end <= part_tiles);
-        part_end = min(tiles, part_end + part_tiles);
-        return done == tiles;
+      load(t + kDeep, full, far);
+      if constexpr (kAt == 0) load_scales(t + 4, sraw);
+      if constexpr (A4) commit(next, coming);
+      multiply(t, cur, now, acc, [&] {
+        if constexpr (kAt == 3) put_scales(x, sraw);
+        exchange(x, (kAt + 1) & 3, coming);
+      });
+    };
+    if (full > 0) {
+      if constexpr (A4) {
+        load(0, full, r0);
+        load(1, full, r1);
+        if constexpr (kDeep == 3) load(2, full, r2);
+        commit(s0, r0);
+        load_scales(0, sraw);
+      } else if constexpr (RING == 2) {
+        load_scales(0, sraw);
+        load(0, full, r0);
+        load(1, full, r1);
+        asm volatile("" ::: "memory");
+        stage_rows(0, full, s0);
+        asm volatile("" ::: "memory");
+        load(2, full, r2);
+      } else {
+        uint4* const st[3] = {s0, s1, s2};
+        Regs* const reg[3] = {&r0, &r1, &r2};
+        load_scales(0, sraw);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          stage_rows(t, full, st[t]);
+          asm volatile("" ::: "memory");
+          load(t, full, *reg[t]);
+          asm volatile("" ::: "memory");
+        }
+      }
+      put_scales(x, sraw);
+      exchange(x, 0, r0);
+      // The stages and the tiles by name, in turns of four, and one way out of the loop: the compiler then waits for what a
+      // step reads and no more.
+      int t = 0, part_end = part_tiles;
+      auto turn = [&](int steps) {   // `steps` is a constant where this is inlined, or the last turn's
+        step(t, std::integral_constant<int, 0>{}, s0, RING == 2 ? s1 : s3, r0, r1, kDeep == 2 ? r2 : r3);
+        if (steps == 1) return;
+        step(t + 1, std::integral_constant<int, 1>{}, s1, s0, r1, r2, kDeep == 2 ? r3 : r0);
+        if (steps == 2) return;
+        step(t + 2, std::integral_constant<int, 2>{}, RING == 2 ? s0 : s2, s1, r2, r3, kDeep == 2 ? r0 : r1);
+        if (steps == 3) return;
+        step(t + 3, std::integral_constant<int, 3>{}, RING == 2 ? s1 : s3, RING == 2 ? s0 : s2, r3, r0, kDeep == 2 ? r1 : r2);
       };
-      for (int t = 0;;) {   // the stages by name: the compiler then knows that a read of one need not wait for loads to the other
-        step(t, lds0, lds1);
-        if (ends(++t)) break;
-        step(t, lds1, lds0);
-        if (ends(++t)) break;
+      for (; t + 4 <= full;) {
+        turn(4);
+        t += 4;
+        if (t == part_end) {   // parts are whole turns
+          add_part(t == part_tiles);
+          part_end += part_tiles;
+        }
       }
+      if (t < full) turn(full - t);
+      tiled_barrier<0>();   // nothing is on its way to a stage, and no wavefront reads one
     }
-    __syncthreads();   // the stages are free for the next pass
+    for (int t = full; t < g.steps; ++t) {
+      load_rest(t, r0);
+      if constexpr (A4) commit(s0, r0);
+      else stage_rest(t, s0);
+      __syncthreads();
+      multiply(t, s0, r0, acc, [] {});
+      __syncthreads();
+      if ((t + 1) % part_tiles == 0 || t + 1 == g.steps) add_part(t < part_tiles);
+    }
+    if (full == g.steps && full % part_tiles != 0) add_part(full < part_tiles);
   }
 };
 
@@ -322,15 +525,25 @@ struct TiledOut {
   float limit;
   const float* a4_gs;
 };
+// A block's LDS stages, as large as the widest pass wants them: four, two where the rows pass registers (A4) and where four
+// would leave room for one block per CU.
+template <int FMT, bool A4>
+struct TiledStages {
+  static constexpr int kUnits = kTiledCols * MTraits<FMT>::kStepElems / 8;
+  static constexpr int kRing = A4 || kUnits > 1024 ? 2 : 4;
+  uint4 *s0, *s1, *s2, *s3;
+  typename TiledPass<FMT, A4, 8, kRing>::Exchange* x;   // of each wavefront
+};
 template <int FMT, bool GU, bool A4, int CT>
 __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
-                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds0,
-                                           uint4* __restrict__ lds1) {
-  TiledPass<FMT, A4, CT> pass;
+                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o,
+                                           const TiledStages<FMT, A4>& st) {
+  TiledPass<FMT, A4, CT, TiledStages<FMT, A4>::kRing> pass;
   f32x4_t sum[2][CT];
-  pass.run(rows, n, k, act, act_stride_bytes, act_rows, act_row0, mt, a4, g, lds0, lds1, sum);
-  const int lane = threadIdx.x & (kWave - 1);
+  pass.run(rows, n, k, act, act_stride_bytes, act_rows, act_row0, mt, a4, g, st.s0, st.s1, st.s2, st.s3,
+           reinterpret_cast<typename TiledPass<FMT, A4, CT, TiledStages<FMT, A4>::kRing>::Exchange&>(st.x[threadIdx.x >> 6]), sum);
+  const int lane = pass.tid & (kWave - 1);
   const bool vec = ((reinterpret_cast<uintptr_t>(o.out) | (GU ? reinterpret_cast<uintptr_t>(o.out_up) : 0)) & 15u) == 0 &&
                    (o.out_stride & 3u) == 0;
 #pragma unroll
@@ -376,15 +589,23 @@ __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&
 template <int FMT, bool GU, bool A4>
 __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
-                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o, uint4* __restrict__ lds0,
-                                           uint4* __restrict__ lds1) {
+                                           int mt, const A4Src& a4, const MGeom& g, const TiledOut& o,
+                                           const TiledStages<FMT, A4>& st) {
   if (mt > 64)
-    tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
+    tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
   else if (mt > 32)
-    tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
+    tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
   else
-    tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, lds0, lds1);
+    tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
 }
+
+// The kernel's stages and exchange regions, by name.
+#define DGPP_TILED_STAGES(st, FMT, A4)                                                                               \
+  using Stages = TiledStages<FMT, A4>;                                                                               \
+  __shared__ uint4 stage0[Stages::kUnits], stage1[Stages::kUnits];                                                   \
+  __shared__ uint4 stage2[Stages::kRing == 4 ? Stages::kUnits : 1], stage3[Stages::kRing == 4 ? Stages::kUnits : 1]; \
+  __shared__ typename TiledPass<FMT, A4, 8, Stages::kRing>::Exchange exchange[kWavesPerBlock];                       \
+  const Stages st = {stage0, stage1, stage2, stage3, exchange}
 
 // Consecutive workgroups go to the eight XCDs in turn. Blocks of one segment share its activation rows and blocks of one
 // row tile its weights, so the linear index is dealt such that an XCD (its own L2) keeps a segment's row tiles, or a row
@@ -449,7 +670,7 @@ static_assert(kXcds == 8, "the shifts above");
 
 template <int FMT, bool GU, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, TiledDeal deal) {
-  __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
+  DGPP_TILED_STAGES(st, FMT, A4);
   const TiledPlace at = tiled_place(deal, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y));
   if (at.seg < 0) return;
   const DgppMoeSegment seg = a.segs[at.seg];
@@ -472,15 +693,15 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(Grouped
   for (int c0 = first_pass; c0 < seg.rows; c0 += at.slots * kTiledCols) {
     const int first = seg.row0 + c0;
     tiled_rows<FMT, GU, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
-                            a.act_rows ? a.act_rows + first : nullptr, first, static_cast<size_t>(first),
-                            min(kTiledCols, seg.rows - c0), src, g, o, lds0, lds1);
+                                   a.act_rows ? a.act_rows + first : nullptr, first, static_cast<size_t>(first),
+                                   min(kTiledCols, seg.rows - c0), src, g, o, st);
   }
 }
 
 // grid.x = kXcds * ceil(row tiles / kXcds) * column passes.
 template <int FMT, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs a, MGeom g, int row_tiles, int passes) {
-  __shared__ uint4 lds0[kTiledStage], lds1[kTiledStage];
+  DGPP_TILED_STAGES(st, FMT, A4);
   const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
   const int tile = idx / passes * kXcds + lin % kXcds, c0 = idx % passes * kTiledCols;
   if (tile >= row_tiles) return;
@@ -498,7 +719,7 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
   src.scale_stride = a.a4_scale_stride;
   const TiledOut o = {a.out, nullptr, a.out_stride, a.out_f32, 0, 0.f, a.a4_gs};
   tiled_rows<FMT, false, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
-                             nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, lds0, lds1);
+                                    nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, st);
 }
 
 }  // namespace dgpp_amd

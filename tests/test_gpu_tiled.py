@@ -258,3 +258,24 @@ def test_a_layer_with_an_mxfp8_shared_expert_does_not_depend_on_its_projections_
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][0], got[2][0])
     assert got[1][1] - got[0][1] == 3 and got[2][1] == got[1 if T == 200 else 0][1]
     layer.close()
+
+
+@pytest.mark.parametrize("kind", ["fp8", "mxfp4"])
+def test_activation_rows_beyond_four_gigabytes(gpu, kind):
+    """Rows that a buffer load does not reach, alone in a pass and beside near ones, and rows that end at its edge."""
+    import torch
+    H, I, E, T = 1152, 576, 2, 1_900_000
+    if T * H * 2 * 1.1 > torch.cuda.mem_get_info()[0]:
+        pytest.skip("not enough memory")
+    p = moe_data.make_problem(E, H, I, 1, 4, kind, 5, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    edge = (1 << 32) // (2 * H)
+    rows = np.array([0, 1, edge - 2, edge - 1] + [edge, edge + 1, T - 1, 3], np.int32)
+    x = torch.empty((T, H), dtype=torch.bfloat16, device=d.x.device)
+    x[torch.from_numpy(rows).long().to(x.device)] = dev(hg.normal_bf16(0x99, (len(rows), H))).view(torch.bfloat16)
+    segs = dev(np.array([[0, 3, 0], [3, 5, 1]], np.int32))
+    act = dev_empty((len(rows), I), np.uint16)
+    gu = L.launch_moe_grouped_mma_gate_up_swiglu if kind == "fp8" else L.launch_moe_grouped_mma_gate_up_swiglu_fp4
+    more = () if kind == "fp8" else (d.fp4_group,)
+    idx = dev(rows)
+    same(lambda: gu(x, H, segs, E, 5, 0, d.views, act, I, I, H, 7.0, None, idx, *more), kind, act)
