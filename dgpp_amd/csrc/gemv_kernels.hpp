@@ -1199,9 +1199,9 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
   const MGeom g = mgeom<FMT>(a.k);
   const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
   const int row_tiles = (a.n + block_rows - 1) / block_rows;
-  const TiledDeal deal = tiled_deal(n_segs, a.long_segs, row_tiles, max_rows, tune_get(kTuneTiledPasses));
+  const TiledPlan plan = tiled_plan(n_segs, a.long_segs, row_tiles, max_rows, a.total_rows, tune_get(kTuneTiledPasses));
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(deal.grid_x(), deal.grid_y()), dim3(kBlockThreads), 0, stream, a, g, deal);
+    hipLaunchKernelGGL(kern, plan.grid(), dim3(kBlockThreads), 0, stream, a, g, plan);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {

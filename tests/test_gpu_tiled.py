@@ -260,6 +260,29 @@ def test_a_layer_with_an_mxfp8_shared_expert_does_not_depend_on_its_projections_
     layer.close()
 
 
+@pytest.mark.parametrize("kind", ["fp8", "mxfp4", "nvfp4", "w4a4"])
+@pytest.mark.parametrize("E,T,K", [(70, 301, 5), (300, 700, 3)])
+def test_sorted_passes_of_a_skewed_table_are_bitwise_the_16_row_form(gpu, kind, E, T, K):
+    """A table of passes enough to be sorted by width: an expert with all tokens, some with 33 to 128, with fewer and with
+    none; more segments than a block has threads."""
+    p = moe_data.make_problem(E, 512, 512, K, T, "nvfp4" if kind == "w4a4" else kind, 31 + E, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    layer = make_layer(p, d, L.ROUTER_SOFTMAX_TOPK, 1.0, T)
+    rng = np.random.default_rng(E)
+    popular = 1.0 / np.arange(1, E - 9) ** 1.1      # the last ten have no rows
+    ids = np.stack([np.concatenate([[0], 1 + rng.choice(E - 10, K - 1, replace=False, p=popular / popular.sum())]) for _ in range(T)])
+    counts = np.bincount(ids.reshape(-1), minlength=E)
+    assert counts[0] == T and (counts == 0).any() and ((counts > 64) & (counts <= 128)).any() and ((counts > 0) & (counts <= 32)).any()
+    ids_d = dev(ids.astype(np.int32))
+    w = dev(rng.uniform(0.1, 1.0, (T, K)).astype(np.float32))
+    out = dev_empty((T, 512), np.uint16)
+    if kind == "w4a4":
+        same(lambda: layer.enqueue_prefill_routed_w4a4(d.x, 512, ids_d, w, out, T), kind, out, tiled=3)
+    else:
+        same(lambda: layer.enqueue_prefill_routed(d.x, 512, ids_d, w, out, T), kind, out, tiled=2)
+    layer.close()
+
+
 @pytest.mark.parametrize("kind", ["fp8", "mxfp4"])
 def test_activation_rows_beyond_four_gigabytes(gpu, kind):
     """Rows that a buffer load does not reach, alone in a pass and beside near ones, and rows that end at its edge."""
