@@ -181,9 +181,15 @@ namespace {
 //   matrices of 64 M weights from four (FP8) or five (FP4) rows on; otherwise only matrices of 64 M weights and
 //   more, from five rows on;
 // * up to four rows (three of a large matrix): the vector core.
+// `streams`: the rows are whole 16-byte vectors, which the streaming form of the matrix core (stream_dense_kernel) reads: its
+// time hardly grows with the rows, the vector core's by a dot chain per row. Measured, us, vector core -> streaming, five
+// rows: 4096 x 4096, NVFP4 9.5 -> 7.7, MXFP4 8.7 -> 5.5, block FP8 12.7 -> 7.7; 6144 x 5120 13.9 -> 9.7, 13.0 -> 7.5, 21.4 -> 9.2: from five rows
+// on for 16 M weights. Smaller matrices and fewer rows would gain less or nothing (4096 x 1024, 8 rows 8.7 -> 7.8 and 7.2 -> 8.0) and keep
+// the bits that the vector core's fused launches share with it.
 constexpr int kVectorPassRows = kMaxActRows;
-bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool have_ws, int from_rows) {
+bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool have_ws, int from_rows, bool streams) {
   if (m > kVectorPassRows || m > max_stage_rows(k)) return true;
+  if (streams && m >= 5 && k >= 4096 && static_cast<size_t>(n) * static_cast<size_t>(k) >= (16u << 20)) return true;
   if (from_rows > 0 && m >= from_rows) return true;   // the caller's own boundary (the reference's mma_from_rows)
   const size_t weights = static_cast<size_t>(n) * static_cast<size_t>(k);
   int parts = 1;
@@ -209,7 +215,7 @@ int dense_rows(int fmt, const uint16_t* act, size_t act_stride, const MatRef& ma
                size_t out_stride, int out_f32, int m, int n, int k, hipStream_t stream, const char* who, int from_rows,
                void* ws = nullptr, size_t ws_bytes = 0, bool beside = false) {
   const int core = tune_get(kTuneCore);   // bench switch: 1 pins the vector core, 2 the matrix core
-  if (core != 1 && (core == 2 || dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, from_rows))) {
+  if (core != 1 && (core == 2 || dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, from_rows, rows_stream(act, act_stride)))) {
     if ((m + kTileCols - 1) / kTileCols > 65535) return fail_arg(std::string(who) + ": grid dimension overflow");
     DenseArgs a;
     a.act = act;
@@ -1212,7 +1218,7 @@ static int mma_gemv_fp8(const uint16_t* act, size_t act_stride, const uint8_t* p
                         void* stream, const char* who) {
   if (m <= 0 || n <= 0) return DGPP_OK;
   const int fmt = e8m0 ? kFmtFp8E8M0 : kFmtFp8F32;
-  if (tune_get(kTuneCore) == 2 || k <= 0 || (tune_get(kTuneCore) != 1 && dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, 0)))
+  if (tune_get(kTuneCore) == 2 || k <= 0 || (tune_get(kTuneCore) != 1 && dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, 0, rows_stream(act, act_stride))))
     return dense_mma_fp8(act, act_stride, payload, scales, e8m0, out, out_f32, m, n, k, out_stride, rs, cs, ws, ws_bytes, stream,
                          who);
   if (!act || !payload || !scales || !out) return fail_arg(std::string(who) + ": null pointer");
@@ -1266,11 +1272,11 @@ int dgpp_launch_mma_gemv_fp8_bf16_pair(const uint16_t* a0, const uint8_t* w0, co
   // Each problem takes the core its single launch would take (so that its bits are that launch's): both on the vector
   // core -> one vector-core launch over both; both on the matrix core -> one matrix-core launch; one each -> two launches.
   const int core = tune_get(kTuneCore);
-  auto takes_mma = [&](int n) {
+  auto takes_mma = [&](const uint16_t* act, int n) {
     if (core == 2) return true;
-    return dense_takes_matrix_core(kFmtFp8F32, m, n, k, ws_bytes, ws != nullptr, 0);
+    return dense_takes_matrix_core(kFmtFp8F32, m, n, k, ws_bytes, ws != nullptr, 0, rows_stream(act, act_stride));
   };
-  const bool mma0 = takes_mma(n0), mma1 = takes_mma(n1);
+  const bool mma0 = takes_mma(a0, n0), mma1 = takes_mma(a1, n1);
   if (mma0 != mma1 || core == 1) {   // (the bench switch that pins the vector core: the single launchers know how)
     const int rc = dgpp_launch_mma_gemv_fp8_bf16(a0, act_stride, w0, s0, o0, m, n0, k, stride0, rs, cs, stream, ws, ws_bytes);
     if (rc != DGPP_OK) return rc;

@@ -1067,6 +1067,11 @@ inline int max_stage_rows(int k) {
   return static_cast<int>(fit < 1 ? 1 : (fit > kMaxActRows ? kMaxActRows : fit));
 }
 
+// Whether the streaming form reads such rows: whole 16-byte vectors, sixteen rows within the reach of a buffer load.
+inline bool rows_stream(const uint16_t* act, size_t act_stride) {
+  return (reinterpret_cast<uintptr_t>(act) & 15u) == 0 && (act_stride & 7u) == 0 && act_stride < (1u << 26);
+}
+
 // Blocks of the 16-row dense form: 64 weight rows x 16 activation rows each.
 inline size_t dense_mfma_tiles(int m, int n) {
   return static_cast<size_t>((n + 63) / 64) * static_cast<size_t>((m + 15) / 16);
@@ -1174,6 +1179,19 @@ inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
   return grouped_fills_tiles(FMT, a.a4_scales != nullptr, a.gate_up != 0, n_segs, a.k, a.max_rows, a.total_rows, a.long_segs);
 }
 
+// Where the tiles do not take the launch, the plain product streams its weights (stream_dense_kernel). Measured, us, the
+// forms before it (parts side by side, over a workspace, row tiles) -> streaming, NVFP4, MXFP4, block FP8: 512 x 4096, 20 rows 15.0 ->
+// 8.0, 13.6 -> 6.0, 13.6 -> 8.0; 4096 x 4096, 20 rows 15.1 -> 8.8, 14.0 -> 6.6, 14.1 -> 8.8, 100 rows 26.8 -> 19.2, 26.0 -> 15.3, 28.2 -> 19.7;
+// 17408 x 5120, 6 rows 26.0 -> 21.6, 28.4 -> 18.8, 27.8 -> 29.0, 64 rows 74 -> 51, 77 -> 45, 72 -> 61; 16000 x 1024, 32 rows 10.6 -> 8.3, 11.2 ->
+// 6.4, 11.5 -> 8.9. Two corners stay as they were: block FP8 of up to eight rows just over one round of the chip (17408 rows
+// above), and NVFP4 with one part of K and few blocks (4096 x 1024, 20 rows 7.7 against 8.4). `act_up` and rows that are no
+// whole 16-byte vectors have no streaming form. Bench / test switch 11: 0, or one of the other forms.
+template <int FMT>
+inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g) {
+  if (tune_get(kTuneTeams) != 0 || a.act_up != nullptr || a.a4_scales != nullptr || !rows_stream(a.act, a.act_stride)) return false;
+  if (FMT == kFmtFp8F32 && dense_mfma_team_row_groups(g.parts, a.m, a.n, true) == 2) return false;
+  return !(FMT == kFmtNvfp4 && g.parts == 1 && a.m > kTileCols && dense_mfma_tiles(a.m, a.n) <= 256);
+}
 template <int FMT>
 hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
   note_tiled_launch();
@@ -1218,6 +1236,13 @@ template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
   if (dense_takes_tiled<FMT>(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
+  if (dense_takes_stream<FMT>(a, g)) {
+    const int rows = kWavesPerBlock / g.parts * 2 * kGroupRows, col_tiles = (a.m + kTileCols - 1) / kTileCols;
+    const dim3 grid(static_cast<unsigned>(((a.n + rows - 1) / rows + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(col_tiles));
+    if (a.m <= 8) hipLaunchKernelGGL((stream_dense_kernel<FMT, 8>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
+    else hipLaunchKernelGGL((stream_dense_kernel<FMT, 16>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
+    return hipGetLastError();
+  }
   const unsigned gx = static_cast<unsigned>((a.n + 63) / 64), gy = static_cast<unsigned>((a.m + kTileCols - 1) / kTileCols);
   const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
   const bool split = ws != nullptr && ws_bytes >= need && dense_mfma_would_split(g.parts, a.m, a.n) && a.a4_scales == nullptr;

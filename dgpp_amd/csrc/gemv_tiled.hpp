@@ -338,16 +338,8 @@ struct TiledPass {
     }
   }
 
-  // `sum` receives the wavefront's two row groups against mt activation rows (row c: act_rows[c] when given, else c).
-  // Rows from mt on repeat row mt - 1; their sums are not stored. Every thread of the block must call.
-  __device__ __forceinline__ void run(const TiledRows& rows, int n, int k_, const uint8_t* act_, size_t act_stride_bytes,
-                                      const int32_t* act_rows, int act_row0, int mt, const A4Src& a4, const MGeom& g,
-                                      uint4* __restrict__ s0, uint4* __restrict__ s1, uint4* __restrict__ s2,
-                                      uint4* __restrict__ s3, Exchange& __restrict__ x, f32x4_t (&sum)[2][CT]) {
-    // A loop over passes would otherwise keep what every width computes from the thread's number in registers around all of them.
-    tid = static_cast<int>(threadIdx.x);
-    asm volatile("" : "+v"(tid));
-    const int lane = tid & (kWave - 1), q = lane >> 4;
+  __device__ __forceinline__ void set_weights(const TiledRows& rows, int n, int k_) {   // once tid is set
+    const int lane = tid & (kWave - 1);
     k = k_;
     chunks = k / MTraits<FMT>::kLoadElems;
 #pragma unroll
@@ -363,6 +355,19 @@ struct TiledPass {
       else soff[i] = (row_at[i] >> rows.mat[i].rs) * ((static_cast<uint32_t>(k) + (1u << cs[i]) - 1) >> cs[i]) * (FMT == kFmtFp8F32 ? 4u : 1u);
     }
     scale_bytes = static_cast<uint32_t>(n) * static_cast<uint32_t>(k / (FMT == kFmtNvfp4 ? 16 : 32));
+  }
+
+  // `sum` receives the wavefront's two row groups against mt activation rows (row c: act_rows[c] when given, else c).
+  // Rows from mt on repeat row mt - 1; their sums are not stored. Every thread of the block must call.
+  __device__ __forceinline__ void run(const TiledRows& rows, int n, int k_, const uint8_t* act_, size_t act_stride_bytes,
+                                      const int32_t* act_rows, int act_row0, int mt, const A4Src& a4, const MGeom& g,
+                                      uint4* __restrict__ s0, uint4* __restrict__ s1, uint4* __restrict__ s2,
+                                      uint4* __restrict__ s3, Exchange& __restrict__ x, f32x4_t (&sum)[2][CT]) {
+    // A loop over passes would otherwise keep what every width computes from the thread's number in registers around all of them.
+    tid = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & (kWave - 1);
+    set_weights(rows, n, k_);
     act = uniform(act_ + (act_rows ? 0 : static_cast<size_t>(act_row0) * act_stride_bytes));
     if constexpr (A4) act_scales = uniform(a4.scales + (act_rows ? 0 : static_cast<size_t>(act_row0) * a4.scale_stride));
 #pragma unroll
@@ -816,6 +821,148 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
   const TiledOut o = {a.out, nullptr, a.out_stride, a.out_f32, 0, 0.f, a.a4_gs};
   tiled_rows<FMT, false, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
                                     nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, st);
+}
+
+// ---- up to sixteen activation rows ------------------------------------------------------------------------------------
+// A dense product of one column tile reads every weight once and is bound by that read, if enough of it is on its way: a
+// wavefront takes two row groups and ONE part of K, three tiles ahead, and meets nobody until the parts are folded, in
+// the order of the forms above. The activation rows, the same few KB for all, come the way of the weights: asked for row by
+// row and turned in LDS of the wavefront's own (in the matrix core's order, sixteen rows side by side, their loads took
+// longer than the weights'). No barrier in the walk. 32 rows x 4 parts to a block of four wavefronts: a matrix of 17408
+// rows has 544 blocks, all resident at once (three to a CU), where the blocks of sixteen wavefronts of the form with
+// the parts side by side made just over one round. More rows go in column tiles, the weights out of the XCD's L2.
+//
+// What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and for the large
+// matrices the memory pipe, 2.3 to 3.1 TB/s (17408 x 5120, 8 rows: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
+// slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half.
+// ROWS: activation rows that are loaded, 8 or 16 (those from m on repeat the last).
+template <int FMT, int ROWS>
+__global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(DenseArgs a, MGeom g, int col_tiles) {
+  // An XCD keeps a row tile's column tiles to itself, one after the other.
+  const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
+  const int tile = idx / col_tiles * kXcds + lin % kXcds, c0 = idx % col_tiles * kTileCols;
+  a.act += static_cast<size_t>(c0) * a.act_stride;
+  a.m = min(a.m - c0, kTileCols);
+  using Weights = TiledPass<FMT, false, 2, 2>;
+  using Regs = typename Weights::Regs;
+  constexpr int kSub = Weights::kSub, kUnits = Weights::kUnits, kActLoads = ROWS * kUnits / kWave;
+  static_assert(kActLoads * kWave == ROWS * kUnits && kWave / kUnits * 2 >= 8, "whole loads, whose rows fold alike");
+  __shared__ typename Weights::Exchange exchange[kWavesPerBlock];
+  __shared__ uint4 act_rows[kWavesPerBlock][2][ROWS * kUnits];   // of two tiles
+  __shared__ f32x4_t fold[kWavesPerBlock][2][kWave];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wave % g.parts;
+  const int row0 = (tile * (kWavesPerBlock / g.parts) + wave / g.parts) * 2 * kGroupRows;
+  Weights w;
+  w.tid = static_cast<int>(threadIdx.x);
+  w.set_weights({{a.mat, a.mat}, {row0, row0 + kGroupRows}}, a.n, a.k);
+  const int lane = threadIdx.x & (kWave - 1), c = lane & 15, q = lane >> 4;
+  const int lo = min(part * g.part_steps, g.steps), hi = min(lo + g.part_steps, g.steps);
+  const int full = min(a.k / Weights::kTileElems, hi);
+  const uint8_t* act = Weights::uniform(a.act);
+  uint32_t act_off[kActLoads];
+  int act_k[kActLoads];   // first element of the tile that the lane loads
+#pragma unroll
+  for (int i = 0; i < kActLoads; ++i) {
+    const int row = i * (kWave / kUnits) + lane / kUnits, unit = Weights::unit_at(lane % kUnits, row);
+    act_k[i] = unit * 8;
+    act_off[i] = static_cast<uint32_t>(min(row, a.m - 1)) * static_cast<uint32_t>(a.act_stride * 2) + unit * 16;
+  }
+  typename Weights::Exchange& x = exchange[wave];
+  struct Acts { uint4 v[kActLoads]; };
+  auto load_acts = [&](int tile, Acts& to) {
+#pragma unroll
+    for (int i = 0; i < kActLoads; ++i) {
+      const typename Weights::u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(Weights::buffer(act, tile < full), act_off[i], tile * Weights::kTileElems * 2, 0);
+      to.v[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  };
+  auto put_acts = [&](int half, const Acts& from) {
+#pragma unroll
+    for (int i = 0; i < kActLoads; ++i) act_rows[wave][half][i * kWave + lane] = from.v[i];
+  };
+  const int act_row = c & (ROWS - 1);
+  f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  auto multiply = [&](int tile, int half, const Regs& r) {
+    uint4 b[kSub];
+#pragma unroll
+    for (int j = 0; j < kSub; ++j) b[j] = act_rows[wave][half][act_row * kUnits + Weights::place(q, j, act_row)];
+    Frag f[2][kSub];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ChunkRegs ch;
+      ch.w = r.w[i];
+      ch.s = w.scale_of(i, tile, r.s[i]);
+      decode_frags<FMT>(ch, f[i]);
+    }
+#pragma unroll
+    for (int j = 0; j < kSub; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = mfma_bf16(f[i][j], b[j], acc[i]);
+  };
+  Regs r0, r1, r2, r3;
+  Acts b0, b1, b2, b3;
+  typename Weights::ScaleWord sraw[2];
+  auto step = [&](int t, auto at, const Regs& now, Regs& coming, Regs& far, const Acts& coming_b, Acts& far_b) {
+    constexpr int kAt = decltype(at)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    w.load(t + 3, full, far);
+    load_acts(t + 3, far_b);
+    if constexpr (kAt == 0) w.load_scales(t + 4, sraw);
+    multiply(t, kAt & 1, now);
+    if constexpr (kAt == 3) w.put_scales(x, sraw);
+    w.exchange(x, (kAt + 1) & 3, coming);
+    put_acts((kAt + 1) & 1, coming_b);
+  };
+  if (lo < full) {
+    w.load_scales(lo, sraw);
+    w.load(lo, full, r0);
+    load_acts(lo, b0);
+    w.load(lo + 1, full, r1);
+    load_acts(lo + 1, b1);
+    w.load(lo + 2, full, r2);
+    load_acts(lo + 2, b2);
+    w.put_scales(x, sraw);
+    w.exchange(x, 0, r0);
+    put_acts(0, b0);
+    int t = lo;
+    auto turn = [&](int steps) {   // a constant where this is inlined, or the last turn's
+      step(t, std::integral_constant<int, 0>{}, r0, r1, r3, b1, b3);
+      if (steps == 1) return;
+      step(t + 1, std::integral_constant<int, 1>{}, r1, r2, r0, b2, b0);
+      if (steps == 2) return;
+      step(t + 2, std::integral_constant<int, 2>{}, r2, r3, r1, b3, b1);
+      if (steps == 3) return;
+      step(t + 3, std::integral_constant<int, 3>{}, r3, r0, r2, b0, b2);
+    };
+    for (; t + 4 <= full; t += 4) turn(4);
+    if (t < full) turn(full - t);
+  }
+  if (full < hi) {   // the part of a tile past the last whole one
+    w.load_rest(full, r0);
+#pragma unroll
+    for (int i = 0; i < kActLoads; ++i) {
+      b0.v[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (full * Weights::kTileElems + act_k[i] < a.k)
+        b0.v[i] = *reinterpret_cast<const uint4*>(act + act_off[i] + static_cast<size_t>(full) * Weights::kTileElems * 2);
+    }
+    put_acts(0, b0);
+    multiply(full, 0, r0);
+  }
+  if (g.parts > 1) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fold[wave][i][lane] = acc[i];
+    __syncthreads();
+    if (part != 0) return;
+  }
+  const float divisor = load_divisor<FMT>(a.global);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f32x4_t s = acc[i];
+    if (g.parts >= 2) s = s + fold[wave + 1][i][lane];
+    if (g.parts == 4) s = (s + fold[wave + 2][i][lane]) + fold[wave + 3][i][lane];
+    store_tile<FMT>(s, divisor, a.out, a.out_f32, static_cast<size_t>(c0 + c) * a.out_stride, row0 + i * kGroupRows, a.n, c < a.m);
+  }
 }
 
 }  // namespace dgpp_amd

@@ -302,3 +302,54 @@ def test_activation_rows_beyond_four_gigabytes(gpu, kind):
     more = () if kind == "fp8" else (d.fp4_group,)
     idx = dev(rows)
     same(lambda: gu(x, H, segs, E, 5, 0, d.views, act, I, I, H, 7.0, None, idx, *more), kind, act)
+
+
+@pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "mxfp8"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4096), (8, 33, 5120), (9, 31, 2048), (16, 130, 1152), (17, 64, 2304), (33, 300, 512), (70, 257, 8192),
+                                   (5, 40, 64), (3, 96, 4224)])
+def test_streaming_dense_form_is_bitwise_the_row_tile_form(gpu, kind, m, n, k):
+    """The dense launch that streams its weights, a part of K to a wavefront, against the form that walks the parts in turn
+    (bench switch 11: 1): one to four parts, an empty one, row groups and column tiles at their edges, tiles of k that are
+    whole, part and none, rows that no vector load reads."""
+    if kind in ("nvfp4", "mxfp4"):
+        group = 16 if kind == "nvfp4" else 32
+        k = {"nvfp4": {1152: 1536, 2304: 640, 64: 512, 4224: 7168, 8192: 3072}, "mxfp4": {64: 576, 4224: 1152, 8192: 2304}}[kind].get(k, k)
+        act, payload, scales, glob = make_fp4(m, n, k, 0xE10 + n + k, group)
+        p_d, s_d = dev(payload), dev(scales)
+        w = fp4_matrix(p_d, s_d, dev(glob) if glob is not None else None, n, k, group)
+        run = lambda a, stride, out: L.launch_mma_gemv_fp4_f32(a, stride, w, out, m, n, k, n + 3)
+    else:
+        act = hg.normal_bf16(0xE11 + n, (m, k))
+        wf = hg.normal_f32(0xE12 + n + k, (n, k), 0.02)
+        if kind == "mxfp8":
+            payload, scales = hg.encode_mxfp8(wf)
+            fn, rs, cs = L.launch_mma_gemv_fp8e8m0_f32, 0, 5
+        else:
+            k_used = k - 16 if k > 64 else k
+            act, wf, k = np.ascontiguousarray(act[:, :k_used]), np.ascontiguousarray(wf[:, :k_used]), k_used
+            payload, _ = hg.encode_fp8_blocks(hg.f32_to_bf16(wf), 128, 128)
+            scales = np.random.default_rng(n).uniform(0.5, 2.0, ((n + 127) >> 7, (k + 127) >> 7)).astype(np.float32) * 1e-3
+            fn, rs, cs = L.launch_mma_gemv_fp8_f32, 7, 7
+        p_d, s_d = dev(payload), dev(scales)
+        run = lambda a, stride, out: fn(a, stride, p_d, s_d, out, m, n, k, n + 3, rs, cs)
+    wide = np.zeros((m, k + 1), np.uint16)
+    wide[:, :k] = act
+    rows = [(dev(act), k), (dev(wide), k + 1)]
+    lib, got = _lib.load(), []
+    lib.dgpp_tune_set(5, 2)
+    lib.dgpp_tune_set(15, 1)
+    try:
+        for knob in (1, 0):
+            for a, stride in rows:
+                lib.dgpp_tune_set(11, knob)
+                out = dev_empty((m, n + 3), np.float32)
+                out.fill_(-7.0)
+                run(a, stride, out)
+                sync()
+                got.append(host(out).copy())
+    finally:
+        for key in (5, 11, 15):
+            lib.dgpp_tune_set(key, 0)
+    assert (got[0][:, :n] != -7.0).all() and (got[0][:, n:] == -7.0).all()
+    for g in got[1:]:
+        assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
