@@ -321,6 +321,39 @@ def test_router_tiled_dots_are_bitwise_the_one_row_form(gpu, mode, E, H, T):
         assert not np.any(other[0] == -7.0), "every score of the batch is written"
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("E,H,T", [(96, 512, 16), (258, 1024, 37), (30, 4096, 64), (33, 2112, 300), (64, 64, 31), (1, 6080, 33), (40, 4160, 257),
+                                   (70, 448, 1), (256, 6144, 290)])
+def test_router_chains_are_bitwise_the_tiled_form(gpu, mode, E, H, T):
+    """The matrix-core form of the score rows, tiles of 16 and 32 tokens (bench switch 10: 16, 32), against sums in one
+    wavefront's lanes (4): tile edges, chains of unequal and of no length, rows with an infinity, a NaN and subnormal numbers."""
+    x = hg.normal_bf16(mode + 11 + E, (T, H))
+    gate = hg.normal_bf16(mode + 19 + H, (E, H), 1.0 / np.sqrt(H))
+    x[0, : H // 2] = 1                       # subnormal
+    if T > 3:
+        x[2, 5], x[3, H - 1] = 0x7F80, 0x7FC0
+    bias = hg.normal_f32(mode + 5, (E,), 0.02)
+    cfg = L.make_config(H, 64, E, 1, router_mode=mode, routed_scaling_factor=1.0 if mode == 1 else 2.5)
+    x_d, g_d, b_d = dev(x), dev(gate), (None if mode == 1 else dev(bias))
+    from dgpp_amd import _lib
+    res = []
+    for tile in (4, 16, 32):
+        sc_d, bi_d = dev_empty((T + 1, E), np.float32), dev_empty((T + 1, E), np.float32)
+        sc_d.fill_(-7.0), bi_d.fill_(-7.0)
+        _lib.load().dgpp_tune_set(10, tile)
+        try:
+            L.launch_moe_router_dots(x_d, g_d, b_d, sc_d, bi_d, cfg, T)
+        finally:
+            _lib.load().dgpp_tune_set(10, 0)
+        sync()
+        res.append([host(t).copy() for t in (sc_d, bi_d)])
+    for other in res[1:]:
+        for a, b, name in zip(res[0], other, ("scores", "biased")):
+            assert np.array_equal(np.isnan(a), np.isnan(b)), name
+            assert np.array_equal(a.view(np.uint32)[~np.isnan(a)], b.view(np.uint32)[~np.isnan(b)]), name
+            assert (b[T] == -7.0).all(), "nothing is written past the batch"
+
+
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("T,E,K,vocab", [(9, 40, 6, 17), (300, 256, 8, 1000), (1, 384, 16, 3)])
 def test_hash_routes_bit_exact(gpu, norm, T, E, K, vocab):
