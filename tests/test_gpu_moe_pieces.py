@@ -228,6 +228,20 @@ def test_gather_accum_round_bit_exact(gpu):
     assert np.array_equal(host(out, np.uint16), hg.f32_to_bf16(want))
 
 
+@pytest.mark.parametrize("T,H,K", [(32768, 8, 2), (32769, 8, 2), (70000, 5, 1), (3, 256, 8), (2, 260, 16), (7, 1, 9)])
+def test_slot_accum_at_the_seams_of_its_grid(gpu, T, H, K):
+    """Tokens past one slice of the grid, columns at the edge of a 256-column tile, bit for bit the oracle."""
+    rng = np.random.default_rng(T + H)
+    contrib = rng.normal(size=(T * (K + 1), H)).astype(np.float32)
+    w = rng.uniform(0, 1, (T, K)).astype(np.float32)
+    f32_want, bf_want = np.empty((T, H), np.float32), np.empty((T, H), np.uint16)
+    orc.oracle().orc_slot_accum(orc.p(contrib), orc.p(w), T, H, K, 1, orc.p(f32_want), orc.p(bf_want))
+    out = dev_empty((T, H), np.uint16)
+    L.launch_moe_slot_accum(out, dev(contrib), dev(w), T, H, K, None)
+    sync()
+    assert np.array_equal(host(out, np.uint16), bf_want)
+
+
 @pytest.mark.parametrize("T,H,K", [(1, 4096, 8), (8, 4096, 8), (5, 333, 3), (64, 6144, 8)])
 def test_slot_accum_and_ordered_accum_bit_exact(gpu, T, H, K):
     rng = np.random.default_rng(T + H)
