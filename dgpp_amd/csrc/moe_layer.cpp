@@ -68,6 +68,15 @@ Layout layout_of(const GlmMoeConfig& c, int max_tokens, int shared_inter, size_t
   return l;
 }
 
+bool is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {   // the default stream while another one is captured
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 // A branch of work on the side stream: forked from the caller's stream and joined to it again on EVERY way out of the
 // scope that opened it (a launcher that throws between fork and join must not leave a captured graph with an
 // unjoined branch).
@@ -365,9 +374,13 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
   if (sel_scores != nullptr && !fused) throw std::logic_error("GlmMoeLayer: fused selection outside its form");
   // The shared expert's gate/up and down passes read nothing the routed passes write (disjoint slot rows): they run
   // on the side stream beside them, forked here and joined before the accumulation. One launcher call per pass.
-  // From a few tokens on: the two cross-stream dependencies cost more than the two hand-overs they take off the
-  // chain while a pass is only a few microseconds long (measured: slower at one token, level at two).
-  const bool split = slot_shared && side_ != nullptr && dgpp_tune_get(9) != 1 && (tokens >= 3 || dgpp_tune_get(9) == 2);
+  // In a captured step from three tokens on (level at two, slower at one). Launched one by one, a dependency between streams
+  // costs the chain more: from sixteen tokens on, or where the shared weights are long. Measured, us, one stream / beside, two
+  // layers of 288 x 512 x 4096 NVFP4 experts with an FP8 one of 512: launched 3 tokens 103 / 118, 8 151 / 158, 14 203 / 203, 18 338 / 278,
+  // captured 3 tokens 107 / 101, 8 155 / 139; 64 x 1024 x 4096 and 2048: launched 141 / 150, 248 / 255, 364 / 362, 557 / 408, captured 146 /
+  // 132, 252 / 233; 128 x 2048 x 6144 and 2048 (38 M shared weights): launched 255 / 252, 516 / 512, captured 260 / 233.
+  const bool beside_pays = tokens >= 3 && (tokens >= 16 || 3ll * H * w_.shared_inter > (32 << 20) || is_capturing(stream));
+  const bool split = slot_shared && side_ != nullptr && dgpp_tune_get(9) != 1 && (beside_pays || dgpp_tune_get(9) == 2);
   // On one stream the shared down pass ends with the token's accumulation (no launch of its own).
   // (One token, where a launch is a fifth of the step; measured level at two tokens. Bench switch 9 = 4 folds at any
   // batch size, 3 never.)

@@ -145,7 +145,7 @@ def test_shared_expert_passes_beside_the_routed_ones_give_the_same_bits(gpu, E, 
     expert_budget(want_h, raw, "shared-expert layer on one stream")
     s = torch.cuda.Stream()
     got = dev_empty((T, H), np.uint16)
-    _lib.load().dgpp_tune_set(9, 2)           # the two-stream form at every batch size (default: from three tokens on)
+    _lib.load().dgpp_tune_set(9, 2)           # the two-stream form at every batch size
     try:
         _two_stream_runs(layer, d, got, want_h, T, H, s)
     finally:
@@ -170,6 +170,25 @@ def _two_stream_runs(layer, d, got, want_h, T, H, s):
             g.replay()
             s.synchronize()
             assert np.array_equal(host(got, np.uint16), want_h), "graph replay"
+
+
+@pytest.mark.parametrize("T,H,sI", [(2, 256, 128), (3, 256, 128), (15, 512, 128), (16, 256, 128), (3, 512, 24576)])
+def test_shared_expert_streams_by_batch_and_capture_give_the_same_bits(gpu, T, H, sI):
+    """Without a switch the launched step and the captured one may order the shared passes on different streams: few tokens,
+    many, one or a wide shared expert. Same bits as on one stream."""
+    from dgpp_amd import _lib
+    p = moe_data.make_problem(8, H, 128, 4, T, "fp8", 900 + T + H, shared_kind="fp8", shared_I=sI, limit=10.0, std=0.05)
+    d = DeviceMoe(p)
+    layer = make_layer(p, d, 0, 2.5, T)
+    want = dev_empty((T, H), np.uint16)
+    _lib.load().dgpp_tune_set(9, 1)
+    try:
+        layer.enqueue_decode(d.x, H, want, T)
+        sync()
+    finally:
+        _lib.load().dgpp_tune_set(9, 0)
+    _two_stream_runs(layer, d, dev_empty((T, H), np.uint16), host(want, np.uint16).copy(), T, H, torch.cuda.Stream())
+    layer.close()
 
 
 GOLDEN_CASES = sorted((__import__("pathlib").Path(__file__).resolve().parent / "golden").glob("moe_*.npz"))
