@@ -40,6 +40,7 @@
 namespace dgpp_amd {
 
 constexpr int kTiledCols = 128;                   // activation rows of the widest pass
+constexpr int kNarrowCols = 32;                   // of the kernel for short segments
 constexpr int kTiledRows = 128;                   // weight rows of a block (gate + up: 64 of each)
 
 // The two row groups of a wavefront: two groups of one matrix, or one of gate and one of up.
@@ -533,22 +534,22 @@ struct TiledOut {
 };
 // A block's LDS stages, as large as the widest pass wants them: four, two where the rows pass registers (A4) and where four
 // would leave room for one block per CU.
-template <int FMT, bool A4>
+template <int FMT, bool A4, int COLS>
 struct TiledStages {
-  static constexpr int kUnits = kTiledCols * MTraits<FMT>::kStepElems / 8;
+  static constexpr int kUnits = COLS * MTraits<FMT>::kStepElems / 8;
   static constexpr int kRing = A4 || kUnits > 1024 ? 2 : 4;
   uint4 *s0, *s1, *s2, *s3;
-  typename TiledPass<FMT, A4, 8, kRing>::Exchange* x;   // of each wavefront
+  typename TiledPass<FMT, A4, COLS / kTileCols, kRing>::Exchange* x;   // of each wavefront
 };
-template <int FMT, bool GU, bool A4, int CT>
+template <int FMT, bool GU, bool A4, int CT, int COLS>
 __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
                                            int mt, const A4Src& a4, const MGeom& g, const TiledOut& o,
-                                           const TiledStages<FMT, A4>& st) {
-  TiledPass<FMT, A4, CT, TiledStages<FMT, A4>::kRing> pass;
+                                           const TiledStages<FMT, A4, COLS>& st) {
+  TiledPass<FMT, A4, CT, TiledStages<FMT, A4, COLS>::kRing> pass;
   f32x4_t sum[2][CT];
   pass.run(rows, n, k, act, act_stride_bytes, act_rows, act_row0, mt, a4, g, st.s0, st.s1, st.s2, st.s3,
-           reinterpret_cast<typename TiledPass<FMT, A4, CT, TiledStages<FMT, A4>::kRing>::Exchange&>(st.x[threadIdx.x >> 6]), sum);
+           reinterpret_cast<typename TiledPass<FMT, A4, CT, TiledStages<FMT, A4, COLS>::kRing>::Exchange&>(st.x[threadIdx.x >> 6]), sum);
   const int lane = pass.tid & (kWave - 1);
   const bool vec = ((reinterpret_cast<uintptr_t>(o.out) | (GU ? reinterpret_cast<uintptr_t>(o.out_up) : 0)) & 15u) == 0 &&
                    (o.out_stride & 3u) == 0;
@@ -592,12 +593,14 @@ __device__ __forceinline__ void tiled_pass(const TiledRows& rows, const float (&
 }
 
 // The narrowest pass that holds mt rows.
-template <int FMT, bool GU, bool A4>
+template <int FMT, bool GU, bool A4, int COLS>
 __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&divisor)[2], int n, int k, const uint8_t* act,
                                            size_t act_stride_bytes, const int32_t* act_rows, int act_row0, size_t out_row0,
                                            int mt, const A4Src& a4, const MGeom& g, const TiledOut& o,
-                                           const TiledStages<FMT, A4>& st) {
-  if (mt > 64)
+                                           const TiledStages<FMT, A4, COLS>& st) {
+  if constexpr (COLS == kNarrowCols)
+    tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
+  else if (mt > 64)
     tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
   else if (mt > 32)
     tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
@@ -606,11 +609,11 @@ __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&
 }
 
 // The kernel's stages and exchange regions, by name.
-#define DGPP_TILED_STAGES(st, FMT, A4)                                                                               \
-  using Stages = TiledStages<FMT, A4>;                                                                               \
+#define DGPP_TILED_STAGES(st, FMT, A4, COLS)                                                                         \
+  using Stages = TiledStages<FMT, A4, COLS>;                                                                         \
   __shared__ uint4 stage0[Stages::kUnits], stage1[Stages::kUnits];                                                   \
   __shared__ uint4 stage2[Stages::kRing == 4 ? Stages::kUnits : 1], stage3[Stages::kRing == 4 ? Stages::kUnits : 1]; \
-  __shared__ typename TiledPass<FMT, A4, 8, Stages::kRing>::Exchange exchange[kWavesPerBlock];                       \
+  __shared__ typename TiledPass<FMT, A4, COLS / kTileCols, Stages::kRing>::Exchange exchange[kWavesPerBlock];         \
   const Stages st = {stage0, stage1, stage2, stage3, exchange}
 
 // Consecutive workgroups go to the eight XCDs in turn. Blocks of one segment share its activation rows and blocks of one
@@ -643,8 +646,9 @@ struct TiledDeal {
   unsigned grid_y() const { return static_cast<unsigned>(slots > 1 ? slots : 1); }
 };
 // max_rows: no segment has more; long_segs: so many at the table's end have that many. tuned > 0: slots (bench switch 16).
-inline TiledDeal tiled_deal(int n_segs, int long_segs, int row_tiles, int max_rows, int tuned) {
-  const int passes = (max_rows + kTiledCols - 1) / kTiledCols;
+// cols: rows of a pass.
+inline TiledDeal tiled_deal(int n_segs, int long_segs, int row_tiles, int max_rows, int tuned, int cols = kTiledCols) {
+  const int passes = (max_rows + cols - 1) / cols;
   auto side_by_side = [&](int64_t blocks) {   // all passes where the blocks of one slot are few, else some
     const int64_t want = tuned > 0 ? tuned : 8192 / blocks;
     return static_cast<int>(want < 1 ? 1 : (want < passes ? want : passes));
@@ -691,22 +695,23 @@ struct TiledPlan {
   }
 };
 // Sorted once every XCD has several items; with fewer, and where the rows are not known, by the deal.
-inline TiledPlan tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int tuned) {
-  const int64_t items = total_rows > 0 && tuned == 0 ? n_segs + total_rows / kTiledCols : 0;
-  return {tiled_deal(n_segs, long_segs, row_tiles, max_rows, tuned),
+inline TiledPlan tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int tuned, int cols) {
+  const int64_t items = total_rows > 0 && tuned == 0 ? n_segs + total_rows / cols : 0;
+  return {tiled_deal(n_segs, long_segs, row_tiles, max_rows, tuned, cols),
           items >= 8 * kXcds && items * row_tiles <= 1 << 24 ? static_cast<int>(items) : 0, n_segs};
 }
 struct TiledItem {
   int expert, row0, rows;
 };
+template <int COLS>
 __device__ __forceinline__ bool sorted_item(const DgppMoeSegment* segs, int n_segs, int item, TiledItem& out) {
   __shared__ int totals[2][kWavesPerBlock], found[2];
   const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6;
-  int wide = 0, rest = 0;   // passes of more than 64 rows; of more than 32 (upper half) and fewer
-  auto wide_of = [](int rows) { return rows / kTiledCols + (rows % kTiledCols > 64 ? 1 : 0); };
+  int wide = 0, rest = 0;   // passes more than half full; more than a quarter (upper half) and less
+  auto wide_of = [](int rows) { return rows / COLS + (rows % COLS > COLS / 2 ? 1 : 0); };
   auto rest_of = [](int rows) {
-    const int r = rows % kTiledCols;
-    return r > 64 ? 0 : r > 32 ? 1 << 16 : r > 0 ? 1 : 0;
+    const int r = rows % COLS;
+    return r > COLS / 2 ? 0 : r > COLS / 4 ? 1 << 16 : r > 0 ? 1 : 0;
   };
   for (int s = tid; s < n_segs; s += kBlockThreads) {
     const int rows = segs[s].rows;
@@ -740,13 +745,13 @@ __device__ __forceinline__ bool sorted_item(const DgppMoeSegment* segs, int n_se
     if (item >= before && item < before + (rest >> shift & 0xffff)) {
       for (int s = tid; s < n_segs; s += kBlockThreads) {
         const int rows = segs[s].rows;
-        if ((rest_of(rows) >> shift & 0xffff) != 0 && before++ == item) found[0] = s, found[1] = rows / kTiledCols * kTiledCols;
+        if ((rest_of(rows) >> shift & 0xffff) != 0 && before++ == item) found[0] = s, found[1] = rows / COLS * COLS;
       }
     }
   } else if (item >= wide_before && item < wide_before + wide) {
     for (int s = tid; s < n_segs; s += kBlockThreads) {
       const int n = wide_of(segs[s].rows);
-      if (item >= wide_before && item < wide_before + n) found[0] = s, found[1] = (item - wide_before) * kTiledCols;
+      if (item >= wide_before && item < wide_before + n) found[0] = s, found[1] = (item - wide_before) * COLS;
       wide_before += n;
     }
   }
@@ -754,27 +759,28 @@ __device__ __forceinline__ bool sorted_item(const DgppMoeSegment* segs, int n_se
   const int s = __builtin_amdgcn_readfirstlane(found[0]), c0 = __builtin_amdgcn_readfirstlane(found[1]);
   if (s < 0) return false;
   const DgppMoeSegment seg = segs[s];
-  out = {seg.expert, seg.row0 + c0, min(kTiledCols, seg.rows - c0)};
+  out = {seg.expert, seg.row0 + c0, min(COLS, seg.rows - c0)};
   return true;
 }
 
-template <int FMT, bool GU, bool A4>
-__global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, TiledPlan plan) {
-  DGPP_TILED_STAGES(st, FMT, A4);
+// COLS: rows of a pass at most, 128, or 32 for short segments (three blocks per CU instead of two).
+template <int FMT, bool GU, bool A4, int COLS>
+__global__ __launch_bounds__(kBlockThreads, COLS == kNarrowCols ? 3 : 2) void tiled_grouped_kernel(GroupedArgs a, MGeom g, TiledPlan plan) {
+  DGPP_TILED_STAGES(st, FMT, A4, COLS);
   TiledItem it;
   int tile, step;
   if (plan.items > 0) {
     const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
     tile = idx % plan.deal.row_tiles;
-    step = kTiledCols;
-    if (!sorted_item(a.segs, plan.n_segs, idx / plan.deal.row_tiles * kXcds + lin % kXcds, it)) return;
+    step = COLS;
+    if (!sorted_item<COLS>(a.segs, plan.n_segs, idx / plan.deal.row_tiles * kXcds + lin % kXcds, it)) return;
   } else {
     const TiledPlace at = tiled_place(plan.deal, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y));
     if (at.seg < 0) return;
     const DgppMoeSegment seg = a.segs[at.seg];
     tile = at.tile;
-    step = at.slots * kTiledCols;
-    it = {seg.expert, seg.row0 + at.slot * kTiledCols, seg.rows - at.slot * kTiledCols};
+    step = at.slots * COLS;
+    it = {seg.expert, seg.row0 + at.slot * COLS, seg.rows - at.slot * COLS};
     if (it.rows <= 0) return;
   }
   const int wave = threadIdx.x >> 6;
@@ -793,16 +799,16 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_grouped_kernel(Grouped
   const TiledOut o = {a.out, a.out_up, a.out_stride, a.out_f32, a.gate_up, a.limit, a.a4_gs};
   for (int c0 = 0; c0 < it.rows; c0 += step) {
     const int first = it.row0 + c0;
-    tiled_rows<FMT, GU, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
+    tiled_rows<FMT, GU, A4, COLS>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
                                    a.act_rows ? a.act_rows + first : nullptr, first, static_cast<size_t>(first),
-                                   min(kTiledCols, it.rows - c0), src, g, o, st);
+                                   min(COLS, it.rows - c0), src, g, o, st);
   }
 }
 
 // grid.x = kXcds * ceil(row tiles / kXcds) * column passes.
 template <int FMT, bool A4>
 __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs a, MGeom g, int row_tiles, int passes) {
-  DGPP_TILED_STAGES(st, FMT, A4);
+  DGPP_TILED_STAGES(st, FMT, A4, kTiledCols);
   const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
   const int tile = idx / passes * kXcds + lin % kXcds, c0 = idx % passes * kTiledCols;
   if (tile >= row_tiles) return;
@@ -819,7 +825,7 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
   src.scales = a.a4_scales;
   src.scale_stride = a.a4_scale_stride;
   const TiledOut o = {a.out, nullptr, a.out_stride, a.out_f32, 0, 0.f, a.a4_gs};
-  tiled_rows<FMT, false, A4>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
+  tiled_rows<FMT, false, A4, kTiledCols>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
                                     nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, st);
 }
 

@@ -283,6 +283,37 @@ def test_sorted_passes_of_a_skewed_table_are_bitwise_the_16_row_form(gpu, kind, 
     layer.close()
 
 
+@pytest.mark.parametrize("kind", ["fp8", "mxfp4", "nvfp4", "w4a4"])
+@pytest.mark.parametrize("E,T,K,H,I", [(70, 301, 5, 512, 512), (300, 700, 3, 512, 576), (12, 40, 3, 2048, 640), (5, 33, 1, 1152, 576), (64, 16, 8, 4096, 320)])
+def test_narrow_passes_are_bitwise_the_16_row_form(gpu, kind, E, T, K, H, I):
+    """The kernel of 32-row passes (bench switch 15: 3): dealt by segment and sorted, segments of no row, one, 16, 17, 32, 33 and
+    of every token, one, two and four parts of k, k tiles whole and in part."""
+    if kind in ("nvfp4", "w4a4") and H == 1152:
+        H = 1536
+    p = moe_data.make_problem(E, H, I, K, T, "nvfp4" if kind == "w4a4" else kind, 77 + E, shared_kind=None, limit=7.0, std=0.05)
+    d = DeviceMoe(p)
+    layer = make_layer(p, d, L.ROUTER_SOFTMAX_TOPK, 1.0, T)
+    rng = np.random.default_rng(E)
+    popular = 1.0 / np.arange(1, E) ** 1.1
+    ids = np.stack([np.concatenate([[0], 1 + rng.choice(E - 1, K - 1, replace=False, p=popular / popular.sum())]) for _ in range(T)])
+    ids_d, w = dev(ids.astype(np.int32)), dev(rng.uniform(0.1, 1.0, (T, K)).astype(np.float32))
+    out, got = dev_empty((T, H), np.uint16), []
+    for form in (1, 3):
+        out.fill_(0x55)
+        _lib.load().dgpp_tune_set(15, form)
+        try:
+            if kind == "w4a4":
+                layer.enqueue_prefill_routed_w4a4(d.x, H, ids_d, w, out, T)
+            else:
+                layer.enqueue_prefill_routed(d.x, H, ids_d, w, out, T)
+        finally:
+            _lib.load().dgpp_tune_set(15, 0)
+        sync()
+        got.append(host(out, np.uint16).copy())
+    layer.close()
+    assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("kind", ["fp8", "mxfp4"])
 def test_activation_rows_beyond_four_gigabytes(gpu, kind):
     """Rows that a buffer load does not reach, alone in a pass and beside near ones, and rows that end at its edge."""
