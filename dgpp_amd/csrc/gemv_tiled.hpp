@@ -838,8 +838,9 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
 // rows has 544 blocks, all resident at once (three to a CU), where the blocks of sixteen wavefronts of the form with
 // the parts side by side made just over one round. More rows go in column tiles, the weights out of the XCD's L2.
 //
-// What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and for the large
-// matrices the memory pipe, 2.3 to 3.1 TB/s (17408 x 5120, 8 rows: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
+// What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and for larger FP4
+// matrices the decoding, a block at a time on each CU: NVFP4, K = 5120, 8 rows took 10.7 us for 256 blocks, 17.6 for 512 and 23 for 768, 3
+// to 4.6 of them the memory's (17408 x 5120, 544 blocks: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
 // slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half.
 // ROWS: activation rows that are loaded, 8 or 16 (those from m on repeat the last).
 template <int FMT, int ROWS>
