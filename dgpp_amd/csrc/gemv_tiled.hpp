@@ -945,7 +945,7 @@ __global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(DenseArg
     for (; t + 4 <= full; t += 4) turn(4);
     if (t < full) turn(full - t);
   }
-  if (full < hi) {   // the part of a tile past the last whole one
+  if (lo <= full && full < hi) {   // the part of a tile past the last whole one, in the part of K that it belongs to (a part may be empty)
     w.load_rest(full, r0);
 #pragma unroll
     for (int i = 0; i < kActLoads; ++i) {

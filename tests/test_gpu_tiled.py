@@ -335,13 +335,16 @@ def test_activation_rows_beyond_four_gigabytes(gpu, kind):
     same(lambda: gu(x, H, segs, E, 5, 0, d.views, act, I, I, H, 7.0, None, idx, *more), kind, act)
 
 
+STREAM_SHAPES = [(1, 1, 4096), (8, 33, 5120), (9, 31, 2048), (16, 130, 1152), (17, 64, 2304), (33, 300, 512), (70, 257, 8192), (5, 40, 64),
+                 (3, 96, 4224), (20, 70, 4160), (7, 33, 4576), (6, 50, 4352)]
+
+
 @pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "mxfp8"])
-@pytest.mark.parametrize("m,n,k", [(1, 1, 4096), (8, 33, 5120), (9, 31, 2048), (16, 130, 1152), (17, 64, 2304), (33, 300, 512), (70, 257, 8192),
-                                   (5, 40, 64), (3, 96, 4224)])
+@pytest.mark.parametrize("m,n,k", STREAM_SHAPES)
 def test_streaming_dense_form_is_bitwise_the_row_tile_form(gpu, kind, m, n, k):
     """The dense launch that streams its weights, a part of K to a wavefront, against the form that walks the parts in turn
-    (bench switch 11: 1): one to four parts, an empty one, row groups and column tiles at their edges, tiles of k that are
-    whole, part and none, rows that no vector load reads."""
+    (bench switch 11: 1): one to four parts, row groups and column tiles at their edges, tiles of k that are whole, part and
+    none, rows that no vector load reads; FP4 at 4352, 4160 and 4576 has an empty part, the last two with a part tile before it."""
     if kind in ("nvfp4", "mxfp4"):
         group = 16 if kind == "nvfp4" else 32
         k = {"nvfp4": {1152: 1536, 2304: 640, 64: 512, 4224: 7168, 8192: 3072}, "mxfp4": {64: 576, 4224: 1152, 8192: 2304}}[kind].get(k, k)

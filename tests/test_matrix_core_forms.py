@@ -92,3 +92,14 @@ def test_tiled_grouped_blocks_cover_every_pass_once_and_spread_long_segments(n_s
     # the others stay on one XCD each, with their activation rows
     for seg in range(spread_from):
         assert {x for (s, _, _), x in seen.items() if s == seg} == {seg % 8}
+
+
+def test_the_streamed_shapes_hold_the_empty_parts_that_their_test_names():
+    """K is cut in four parts of whole turns of four steps from 4096 elements on; FP4 steps are of 128."""
+    from test_gpu_tiled import STREAM_SHAPES
+    empty, with_part_tile = set(), set()
+    for k in {k for _, _, k in STREAM_SHAPES if k >= 4096}:
+        steps = -(-k // 128)
+        if 3 * (-(-steps // 4) + 3 & ~3) >= steps:
+            (with_part_tile if k % 128 else empty).add(k)
+    assert empty >= {4352} and with_part_tile >= {4160, 4576}
