@@ -291,6 +291,15 @@ struct TiledPass {
     }
   }
 
+  // A use of a tile's weights and scales that costs nothing once they have arrived.
+  __device__ __forceinline__ void keep(const Regs& r) const {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      asm volatile("" ::"v"(r.w[g].x), "v"(r.w[g].y), "v"(r.w[g].z), "v"(r.w[g].w));
+      if constexpr (!kFp4) asm volatile("" ::"v"(r.s[g]));
+    }
+  }
+
   // The products of a tile. The operands from LDS are asked for kAhead products early, in an order that the compiler is held
   // to: left alone it reads one, waits for it and uses it, with one other wavefront on the SIMD to cover the wait.
   static constexpr int kAhead = CT < 4 ? CT * 2 : 4;
@@ -410,14 +419,18 @@ struct TiledPass {
     // those may still be on their way then that are younger than its loads to the stage: the weights (and block-FP8 scales)
     // that followed those, and what the RING - 2 steps between asked for. (The FP4 scales of a turn are not counted: where
     // they are among them, up to two fewer may be left.)
+    // The count stands on every one of those loads being in the program. Those of a whole turn are, all of them are read
+    // on both ways out of the loop below. Those of the last turn are not: what it asks for past the last tile nobody reads,
+    // and the compiler leaves out as much of it as it can tell. Its steps, three of a pass at most, wait for everything.
     constexpr int kTileLoads = kFp4 ? 2 : 4;
     constexpr int kYounger = kTileLoads + (RING - 2) * (kRowLoads + kTileLoads);
-    auto step = [&](int t, auto at, const uint4* __restrict__ cur, uint4* __restrict__ next, const Regs& now, Regs& coming, Regs& far) {
+    auto step = [&](int t, auto at, auto last, const uint4* __restrict__ cur, uint4* __restrict__ next, const Regs& now, Regs& coming,
+                    Regs& far) {
       constexpr int kAt = decltype(at)::value;   // in its turn
       if constexpr (A4) {
         tiled_barrier<63>();
       } else {
-        tiled_barrier<kYounger>();
+        tiled_barrier<decltype(last)::value ? 0 : kYounger>();
         stage_rows(t + RING - 1, full, next);
         asm volatile("" ::: "memory");   // the weights are asked for after the rows: kYounger
       }
@@ -461,25 +474,32 @@ struct TiledPass {
       // The stages and the tiles by name, in turns of four, and one way out of the loop: the compiler then waits for what a
       // step reads and no more.
       int t = 0, part_end = part_tiles;
-      auto turn = [&](int steps) {   // `steps` is a constant where this is inlined, or the last turn's
-        step(t, std::integral_constant<int, 0>{}, s0, RING == 2 ? s1 : s3, r0, r1, kDeep == 2 ? r2 : r3);
+      auto turn = [&](int steps, auto last) {   // whole: four steps; the last: one to three
+        step(t, std::integral_constant<int, 0>{}, last, s0, RING == 2 ? s1 : s3, r0, r1, kDeep == 2 ? r2 : r3);
         if (steps == 1) return;
-        step(t + 1, std::integral_constant<int, 1>{}, s1, s0, r1, r2, kDeep == 2 ? r3 : r0);
+        step(t + 1, std::integral_constant<int, 1>{}, last, s1, s0, r1, r2, kDeep == 2 ? r3 : r0);
         if (steps == 2) return;
-        step(t + 2, std::integral_constant<int, 2>{}, RING == 2 ? s0 : s2, s1, r2, r3, kDeep == 2 ? r0 : r1);
-        if (steps == 3) return;
-        step(t + 3, std::integral_constant<int, 3>{}, RING == 2 ? s1 : s3, RING == 2 ? s0 : s2, r3, r0, kDeep == 2 ? r1 : r2);
+        step(t + 2, std::integral_constant<int, 2>{}, last, RING == 2 ? s0 : s2, s1, r2, r3, kDeep == 2 ? r0 : r1);
+        if constexpr (!decltype(last)::value)
+          step(t + 3, std::integral_constant<int, 3>{}, last, RING == 2 ? s1 : s3, RING == 2 ? s0 : s2, r3, r0, kDeep == 2 ? r1 : r2);
       };
       for (; t + 4 <= full;) {
-        turn(4);
+        turn(4, std::false_type{});
         t += 4;
         if (t == part_end) {   // parts are whole turns
           add_part(t == part_tiles);
           part_end += part_tiles;
         }
       }
-      if (t < full) turn(full - t);
+      if (t < full) turn(full - t, std::true_type{});
       tiled_barrier<0>();   // nothing is on its way to a stage, and no wavefront reads one
+      if constexpr (!A4) {
+        if (t == full) {    // what the last whole turn asked for is read here, by an instruction that is none (kYounger)
+          keep(r0);
+          keep(r1);
+          keep(r2);
+        }
+      }
     }
     for (int t = full; t < g.steps; ++t) {
       load_rest(t, r0);

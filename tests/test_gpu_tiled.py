@@ -387,3 +387,39 @@ def test_streaming_dense_form_is_bitwise_the_row_tile_form(gpu, kind, m, n, k):
     assert (got[0][:, :n] != -7.0).all() and (got[0][:, n:] == -7.0).all()
     for g in got[1:]:
         assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "mxfp8"])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 5, 6, 7, 11, 66])
+def test_walks_that_end_with_part_of_a_turn_are_bitwise_the_16_row_form(gpu, kind, tiles):
+    """Whole tiles of k that are no whole turns of four: the walk's last steps, where less is on its way than its counted waits
+    stand on. Every pass width, the 128-row passes and (grouped) the 32-row ones; 66 tiles in two (block FP8, MXFP8) or four parts."""
+    k = tiles * (64 if kind in ("fp8", "mxfp8") else 128)
+    n, rows = 140, [32, 64, 128, 5, 96]
+    if kind == "mxfp8":
+        payload, scales = hg.encode_mxfp8(hg.normal_f32(0xF10 + k, (n, k), 0.02))
+        p_d, s_d = dev(payload), dev(scales)
+        for m in rows[:3]:
+            x, out = dev(hg.normal_bf16(0xF11 + m, (m, k))), dev_empty((m, n), np.uint16)
+            same(lambda: L.launch_mma_gemv_fp8e8m0_bf16(x, k, p_d, s_d, out, m, n, k, n, 0, 5), f"{m} rows", out)
+        return
+    E, total = len(rows), sum(rows)
+    d = DeviceMoe(moe_data.make_problem(E, k, 128, 2, 4, kind, 0xF20 + tiles, shared_kind=None, limit=7.0, std=0.05))
+    x = dev(hg.normal_bf16(0xF21 + k, (total, k)))
+    starts = np.concatenate([[0], np.cumsum(rows)[:-1]])
+    segs = dev(np.array([[starts[i], rows[i], (i * 2) % E] for i in range(E)], np.int32))
+    plain = L.launch_moe_grouped_mma_f32 if kind == "fp8" else L.launch_moe_grouped_mma_fp4_f32
+    more = () if kind == "fp8" else (d.fp4_group,)
+    out, got = dev_empty((total, 128), np.float32), []
+    for form in (1, 2, 3):
+        out.fill_(-7.0)
+        _lib.load().dgpp_tune_set(15, form)
+        try:
+            plain(x, k, segs, E, max(rows), 0, d.views, 1, out, 128, 128, k, None, None, *more)
+        finally:
+            _lib.load().dgpp_tune_set(15, 0)
+        sync()
+        got.append(host(out).copy())
+    assert (got[0] != -7.0).all()
+    for g in got[1:]:
+        assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
