@@ -182,6 +182,9 @@ struct TiledPass {
     }
   }
   // A tile's weights, from as they were loaded to as they are multiplied, and its FP4 scales (`at`: which tile of its turn).
+  // LOADS: loads to LDS may be on their way. A scale is then read as the word that was written: a read of its bytes could, for
+  // the compiler, be one of the stage that is being loaded, and waited for every load (MXFP4 2048 tokens 854 us for 833 so).
+  template <bool LOADS = !A4>
   __device__ __forceinline__ void exchange(Exchange& x, int at, Regs& r) const {
     const int lane = tid & 63, row = lane & 15, q = lane >> 4;
 #pragma unroll
@@ -191,9 +194,15 @@ struct TiledPass {
     if constexpr (kFp4) {
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        const uint8_t* p = reinterpret_cast<const uint8_t*>(x.s[g]) + (row * 4 + at) * kTileScale;
-        if constexpr (FMT == kFmtNvfp4) r.s[g] = *reinterpret_cast<const uint16_t*>(p + q * 2);
-        else r.s[g] = p[q];
+        if constexpr (LOADS) {
+          const ScaleWord w = x.s[g][row * 4 + at];
+          if constexpr (FMT == kFmtNvfp4) r.s[g] = ((q & 2) != 0 ? w.y : w.x) >> (q & 1) * 16 & 0xffffu;
+          else r.s[g] = w >> q * 8 & 0xffu;
+        } else {
+          const uint8_t* p = reinterpret_cast<const uint8_t*>(x.s[g]) + (row * 4 + at) * kTileScale;
+          if constexpr (FMT == kFmtNvfp4) r.s[g] = *reinterpret_cast<const uint16_t*>(p + q * 2);
+          else r.s[g] = p[q];
+        }
       }
     }
   }
@@ -938,7 +947,7 @@ __global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(DenseArg
     if constexpr (kAt == 0) w.load_scales(t + 4, sraw);
     multiply(t, kAt & 1, now);
     if constexpr (kAt == 3) w.put_scales(x, sraw);
-    w.exchange(x, (kAt + 1) & 3, coming);
+    w.template exchange<false>(x, (kAt + 1) & 3, coming);
     put_acts((kAt + 1) & 1, coming_b);
   };
   if (lo < full) {
@@ -950,7 +959,7 @@ __global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(DenseArg
     w.load(lo + 2, full, r2);
     load_acts(lo + 2, b2);
     w.put_scales(x, sraw);
-    w.exchange(x, 0, r0);
+    w.template exchange<false>(x, 0, r0);
     put_acts(0, b0);
     int t = lo;
     auto turn = [&](int steps) {   // a constant where this is inlined, or the last turn's
