@@ -172,26 +172,25 @@ namespace {
 //
 // Which form, measured on this chip (cold weights; 2048 x 4096 ... 17408 x 5120, one to eight rows):
 // * more rows than one vector pass holds: the matrix core (the vector core would read the weights again per pass);
-// * five to eight rows: the vector core pays a dot chain per row and weight, the matrix core one decode per weight -
-//   but an unsplit matrix-core launch has one block per 64 weight rows, too few to fill the chip unless the matrix is
-//   large: with a split-K workspace the matrix core wins from five rows on (from three for matrices of 48 M weights and
-//   more). Without one, rows of 4096 elements and more run the four parts of K side by side inside a block while the
-//   row tiles fit one round of the chip (dense_mfma_team_row_groups): then six rows and more take the matrix core for
-//   matrices of 8 M weights (block FP8: the vector core needs two passes there) or 32 M weights (FP4) and more, and
-//   matrices of 64 M weights from four (FP8) or five (FP4) rows on; otherwise only matrices of 64 M weights and
-//   more, from five rows on;
+// * five to eight rows: the vector core pays a dot chain per row and weight, the matrix core's streaming form
+//   (stream_dense_kernel) hardly grows with the rows. Vector core -> streaming, us, five rows: 4096 x 4096, NVFP4 9.5 -> 7.7,
+//   MXFP4 8.7 -> 5.5, block FP8 12.7 -> 7.7; 6144 x 5120 13.9 -> 9.7, 13.0 -> 7.5, 21.4 -> 9.2: the matrix core from 16 M
+//   weights on with rows of 4096 elements and more, else from 64 M on. Smaller matrices would gain less or nothing (4096 x
+//   1024, 8 rows 8.7 -> 7.8 and 7.2 -> 8.0) and keep the bits that the vector core's fused launches share with it. With a
+//   split-K workspace the matrix core wins from five rows on at any size, from three for matrices of 48 M weights and more;
+//   block FP8, whose second vector pass starts at six rows, from six rows on for 8 M weights, from four for 64 M, while the
+//   parts of K side by side fit one round of the chip (dense_mfma_team_row_groups);
 // * up to four rows (three of a large matrix): the vector core.
-// `streams`: the rows are whole 16-byte vectors, which the streaming form of the matrix core (stream_dense_kernel) reads: its
-// time hardly grows with the rows, the vector core's by a dot chain per row. Measured, us, vector core -> streaming, five
-// rows: 4096 x 4096, NVFP4 9.5 -> 7.7, MXFP4 8.7 -> 5.5, block FP8 12.7 -> 7.7; 6144 x 5120 13.9 -> 9.7, 13.0 -> 7.5, 21.4 -> 9.2: from five rows
-// on for 16 M weights. Smaller matrices and fewer rows would gain less or nothing (4096 x 1024, 8 rows 8.7 -> 7.8 and 7.2 -> 8.0) and keep
-// the bits that the vector core's fused launches share with it.
+// Which form is a function of m, n, k, the format and the workspace, so that a row's bits do not depend on where it lies. Rows that
+// are no whole 16-byte vectors have no streaming form, but the vector core loses more by them than the matrix core's other
+// forms: vector -> matrix core, us, such rows, five of 4096 x 4096: block FP8 34.7 -> 14.3, MXFP8 33.6 -> 19.9, NVFP4 20.1 -> 14.9, MXFP4
+// 19.5 -> 14.2; eight of 12288 x 4096: 163 -> 18, 162 -> 24, 86 -> 17.
 constexpr int kVectorPassRows = kMaxActRows;
-bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool have_ws, int from_rows, bool streams) {
+bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool have_ws, int from_rows) {
   if (m > kVectorPassRows || m > max_stage_rows(k)) return true;
-  if (streams && m >= 5 && k >= 4096 && static_cast<size_t>(n) * static_cast<size_t>(k) >= (16u << 20)) return true;
   if (from_rows > 0 && m >= from_rows) return true;   // the caller's own boundary (the reference's mma_from_rows)
   const size_t weights = static_cast<size_t>(n) * static_cast<size_t>(k);
+  if (m >= 5 && weights >= ((k >= 4096 ? 16u : 64u) << 20)) return true;
   int parts = 1;
   switch (fmt) {
     case kFmtFp8F32: parts = mgeom<kFmtFp8F32>(k).parts; break;
@@ -202,20 +201,15 @@ bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool
   const bool split = have_ws && parts > 1 && (n + 63) / 64 < 1024 &&
                      ws_bytes >= static_cast<size_t>(parts) * m * static_cast<size_t>(n) * sizeof(float);
   if (split) return m >= 5 || (m >= 3 && weights >= (48u << 20));
-  if (dense_mfma_team_row_groups(parts, m, n, true) != 0) {
-    // the parts of K side by side inside a block: block FP8 from six rows on (the vector core takes two passes there),
-    // FP4 from six rows on for matrices of 32 M weights and more; large matrices from four rows on
-    const bool fp8 = fmt == kFmtFp8F32 || fmt == kFmtFp8E8M0;
-    if (m >= 6 && weights >= ((fp8 ? 8u : 32u) << 20)) return true;
-    return m >= (fp8 ? 4 : 5) && weights >= (64u << 20);
-  }
-  return m >= 5 && weights >= (64u << 20);
+  const bool fp8 = fmt == kFmtFp8F32 || fmt == kFmtFp8E8M0;
+  return fp8 && dense_mfma_team_row_groups(parts, m, n, true) != 0 &&
+         ((m >= 6 && weights >= (8u << 20)) || (m >= 4 && weights >= (64u << 20)));
 }
 int dense_rows(int fmt, const uint16_t* act, size_t act_stride, const MatRef& mat, const float* global, void* out,
                size_t out_stride, int out_f32, int m, int n, int k, hipStream_t stream, const char* who, int from_rows,
                void* ws = nullptr, size_t ws_bytes = 0, bool beside = false) {
   const int core = tune_get(kTuneCore);   // bench switch: 1 pins the vector core, 2 the matrix core
-  if (core != 1 && (core == 2 || dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, from_rows, rows_stream(act, act_stride)))) {
+  if (core != 1 && (core == 2 || dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, from_rows))) {
     if ((m + kTileCols - 1) / kTileCols > 65535) return fail_arg(std::string(who) + ": grid dimension overflow");
     DenseArgs a;
     a.act = act;
@@ -1210,15 +1204,14 @@ static int dense_mma_fp8(const uint16_t* act, size_t act_stride, const uint8_t* 
                    out_f32, out_stride, m, n, k, ws, ws_bytes, stream, who, act_up, limit);
 }
 // The reference's streaming tensor-core GEMV (launch_mma_gemv_fp8{,e8m0}_*) is its decode form for FP8 weights at every
-// row count. Here a batch that fits one vector-core pass (up to eight rows) runs on the vector core, which is the
-// faster form for it on this chip; from nine rows on the matrix core takes over (ws: its split-K workspace). As with the
-// GEMV-named launchers the two cores differ in summation order and meet the same tolerance.
+// row count. Here it has the GEMV-named launchers' dispatch (dense_takes_matrix_core; ws: the split-K workspace): the two
+// cores differ in summation order and meet the same tolerance.
 static int mma_gemv_fp8(const uint16_t* act, size_t act_stride, const uint8_t* payload, const void* scales, int e8m0, void* out,
                         int out_f32, int m, int n, int k, size_t out_stride, int rs, int cs, void* ws, size_t ws_bytes,
                         void* stream, const char* who) {
   if (m <= 0 || n <= 0) return DGPP_OK;
   const int fmt = e8m0 ? kFmtFp8E8M0 : kFmtFp8F32;
-  if (tune_get(kTuneCore) == 2 || k <= 0 || (tune_get(kTuneCore) != 1 && dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, 0, rows_stream(act, act_stride))))
+  if (tune_get(kTuneCore) == 2 || k <= 0 || (tune_get(kTuneCore) != 1 && dense_takes_matrix_core(fmt, m, n, k, ws_bytes, ws != nullptr, 0)))
     return dense_mma_fp8(act, act_stride, payload, scales, e8m0, out, out_f32, m, n, k, out_stride, rs, cs, ws, ws_bytes, stream,
                          who);
   if (!act || !payload || !scales || !out) return fail_arg(std::string(who) + ": null pointer");
@@ -1272,11 +1265,11 @@ int dgpp_launch_mma_gemv_fp8_bf16_pair(const uint16_t* a0, const uint8_t* w0, co
   // Each problem takes the core its single launch would take (so that its bits are that launch's): both on the vector
   // core -> one vector-core launch over both; both on the matrix core -> one matrix-core launch; one each -> two launches.
   const int core = tune_get(kTuneCore);
-  auto takes_mma = [&](const uint16_t* act, int n) {
+  auto takes_mma = [&](int n) {
     if (core == 2) return true;
-    return dense_takes_matrix_core(kFmtFp8F32, m, n, k, ws_bytes, ws != nullptr, 0, rows_stream(act, act_stride));
+    return dense_takes_matrix_core(kFmtFp8F32, m, n, k, ws_bytes, ws != nullptr, 0);
   };
-  const bool mma0 = takes_mma(a0, n0), mma1 = takes_mma(a1, n1);
+  const bool mma0 = takes_mma(n0), mma1 = takes_mma(n1);
   if (mma0 != mma1 || core == 1) {   // (the bench switch that pins the vector core: the single launchers know how)
     const int rc = dgpp_launch_mma_gemv_fp8_bf16(a0, act_stride, w0, s0, o0, m, n0, k, stride0, rs, cs, stream, ws, ws_bytes);
     if (rc != DGPP_OK) return rc;

@@ -432,9 +432,8 @@ int dgpp_launch_mma_gemv_fp4_bf16_static(const uint16_t* act, size_t act_stride,
 int dgpp_static_scratch_release(void);
 /* src/kernels/mma_gemv.hpp:70-94 (launch_mma_gemv_fp8{,e8m0}_{bf16,f32}): the reference's streaming tensor-core GEMV for
  * FP8 weights. The same dispatch as dgpp_launch_scale_gemm_bf16 here: small batches run on the vector core where that
- * is the faster form on this chip (always up to four rows; five to eight rows without a workspace unless the matrix is
- * large), the rest on the matrix core with `ws` as its split-K workspace. The two cores differ in fp32 summation order;
- * both meet the same tolerance against the fp64 oracle. */
+ * is the faster form on this chip, the rest on the matrix core with `ws` as its split-K workspace. The two cores differ in
+ * fp32 summation order; both meet the same tolerance against the fp64 oracle. */
 int dgpp_launch_mma_gemv_fp8_bf16(const uint16_t* act, size_t act_stride, const uint8_t* w, const float* scales,
                                   uint16_t* out, int m, int n, int k, size_t out_stride, int rs, int cs, void* stream,
                                   void* ws, size_t ws_bytes);
@@ -514,12 +513,10 @@ int dgpp_launch_moe_grouped_mma_fp4_f32(const uint16_t* act, size_t act_stride, 
                                         int fp4_group, int tile_rows);
 
 /* src/kernels/fp4_gemv.hpp:23-32. `w` is a HOST struct holding device pointers.
- * Dispatch between the vector-core GEMV (up to eight rows per pass over the weights) or the matrix-core form (16 rows
+ * Dispatch between the vector-core GEMV (up to eight rows per pass over the weights) and the matrix-core form (16 rows
  * per pass), chosen by what was measured faster on this chip: more rows than one vector pass holds -> matrix core; five
- * to eight rows -> matrix core when a split-K workspace is there (then from three rows on for matrices of 48 M weights
- * and more) or, without one, when the matrix has 64 M weights and more (an unsplit matrix-core launch has one block per
- * 64 weight rows: too few to fill the chip for smaller matrices); otherwise the vector core.
- * (This signature carries no workspace.) The reference moves to its tensor-core form as m grows in the same way
+ * to eight rows -> matrix core for matrices of 64 M weights and more, from 16 M on with k >= 4096; otherwise the vector core.
+ * The reference moves to its tensor-core form as m grows in the same way
  * (src/kernels/glm_moe_launch.hpp:363). The two forms sum in different fp32 orders: a row's bits depend on which form
  * its call takes (a function of m, n, k only); both are held to the same oracle tolerance. */
 int dgpp_launch_fp4_gemv_bf16(const uint16_t* act, size_t act_row_stride_elems,
@@ -534,9 +531,9 @@ int dgpp_fp4_gemv_accepts(const DgppFp4Matrix* w);
 /* src/kernels/scale_gemm.hpp:57-79. Dispatch (reference: src/kernels/scale_gemm.cu:296-339) between
  * the vector-core GEMV (up to eight rows per pass over the weights) or the matrix-core form (16 rows
  * per pass), chosen by what was measured faster on this chip: more rows than one vector pass holds -> matrix core; five
- * to eight rows -> matrix core when a split-K workspace is there (then from three rows on for matrices of 48 M weights
- * and more) or, without one, when the matrix has 64 M weights and more (an unsplit matrix-core launch has one block per
- * 64 weight rows: too few to fill the chip for smaller matrices); otherwise the vector core.
+ * to eight rows -> matrix core for matrices of 64 M weights and more, from 16 M on with k >= 4096, at any size when a split-K
+ * workspace is there (then from three rows on for matrices of 48 M weights and more); with k >= 4096 and n <= 20480 also
+ * from six rows on for 8 M weights and from four for 64 M; otherwise the vector core.
  * A positive mma_from_rows adds the calls with m >= mma_from_rows to the matrix-core side. `ws` / `ws_bytes` (nullable;
  * parts(k) * m * n floats) is the split-K workspace. Split and unsplit give the same bits; the two cores sum in
  * different fp32 orders (both held to the same oracle tolerance), so a row's bits depend on which form its call takes

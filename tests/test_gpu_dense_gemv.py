@@ -266,6 +266,48 @@ def test_fp8_dequant_bridge_is_bit_exact(gpu):
     assert np.array_equal(got[ok], want[ok])
 
 
+@pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "mxfp8"])
+@pytest.mark.parametrize("m,n,k", [(4, 4096, 4096), (5, 4096, 4096), (8, 4096, 4096), (6, 2048, 4096), (5, 256, 1024)])
+def test_a_rows_bits_do_not_depend_on_where_it_lies(gpu, kind, m, n, k):
+    """Which core a call takes is a function of its sizes: rows that are no whole 16-byte vectors give the bits of those that are, at
+    the sizes where the dispatch turns from one core to the other and beside them."""
+    w = hg.normal_f32(0x3C00 + k, (64, k), 0.02)      # 64 rows of weights, repeated
+    act = hg.normal_bf16(0x3C01 + m, (m, k))
+    wide = np.zeros((m, k + 1), np.uint16)
+    wide[:, :k] = act
+    if kind in ("nvfp4", "mxfp4"):
+        group = 16 if kind == "nvfp4" else 32
+        if group == 16:
+            payload, scales, ws2 = hg.encode_nvfp4(w)
+            glob = np.array([1.0 / np.float32(ws2)], np.float32)
+        else:
+            (payload, scales), glob = hg.encode_mxfp4(w), None
+        raw = orc.gemv_fp4(act, payload, scales, float(glob[0]) if glob is not None else 1.0, group, m, 64, k)
+        p_d, s_d, g_d = dev(np.tile(payload, (n // 64, 1))), dev(np.tile(scales, (n // 64, 1))), dev(glob) if glob is not None else None
+        mat = fp4_matrix(p_d, s_d, g_d, n, k, group)
+        run = lambda a, stride, out: L.launch_fp4_gemv_bf16(a, stride, mat, out, m, n, k)
+    elif kind == "mxfp8":
+        payload, scales = hg.encode_mxfp8(w)
+        raw = None
+        p_d, s_d = dev(np.tile(payload, (n // 64, 1))), dev(np.tile(scales, (n // 64, 1)))
+        run = lambda a, stride, out: L.launch_scale_gemm_grid_e8m0_bf16(a, stride, p_d, s_d, out, m, n, k, None, n, 0, 5)
+    else:
+        payload, scales = hg.encode_fp8_blocks(hg.f32_to_bf16(w), 64, 128)
+        raw = orc.gemv_fp8(act, payload, scales, m, 64, k, 6, 7, True)
+        p_d, s_d = dev(np.tile(payload, (n // 64, 1))), dev(np.tile(scales, (n // 64, 1)))
+        run = lambda a, stride, out: L.launch_scale_gemm_grid_bf16(a, stride, p_d, s_d, out, m, n, k, None, n, 6, 7)
+    got = []
+    for a, stride in ((dev(act), k), (dev(wide), k + 1)):
+        out = dev_empty((m, n), np.uint16)
+        run(a, stride, out)
+        sync()
+        got.append(host(out, np.uint16).copy())
+    assert np.array_equal(got[0], got[1])
+    assert np.array_equal(got[0], np.tile(got[0][:, :64], (1, n // 64))), "the same weights give the same bits in every tile"
+    if raw is not None:
+        check(np.ascontiguousarray(got[0][:, :64]), raw, kind)
+
+
 def test_fp8_gemv_multi_is_bitwise_the_single_launches(gpu):
     """launch_scale_gemv_multi_bf16 (reference: src/kernels/scale_gemm.hpp:88-107, its test
     scale_gemm_gemv_multi_is_bitwise_the_single_launches): up to four [n_i, k] matrices against the same rows, every
