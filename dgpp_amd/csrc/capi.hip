@@ -1709,34 +1709,43 @@ int dgpp_launch_scale_gemv_multi_bf16(const DgppFp8GemvProblem* problems, int n_
     if (!p.payload || !p.scales || !p.out || p.n <= 0) return fail_arg(std::string(who) + ": null pointer");
     if (!fp8_shape_ok(p.payload, k)) return fail_arg(std::string(who) + ": k must be a multiple of 16 with aligned payloads");
   }
-  // One launch over all problems' row tiles where the rows fit one stage (the decode case); otherwise one launch each.
-  if (tune_get(kTuneCore) != 2 && rows <= max_stage_rows(k)) {
-    DenseArgs d[kMaxDenseProblems];
-    for (int i = 0; i < n_problems; ++i) {
-      const DgppFp8GemvProblem& p = problems[i];
-      const size_t out_stride = p.out_stride ? p.out_stride : static_cast<size_t>(p.n);
-      if (out_stride < static_cast<size_t>(p.n)) return fail_arg(std::string(who) + ": output row stride narrower than n");
-      d[i].act = act;
-      d[i].act_stride = act_row_stride_elems;
-      d[i].mat = fp8_mat(p.payload, p.scales, p.rs, p.cs);
-      d[i].global = nullptr;
-      d[i].out = p.out;
-      d[i].out_stride = out_stride;
-      d[i].out_f32 = 0;
-      d[i].m = rows;
-      d[i].n = p.n;
-      d[i].k = k;
-      d[i].once = 1;
-    }
-    return finish(launch_dense_multi(kFmtFp8F32, d, n_problems, as_stream(stream)), who);
-  }
+  // A problem takes the core that its single launch takes, those of a core together in one launch.
+  DenseArgs d[2][kMaxDenseProblems];
+  int count[2] = {0, 0};   // on the vector core, on the matrix core
+  const int core = tune_get(kTuneCore);
   for (int i = 0; i < n_problems; ++i) {
     const DgppFp8GemvProblem& p = problems[i];
-    const int rc = scale_gemm(act, act_row_stride_elems, p.payload, p.scales, 0, p.out, 0, rows, p.n, k, stream,
-                              p.out_stride, p.rs, p.cs, 0, -1, false, who);
-    if (rc != DGPP_OK) return rc;
+    const size_t out_stride = p.out_stride ? p.out_stride : static_cast<size_t>(p.n);
+    if (out_stride < static_cast<size_t>(p.n)) return fail_arg(std::string(who) + ": output row stride narrower than n");
+    const bool mma = core != 1 && (core == 2 || dense_takes_matrix_core(kFmtFp8F32, rows, p.n, k, 0, false, 0));
+    DenseArgs& a = d[mma][count[mma]++];
+    a.act = act;
+    a.act_stride = act_row_stride_elems;
+    a.mat = fp8_mat(p.payload, p.scales, p.rs, p.cs);
+    a.global = nullptr;
+    a.out = p.out;
+    a.out_stride = out_stride;
+    a.out_f32 = 0;
+    a.m = rows;
+    a.n = p.n;
+    a.k = k;
+    a.once = 1;
   }
-  return DGPP_OK;
+  int rc = DGPP_OK;
+  auto one_by_one = [&](int which) {   // (dense_rows comes to the same core)
+    for (int i = 0; i < count[which] && rc == DGPP_OK; ++i) {
+      const DenseArgs& a = d[which][i];
+      rc = dense_rows(kFmtFp8F32, act, act_row_stride_elems, a.mat, nullptr, a.out, a.out_stride, 0, rows, a.n, k, as_stream(stream), who, 0);
+    }
+  };
+  if (count[1] > 1 && dense_mma_multi_fp8_takes(d[1], count[1]))
+    rc = finish(launch_dense_mma_multi_fp8(d[1], count[1], as_stream(stream)), who);
+  else
+    one_by_one(1);
+  if (rc != DGPP_OK || count[0] == 0) return rc;
+  if (rows <= max_stage_rows(k)) return finish(launch_dense_multi(kFmtFp8F32, d[0], count[0], as_stream(stream)), who);
+  one_by_one(0);   // the vector core pinned by the bench switch, in passes of the rows that it stages
+  return rc;
 }
 
 int dgpp_fp8_gemv_can_stage(const void* w_payload, int k) { return fp8_shape_ok(w_payload, k) ? 1 : 0; }

@@ -1000,6 +1000,9 @@ template <int FMT> hipError_t launch_token_down_fmt(const TokenDownArgs& a, hipS
 
 // The matrix-core launchers proper (the *_mma_* entry points).
 hipError_t launch_dense_mma(int fmt, const DenseArgs& a, float* ws, size_t ws_bytes, hipStream_t stream);
+// Up to four FP8 (F32 grid) problems of one k and m streamed in one launch, and whether they take it.
+bool dense_mma_multi_fp8_takes(const DenseArgs* problems, int count);
+hipError_t launch_dense_mma_multi_fp8(const DenseArgs* problems, int count, hipStream_t stream);
 // Two FP8 (F32 grid) problems of one k and m in one launch; ws as in launch_dense_mma (both problems' partials).
 hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, float* ws, size_t ws_bytes, hipStream_t stream);
 hipError_t launch_grouped_mma(int fmt, const GroupedArgs& a, int n_segs, int z_ext, hipStream_t stream);
@@ -1134,6 +1137,7 @@ inline bool grouped_fills_tiles(int fmt, bool a4, bool gate_up, int n_segs, int 
 // for up to eight activation rows when the row tiles just exceed a round. Bench switch 11: 1 never, 2 four, 3 two.
 constexpr size_t kTeamsMaxTiles = 256;
 constexpr size_t kTeamsMaxTilesHalf = 320;
+constexpr size_t kPairStreamTiles = 384;
 inline int dense_mfma_team_row_groups(int parts, int m, int n, bool plain) {
   const int knob = tune_get(kTuneTeams);
   if (!plain || parts != 4 || knob == 1) return 0;
@@ -1266,15 +1270,20 @@ hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, 
   return hipGetLastError();
 }
 
+// Blocks of a product's streaming form: whole rounds of the XCDs.
+inline int64_t stream_blocks(const DenseArgs& a, const MGeom& g) {
+  const int rows = kWavesPerBlock / g.parts * 2 * kGroupRows;
+  return static_cast<int64_t>(((a.n + rows - 1) / rows + kXcds - 1) / kXcds * kXcds) * ((a.m + kTileCols - 1) / kTileCols);
+}
 template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
   if (dense_takes_tiled<FMT>(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
   if (dense_takes_stream<FMT>(a, g)) {
-    const int rows = kWavesPerBlock / g.parts * 2 * kGroupRows, col_tiles = (a.m + kTileCols - 1) / kTileCols;
-    const dim3 grid(static_cast<unsigned>(((a.n + rows - 1) / rows + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(col_tiles));
-    if (a.m <= 8) hipLaunchKernelGGL((stream_dense_kernel<FMT, 8>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
-    else hipLaunchKernelGGL((stream_dense_kernel<FMT, 16>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
+    const int col_tiles = (a.m + kTileCols - 1) / kTileCols;
+    const dim3 grid(static_cast<unsigned>(stream_blocks(a, g)));
+    if (a.m <= 8) hipLaunchKernelGGL((stream_dense_kernel<FMT, 8, DenseArgs>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
+    else hipLaunchKernelGGL((stream_dense_kernel<FMT, 16, DenseArgs>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
     return hipGetLastError();
   }
   const unsigned gx = static_cast<unsigned>((a.n + 63) / 64), gy = static_cast<unsigned>((a.m + kTileCols - 1) / kTileCols);
@@ -1324,6 +1333,33 @@ hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, 
 }
 
 #ifdef DGPP_GEMV_PAIR
+// Several products in one streamed launch: their blocks are one grid, so that small products fill the chip together and a launch
+// each is saved. Measured, us, block FP8: two of 4096 x 4096, five rows 23.9 (the row tiles of both in one launch) or 18.7 (a streamed
+// launch each) -> 11.9; four of them, eight rows 77.6 (one vector-core launch) or 37.6 -> 18.9; four of 2048 x 4096, six rows 27.0 or
+// 35.2 -> 11.0. One part of K (k < 2048) gains nothing (2 x 8192 x 1024, 12 rows 9.0 against 9.4).
+bool dense_mma_multi_fp8_takes(const DenseArgs* p, int count) {
+  if (tune_get(kTuneTeams) != 0 || mgeom<kFmtFp8F32>(p[0].k).parts == 1) return false;
+  for (int i = 0; i < count; ++i)
+    if (!rows_stream(p[i].act, p[i].act_stride)) return false;
+  return true;
+}
+hipError_t launch_dense_mma_multi_fp8(const DenseArgs* p, int count, hipStream_t stream) {
+  constexpr int FMT = kFmtFp8F32;
+  const MGeom g = mgeom<FMT>(p[0].k);
+  DenseMultiArgs ma{};
+  ma.count = count;
+  int64_t end = 0;
+  for (int i = 0; i < count; ++i) {
+    ma.p[i] = p[i];
+    end += stream_blocks(p[i], g);
+    ma.tile_end[i] = static_cast<int>(end);
+  }
+  const int col_tiles = (p[0].m + kTileCols - 1) / kTileCols;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(end)), dim3(kBlockThreads), 0, stream, ma, g, col_tiles); };
+  if (p[0].m <= 8) go(stream_dense_kernel<FMT, 8, DenseMultiArgs>);
+  else go(stream_dense_kernel<FMT, 16, DenseMultiArgs>);
+  return hipGetLastError();
+}
 hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, float* ws, size_t ws_bytes, hipStream_t stream) {
   constexpr int FMT = kFmtFp8F32;
   const MGeom g = mgeom<FMT>(a0.k);
@@ -1331,6 +1367,12 @@ hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, f
   const unsigned gy = static_cast<unsigned>((a0.m + kTileCols - 1) / kTileCols);
   const size_t need = static_cast<size_t>(g.parts) * a0.m * (static_cast<size_t>(a0.n) + a1.n) * sizeof(float);
   const bool split = ws != nullptr && g.parts > 1 && ws_bytes >= need && static_cast<size_t>(t0 + t1) * gy < 1024;
+  // Without a workspace that both split over: streamed while the row tiles are no more than a round and a half of the chip.
+  // Row tiles -> streamed, us, at so many tiles: 64 (2048 x 4096, six rows) 16.3 -> 9.5, 128 24.1 -> 10.9, 256 25.9 -> 18.1, 384 26.6 ->
+  // 22.9 and 31.3 -> 31.5, 512 26.9 -> 27.9 and 18.6 -> 21.4, 768 34.6 -> 40.7.
+  const DenseArgs pair[2] = {a0, a1};
+  if (!split && static_cast<size_t>(t0 + t1) * gy <= kPairStreamTiles && dense_mma_multi_fp8_takes(pair, 2))
+    return launch_dense_mma_multi_fp8(pair, 2, stream);
   const dim3 grid(t0 + t1, gy, split ? g.parts : 1);
   hipError_t err = hipSuccess;
   dispatch_bool(a0.once != 0, [&](auto ntc) {

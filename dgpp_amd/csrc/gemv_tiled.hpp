@@ -858,6 +858,17 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
                                     nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, st);
 }
 
+// A streamed launch's product that the block belongs to; `lin`: the block's number in it.
+__device__ __forceinline__ const DenseArgs& stream_problem(const DenseArgs& a, int&) { return a; }
+__device__ __forceinline__ const DenseArgs& stream_problem(const DenseMultiArgs& ma, int& lin) {
+  int which = 0;
+#pragma unroll
+  for (int i = 0; i + 1 < kMaxDenseProblems; ++i)
+    if (i + 1 < ma.count && lin >= ma.tile_end[i]) which = i + 1;
+  if (which != 0) lin -= ma.tile_end[which - 1];
+  return ma.p[which];
+}
+
 // ---- up to sixteen activation rows ------------------------------------------------------------------------------------
 // A dense product of one column tile reads every weight once and is bound by that read, if enough of it is on its way: a
 // wavefront takes two row groups and ONE part of K, three tiles ahead, and meets nobody until the parts are folded, in
@@ -872,10 +883,14 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
 // to 4.6 of them the memory's (17408 x 5120, 544 blocks: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
 // slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half.
 // ROWS: activation rows that are loaded, 8 or 16 (those from m on repeat the last).
-template <int FMT, int ROWS>
-__global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(DenseArgs a, MGeom g, int col_tiles) {
+// Args: DenseArgs, or DenseMultiArgs: up to four products of one k and one row count in one launch, their blocks one after the other
+// (whole rounds of the XCDs each), each output bitwise its single launch's.
+template <int FMT, int ROWS, class Args>
+__global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(Args args, MGeom g, int col_tiles) {
+  int lin = static_cast<int>(blockIdx.x);
+  DenseArgs a = stream_problem(args, lin);
   // An XCD keeps a row tile's column tiles to itself, one after the other.
-  const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
+  const int idx = lin / kXcds;
   const int tile = idx / col_tiles * kXcds + lin % kXcds, c0 = idx % col_tiles * kTileCols;
   a.act += static_cast<size_t>(c0) * a.act_stride;
   a.m = min(a.m - c0, kTileCols);

@@ -455,8 +455,8 @@ int dgpp_launch_moe_grouped_mma_f32(const uint16_t* act, size_t act_stride, cons
                                     size_t out_stride, int n, int k, void* stream, const int32_t* act_rows);
 /* src/kernels/mma_gemv.hpp:103-104, :119-130 (mma_gemv_shape_ok, mma_gemv_pair_ok, launch_mma_gemv_fp8_bf16_pair): two
  * FP8 projections of one k against one batch in ONE launch - two dependent-free GEMVs sharing one ramp and drain.
- * Each row's bits are those of dgpp_launch_mma_gemv_fp8_bf16 on its own problem (up to eight rows: both problems in one
- * vector-core launch; more: one matrix-core launch). act_stride is both activations';
+ * Each row's bits are those of dgpp_launch_mma_gemv_fp8_bf16 on its own problem: both problems in one launch of the core that
+ * the single launches take, two launches where they take different ones. act_stride is both activations';
  * ws (nullable here) holds both problems' K-part sums: parts(k) * m * (n0 + n1) floats. pair_ok mirrors the reference's
  * conditions that carry over (a workspace, 1 <= m <= 32, both shapes taken, the workspace large enough). */
 int dgpp_mma_gemv_shape_ok(const void* w, const void* act, size_t act_stride, int m, int k);
@@ -577,8 +577,9 @@ int dgpp_launch_scale_gemm_tile_bf16(const uint16_t* act, size_t act_row_stride_
                                      const float* w_scales, uint16_t* out, int m, int n, int k, void* stream, int rs, int cs);
 int dgpp_launch_scale_gemm_tile_f32(const uint16_t* act, size_t act_row_stride_elems, const uint8_t* w_payload,
                                     const float* w_scales, float* out, int m, int n, int k, void* stream, int rs, int cs);
-/* src/kernels/scale_gemm.hpp:85-107: up to four [n_i, k] fp8 matrices against the same rows, ONE launch (the grid is the
- * problems' row tiles laid end to end); each output is bitwise the single launcher's.
+/* src/kernels/scale_gemm.hpp:85-107: up to four [n_i, k] fp8 matrices against the same rows, in one launch where their
+ * single launches take the same core (the grid is the problems' row tiles laid end to end; up to four rows always the vector
+ * core), else in a launch per core; each output is bitwise the single launcher's (without a workspace).
  * `problems` is a HOST array. bf16_weight must be null (that form is outside this path). */
 typedef struct DgppFp8GemvProblem {
   const uint8_t* payload;

@@ -348,6 +348,31 @@ def test_fp8_gemv_multi_is_bitwise_the_single_launches(gpu):
         L.launch_scale_gemv_multi_bf16([bad], act, k + 16, 1, k)                          # a bf16-weight problem
 
 
+@pytest.mark.parametrize("rows,k,ns,pad", [(5, 4096, (4096, 64, 4096), 0), (8, 4096, (2048, 4096, 1024, 2112), 0), (6, 5120, (4096, 3328), 1),
+                                           (4, 4096, (4096, 4096), 0), (5, 1024, (65536, 72), 0)])
+def test_fp8_gemv_multi_is_bitwise_the_single_launches_where_those_leave_the_vector_core(gpu, rows, k, ns, pad):
+    """Problems whose single launches take the matrix core (16 M weights from five rows on, 8 M from six), beside ones that do not, with
+    rows that are whole vectors and rows that are not (pad)."""
+    from dgpp_amd import _lib
+    rng = np.random.default_rng(k + rows)
+    act = dev(hg.normal_bf16(0x3D01 + rows, (rows, k + pad)))
+    outs, singles, problems, keep = [], [], [], []
+    for i, n in enumerate(ns):
+        codes = rng.integers(0, 120, (n, k), np.uint8) | (rng.integers(0, 2, (n, k), np.uint8) << 7)   # either sign, no NaN
+        p_d, s_d = dev(codes), dev(rng.uniform(0.5, 2.0, (-(-n // 64), -(-k // 128))).astype(np.float32) * np.float32(1e-3))
+        o, one = dev_empty((rows, n + 8), np.uint16), dev_empty((rows, n), np.uint16)
+        o.zero_()
+        problems.append(_lib.Fp8GemvProblem(p_d.data_ptr(), s_d.data_ptr(), o.data_ptr(), n, 0, n + 8, 6, 7, None))
+        L.launch_scale_gemm_grid_bf16(act, k + pad, p_d, s_d, one, rows, n, k, None, 0, 6, 7)
+        outs.append(o), singles.append(one), keep.append((p_d, s_d))
+    L.launch_scale_gemv_multi_bf16(problems, act, k + pad, rows, k)
+    sync()
+    for n, o, one in zip(ns, outs, singles):
+        got = host(o, np.uint16)
+        assert np.array_equal(got[:, :n], host(one, np.uint16)), f"n {n}"
+        assert not got[:, n:].any(), "columns past n stay untouched"
+
+
 def test_fp8_saturation_extremes(gpu):
     """The reference's scale_gemm_saturation_extremes (tests/cuda/scale_gemm_test.cu:501-532): all-maximum payloads
     (0x7E = 448) with scales of 1e30 (products near 1e35 stay finite in bf16 and fp32), and the minimum subnormal

@@ -315,7 +315,8 @@ def test_try_dense_fp4_decode_follows_the_shape_rule(gpu):
 
 
 @pytest.mark.parametrize("m,n0,n1,k,with_ws", [(1, 1536, 576, 7168, True), (8, 200, 130, 2048, False), (20, 96, 300, 1024, True),
-                                                (32, 64, 64, 4096, True)])
+                                                (32, 64, 64, 4096, True), (9, 200, 130, 2048, False), (17, 33, 64, 4096, False),
+                                                (30, 96, 300, 1024, False), (12, 40, 264, 5120, False)])
 def test_fp8_pair_launch_is_bitwise_the_two_single_launches(gpu, m, n0, n1, k, with_ws):
     """src/kernels/mma_gemv.hpp:119-130: two projections in one launch, each row's chain its single launch's."""
     acts = [hg.normal_bf16(0x6B0 + i + n0, (m, k)) for i in range(2)]
