@@ -466,6 +466,13 @@ int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_row
   }
   return blocks;
 }
+int dgpp_bench_tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int cols, int64_t* blocks) {
+  if (n_segs <= 0 || long_segs < 0 || long_segs > n_segs || row_tiles <= 0 || max_rows <= 0 || total_rows < 0 || (cols != kTiledCols && cols != kNarrowCols))
+    return -1;
+  const TiledPlan plan = tiled_plan(n_segs, long_segs, row_tiles, max_rows, total_rows, 0, cols);
+  if (blocks) *blocks = plan.items > 0 ? static_cast<int64_t>(plan.items) * row_tiles : 0;
+  return plan.items;
+}
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k) { return dense_fills_tiles(fmt, m, n, k) ? 1 : 0; }
 
 int dgpp_moe_config_validate(const DgppMoeConfig* c) {

@@ -716,18 +716,21 @@ static_assert(kXcds == 8, "the shifts above");
 // down 339 -> 323; NVFP4, 288 experts, 4096 tokens 549 -> 430; block FP8, 128 experts, 777 tokens 141 -> 132 and 80 -> 77.
 struct TiledPlan {
   TiledDeal deal;
-  int items;          // 0: by the deal; else no fewer than there are passes
+  int items;          // 0: by the deal; else no fewer than there are passes, a multiple of the XCDs
   int n_segs;
   dim3 grid() const {
-    return items > 0 ? dim3(static_cast<unsigned>((items + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(deal.row_tiles))
-                     : dim3(deal.grid_x(), deal.grid_y());
+    return items > 0 ? dim3(static_cast<unsigned>(items) * static_cast<unsigned>(deal.row_tiles)) : dim3(deal.grid_x(), deal.grid_y());
   }
 };
-// Sorted once every XCD has several items; with fewer, and where the rows are not known, by the deal.
+constexpr int kSortedSegs = 1 << 15;            // sorted_item counts segments in the halves of a word
+constexpr int64_t kSortedBlocks = 1 << 24;      // a launch takes fewer than 2^32 threads
+// Sorted once every XCD has several items; with fewer, where the rows are not known and beyond what it counts, by the deal.
 inline TiledPlan tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int tuned, int cols) {
-  const int64_t items = total_rows > 0 && tuned == 0 ? n_segs + total_rows / cols : 0;
-  return {tiled_deal(n_segs, long_segs, row_tiles, max_rows, tuned, cols),
-          items >= 8 * kXcds && items * row_tiles <= 1 << 24 ? static_cast<int>(items) : 0, n_segs};
+  int64_t items = total_rows > 0 && tuned == 0 ? n_segs + total_rows / cols : 0;
+  if (items < 8 * kXcds || n_segs >= kSortedSegs) items = 0;
+  items = (items + kXcds - 1) / kXcds * kXcds;
+  if (items >= kSortedBlocks || items * row_tiles >= kSortedBlocks) items = 0;
+  return {tiled_deal(n_segs, long_segs, row_tiles, max_rows, tuned, cols), static_cast<int>(items), n_segs};
 }
 struct TiledItem {
   int expert, row0, rows;

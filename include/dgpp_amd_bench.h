@@ -72,6 +72,10 @@ int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_se
  * (-1: nothing), row tile, first pass and step of its passes of 128 rows. Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */
 int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place);
 
+/* How many items the passes of a grouped launch of known rows are sorted into (0: dealt by segment): no fewer than a table of
+ * total_rows rows has passes of `cols` (128 or 32) rows. blocks: of that launch. -1: arguments out of range. Host arithmetic only. */
+int dgpp_bench_tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int cols, int64_t* blocks);
+
 /* Measurement aid with no counterpart in the reference: a plain streaming copy of `bytes`
  * (a multiple of 16; both pointers 16-byte aligned) on `stream`. A profiler's HBM byte counters
  * are calibrated against it: it reads `bytes` and writes `bytes`, nothing else. */

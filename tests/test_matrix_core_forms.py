@@ -94,6 +94,20 @@ def test_tiled_grouped_blocks_cover_every_pass_once_and_spread_long_segments(n_s
         assert {x for (s, _, _), x in seen.items() if s == seg} == {seg % 8}
 
 
+@pytest.mark.parametrize("cols", [32, 128])
+@pytest.mark.parametrize("n_segs,row_tiles,total_rows", [
+    (1, 4, 4096), (63, 8, 31), (64, 8, 1), (256, 32, 16384), (289, 64, 36864), (1024, 56, 655360), (32767, 1, 100), (32768, 1, 100),
+    (65535, 2, 100000), (64, 262143, 1), (64, 262144, 1), (56, 262144, 8 * 128), (61, 262144, 1), (1, 1, 1 << 29), (1, 2, 1 << 30)])
+def test_sorted_passes_hold_every_pass_within_what_they_count_and_what_a_launch_takes(cols, n_segs, row_tiles, total_rows):
+    blocks = np.zeros(1, np.int64)
+    items = _lib.load().dgpp_bench_tiled_plan(n_segs, 0, row_tiles, min(total_rows, 1 << 20), total_rows, cols, blocks.ctypes.data)
+    least = n_segs + total_rows // cols                     # passes of any table of so many segments and rows, at most
+    sorts = least >= 64 and n_segs < 1 << 15 and -(-least // 8) * 8 * row_tiles < 1 << 24
+    assert (items > 0) == sorts
+    if sorts:
+        assert items >= least and items % 8 == 0 and blocks[0] == items * row_tiles and blocks[0] * 256 < 1 << 32
+
+
 def test_the_streamed_shapes_hold_the_empty_parts_that_their_test_names():
     """K is cut in four parts of whole turns of four steps from 4096 elements on; FP4 steps are of 128."""
     from test_gpu_tiled import STREAM_SHAPES
