@@ -249,6 +249,7 @@ BENCH_SIGNATURES = {
     "dgpp_tune_get": (_I, [_I]),
     "dgpp_tune_enabled": (_I, []),
     "dgpp_bench_tiled_launches": (_I, []),
+    "dgpp_bench_form_launches": (_I, [_I]),
     "dgpp_bench_dense_takes_tiles": (_I, [_I, _I, _I, _I]),
     "dgpp_bench_grouped_takes_tiles": (_I, [_I, _I, _I, _I, _I, _I, _I, _I]),
     "dgpp_bench_tiled_place": (_I, [_I, _I, _I, _I, _I, _P]),

@@ -69,13 +69,13 @@ namespace dgpp_amd {
 // switch once). A build with -DDGPP_NO_TUNE compiles them out: every switch reads 0 and dgpp_tune_set does nothing.
 #ifdef DGPP_NO_TUNE
 int tune_get(int) { return 0; }
-void note_tiled_launch() {}
+void note_launch(int) {}
 #else
 static std::atomic<int> g_tune[kTuneCount];
 int tune_get(int key) { return key >= 0 && key < kTuneCount ? g_tune[key].load(std::memory_order_relaxed) : 0; }
-static std::atomic<int> g_tiled_launches;
-void note_tiled_launch() {
-  if (dgpp_tune_enabled()) g_tiled_launches.fetch_add(1, std::memory_order_relaxed);
+static std::atomic<int> g_launches[kFormCount];
+void note_launch(int form) {
+  if (dgpp_tune_enabled()) g_launches[form].fetch_add(1, std::memory_order_relaxed);
 }
 #endif
 
@@ -442,13 +442,15 @@ void dgpp_tune_set(int key, int value) {
 #endif
 }
 int dgpp_tune_get(int key) { return tune_get(key); }
-int dgpp_bench_tiled_launches(void) {
+int dgpp_bench_form_launches(int form) {
 #ifdef DGPP_NO_TUNE
+  (void)form;
   return 0;
 #else
-  return g_tiled_launches.load(std::memory_order_relaxed);
+  return form >= 0 && form < kFormCount ? g_launches[form].load(std::memory_order_relaxed) : 0;
 #endif
 }
+int dgpp_bench_tiled_launches(void) { return dgpp_bench_form_launches(kFormTiles); }
 int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_segs, int k, int max_rows, int total_rows,
                                    int long_segs) {
   return grouped_fills_tiles(fmt, act_nvfp4 != 0, gate_up != 0, n_segs, k, max_rows, total_rows, long_segs) ? 1 : 0;

@@ -1219,20 +1219,42 @@ inline bool grouped_takes_narrow(const GroupedArgs& a, int n_segs) {
 
 // Where the tiles do not take the launch, the plain product streams its weights (stream_dense_kernel). Measured, us, the
 // forms before it (parts side by side, over a workspace, row tiles) -> streaming, NVFP4, MXFP4, block FP8: 512 x 4096, 20 rows 15.0 ->
-// 8.0, 13.6 -> 6.0, 13.6 -> 8.0; 4096 x 4096, 20 rows 15.1 -> 8.8, 14.0 -> 6.6, 14.1 -> 8.8, 100 rows 26.8 -> 19.2, 26.0 -> 15.3, 28.2 -> 19.7;
-// 17408 x 5120, 6 rows 26.0 -> 21.6, 28.4 -> 18.8, 27.8 -> 29.0, 64 rows 74 -> 51, 77 -> 45, 72 -> 61; 16000 x 1024, 32 rows 10.6 -> 8.3, 11.2 ->
-// 6.4, 11.5 -> 8.9. Two corners stay as they were: block FP8 of up to eight rows just over one round of the chip (17408 rows
-// above), and NVFP4 with one part of K and few blocks (4096 x 1024, 20 rows 7.7 against 8.4). `act_up` and rows that are no
-// whole 16-byte vectors have no streaming form. Bench / test switch 11: 0, or one of the other forms.
+// 8.0, 13.6 -> 6.0, 13.6 -> 8.0; 4096 x 4096, 20 rows 15.1 -> 8.8, 14.0 -> 6.6, 14.1 -> 8.8; 17408 x 5120, 6 rows 26.0 -> 21.6, 28.4 ->
+// 18.8, 64 rows 74 -> 51, 77 -> 45; 16000 x 1024, 32 rows 10.6 -> 8.3, 11.2 -> 6.4, 11.5 -> 8.9.
+// Not where another form fills the chip better. A streaming block is 32, 64 or 128 rows with four, two or one parts of K, and takes
+// about as long beside another one on its CU as alone, so that just over a block per CU is its worst size. Time of the other form over
+// streaming's, over 500 shapes of 512 to 17408 rows of weights, 9 to 200 of activations (NVFP4 from one), by 64 x 16 tiles:
+// * block FP8 and MXFP8, one column tile, four parts: up to 128 tiles 1.1 to 2.1 (over a workspace 0.86 to 1.3), 129 to 256 0.79 to 0.97
+//   (0.74 to 1.0; block FP8 at 272 0.92 to 0.99 and 0.78, MXFP8 1.26 and 0.95), more column tiles 0.95 to 1.5. Two parts, block FP8: up
+//   to 256 tiles 1.3 to 1.8 (0.92 to 1.3), 257 to 288 0.86 (0.80);
+// * both over a workspace, longer rows, two to four column tiles, 129 to 192 tiles 0.82 to 1.1, on average 0.95 and 0.92; one column tile
+//   of more than ten rows, 33 to 64 tiles 0.86 to 0.96;
+// * both with one part, more than 512 and up to 768 tiles 0.72 to 1.08, on average 0.85 and 0.90; one column tile of 97 to 256 tiles 0.91 to 0.98;
+// * NVFP4 of one part, k up to 1024, up to 256 tiles 0.82 to 1.02, on average 0.93 (k = 1536 0.98 to 1.1); over a workspace, longer rows,
+//   one column tile of 129 to 160 tiles 0.85 to 1.0.
+// `act_up` and rows that are no whole 16-byte vectors have no streaming form. The bits are those of every other form.
+// Bench / test switch 11: 4 always (where it can), 1 to 3 one of the other forms. `split`: the workspace holds the parts of K.
 template <int FMT>
-inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g) {
-  if (tune_get(kTuneTeams) != 0 || a.act_up != nullptr || a.a4_scales != nullptr || !rows_stream(a.act, a.act_stride)) return false;
-  if (FMT == kFmtFp8F32 && dense_mfma_team_row_groups(g.parts, a.m, a.n, true) == 2) return false;
-  return !(FMT == kFmtNvfp4 && g.parts == 1 && a.m > kTileCols && dense_mfma_tiles(a.m, a.n) <= 256);
+inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g, bool split) {
+  const int knob = tune_get(kTuneTeams);
+  if (a.act_up != nullptr || a.a4_scales != nullptr || !rows_stream(a.act, a.act_stride) || (knob != 0 && knob != 4)) return false;
+  if (FMT == kFmtMxfp4 || knob == 4) return true;
+  const size_t tiles = dense_mfma_tiles(a.m, a.n);
+  const bool column = a.m <= kTileCols, longer = split && a.k > 4096;   // (k > 4096: four parts)
+  if constexpr (FMT == kFmtNvfp4) {
+    if (g.parts == 1) return a.k > 1024 || tiles > 256;
+    return !(longer && column && tiles > 128 && tiles <= 160);
+  }
+  if (g.parts == 1) return !(column && tiles > 96 && tiles <= 256) && !(tiles > 512 && tiles <= 768);
+  if (longer && a.m <= 4 * kTileCols && tiles > 128 && tiles <= 192) return false;
+  if (longer && column && a.m > 10 && tiles > 32 && tiles <= 64) return false;
+  if (!column) return true;
+  const size_t blocks = tiles * static_cast<size_t>(g.parts) / 2;
+  return blocks <= 256 || (FMT == kFmtFp8F32 ? blocks > 640 : g.parts == 2 || blocks > 512);
 }
 template <int FMT>
 hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
-  note_tiled_launch();
+  note_launch(kFormTiles);
   const MGeom g = mgeom<FMT>(a.k);
   const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows, passes = (a.m + kTiledCols - 1) / kTiledCols;
   const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
@@ -1251,7 +1273,7 @@ hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
 
 template <int FMT, int COLS>
 hipError_t launch_grouped_tiled(const GroupedArgs& a, int n_segs, int max_rows, hipStream_t stream) {
-  if (COLS == kTiledCols) note_tiled_launch();
+  note_launch(COLS == kTiledCols ? kFormTiles : kFormNarrow);
   const MGeom g = mgeom<FMT>(a.k);
   const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
   const int row_tiles = (a.n + block_rows - 1) / block_rows;
@@ -1279,7 +1301,10 @@ template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
   if (dense_takes_tiled<FMT>(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
-  if (dense_takes_stream<FMT>(a, g)) {
+  const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
+  const bool split = ws != nullptr && ws_bytes >= need && dense_mfma_would_split(g.parts, a.m, a.n) && a.a4_scales == nullptr;
+  if (dense_takes_stream<FMT>(a, g, split)) {
+    note_launch(kFormStreamed);
     const int col_tiles = (a.m + kTileCols - 1) / kTileCols;
     const dim3 grid(static_cast<unsigned>(stream_blocks(a, g)));
     if (a.m <= 8) hipLaunchKernelGGL((stream_dense_kernel<FMT, 8, DenseArgs>), grid, dim3(kBlockThreads), 0, stream, a, g, col_tiles);
@@ -1287,8 +1312,6 @@ hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, 
     return hipGetLastError();
   }
   const unsigned gx = static_cast<unsigned>((a.n + 63) / 64), gy = static_cast<unsigned>((a.m + kTileCols - 1) / kTileCols);
-  const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
-  const bool split = ws != nullptr && ws_bytes >= need && dense_mfma_would_split(g.parts, a.m, a.n) && a.a4_scales == nullptr;
   const dim3 grid(gx, gy, split ? g.parts : 1);
   hipError_t err = hipSuccess;
   // Without a workspace the four parts of K run side by side inside a block while the row tiles alone would leave
@@ -1325,6 +1348,7 @@ hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, 
   });
   if (err != hipSuccess) return err;
   if (split) {
+    note_launch(kFormSplit);
     const int64_t total = static_cast<int64_t>(a.m) * a.n;
     hipLaunchKernelGGL(fold_parts_kernel<FMT>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, stream, ws,
                        g.parts, a.m, a.n, a.global, a.out, a.out_f32, a.out_stride);
@@ -1338,13 +1362,14 @@ hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, 
 // launch each) -> 11.9; four of them, eight rows 77.6 (one vector-core launch) or 37.6 -> 18.9; four of 2048 x 4096, six rows 27.0 or
 // 35.2 -> 11.0. One part of K (k < 2048) gains nothing (2 x 8192 x 1024, 12 rows 9.0 against 9.4).
 bool dense_mma_multi_fp8_takes(const DenseArgs* p, int count) {
-  if (tune_get(kTuneTeams) != 0 || mgeom<kFmtFp8F32>(p[0].k).parts == 1) return false;
+  if ((tune_get(kTuneTeams) & 3) != 0 || mgeom<kFmtFp8F32>(p[0].k).parts == 1) return false;
   for (int i = 0; i < count; ++i)
     if (!rows_stream(p[i].act, p[i].act_stride)) return false;
   return true;
 }
 hipError_t launch_dense_mma_multi_fp8(const DenseArgs* p, int count, hipStream_t stream) {
   constexpr int FMT = kFmtFp8F32;
+  note_launch(kFormStreamed);
   const MGeom g = mgeom<FMT>(p[0].k);
   DenseMultiArgs ma{};
   ma.count = count;
@@ -1384,6 +1409,7 @@ hipError_t launch_dense_mma_pair_fp8(const DenseArgs& a0, const DenseArgs& a1, f
   });
   if (err != hipSuccess) return err;
   if (split) {
+    note_launch(kFormSplit);
     const DenseArgs* both[2] = {&a0, &a1};
     float* at = ws;
     for (const DenseArgs* a : both) {

@@ -424,7 +424,7 @@ summed:
 template <typename Out, int WN, int WM, int DEPTH>
 hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* ws, Out* out, int m, int n,
                              int k, size_t stride, hipStream_t stream) {
-  note_tiled_launch();
+  note_launch(kFormTiles);
   constexpr int tn = 32 * WN, tm = 32 * WM;
   const int row_tiles = (n + tn - 1) / tn, passes = (m + tm - 1) / tm;
   const dim3 grid(static_cast<unsigned>((row_tiles + 7) / 8 * 8) * static_cast<unsigned>(passes));

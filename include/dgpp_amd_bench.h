@@ -31,10 +31,11 @@ extern "C" {
  * on the caller's stream, 2 moves them to a second stream beside the routed passes at every batch size (default:
  * from three tokens on); 3 and 4 keep one stream and never / always fold the accumulation into the shared down pass
  * (default: at one token); key 10: 2 or 4 runs the router's token-tiled score kernel at every batch size with that many tokens per
- * wavefront (0 = automatic: tiled from 32 rows on, 4 tokens from 128 rows on); key 11: the dense matrix-core launch
- * without a workspace that runs the four parts of K side by side inside a block: 1 never, 2 always with four row groups
- * per block, 3 with two for up to eight rows (0 = automatic: four while the row tiles fit one round of the chip, two for up
- * to a round and a quarter); key 12: 1 makes dgpp_launch_moe_slot_chain* run the launches the one-launch chain stands for, 2 makes
+ * wavefront (0 = automatic: tiled from 32 rows on, 4 tokens from 128 rows on); key 11: the form of the dense matrix-core
+ * launch below the tiles: 4 streamed wherever the rows are whole 16-byte vectors, 1 to 3 not streamed; without a workspace 1
+ * row tiles, 2 the four parts of K side by side inside a block of four row groups, 3 of two for up to eight rows (0 = automatic:
+ * streamed except where another form fills the chip better; else four row groups while the row tiles fit one round of the chip,
+ * two up to a round and a quarter); key 12: 1 makes dgpp_launch_moe_slot_chain* run the launches the one-launch chain stands for, 2 makes
  * the layer driver take the one-launch chain for small routed-only decode batches (default: the driver runs the
  * launches; the chain measured slower); key 13: row steps per wavefront of the chain's down part (0 = automatic);
  * key 14: the fused gate + up matrix-core grouped launch: 1 = every wavefront walks both matrices in turn, 2 = the block's
@@ -57,6 +58,9 @@ int dgpp_tune_enabled(void);
 
 /* How many launches took a form of key 15's tiles so far, counted in a process that enabled the switches. */
 int dgpp_bench_tiled_launches(void);
+/* Likewise by form: 0 those, 1 the grouped passes of 32 rows, 2 streamed dense products, 3 dense products whose parts of K were
+ * split over a workspace. */
+int dgpp_bench_form_launches(int form);
 
 /* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):
  * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a

@@ -301,6 +301,7 @@ def test_narrow_passes_are_bitwise_the_16_row_form(gpu, kind, E, T, K, H, I):
     for form in (1, 3):
         out.fill_(0x55)
         _lib.load().dgpp_tune_set(15, form)
+        before = _lib.load().dgpp_bench_form_launches(1)
         try:
             if kind == "w4a4":
                 layer.enqueue_prefill_routed_w4a4(d.x, H, ids_d, w, out, T)
@@ -309,6 +310,7 @@ def test_narrow_passes_are_bitwise_the_16_row_form(gpu, kind, E, T, K, H, I):
         finally:
             _lib.load().dgpp_tune_set(15, 0)
         sync()
+        assert _lib.load().dgpp_bench_form_launches(1) - before == (0 if form == 1 else 3 if kind == "w4a4" else 2)
         got.append(host(out, np.uint16).copy())
     layer.close()
     assert np.array_equal(got[0], got[1])
@@ -343,7 +345,7 @@ STREAM_SHAPES = [(1, 1, 4096), (8, 33, 5120), (9, 31, 2048), (16, 130, 1152), (1
 @pytest.mark.parametrize("m,n,k", STREAM_SHAPES)
 def test_streaming_dense_form_is_bitwise_the_row_tile_form(gpu, kind, m, n, k):
     """The dense launch that streams its weights, a part of K to a wavefront, against the form that walks the parts in turn
-    (bench switch 11: 1): one to four parts, row groups and column tiles at their edges, tiles of k that are whole, part and
+    (bench switch 11: 4, 1): one to four parts, row groups and column tiles at their edges, tiles of k that are whole, part and
     none, rows that no vector load reads; FP4 at 4352, 4160 and 4576 has an empty part, the last two with a part tile before it."""
     if kind in ("nvfp4", "mxfp4"):
         group = 16 if kind == "nvfp4" else 32
@@ -373,13 +375,15 @@ def test_streaming_dense_form_is_bitwise_the_row_tile_form(gpu, kind, m, n, k):
     lib.dgpp_tune_set(5, 2)
     lib.dgpp_tune_set(15, 1)
     try:
-        for knob in (1, 0):
+        for knob in (1, 4):
             for a, stride in rows:
+                before = lib.dgpp_bench_form_launches(2)
                 lib.dgpp_tune_set(11, knob)
                 out = dev_empty((m, n + 3), np.float32)
                 out.fill_(-7.0)
                 run(a, stride, out)
                 sync()
+                assert lib.dgpp_bench_form_launches(2) - before == (knob == 4 and stride == k), "streamed, if the rows are whole vectors"
                 got.append(host(out).copy())
     finally:
         for key in (5, 11, 15):
@@ -414,11 +418,13 @@ def test_walks_that_end_with_part_of_a_turn_are_bitwise_the_16_row_form(gpu, kin
     for form in (1, 2, 3):
         out.fill_(-7.0)
         _lib.load().dgpp_tune_set(15, form)
+        before = [_lib.load().dgpp_bench_form_launches(f) for f in (0, 1)]
         try:
             plain(x, k, segs, E, max(rows), 0, d.views, 1, out, 128, 128, k, None, None, *more)
         finally:
             _lib.load().dgpp_tune_set(15, 0)
         sync()
+        assert [_lib.load().dgpp_bench_form_launches(f) - b for f, b in zip((0, 1), before)] == [form == 2, form == 3]
         got.append(host(out).copy())
     assert (got[0] != -7.0).all()
     for g in got[1:]:
