@@ -15,6 +15,19 @@ from test_gpu_dense_gemv import check, make_fp4
 
 pytestmark = pytest.mark.gpu
 
+def over_the_workspace(run, splits):
+    """run() with the streaming form off (bench switch 11: 1), which would not use the workspace; `splits`: whether each launch of it
+    has its parts of K in separate blocks then."""
+    lib = _lib.load()
+    lib.dgpp_tune_set(11, 1)
+    before = lib.dgpp_bench_form_launches(3)
+    try:
+        launches = run()
+    finally:
+        lib.dgpp_tune_set(11, 0)
+    assert lib.dgpp_bench_form_launches(3) - before == (launches if splits else 0)
+
+
 FP4_SHAPES = [(1, 520, 4096), (5, 200, 1024), (16, 100, 2048), (37, 130, 5120), (8, 64, 160), (3, 33, 576),
               (20, 77, 6144), (2, 16, 32), (4, 45, 4160), (19, 40, 4576)]   # the last two: an empty part of k behind a part of a step
 
@@ -43,6 +56,17 @@ def test_dense_mma_fp4_matches_oracle_and_rows_are_independent(gpu, group, m, n,
     assert np.array_equal(hg.f32_to_bf16(host(outsf)[:, :n]), got), "the split form's unrounded output rounds to the same bits"
     check(got, raw, f"dense mma fp4 g{group} {m}x{n}x{k}")
     assert np.array_equal(hg.f32_to_bf16(host(outf)), got), "bf16(out_f32) == out_bf16"
+    for t in (outs, outsf, ws):
+        t.fill_(0x55)
+
+    def split():
+        L.launch_mma_gemv_fp4_bf16(act_d, k, w, outs, m, n, k, n + 8, None, ws, 4 * m * n * 4)
+        L.launch_mma_gemv_fp4_f32(act_d, k, w, outsf, m, n, k, n + 8, None, ws, 4 * m * n * 4)
+        return 2
+    over_the_workspace(split, k >= 2048)
+    sync()
+    assert np.array_equal(host(outs, np.uint16)[:, :n], got), "parts of K in separate blocks: the same bits"
+    assert np.array_equal(hg.f32_to_bf16(host(outsf)[:, :n]), got)
     assert np.array_equal(host(one, np.uint16)[0], got[m - 1]), "a row's bits do not depend on the rows beside it"
 
 
@@ -78,6 +102,15 @@ def test_mma_gemv_fp8_matches_oracle_split_and_unsplit(gpu, e8m0, rs, cs, m, n, 
     check(got, raw, f"mma gemv fp8 e8m0={e8m0} {m}x{n}x{k} rs{rs} cs{cs}")
     assert np.array_equal(hg.f32_to_bf16(host(outf)), got)
     assert np.array_equal(host(outs, np.uint16), got), "the split form's bits are the unsplit form's"
+    for t in (outs, ws):
+        t.fill_(0x55)
+
+    def split():
+        fn_b(a_d, k, p_d, s_d, outs, m, n, k, 0, rs, cs, None, ws, 4 * m * n * 4)
+        return 1
+    over_the_workspace(split, k >= 2048 and m >= 5)   # fewer rows keep to the vector core
+    sync()
+    assert np.array_equal(host(outs, np.uint16), got), "parts of K in separate blocks: the same bits"
     if not e8m0 and rs == 7 and cs == 7:
         outd, outdf = dev_empty((m, n), np.uint16), dev_empty((m, n), np.float32)
         L.launch_dense_mma_bf16(a_d, k, p_d, s_d, outd, m, n, k, None)
