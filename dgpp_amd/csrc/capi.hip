@@ -455,6 +455,10 @@ int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_se
                                    int long_segs) {
   return grouped_fills_tiles(fmt, act_nvfp4 != 0, gate_up != 0, n_segs, k, max_rows, total_rows, long_segs) ? 1 : 0;
 }
+int dgpp_bench_grouped_takes_narrow(int fmt, int act_nvfp4, int gate_up, int n_segs, int n, int k, int max_rows, int total_rows,
+                                    int long_segs) {
+  return grouped_fills_narrow(fmt, act_nvfp4 != 0, gate_up != 0, n_segs, n, k, max_rows, total_rows, long_segs) ? 1 : 0;
+}
 int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place) {
   if (n_segs <= 0 || long_segs < 0 || long_segs > n_segs || row_tiles <= 0 || max_rows <= 0) return 0;
   const TiledDeal d = tiled_deal(n_segs, long_segs, row_tiles, max_rows, 0);
@@ -1442,7 +1446,8 @@ int dgpp_launch_mma_gemv_fp4_bf16_static(const uint16_t* act, size_t act_stride,
   if (k <= 0 || k % 32 != 0) return fail_arg(std::string(who) + ": k must be a positive multiple of 32");
   const int parts = w && w->scale_group == 32 ? mgeom<kFmtMxfp4>(k).parts : mgeom<kFmtNvfp4>(k).parts;
   // Only the split form uses the workspace: a launch that would run unsplit anyway (one part, or row tiles that fill
-  // the chip by themselves) needs none and is never refused for its size.
+  // the chip by themselves) needs none and is never refused for its size. Whether the rows let the launch stream is not asked:
+  // what is refused must not depend on where they lie.
   if (!dense_mma_would_split(parts, m, n)) return dense_mma_fp4(act, act_stride, w, out, 0, m, n, k, stream, out_stride, nullptr, 0);
   const size_t need = static_cast<size_t>(parts) * static_cast<size_t>(m) * static_cast<size_t>(n) * sizeof(float);
   if (need > kStaticScratchBytes)

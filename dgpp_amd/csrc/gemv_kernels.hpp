@@ -1099,9 +1099,10 @@ inline bool dense_fills_tiles(int fmt, int m, int n, int k) {
 }
 
 // Whether a grouped launch takes the tiles of up to 128 activation rows (gemv_tiled.hpp) or the 16-row form, where the passes of 32
-// rows (grouped_takes_narrow) do not come first: by the rows of a segment on average. The figures are of tiles with one tile on
-// its way; with three the 128-row passes are level with the 16-row form at half of these rows, which the 32-row passes now take.
-// A pass of the tiles costs the same for a few rows as for 32, the 16-row form grows with every 16. A block of
+// rows (grouped_fills_narrow, below) do not come first: by the rows of a segment on average. They come first wherever the rows are
+// known and few, so this line decides for the layer driver between those passes and the 128-row ones from `most` rows on, and for the
+// entry points, which do not know the rows, between 128-row passes and the 16-row form. The figures are of tiles with one tile on
+// its way; with three the 128-row passes are level with the 16-row form at half of these rows. A pass of the tiles costs the same for a few rows as for 32, the 16-row form grows with every 16. A block of
 // the tiles spends its start on a pass that a short k does not repay, so the line rises as k falls; gate + up in one launch
 // walks twice the weights per start, and the 16-row form holds half as many of them: its line is lower. Measured, time of the
 // tiles over the 16-row form's, 128 and 288 segments, n = 384 to 7168, at rows per segment:
@@ -1129,6 +1130,34 @@ inline bool grouped_fills_tiles(int fmt, bool a4, bool gate_up, int n_segs, int 
   else if (fmt == kFmtMxfp4) least = gate_up ? 7 : 9, start = gate_up ? 0 : 8192;
   else least = gate_up ? 11 : 12, start = gate_up ? 6144 : 20480;
   return rows * k >= n_segs * (least * k + start);
+}
+
+// Whether a grouped launch of a known number of rows takes the kernel of 32-row passes: three blocks per CU and four stages of
+// LDS where the 128-row passes have two and two, but a weight decoded once per 32 rows. Short segments: against the 16-row form
+// below the line above, and against the 128-row passes up to `most` rows a segment, twice that where a pass's walk of k is short;
+// segments of up to 128 rows, and those that the 16-row form would take, at any length. Fewer segments than XCDs (a shared
+// expert's own): where the 128-row passes would be one round of the chip at most. A block-FP8 shared expert beside 16 x 768 x
+// 2048, whole layer, 16-row form / 128-row / 32-row passes, us: 40 tokens 137 / 80 / 74, 100 266 / 110 / 85, 256 579 / 128 / 117. Measured over whole layers, time over the 16-row form's, 128-row / 32-row passes, at rows
+// per segment (experts x inter x hidden):
+//   NVFP4      128 x 512 x 4096   1: 1.11 / 0.94, 4: 0.98 / 0.88, 16: 0.63 / 0.55, 25: 0.46 / 0.45, 44: 0.42 / 0.43
+//              256 x 2048 x 6144  1.2: 1.09 / 0.97, 5: 0.95 / 0.88, 12: 0.63 / 0.60, 22: 0.55 / 0.58; 9 experts, 36: 0.50 / 0.53
+//   MXFP4      256 x 1024 x 4096  0.5: 0.90 / 0.81, 5: 0.70 / 0.65, 12: 0.53 / 0.51, 22: 0.44 / 0.45
+//   block FP8  128 x 768 x 2048   2.5: 1.00 / 0.95, 6: 0.84 / 0.79, 16: 0.58 / 0.55, 25: 0.47 / 0.49
+//              256 x 2048 x 7168  3.1: 1.05 / 1.03, 4: 0.99 / 0.97, 6: 0.93 / 0.91, 10: 0.82 / 0.85
+//   NVFP4 activations, 128 x 2048 x 6144  1: 1.18 / 1.09, 4: 0.95 / 0.88, 16: 0.56 / 0.54, 25: 0.40 / 0.42
+// Bench / test switch 15: 3 always (where it can).
+inline bool grouped_fills_narrow(int fmt, bool a4, bool gate_up, int n_segs, int n, int k, int max_rows, int64_t total_rows, int long_segs) {
+  if (total_rows <= 0) return false;
+  const bool fp4 = fmt == kFmtNvfp4 || fmt == kFmtMxfp4;
+  const int64_t rows = total_rows, least = a4 || !fp4 ? 4 : (fmt == kFmtNvfp4 ? 1 : 0);
+  if (rows < least * n_segs) return false;
+  if (n_segs < kXcds) {
+    const int block_rows = gate_up ? kTiledRows / 2 : kTiledRows;
+    return (n + block_rows - 1) / block_rows * (n_segs + rows / kTiledCols) <= 256;
+  }
+  const int64_t most = (fp4 ? 16 : 8) * (k < 1024 ? 2 : 1);
+  return max_rows <= kTiledCols || rows <= most * n_segs ||
+         !grouped_fills_tiles(fmt, a4, gate_up, n_segs, k, max_rows, total_rows, long_segs);
 }
 
 // Row groups per block of the dense matrix-core launch that runs the four parts of K side by side inside a block
@@ -1185,36 +1214,12 @@ inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
   return grouped_fills_tiles(FMT, a.a4_scales != nullptr, a.gate_up != 0, n_segs, a.k, a.max_rows, a.total_rows, a.long_segs);
 }
 
-// Whether a grouped launch of a known number of rows takes the kernel of 32-row passes: three blocks per CU and four stages of
-// LDS where the 128-row passes have two and two, but a weight decoded once per 32 rows. Short segments: against the 16-row form
-// below the line above, and against the 128-row passes up to `most` rows a segment, twice that where a pass's walk of k is short;
-// segments of up to 128 rows, and those that the 16-row form would take, at any length. Fewer segments than XCDs (a shared
-// expert's own): where the 128-row passes would be one round of the chip at most. A block-FP8 shared expert beside 16 x 768 x
-// 2048, whole layer, 16-row form / 128-row / 32-row passes, us: 40 tokens 137 / 80 / 74, 100 266 / 110 / 85, 256 579 / 128 / 117. Measured over whole layers, time over the 16-row form's, 128-row / 32-row passes, at rows
-// per segment (experts x inter x hidden):
-//   NVFP4      128 x 512 x 4096   1: 1.11 / 0.94, 4: 0.98 / 0.88, 16: 0.63 / 0.55, 25: 0.46 / 0.45, 44: 0.42 / 0.43
-//              256 x 2048 x 6144  1.2: 1.09 / 0.97, 5: 0.95 / 0.88, 12: 0.63 / 0.60, 22: 0.55 / 0.58; 9 experts, 36: 0.50 / 0.53
-//   MXFP4      256 x 1024 x 4096  0.5: 0.90 / 0.81, 5: 0.70 / 0.65, 12: 0.53 / 0.51, 22: 0.44 / 0.45
-//   block FP8  128 x 768 x 2048   2.5: 1.00 / 0.95, 6: 0.84 / 0.79, 16: 0.58 / 0.55, 25: 0.47 / 0.49
-//              256 x 2048 x 7168  3.1: 1.05 / 1.03, 4: 0.99 / 0.97, 6: 0.93 / 0.91, 10: 0.82 / 0.85
-//   NVFP4 activations, 128 x 2048 x 6144  1: 1.18 / 1.09, 4: 0.95 / 0.88, 16: 0.56 / 0.54, 25: 0.40 / 0.42
-// Bench / test switch 15: 3 always (where it can).
 template <int FMT>
 inline bool grouped_takes_narrow(const GroupedArgs& a, int n_segs) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || knob == 2 || a.rows_per_block != INT_MAX || !tiled_rows_aligned(a)) return false;
   if (knob == 3) return true;
-  if (a.total_rows <= 0) return false;
-  const bool a4 = a.a4_scales != nullptr, fp4 = FMT == kFmtNvfp4 || FMT == kFmtMxfp4;
-  const int64_t rows = a.total_rows, least = a4 || !fp4 ? 4 : (FMT == kFmtNvfp4 ? 1 : 0);
-  if (rows < least * n_segs) return false;
-  if (n_segs < kXcds) {
-    const int block_rows = a.gate_up != 0 ? kTiledRows / 2 : kTiledRows;
-    return (a.n + block_rows - 1) / block_rows * (n_segs + rows / kTiledCols) <= 256;
-  }
-  const int64_t most = (fp4 ? 16 : 8) * (a.k < 1024 ? 2 : 1);
-  return a.max_rows <= kTiledCols || rows <= most * n_segs ||
-         !grouped_fills_tiles(FMT, a4, a.gate_up != 0, n_segs, a.k, a.max_rows, a.total_rows, a.long_segs);
+  return grouped_fills_narrow(FMT, a.a4_scales != nullptr, a.gate_up != 0, n_segs, a.n, a.k, a.max_rows, a.total_rows, a.long_segs);
 }
 
 // Where the tiles do not take the launch, the plain product streams its weights (stream_dense_kernel). Measured, us, the

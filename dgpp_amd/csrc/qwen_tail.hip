@@ -3,8 +3,8 @@
 //   out = bf16(fma(sw, act . down_w, routed accumulation))                                         (one launch)
 // Every dot is the dense FP8 GEMV's own chain (the same row geometry and row_dots), the SwiGLU is the
 // slot kernels' epilogue without clamps, the accumulation is the accumulate kernels' fma, so the tail is
-// bitwise the unfused chain of launchers it stands for: two grid GEMVs to BF16, swiglu_clamp, a grid GEMV
-// to F32, the shared gate, accumulate, round.
+// bitwise the unfused chain of launchers it stands for, on the vector core: two grid GEMVs to BF16, swiglu_clamp, a grid
+// GEMV to F32, the shared gate, accumulate, round. (From four tokens on the GEMV launchers take large matrices to the matrix core.)
 //
 // Reference counterparts: src/kernels/qwen_moe.hpp:12-87 (interface), src/kernels/qwen_moe.cu:27-56
 // (shared gate), :60-120 (gate/up + SwiGLU), :122-198 (down with the accumulation in the epilogue),

@@ -399,7 +399,7 @@ int dgpp_launch_moe_grouped_gemv_fp4_f32(const uint16_t* act, size_t act_stride,
  * launchers' (another summation order) and is held to the same oracle tolerance.
  * act_rows (nullable): segment row i reads activation row act_rows[i] (the gather folded in).
  * ws / ws_bytes (nullable): room for parts(k) * m * n floats lets an under-filled grid run the K parts in
- * separate blocks plus one folding launch. rows_per_block: segment rows per z block (0 = all).
+ * separate blocks plus one folding launch, where that is faster than the forms that need no workspace. rows_per_block: segment rows per z block (0 = all).
  * tile_rows is accepted for the signature and ignored. */
 int dgpp_launch_dense_mma_bf16(const uint16_t* act, size_t act_stride, const uint8_t* payload, const float* scales,
                                uint16_t* out, int m, int n, int k, void* stream, size_t out_stride);
@@ -421,7 +421,8 @@ int dgpp_launch_mma_gemv_fp4_f32(const uint16_t* act, size_t act_stride, const D
  * bits. Only launches that would run split use the workspace (more than one K part: parts = 4 from k = 4096, 2 from
  * k = 2048; and fewer than 1024 tiles of 64 weight rows x 16 activation rows); of those, parts(k) * m * n floats
  * beyond the static workspace are refused with DGPP_INVALID_ARGUMENT. Every other launch runs unsplit, uses no
- * workspace and is never refused for its size. Every split call on a GPU shares that GPU's array, so the array is
+ * workspace and is never refused for its size. (The rule is by size: a call that it names is refused and bound as said also
+ * where the launch turns out to stream its weights and to leave the workspace alone.) Every split call on a GPU shares that GPU's array, so the array is
  * BOUND to the stream of the first split call: a split call on another stream of that GPU is refused with
  * DGPP_INVALID_ARGUMENT (calls on two streams could overlap and race on the array; calls on one stream follow each
  * other) until dgpp_static_scratch_release() - to be called once the bound stream's work is done - frees the
@@ -709,7 +710,8 @@ int dgpp_qwen_moe_shared_gate_bf16(const uint16_t* x, const uint16_t* g, float* 
  * tokens <= 8 (one pass over the weights for all of them), H and S multiples of 16, operands 16-byte aligned.
  * Each launch is bitwise the unfused launchers it stands for (dgpp_launch_scale_gemm_grid_bf16 twice,
  * dgpp_launch_moe_swiglu_clamp with an infinite limit, dgpp_launch_scale_gemm_grid_f32, the gate, the accumulate,
- * dgpp_launch_moe_round_bf16). The halves are entries of their own so that gate_up can run beside the routed
+ * dgpp_launch_moe_round_bf16), with the projections on the vector core: from four tokens on dgpp_launch_scale_gemm_grid_*
+ * itself takes large matrices to the matrix core (its comment says from where), which sums in another order. The halves are entries of their own so that gate_up can run beside the routed
  * experts on another stream; the BF16-weight forms of the reference's tail are not provided. */
 int dgpp_qwen_moe_shared_gate_up_decode_fp8(const uint16_t* x, size_t x_stride, const uint8_t* gate_p, const float* gate_s,
                                             const uint8_t* up_p, const float* up_s, const uint16_t* g, uint16_t* act, float* sw,

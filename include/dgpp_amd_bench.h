@@ -15,40 +15,40 @@ extern "C" {
  * the new value), 0 everywhere = the product behaviour. They are inert unless the process opted in through the
  * environment (DGPP_AMD_BENCH=1, see dgpp_tune_enabled); a library built with -DDGPP_NO_TUNE leaves them out
  * (dgpp_tune_set stores nothing, dgpp_tune_get returns 0). The reference keeps such a switch in its launcher header
- * too: moe_set_fp8_ldm, src/kernels/glm_moe_launch.hpp:90.
- * key 0: preferred chunks per lane of the row geometry (0 = default 4); key 1: slots of one expert a
- * decode-slot block serves together (0 = default: 2 gate/up, 4 down; 1 = one slot per block);
- * key 2: row steps per block of the slot launches (0 = automatic); key 3: 1 stages activations before
- * any weight load is issued (default: activation loads, first weight pass, LDS commit); key 4: 1 keeps
- * the layer driver on the two-launch down + accumulate form; key 5: 2 moves every GEMV launcher to the
- * matrix-core form, 1 keeps the dense launchers on the vector core at every row count (default: the dense launchers
- * choose by rows, matrix size and workspace); key 6: 1 makes the layer driver compute the slot order for small decode batches too
- * (default: batches of at most 128 routed slots find the sharers of an expert by ballot, no order);
- * key 7: 1 keeps the selection of a one-token step a launch of its own (default: repeated in the gate/up
- * blocks, dgpp_launch_moe_select_gate_up_swiglu); key 8: row tiles an XCD takes for one token before it turns to the next token in the token-major
- * down + accumulate launch (0 = automatic: 1 from 64 routed slots on, else plain token-major order);
- * key 9: 1 keeps the shared expert's passes of the layer driver
- * on the caller's stream, 2 moves them to a second stream beside the routed passes at every batch size (default:
- * from three tokens on); 3 and 4 keep one stream and never / always fold the accumulation into the shared down pass
- * (default: at one token); key 10: 2 or 4 runs the router's token-tiled score kernel at every batch size with that many tokens per
- * wavefront (0 = automatic: tiled from 32 rows on, 4 tokens from 128 rows on); key 11: the form of the dense matrix-core
- * launch below the tiles: 4 streamed wherever the rows are whole 16-byte vectors, 1 to 3 not streamed; without a workspace 1
- * row tiles, 2 the four parts of K side by side inside a block of four row groups, 3 of two for up to eight rows (0 = automatic:
- * streamed except where another form fills the chip better; else four row groups while the row tiles fit one round of the chip,
- * two up to a round and a quarter); key 12: 1 makes dgpp_launch_moe_slot_chain* run the launches the one-launch chain stands for, 2 makes
- * the layer driver take the one-launch chain for small routed-only decode batches (default: the driver runs the
- * launches; the chain measured slower); key 13: row steps per wavefront of the chain's down part (0 = automatic);
- * key 14: the fused gate + up matrix-core grouped launch: 1 = every wavefront walks both matrices in turn, 2 = the block's
- * wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most 2048 blocks);
- * key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row form, 2 = tiles
- * of 128 activation rows wherever the rows are 16-byte aligned (0 = automatic: dgpp_bench_dense_takes_tiles,
- * dgpp_bench_grouped_takes_tiles). The MXFP8 GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x
- * activation rows; 0 = automatic); key 16: blocks that share the passes of a segment and a row tile in the grouped tiles
- * (0 = automatic); key 17: the MXFP8 shared expert's projections of more than 64 rows on the layer driver's second stream: 1 =
- * the form that is faster alone, 2 = the tiles (0 = automatic). Outputs do not
- * depend on keys 1 - 4 and 6 - 17; keys 0 and
- * 5 change the fp32 summation order (every GEMV launcher follows them alike, so the launchers stay
- * bitwise twins of each other). */
+ * too: moe_set_fp8_ldm, src/kernels/glm_moe_launch.hpp:90. key 0: preferred chunks per lane of the row geometry (0 =
+ * default 4); key 1: slots of one expert a decode-slot block serves together (0 = default: 2 gate/up, 4 down; 1 = one
+ * slot per block); key 2: row steps per block of the slot launches (0 = automatic); key 3: 1 stages activations before
+ * any weight load is issued (default: activation loads, first weight pass, LDS commit); key 4: 1 keeps the layer
+ * driver on the two-launch down + accumulate form; key 5: 2 moves every GEMV launcher to the matrix-core form, 1 keeps
+ * the dense launchers on the vector core at every row count (default: the dense launchers choose by rows, matrix size
+ * and workspace); key 6: 1 makes the layer driver compute the slot order for small decode batches too (default:
+ * batches of at most 128 routed slots find the sharers of an expert by ballot, no order); key 7: 1 keeps the selection
+ * of a one-token step a launch of its own (default: repeated in the gate/up blocks,
+ * dgpp_launch_moe_select_gate_up_swiglu); key 8: row tiles an XCD takes for one token before it turns to the next
+ * token in the token-major down + accumulate launch (0 = automatic: 1 from 64 routed slots on, else plain token-major
+ * order); key 9: 1 keeps the shared expert's passes of the layer driver on the caller's stream, 2 moves them to a
+ * second stream beside the routed passes at every batch size (default: from three tokens on in a captured step or with
+ * more than 32 M shared weights, else from sixteen on); 3 and 4 keep one stream and never / always fold the
+ * accumulation into the shared down pass (default: at one token); key 10: 2 or 4 runs the router's token-tiled score
+ * kernel at every batch size with that many tokens per wavefront, 16 or 32 the one on the matrix core with tiles of
+ * that many (0 = automatic: tiled from 32 rows on, 4 tokens from 128 rows on, the matrix core where its blocks' walk
+ * is shorter than the sums in lanes); key 11: the form of the dense matrix-core launch below the tiles: 4 streamed
+ * wherever the rows are whole 16-byte vectors, 1 to 3 not streamed; without a workspace 1 row tiles, 2 the four parts
+ * of K side by side inside a block of four row groups, 3 of two for up to eight rows (0 = automatic: streamed except
+ * where another form fills the chip better; else four row groups while the row tiles fit one round of the chip, two up
+ * to a round and a quarter); key 12: 1 makes dgpp_launch_moe_slot_chain* run the launches the one-launch chain stands
+ * for, 2 makes the layer driver take the one-launch chain for small routed-only decode batches (default: the driver
+ * runs the launches; the chain measured slower); key 13: row steps per wavefront of the chain's down part (0 =
+ * automatic); key 14: the fused gate + up matrix-core grouped launch: 1 = every wavefront walks both matrices in turn,
+ * 2 = the block's wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most
+ * 2048 blocks); key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row
+ * form, 2 = tiles of 128 activation rows wherever the rows are 16-byte aligned, 3 = grouped passes of 32 there (0 =
+ * automatic: dgpp_bench_dense_takes_tiles, dgpp_bench_grouped_takes_narrow, dgpp_bench_grouped_takes_tiles). The MXFP8
+ * GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows; 0 = automatic);
+ * key 16: blocks that share the passes of a segment and a row tile in the grouped tiles (0 = automatic); key 17: the
+ * MXFP8 shared expert's projections of more than 64 rows on the layer driver's second stream: 1 = the form that is
+ * faster alone, 2 = the tiles (0 = automatic). Outputs do not depend on keys 1 - 4 and 6 - 17; keys 0 and 5 change the
+ * fp32 summation order (every GEMV launcher follows them alike, so the launchers stay bitwise twins of each other). */
 void dgpp_tune_set(int key, int value);
 int dgpp_tune_get(int key);
 /* 1 when the process opted in: the switches take values only if the environment held DGPP_AMD_BENCH=1 at the first
@@ -63,21 +63,26 @@ int dgpp_bench_tiled_launches(void);
 int dgpp_bench_form_launches(int form);
 
 /* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):
- * 1 = tiles of 128 x 128, 0 = the 16-row form (with its K parts in one block, side by side in a block, or split over a
- * workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
+ * 1 = tiles of 128 x 128, 0 = a form of 16-row passes (streamed; or with its K parts in one block, side by side in a block, or
+ * split over a workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k);
-/* Likewise for a grouped matrix-core launch over n_segs segments (act_nvfp4: NVFP4 activations; gate_up: gate and up in one
- * launch) of max_rows rows at most and total_rows together (0: the caller does not know), of which the last long_segs
- * have max_rows: 1 = tiles of up to 128 activation rows, 0 = the 16-row form. */
+/* Likewise for a grouped matrix-core launch, where dgpp_bench_grouped_takes_narrow does not say 1: over n_segs
+ * segments (act_nvfp4: NVFP4 activations; gate_up: gate and up in one launch) of max_rows rows at most and total_rows
+ * together (0: the caller does not know), of which the last long_segs have max_rows: 1 = tiles of up to 128 activation
+ * rows, 0 = the 16-row form. */
 int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_segs, int k, int max_rows, int total_rows,
                                    int long_segs);
+/* Whether that launch, of n weight rows, takes the passes of 32 rows: only if total_rows is known. */
+int dgpp_bench_grouped_takes_narrow(int fmt, int act_nvfp4, int gate_up, int n_segs, int n, int k, int max_rows, int total_rows,
+                                    int long_segs);
 /* What a block of the grouped launch's 128-row form works on (the last long_segs of the table's segments are known to
- * have max_rows rows): place[0 .. 3] = segment
- * (-1: nothing), row tile, first pass and step of its passes of 128 rows. Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */
+ * have max_rows rows): place[0 .. 3] = segment (-1: nothing), row tile, first pass and step of its passes of 128 rows.
+ * Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */
 int dgpp_bench_tiled_place(int n_segs, int long_segs, int row_tiles, int max_rows, int block, int32_t* place);
 
-/* How many items the passes of a grouped launch of known rows are sorted into (0: dealt by segment): no fewer than a table of
- * total_rows rows has passes of `cols` (128 or 32) rows. blocks: of that launch. -1: arguments out of range. Host arithmetic only. */
+/* How many items the passes of a grouped launch of known rows are sorted into (0: dealt by segment): no fewer than a
+ * table of total_rows rows has passes of `cols` (128 or 32) rows. blocks: of that launch. -1: arguments out of range.
+ * Host arithmetic only. */
 int dgpp_bench_tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows, int64_t total_rows, int cols, int64_t* blocks);
 
 /* Measurement aid with no counterpart in the reference: a plain streaming copy of `bytes`

@@ -51,6 +51,33 @@ def test_grouped_tiles_by_rows_per_segment(fmt, a4, gate_up, k, below, above, se
         assert takes(below, 129, 1)   # a shared expert's segment behind the others
 
 
+@pytest.mark.parametrize("fmt,a4,gate_up,segs,n,k,narrow,wide", [
+    (NVFP4, 0, 1, 128, 512, 4096, (1, 4, 16), (25, 44)), (NVFP4, 0, 0, 128, 4096, 512, (1, 4, 16, 25), (44,)),
+    (NVFP4, 0, 1, 256, 2048, 6144, (2, 5, 12), (22,)), (MXFP4, 0, 1, 256, 1024, 4096, (1, 5, 12), (22,)),
+    (FP8, 0, 1, 128, 768, 2048, (6,), (25,)), (FP8, 0, 0, 128, 2048, 768, (6, 16), (48,)), (FP8, 0, 1, 256, 2048, 7168, (4, 6), (14,)),
+    (NVFP4, 1, 0, 128, 2048, 6144, (4, 16), (25,))])
+def test_grouped_passes_of_32_rows_by_rows_per_segment(fmt, a4, gate_up, segs, n, k, narrow, wide):
+    """Measured over whole layers, the 32-row passes are faster than the 16-row form and than the 128-row passes at `narrow` rows per
+    segment, the 128-row passes at `wide`; the rows must be known, and segments of up to 128 rows take them at any number."""
+    lib = _lib.load()
+    def takes(rows, most=1000, total=None):
+        return lib.dgpp_bench_grouped_takes_narrow(fmt, a4, gate_up, segs, n, k, most, rows * segs if total is None else total, 0)
+    for rows in narrow:
+        assert takes(rows) and not takes(rows, total=0)
+    for rows in wide:
+        assert not takes(rows) and takes(rows, most=128)
+        assert lib.dgpp_bench_grouped_takes_tiles(fmt, a4, gate_up, segs, k, 1000, rows * segs, 0)
+
+
+def test_grouped_passes_of_32_rows_not_where_segments_are_nearly_empty_or_alone_and_long():
+    takes = _lib.load().dgpp_bench_grouped_takes_narrow
+    assert not takes(FP8, 0, 1, 128, 768, 2048, 100, 3 * 128, 0) and not takes(NVFP4, 1, 0, 128, 2048, 6144, 100, 3 * 128, 0)
+    assert not takes(NVFP4, 0, 1, 128, 512, 4096, 100, 127, 0) and takes(MXFP4, 0, 1, 256, 1024, 4096, 100, 8, 0)
+    # a shared expert's own launch: while the 128-row passes would be one round of the chip
+    assert takes(FP8, 0, 1, 1, 2048, 4096, 100, 100, 1) and takes(FP8, 0, 1, 1, 512, 4096, 3968, 3968, 1)
+    assert not takes(FP8, 0, 1, 1, 512, 4096, 4096, 4096, 1) and not takes(FP8, 0, 1, 1, 17408, 4096, 129, 129, 1)
+
+
 def test_grouped_tiles_without_the_rows_known():
     takes = _lib.load().dgpp_bench_grouped_takes_tiles
     assert takes(NVFP4, 0, 0, 1, 128, 129, 0, 0) and not takes(NVFP4, 0, 0, 1, 128, 128, 0, 0)   # one segment: a dense product
