@@ -1236,19 +1236,20 @@ inline bool grouped_takes_narrow(const GroupedArgs& a, int n_segs) {
 //   of more than ten rows, 33 to 64 tiles 0.86 to 0.96;
 // * both with one part, more than 512 and up to 768 tiles 0.72 to 1.08, on average 0.85 and 0.90; one column tile of 97 to 256 tiles 0.91 to 0.98;
 // * NVFP4 of one part, k up to 1024, up to 256 tiles 0.82 to 1.02, on average 0.93 (k = 1536 0.98 to 1.1); over a workspace, longer rows,
-//   one column tile of 129 to 160 tiles 0.85 to 1.0.
-// `act_up` and rows that are no whole 16-byte vectors have no streaming form. The bits are those of every other form.
+//   one column tile of 129 to 160 tiles 0.85 to 1.0, of 272 0.94 to 0.98 (236 and 249 1.07 to 1.11).
+// With other work beside it (`beside`) it streams: no second launch, no partial sums. `act_up` and rows that are no whole 16-byte vectors
+// have no streaming form. The bits are those of every other form.
 // Bench / test switch 11: 4 always (where it can), 1 to 3 one of the other forms. `split`: the workspace holds the parts of K.
 template <int FMT>
 inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g, bool split) {
   const int knob = tune_get(kTuneTeams);
   if (a.act_up != nullptr || a.a4_scales != nullptr || !rows_stream(a.act, a.act_stride) || (knob != 0 && knob != 4)) return false;
-  if (FMT == kFmtMxfp4 || knob == 4) return true;
+  if (FMT == kFmtMxfp4 || a.beside || knob == 4) return true;
   const size_t tiles = dense_mfma_tiles(a.m, a.n);
   const bool column = a.m <= kTileCols, longer = split && a.k > 4096;   // (k > 4096: four parts)
   if constexpr (FMT == kFmtNvfp4) {
     if (g.parts == 1) return a.k > 1024 || tiles > 256;
-    return !(longer && column && tiles > 128 && tiles <= 160);
+    return !(longer && column && ((tiles > 128 && tiles <= 160) || (tiles > 256 && tiles <= 288)));
   }
   if (g.parts == 1) return !(column && tiles > 96 && tiles <= 256) && !(tiles > 512 && tiles <= 768);
   if (longer && a.m <= 4 * kTileCols && tiles > 128 && tiles <= 192) return false;

@@ -11,8 +11,8 @@
 // registers, three tiles ahead of their use, two for the widest pass with NVFP4 activations; the block's activation rows
 // go into a ring of LDS stages, three tiles ahead as well (BF16: from memory to LDS without passing registers) where four
 // stages leave room for two blocks per CU, one tile ahead for FP4's widest pass. One barrier per tile, which waits for
-// those of a wavefront's loads that the tile needs and no others: waiting for all of them, the form before this one had
-// one tile on its way and took the latency of a load per tile.
+// those of a wavefront's loads that the tile needs and no others (in the last turn, of up to three tiles, for all): waiting for all
+// of them, the form before this one had one tile on its way and took the latency of a load per tile.
 //
 // Lanes. The matrix core wants 16 rows in 16 adjacent lanes, the memory pipe adjacent lanes in one row. Weights are
 // therefore asked for row by row (four lanes to the 64 bytes of a row's tile), the FP4 scales of four tiles at once, and
@@ -423,7 +423,9 @@ struct TiledPass {
     };
     Regs r0, r1, r2, r3;
     ScaleWord sraw[2];
-    constexpr int kDeep = A4 && CT == 8 ? 2 : 3;   // tiles of weights on their way; a third of the widest with codes would spill
+    // Tiles of weights on their way. The widest pass with codes has two and 32 bytes of scratch a lane as it is, its 32-row form 12, NVFP4's
+    // plain 128-row form 8; the others none.
+    constexpr int kDeep = A4 && CT == 8 ? 2 : 3;
     // One tile: its stage is whole and the one that is filled next is free after the barrier. Of a wavefront's loads
     // those may still be on their way then that are younger than its loads to the stage: the weights (and block-FP8 scales)
     // that followed those, and what the RING - 2 steps between asked for. (The FP4 scales of a turn are not counted: where

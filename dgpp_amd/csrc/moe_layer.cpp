@@ -318,7 +318,9 @@ bool GlmMoeLayer::shared_beside_takes_tiles(int tokens) const {
 }
 void GlmMoeLayer::dense_shared_chain(const uint16_t* x, size_t x_stride, int tokens, hipStream_t st) {
   const int H = cfg_.hidden, SI = w_.shared_inter;
-  const bool beside = st == side_ && shared_beside_takes_tiles(tokens);
+  // (up to 64 rows the tiles are not in question, but a second launch per product and its partial sums are: NVFP4 100 x 512 x 5120 with
+  // 4096, 14 tokens 117 us streamed, 121 split over the workspace)
+  const bool beside = st == side_ && (tokens <= 64 || shared_beside_takes_tiles(tokens));
   auto project = [&](int i, const uint16_t* act, size_t stride, void* out, int f32, int n, int k) {
     detail::check(dgpp_amd::scale_gemm_mxfp8(act, stride, w_.sh_payload[i], w_.sh_scales_e8m0[i], out, f32, tokens, n, k, st,
                                              d_sh_ws_, sh_ws_bytes_, beside));

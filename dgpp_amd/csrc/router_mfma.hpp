@@ -9,7 +9,8 @@
 // bit-reversed order, so that the tree's first three levels (l ^ 32, 16, 8) need three sums in registers; the last three are the
 // eight wavefronts', over LDS. An item is four vectors a chain of the eight chains of one h: four 128-byte lines of every row, loaded
 // to a ring of LDS stages. Tiles of 32 tokens have two stages and two blocks per CU, which cover each other's barriers; tiles of 16,
-// for batches that leave CUs without one of 32, have four stages, three items on their way.
+// for batches that leave CUs without one of 32, have four stages, three items on their way. (Tiles of 32 hold 128 registers and 12 bytes
+// of scratch a lane, at four wavefronts per SIMD.)
 //
 // Lanes. The instruction wants one element of a row from each of four lanes: a lane reads the words that hold its two elements
 // of a vector and places the halves by v_perm. (Whole vectors and swaps between lanes took twice the vector instructions, which
