@@ -31,6 +31,12 @@ def test_segment_bit_exact(gpu, T, K, E):
         assert np.array_equal(host(segs_d), segs)
 
 
+@pytest.mark.parametrize("T,K,E", [(1, 1, 1), (64, 1, 7), (65, 1, 3), (43, 3, 64), (64, 4, 1024)])
+def test_segment_of_one_wavefront_bit_exact(gpu, T, K, E):
+    """Around one read of 64 ids and one wavefront's four."""
+    test_segment_bit_exact(gpu, T, K, E)
+
+
 @pytest.mark.parametrize("T,K,E", [(255, 1, 3), (257, 1, 1), (513, 1, 4), (1365, 3, 130), (4096, 1, 2), (4097, 1, 5),
                                    (2731, 3, 3), (9001, 2, 1024), (4096, 8, 288)])
 def test_segment_over_several_wavefronts_bit_exact(gpu, T, K, E):
