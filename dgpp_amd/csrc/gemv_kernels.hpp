@@ -1151,6 +1151,12 @@ inline bool grouped_fills_narrow(int fmt, bool a4, bool gate_up, int n_segs, int
   const bool fp4 = fmt == kFmtNvfp4 || fmt == kFmtMxfp4;
   const int64_t rows = total_rows, least = a4 || !fp4 ? 4 : (fmt == kFmtNvfp4 ? 1 : 0);
   if (rows < least * n_segs) return false;
+  // A short table leaves CUs without a block or with one: the 16-row form's blocks, of half as many weight rows, are done sooner as long as
+  // they make one pass. 32-row passes over the 16-row form, whole layers, at rows per segment: NVFP4, 8 x 1024 x 4096 2: 1.10, 4: 1.04; 16 x 1024
+  // x 4096 1: 1.09, 2: 1.03, 3: 0.93; 16 x 2048 x 5120 2: 1.15, 3: 0.99; 32 x 512 x 4096 1: 1.12, 2: 1.01, 3: 0.92 (64 experts 1: 0.95); block FP8, 8 x
+  // 1024 x 4096 4: 1.08; 16 x 1024 x 4096 3: 1.00, 4: 0.99. One segment, gate + up and down, us, 16-row form -> 32-row passes: block FP8 2048 x
+  // 5120, 8 rows 44.7 -> 46.7, 14 47.4 -> 46.7, 17 77 -> 49; NVFP4 512 x 4096, 8 rows 26.8 -> 27.7, 12 30.5 -> 27.6. MXFP4 gains at any size.
+  if (fmt != kFmtMxfp4 && n_segs < 64 && rows < 3 * n_segs + (a4 || !fp4 ? 11 : 8)) return false;
   if (n_segs < kXcds) {
     const int block_rows = gate_up ? kTiledRows / 2 : kTiledRows;
     return (n + block_rows - 1) / block_rows * (n_segs + rows / kTiledCols) <= 256;

@@ -78,6 +78,16 @@ def test_grouped_passes_of_32_rows_not_where_segments_are_nearly_empty_or_alone_
     assert not takes(FP8, 0, 1, 1, 512, 4096, 4096, 4096, 1) and not takes(FP8, 0, 1, 1, 17408, 4096, 129, 129, 1)
 
 
+@pytest.mark.parametrize("fmt,a4,segs,wide,short", [(FP8, 0, 1, 14, 13), (FP8, 0, 8, 35, 34), (FP8, 0, 16, 64, 63), (NVFP4, 0, 1, 11, 10),
+                                                    (NVFP4, 0, 8, 32, 31), (NVFP4, 0, 16, 56, 55), (NVFP4, 0, 63, 197, 196), (NVFP4, 0, 64, 64, 63),
+                                                    (NVFP4, 1, 8, 35, 34), (MXFP4, 0, 1, 1, 0), (MXFP4, 0, 16, 1, 0)])
+@pytest.mark.parametrize("gate_up", [0, 1])
+def test_grouped_passes_of_32_rows_of_a_short_table(fmt, a4, segs, wide, short, gate_up):
+    """Measured slower than the 16-row form in tables of few segments until each has some rows, but for MXFP4."""
+    takes = lambda rows: _lib.load().dgpp_bench_grouped_takes_narrow(fmt, a4, gate_up, segs, 1024, 4096, 16, rows, 0)
+    assert takes(wide) and not takes(short)
+
+
 def test_grouped_tiles_without_the_rows_known():
     takes = _lib.load().dgpp_bench_grouped_takes_tiles
     assert takes(NVFP4, 0, 0, 1, 128, 129, 0, 0) and not takes(NVFP4, 0, 0, 1, 128, 128, 0, 0)   # one segment: a dense product
