@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <type_traits>
 
 #include "../../include/dgpp_amd.h"
 #include "capi_errors.hpp"
@@ -421,6 +422,273 @@ summed:
   }
 }
 
+// ---- GEMM, a ring of stages --------------------------------------------------------------------------
+//
+// The tiles above have DEPTH steps on their way in registers. Here the operands go from memory to a ring of STAGES LDS stages without
+// passing registers, and the e8m0 scales of all of a block's rows come once, to a panel whose words hold the scales of a k-block of
+// four steps: the instruction takes the byte. WGN x WGM wavefronts, each WT 16-row tiles of W times MT of A. The chain of an output
+// element is the other forms' (see above); SIDE of them run side by side, so that with four a row is read 512 bytes at a time
+// and sums meet once in four chains.
+//
+// What bounds it: a step's own way, barrier, operands out of LDS, products, about 0.25 us whatever the tile up to 64 x 64 (a CU fetches
+// 50 to 60 of the 130 bytes a ns that its L2 gives), and for cold weights the latency of memory. Reading the operands a step ahead
+// gained nothing, nor did eight stages. n = 4096, k = 6144, us, the tiles above -> here: 64 rows 17.5 -> 15.8, 160 31.5 -> 17.6, 300
+// 41.9 -> 22.3, 1024 66 -> 38; n = 6144, k = 4096: 64 22.0 -> 11.9, 300 31.8 -> 18.9, 1024 76 -> 52.
+
+// 1 KB of a wavefront, a lane's 16 bytes after the other's, from base + offset + at to LDS; zeros from `bytes` on.
+__device__ __forceinline__ void ring_load(const uint8_t* base, int bytes, uint32_t offset, int at, u32x4* to) {
+  const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00027000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)to, 16, offset, at, 0, 0);
+}
+template <int WGN, int WGM, int WT, int MT, int STAGES, int QUADS, int SIDE>
+struct RingShape {
+  static constexpr int kWaves = WGN * WGM, kThreads = kWaves * 64;
+  static constexpr int kTN = 16 * WT * WGN, kTM = 16 * MT * WGM, kRows = kTN + kTM;
+  static constexpr int kUnits = kRows * 8;                     // 16-byte units of a stage: 128 bytes of every row
+  static constexpr int kLoads = kUnits / kThreads;             // of a wavefront and stage, eight rows x 128 bytes each
+  static constexpr int kMaxK = (QUADS < 16 ? QUADS : 16) * 4 * 128;
+  static_assert(kLoads * kThreads == kUnits && kTN % 8 == 0, "whole loads");
+  static_assert(QUADS % 2 == 1 && QUADS <= 17, "sixteen rows of the panel meet no bank twice");
+  static constexpr int kTurns = STAGES == 3 ? 12 : STAGES;     // until the stages and the steps of a quad are in the same places again
+  static_assert((STAGES == 3 || STAGES == 4) && (STAGES - 2) * kLoads < 64, "four named stages; the waits count to 63");
+  static_assert(SIDE == 1 || SIDE == 4, "the panel holds the scales of four steps to a word");
+};
+
+template <int N>
+__device__ __forceinline__ void ring_barrier() {   // all but the newest N loads of the wavefront have arrived; then the block's barrier
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Launched with kThreads threads; the bound of 512 keeps the compiler to 256 registers, and the accumulators out of those
+// that it would have to move sums in and out of.
+template <typename Out, int WGN, int WGM, int WT, int MT, int STAGES, int QUADS, int SIDE, int CHAINS>
+__global__ __launch_bounds__(512) void mxfp8_gemm_ring_kernel(
+    const uint8_t* __restrict__ a, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ w,
+    const uint8_t* __restrict__ w_scales, Out* __restrict__ out, int m, int n, int k, size_t out_stride, int row_tiles,
+    int passes) {
+  using Shape = RingShape<WGN, WGM, WT, MT, STAGES, QUADS, SIDE>;
+  constexpr int kRows = Shape::kRows, kTN = Shape::kTN, kLoads = Shape::kLoads, kWaves = Shape::kWaves;
+  // By name: the compiler then tells a stage that is read from those that are on their way.
+  constexpr int kUnits = Shape::kUnits;
+  __shared__ u32x4 stage0[kUnits], stage1[kUnits], stage2[kUnits], stage3[STAGES == 4 ? kUnits : 1];
+  auto stage = [&](auto turn) -> u32x4* {
+    constexpr int kAt = decltype(turn)::value % STAGES;
+    if constexpr (kAt == 0) return stage0;
+    else if constexpr (kAt == 1) return stage1;
+    else if constexpr (kAt == 2) return stage2;
+    else return stage3;
+  };
+  __shared__ u32x4 panel[kRows * QUADS];
+  // Consecutive workgroups go to the eight XCDs in turn: an XCD keeps the column passes of a row tile to itself.
+  const int lin = static_cast<int>(blockIdx.x), idx = lin / 8;
+  const int row_tile = idx / passes * 8 + lin % 8;
+  if (row_tile >= row_tiles) return;
+  const int n0 = row_tile * kTN, m0 = idx % passes * Shape::kTM;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int kblocks = k >> 5, steps = (kblocks + 3) >> 2;
+
+  // The order of the units, SIDE steps each, which belong to chains SIDE c .. SIDE c + SIDE - 1: c, c + CHAINS / SIDE, ..., then c + 1.
+  const int quads = (steps + 3) >> 2, units = SIDE == 4 ? quads : steps;
+  struct Walk {
+    int at, first;
+    __device__ __forceinline__ bool next(int units) {   // whether that was the last of its chains
+      const bool last = at + CHAINS / SIDE >= units;
+      first += last ? 1 : 0;
+      at = last ? first : at + CHAINS / SIDE;
+      return last;
+    }
+  };
+
+  // The panel: a quad of a row to a thread, words of a step turned into words of a k-block. Where the last step has two blocks, its word
+  // is the row's last, turned so that they come first; past the last step, that one again, which nobody uses. All of a thread's words
+  // are on their way together, and the first stages behind them.
+  struct __attribute__((packed, aligned(1))) Word { uint32_t v; };
+  constexpr int kEach = kRows * 16 / Shape::kThreads;
+  const int quad_of = static_cast<int>(threadIdx.x) & 15, row_of = static_cast<int>(threadIdx.x) >> 4;
+  uint32_t word[kEach][4];
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const int row = row_of + e * (Shape::kThreads / 16);
+    const uint8_t* src = row < kTN ? w_scales + static_cast<size_t>(min(n0 + row, n - 1)) * kblocks
+                                   : a_scales + static_cast<size_t>(min(m0 + row - kTN, m - 1)) * kblocks;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) word[e][i] = reinterpret_cast<const Word*>(src + min(quad_of * 16 + i * 4, kblocks - 4))->v;
+  }
+
+  // Load i of the wavefront: eight rows x 128 bytes of a step, the lane's piece the one that belongs at the lane's place. Where k ends
+  // inside the last step the next row's bytes come along, or zeros behind the last row; multiply() clears them.
+  uint32_t off[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = (i * kWaves + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    const int of = row < kTN ? min(n0 + row, n - 1) - n0 : min(m0 + row - kTN, m - 1) - m0;
+    off[i] = static_cast<uint32_t>(of) * static_cast<uint32_t>(k) + piece * 16;
+  }
+  const uint8_t* wbase = w + static_cast<size_t>(n0) * k;
+  const uint8_t* abase = a + static_cast<size_t>(m0) * k;
+  const int wbytes = min(n - n0, kTN) * k, abytes = min(m - m0, Shape::kTM) * k;
+  Walk ahead = {0, 0}, at = {0, 0};
+  auto load = [&](auto turn) {   // what that turn multiplies
+    constexpr int kStep = decltype(turn)::value % 4;
+    u32x4* const to = stage(turn);
+    const int byte = min(SIDE == 4 ? ahead.at * 4 + kStep : ahead.at, steps - 1) * 128;   // past the last step that one again: the waits count the loads
+    if constexpr (SIDE == 1 || kStep == 3) ahead.next(units);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const bool is_w = kTN / 8 % kWaves == 0 ? i * kWaves < kTN / 8 : (i * kWaves + wave) * 8 < kTN;
+      ring_load(is_w ? wbase : abase, is_w ? wbytes : abytes, off[i], byte, to + (i * kWaves + wave) * 64);
+    }
+  };
+  load(std::integral_constant<int, 0>{});
+  load(std::integral_constant<int, 1>{});
+  if constexpr (STAGES == 4) load(std::integral_constant<int, 2>{});
+  if (quad_of < quads) {
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      uint32_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = __builtin_amdgcn_alignbit(word[e][i], word[e][i], (quad_of * 4 + i) * 4 + 4 > kblocks ? 16 : 0);
+      const uint32_t lo01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400), hi01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602);
+      const uint32_t lo23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400), hi23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602);
+      panel[(row_of + e * (Shape::kThreads / 16)) * QUADS + quad_of] =
+          u32x4{__builtin_amdgcn_perm(lo23, lo01, 0x05040100), __builtin_amdgcn_perm(lo23, lo01, 0x07060302),
+                __builtin_amdgcn_perm(hi23, hi01, 0x05040100), __builtin_amdgcn_perm(hi23, hi01, 0x07060302)};
+    }
+  }
+
+  const int wn = wave % WGN * WT * 16, wm = kTN + wave / WGN * MT * 16;   // first rows of the stage that the wavefront reads
+  v4f acc[SIDE][WT][MT], sum[WT][MT];
+#pragma unroll
+  for (int i = 0; i < WT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+#pragma unroll
+      for (int c = 0; c < SIDE; ++c) acc[c][i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+      sum[i][j] = v4f{-0.f, -0.f, -0.f, -0.f};   // whose sum with a number is the number
+    }
+
+  int ws[WT], as[MT];   // a quad's scales
+  const int* panel_lane = reinterpret_cast<const int*>(panel) + r * (QUADS * 4) + g;
+  auto read_scales = [&](int quad, int shift) {
+#pragma unroll
+    for (int i = 0; i < WT; ++i) ws[i] = panel_lane[(wn + i * 16) * (QUADS * 4) + quad * 4] >> shift;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) as[j] = panel_lane[(wm + j * 16) * (QUADS * 4) + quad * 4] >> shift;
+  };
+  const int cut = (k & 64) != 0 ? steps - 1 : -1;   // the step that k ends inside of
+  int left = SIDE == 4 ? quads * 4 : steps;
+  // A stage is whole for every wavefront after the barrier, which the readers of the one that is filled next have passed.
+  auto turn = [&](auto i) {
+    constexpr int kStep = decltype(i)::value % 4, kByte = SIDE == 4 ? kStep : 0, kChain = SIDE == 4 ? kStep : 0;
+    ring_barrier<(STAGES - 2) * kLoads>();
+    load(std::integral_constant<int, decltype(i)::value + STAGES - 1>{});
+    const u32x4* unit = stage(i);
+    const int s = SIDE == 4 ? at.at * 4 + kStep : min(at.at, steps - 1);
+    if constexpr (SIDE == 1) read_scales(s >> 2, (s & 3) * 8);
+    v8i wv[WT], av[MT];
+#pragma unroll
+    for (int t = 0; t < WT; ++t) wv[t] = as_operand(unit[region_unit(wn + t * 16 + r, g)], unit[region_unit(wn + t * 16 + r, 4 + g)]);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) av[t] = as_operand(unit[region_unit(wm + t * 16 + r, g)], unit[region_unit(wm + t * 16 + r, 4 + g)]);
+    if (s == cut) {   // clears what came from behind k (asm: else every step selects)
+#pragma unroll
+      for (int e = 4; e < 8; ++e) {
+#pragma unroll
+        for (int t = 0; t < WT; ++t) asm volatile("v_mov_b32 %0, 0" : "=v"(wv[t][e]));
+#pragma unroll
+        for (int t = 0; t < MT; ++t) asm volatile("v_mov_b32 %0, 0" : "=v"(av[t][e]));
+      }
+    }
+    if (SIDE == 4 ? s < steps : left > 0) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int t = 0; t < WT; ++t)
+          acc[kChain][t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wv[t], av[j], acc[kChain][t][j], 0, 0, kByte, ws[t], kByte, as[j]);
+    }
+    if constexpr (SIDE == 1 || kStep == 3) {
+      const bool fold = at.next(units);
+      if constexpr (SIDE == 4) read_scales(min(at.at, quads - 1), 0);
+      if (fold && left > 0) {
+#pragma unroll
+        for (int t = 0; t < WT; ++t)
+#pragma unroll
+          for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int c = 0; c < SIDE; ++c) {
+              sum[t][j] = sum[t][j] + acc[c][t][j];
+              acc[c][t][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            }
+      }
+    }
+    --left;
+  };
+  auto four = [&](auto first) {   // whether there are more
+    constexpr int kFirst = decltype(first)::value * 4;
+    turn(std::integral_constant<int, kFirst>{});
+    turn(std::integral_constant<int, kFirst + 1>{});
+    turn(std::integral_constant<int, kFirst + 2>{});
+    turn(std::integral_constant<int, kFirst + 3>{});
+    return left > 0;
+  };
+  if constexpr (SIDE == 4) {   // the panel is whole
+    __syncthreads();
+    read_scales(0, 0);
+  }
+  for (;;) {
+    if (!four(std::integral_constant<int, 0>{})) break;
+    if constexpr (Shape::kTurns > 4) { if (!four(std::integral_constant<int, 1>{})) break; }
+    if constexpr (Shape::kTurns > 8) { if (!four(std::integral_constant<int, 2>{})) break; }
+  }
+  if (SIDE == 1 && steps < CHAINS) {   // the other forms' empty partial sums: -0 becomes +0
+#pragma unroll
+    for (int t = 0; t < WT; ++t)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) sum[t][j] = sum[t][j] + acc[0][t][j];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing is on its way to the LDS when the block ends
+
+  const bool vec = (reinterpret_cast<uintptr_t>(out) & 15u) == 0 && out_stride % 4 == 0;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int a_row = m0 + wm - kTN + j * 16 + r;
+    if (a_row >= m) continue;
+#pragma unroll
+    for (int i = 0; i < WT; ++i) {
+      const int col = n0 + wn + i * 16 + g * 4;
+      Out* dst = out + static_cast<size_t>(a_row) * out_stride + col;
+      if (vec && col + 4 <= n) {
+        struct alignas(4 * sizeof(Out)) Four { Out v[4]; } four;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) put<Out>(&four.v[e], sum[i][j][e]);
+        *reinterpret_cast<Four*>(dst) = four;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + e < n) put<Out>(dst + e, sum[i][j][e]);
+      }
+    }
+  }
+}
+
+template <typename Out, int WGN, int WGM, int WT, int MT, int STAGES, int QUADS, int SIDE>
+hipError_t launch_gemm_ring(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* ws, Out* out, int m, int n,
+                            int k, size_t stride, hipStream_t stream) {
+  using Shape = RingShape<WGN, WGM, WT, MT, STAGES, QUADS, SIDE>;
+  if (k > Shape::kMaxK) return hipErrorInvalidValue;   // tiles_for() asks for no such
+  note_launch(kFormTiles);
+  const int row_tiles = (n + Shape::kTN - 1) / Shape::kTN, passes = (m + Shape::kTM - 1) / Shape::kTM;
+  const dim3 grid(static_cast<unsigned>((row_tiles + 7) / 8 * 8) * static_cast<unsigned>(passes));
+  if (k >= 16 * 128)
+    hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<Out, WGN, WGM, WT, MT, STAGES, QUADS, SIDE, 16>), grid, dim3(Shape::kThreads), 0, stream, a, as, w, ws, out, m, n, k, stride, row_tiles, passes);
+  else
+    hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<Out, WGN, WGM, WT, MT, STAGES, QUADS, SIDE, 4>), grid, dim3(Shape::kThreads), 0, stream, a, as, w, ws, out, m, n, k, stride, row_tiles, passes);
+  return hipGetLastError();
+}
+
 template <typename Out, int WN, int WM, int DEPTH>
 hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* ws, Out* out, int m, int n,
                              int k, size_t stride, hipStream_t stream) {
@@ -435,24 +703,41 @@ hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t*
   return hipGetLastError();
 }
 
-// Which form takes an m x n x k product: 0 the 16-row one, 1 - 3 tiles of 32 x 64, 64 x 64 and 64 x 128 (W x A rows).
-// Measured (us, 16-row form -> the form taken): n = 4096, k = 6144: m = 65 26.2 -> 25.1, 128 33.0 -> 26.4, 300 75 -> 41,
-// 1024 244 -> 62; n = 6144, k = 4096: m = 65 28.4 -> 21.9, 300 78 -> 31, 1024 246 -> 74. A tiled step takes about 0.6 us
-// however few blocks there are (LDS round trip, barrier, operand reads, matrix core in turn), so the 16-row form
-// stays where it has no more work than one round of its blocks (of 64 A rows) on every CU: n = 1536, k = 2048, m = 128
-// 6.9 against 10.7; below k = 2048, whose chains are short, up to 1.75 rounds: n = 4096, k = 1024, m = 100 6.1 against
-// 6.8, m = 128 7.4 against 6.9. Up to 64 rows it
-// reads W once and stays until 64 x 64 tiles fill the chip too: n = 6144, m = 48 16.8 against 21.9, n = 17408 52.8
-// against 42.4. Among the tiles: the smallest while they are no more than the CUs (n = 4096, m = 128: 26.4 against
-// 31.7), the largest once there are two for every CU and little of the last one is padding (m = 1024: 62 against 76).
+// Which form takes an m x n x k product: 0 the 16-row one, 1 - 3 tiles of 32 x 64, 64 x 64 and 64 x 128 (W x A rows) through registers,
+// 4 - 8 the ring's, of 32 x 64, 64 x 64, 64 x 128, 128 x 64 and 128 x 128.
+//
+// The 16-row form stays where its blocks, 16 rows of W each, are one round of the CUs and up to 48 rows of A (us, 16-row form /
+// ring: n = 4096, k = 6144: 17 rows 10.1 / 15.2, 48 13.5 / 15.3, 64 16.6 / 15.8; n = 2048, k = 5184: 32 9.9 / 11.1, 48 12.0 / 11.2), two
+// rounds and up to 16 rows (n = 6144, k = 6144: 1 row 12.7 / 15.5, 16 14.9 / 15.5; three rounds, n = 12288, k = 4096: 16.2 / 13.3 and
+// 18.0 / 13.4), and where k is less than sixteen steps and its passes of 16 x 16 are few (n = 1024, k = 1088: 300 rows 5.5 / 6.0, 1024
+// 12.3 / 6.9). Past one round it loses from 17 rows on (n = 6144, k = 4096: 17 rows 12.4 / 11.5, 64 21.4 / 11.9; n = 12288: 20.2 / 13.6).
+//
+// Among the ring's tiles the one whose rounds of 256 blocks cost least. A round's cost by tile is what it took at k = 6144: 32 x 64
+// 15 us, each further round 9 (two blocks fit a CU); 64 x 64 17; 64 x 128 23; 128 x 64 26; 128 x 128 35. n = 12288, k = 4096: 100
+// rows 64 x 128 18.5 (32 x 64 24, 128 x 128 26), 160 128 x 128 26 (64 x 128 31), 300 128 x 64 36 (128 x 128 50, 64 x 64 46).
+//
+// A panel holds the scales of 8192 of k, 6656 beside the largest tile; past that the tiles through registers: the smallest while
+// they are no more than the CUs, the largest once there are two for every CU.
 int tiles_for(int m, int n, int k) {
   if (k < 128) return 0;   // the tiles read whole words of scales
-  const int knob = tune_get(kTuneTiled);   // bench / test switch: 1 never tiled, 2 - 4 the three tiles
-  if (knob >= 1 && knob <= 4) return knob - 1;
+  const int knob = tune_get(kTuneTiled);   // bench / test switch: 1 never tiled, 2 - 9 the tiles
+  if (knob >= 1 && knob <= (k <= 6656 ? 9 : k <= 8192 ? 8 : 4)) return knob - 1;
   constexpr int64_t kCus = 256;
   auto blocks = [&](int tn, int tm) { return static_cast<int64_t>((n + tn - 1) / tn) * ((m + tm - 1) / tm); };
+  if (k <= 8192) {
+    if (m <= 16 && blocks(16, 64) <= 2 * kCus) return 0;
+    if (m <= 48 && blocks(16, 64) <= kCus) return 0;
+    if (k < 2048 && blocks(16, 16) <= 7 * kCus) return 0;
+    auto rounds = [&](int tn, int tm) { return (blocks(tn, tm) + kCus - 1) / kCus; };
+    const int64_t cost[5] = {6 + 9 * rounds(32, 64), 17 * rounds(64, 64), 23 * rounds(64, 128), 26 * rounds(128, 64),
+                             k <= 6656 ? 35 * rounds(128, 128) : int64_t{1} << 40};
+    int best = 0;
+    for (int i = 1; i < 5; ++i)
+      if (cost[i] < cost[best]) best = i;
+    return 4 + best;
+  }
   if (m <= 32 || (m <= 64 && blocks(64, 64) <= kCus)) return 0;
-  if (m > 64 && blocks(16, 16) <= (k < 2048 ? 7 * kCus : 4 * kCus)) return 0;
+  if (m > 64 && blocks(16, 16) <= 4 * kCus) return 0;
   if (m > 512 && blocks(64, 128) >= 2 * kCus) return 3;
   return blocks(32, 64) <= kCus ? 1 : 2;
 }
@@ -479,6 +764,11 @@ int gemm(const uint8_t* a, const uint8_t* as, const uint8_t* w, const uint8_t* w
     case 1: return report_hip(launch_gemm_tiled<Out, 1, 2, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
     case 2: return report_hip(launch_gemm_tiled<Out, 2, 2, 2>(a, as, w, ws, out, m, n, k, stride, s), who);
     case 3: return report_hip(launch_gemm_tiled<Out, 2, 4, 2>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 4: return report_hip(launch_gemm_ring<Out, 2, 2, 1, 2, 4, 17, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 5: return report_hip(launch_gemm_ring<Out, 4, 2, 1, 2, 4, 17, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 6: return report_hip(launch_gemm_ring<Out, 2, 4, 2, 2, 4, 17, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 7: return report_hip(launch_gemm_ring<Out, 4, 2, 2, 2, 4, 17, 4>(a, as, w, ws, out, m, n, k, stride, s), who);
+    case 8: return report_hip(launch_gemm_ring<Out, 2, 4, 4, 2, 3, 13, 1>(a, as, w, ws, out, m, n, k, stride, s), who);
     default: break;
   }
   const hipError_t err = k >= 16 * 128 ? launch_gemm_waves<Out, 16>(a, as, w, ws, out, m, n, k, stride, s)
