@@ -1514,6 +1514,71 @@ static int grouped_mma_fp4(const uint16_t* act, size_t act_stride, const DgppMoe
                  which, out, out_f32, out_stride, n, k, stream, who, true, act_rows, gate_up_limit, out_up);
 }
 }  // extern "C"
+int dgpp_amd::gate_up_with_shared(int fp4_group, const RouterScores* select, const uint16_t* x, size_t x_stride, const int32_t* ids,
+                                  const DgppMoeExpertView* views, int inter, int hidden, const SharedExpert& shared, uint16_t* act,
+                                  int act_stride, int tokens, int top_k, float limit, void* stream, bool& taken) {
+  taken = false;
+  const int fmt = fp4_group == 0 ? kFmtFp8F32 : fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4, slots = tokens * (top_k + 1);
+  if (tokens <= 0 || tokens > 65535 || top_k <= 0 || !x || !ids || !views || !act || inter <= 0 || hidden <= 0 || shared.inter <= 0 ||
+      act_stride < inter || act_stride < shared.inter || hidden % 16 != 0 || stage_bytes(2, hidden) > kDefaultLdsBytes ||
+      (fp4_group != 0 && (!fp4_k_supported(hidden) || !fp4_k_compiled(hidden, fp4_group))) || !shared.scales[0] || !shared.scales[1] ||
+      !shared.payload[0] || !shared.payload[1] || !fp8_shape_ok(shared.payload[0], hidden) || !fp8_shape_ok(shared.payload[1], hidden))
+    return DGPP_OK;
+  SlotArgs a = slot_args(x, x_stride, ids, nullptr, views, act, act_stride, slots, top_k, limit);
+  a.n = inter;
+  a.k = hidden;
+  a.want_shared = 0;
+  SlotArgs sh = a;
+  sh.n = shared.inter;
+  sh.want_shared = 1;
+  sh.sh[0] = fp8_mat(shared.payload[0], shared.scales[0], shared.rs, shared.cs);
+  sh.sh[1] = fp8_mat(shared.payload[1], shared.scales[1], shared.rs, shared.cs);
+  SelectArgs sel;
+  bool inside = false;
+  hipError_t err = hipSuccess;
+  if (select != nullptr) {
+    const DgppMoeConfig& c = *select->cfg;
+    if (tokens != 1 || dgpp_moe_config_validate(&c) != DGPP_OK || !select->scores || !select->biased || !select->ids || !select->weights)
+      return DGPP_OK;
+    inside = select_gate_up_fits(a, tokens, c.n_experts);
+    sel = {select->scores, select->biased, select->ids, select->weights, c.router_mode, c.n_experts, c.routed_scaling_factor, c.norm_topk_prob ? 1 : 0};
+    if (!inside) {   // a launch of its own
+      if (!launch_gate_up_shared(fmt, a, sh, nullptr, true, as_stream(stream), err)) return DGPP_OK;
+      const int rc = dgpp_launch_moe_router_select(select->scores, select->biased, select->ids, select->weights, &c, tokens, stream);
+      if (rc != DGPP_OK) return rc;
+    }
+  }
+  taken = launch_gate_up_shared(fmt, a, sh, inside ? &sel : nullptr, false, as_stream(stream), err);
+  return taken ? finish(err, "moe_gate_up_with_shared") : DGPP_OK;
+}
+
+int dgpp_amd::down_accum_with_shared(int fp4_group, const uint16_t* act, size_t act_stride, const int32_t* ids,
+                                     const DgppMoeExpertView* views, int hidden, int inter, const SharedExpert& shared, int tokens, int top_k,
+                                     const float* weights, uint16_t* out_bf16, void* stream, bool& taken) {
+  taken = false;
+  const int fmt = fp4_group == 0 ? kFmtFp8F32 : fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4;
+  if (tokens <= 0 || tokens > 65535 || top_k <= 0 || !act || !ids || !views || !weights || !out_bf16 || hidden <= 0 || inter <= 0 ||
+      act_stride < static_cast<size_t>(inter) || act_stride < static_cast<size_t>(shared.inter) ||
+      (fp4_group == 0 ? inter % 16 != 0 : !fp4_k_supported(inter) || !fp4_k_compiled(inter, fp4_group)) || shared.inter <= 0 ||
+      !shared.payload[2] || !shared.scales[2] || !fp8_shape_ok(shared.payload[2], shared.inter))
+    return DGPP_OK;
+  TokenDownArgs a;
+  a.act = act;
+  a.act_stride = act_stride;
+  a.ids = ids;
+  a.views = views;
+  a.weights = weights;
+  a.out = out_bf16;
+  a.out_f32 = 0;
+  a.n = hidden;
+  a.k = inter;
+  a.tokens = tokens;
+  a.top_k = top_k;
+  hipError_t err = hipSuccess;
+  taken = launch_token_down_shared(fmt, a, fp8_mat(shared.payload[2], shared.scales[2], shared.rs, shared.cs), shared.inter, as_stream(stream), err);
+  return taken ? finish(err, "moe_down_accum_with_shared") : DGPP_OK;
+}
+
 int dgpp_amd::grouped_mma(int fp4_group, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,
                           const SegmentRows& rows, const DgppMoeExpertView* views, int which, void* out, int out_f32,
                           size_t out_stride, int n, int k, void* stream, const int32_t* act_rows, const float* gate_up_limit) {

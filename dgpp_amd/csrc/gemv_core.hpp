@@ -69,7 +69,7 @@ struct RowGeom {
 // dgpp_tune_set; launchers read them when they pick a geometry or a kernel form.
 enum : int { kTunePreferP = 0, kTuneSlotRun = 1, kTuneSlotSteps = 2, kTuneSplitStage = 3, kTuneCore = 5, kTuneSelectAlone = 7, kTuneXcdGroup = 8, kTuneRouterTile = 10, kTuneTeams = 11, kTuneChain = 12, kTuneChainDownSteps = 13, kTuneGateUpWalks = 14, kTuneTiled = 15, kTuneTiledPasses = 16, kTuneSharedBeside = 17, kTuneCount = 18 };
 int tune_get(int key);
-enum : int { kFormTiles = 0, kFormNarrow = 1, kFormStreamed = 2, kFormSplit = 3, kFormCount = 4 };
+enum : int { kFormTiles = 0, kFormNarrow = 1, kFormStreamed = 2, kFormSplit = 3, kFormShared = 4, kFormCount = 5 };
 void note_launch(int form);   // counted for the tests while the switches are enabled
 
 __host__ __device__ inline RowGeom row_geom(int chunks, int prefer_p = 4) {

@@ -493,6 +493,31 @@ __global__ __launch_bounds__(kBlockThreads, kMinWavesPerSimd) void slot_gate_up_
     act[tile_row0 + r] = GATE_FP4 ? swiglu_bf16(d4[r], d8[r], a.limit) : swiglu_bf16(d8[r], d4[r], a.limit);
 }
 
+// One wavefront's selection, to `ids` in LDS; `first`: this block stores ids and weights.
+__device__ __forceinline__ void select_to_lds(const SelectArgs& sel, int top_k, int32_t* ids, bool first) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int id;
+  float w;
+  if (sel.n_experts <= 4 * kWave) {
+    if (sel.mode == DGPP_ROUTER_SOFTMAX_TOPK)
+      rsel::select_token<DGPP_ROUTER_SOFTMAX_TOPK, 4>(sel.scores, sel.biased, sel.n_experts, top_k, sel.scaling, sel.norm_topk, lane, id, w);
+    else
+      rsel::select_token<DGPP_ROUTER_SIGMOID_BIAS, 4>(sel.scores, sel.biased, sel.n_experts, top_k, sel.scaling, sel.norm_topk, lane, id, w);
+  } else {
+    if (sel.mode == DGPP_ROUTER_SOFTMAX_TOPK)
+      rsel::select_token<DGPP_ROUTER_SOFTMAX_TOPK, 8>(sel.scores, sel.biased, sel.n_experts, top_k, sel.scaling, sel.norm_topk, lane, id, w);
+    else
+      rsel::select_token<DGPP_ROUTER_SIGMOID_BIAS, 8>(sel.scores, sel.biased, sel.n_experts, top_k, sel.scaling, sel.norm_topk, lane, id, w);
+  }
+  if (lane < top_k) {
+    ids[lane] = id;
+    if (first) {
+      sel.ids[lane] = id;
+      sel.weights[lane] = w;
+    }
+  }
+}
+
 // The router's selection and the routed gate/up pass of a ONE-token decode step in one launch: the first
 // wavefront of every block repeats the selection (whole score row in registers: the selection kernel's own
 // code), the ids go to LDS behind the activation stage and the block goes on as slot_gate_up_kernel does.
@@ -505,29 +530,7 @@ __global__ __launch_bounds__(kBlockThreads, kMinWavesPerSimd) void select_gate_u
   extern __shared__ uint4 lds[];
   const int chunks = a.k / FmtTraits<FMT>::kElemsPerChunk;
   int32_t* ids = reinterpret_cast<int32_t*>(lds + FmtTraits<FMT>::kPieces * chunks);
-  const int lane = threadIdx.x & (kWave - 1);
-  if (threadIdx.x < kWave) {
-    int id;
-    float w;
-    if (sel.n_experts <= 4 * kWave) {
-      if (sel.mode == DGPP_ROUTER_SOFTMAX_TOPK)
-        rsel::select_token<DGPP_ROUTER_SOFTMAX_TOPK, 4>(sel.scores, sel.biased, sel.n_experts, a.top_k, sel.scaling, sel.norm_topk, lane, id, w);
-      else
-        rsel::select_token<DGPP_ROUTER_SIGMOID_BIAS, 4>(sel.scores, sel.biased, sel.n_experts, a.top_k, sel.scaling, sel.norm_topk, lane, id, w);
-    } else {
-      if (sel.mode == DGPP_ROUTER_SOFTMAX_TOPK)
-        rsel::select_token<DGPP_ROUTER_SOFTMAX_TOPK, 8>(sel.scores, sel.biased, sel.n_experts, a.top_k, sel.scaling, sel.norm_topk, lane, id, w);
-      else
-        rsel::select_token<DGPP_ROUTER_SIGMOID_BIAS, 8>(sel.scores, sel.biased, sel.n_experts, a.top_k, sel.scaling, sel.norm_topk, lane, id, w);
-    }
-    if (lane < a.top_k) {
-      ids[lane] = id;
-      if (blockIdx.x == 0 && blockIdx.y == 0) {
-        sel.ids[lane] = id;
-        sel.weights[lane] = w;
-      }
-    }
-  }
+  if (threadIdx.x < kWave) select_to_lds(sel, a.top_k, ids, blockIdx.x == 0 && blockIdx.y == 0);
   __syncthreads();
   SlotArgs b = a;
   b.ids = ids;
@@ -983,6 +986,9 @@ inline int pick_steps(long long block_steps_total) {
 }
 
 hipError_t launch_dense(int fmt, const DenseArgs& a, hipStream_t stream);
+// A pass of the routed and of a block-FP8 shared expert in one launch (gemv_shared.hpp); false, and nothing launched: not of this form.
+bool launch_gate_up_shared(int fmt, const SlotArgs& a, const SlotArgs& sh, const SelectArgs* sel, bool ask, hipStream_t stream, hipError_t& err);
+bool launch_token_down_shared(int fmt, const TokenDownArgs& a, const MatRef& shared, int k_shared, hipStream_t stream, hipError_t& err);
 // `count` problems (<= kMaxDenseProblems) of one k, one row count (<= the rows one stage holds) in one vector-core launch.
 hipError_t launch_dense_multi(int fmt, const DenseArgs* problems, int count, hipStream_t stream);
 template <int FMT> hipError_t launch_dense_multi_fmt(const DenseArgs* problems, int count, hipStream_t stream);

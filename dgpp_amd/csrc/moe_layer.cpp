@@ -392,6 +392,33 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
   if (slot_shared && out_f32 != nullptr)
     throw std::invalid_argument("GlmMoeLayer: an unrounded output with a shared expert is not a decode form");
   if (out_bf16 == nullptr && out_f32 == nullptr) throw std::invalid_argument("GlmMoeLayer: no output buffer");
+  // A block-FP8 shared expert and the routed ones in one launch per pass, where the batch is small enough to need no slot order.
+  // Down comes with the accumulation then, token by token: it reads an expert once per slot and the shared rows once per token, which
+  // NVFP4, bound by its decoding, does not feel while few slots share an expert, the others from about 100 MB of routed rows on. Measured, us,
+  // two layers, a launch for each / gate + up in one / both in one: NVFP4 288 x 512 x 4096, 2 tokens 93 / 82 / 65, 8 155 / 140 / 135, 12 191 /
+  // 175 / 177; 256 x 2048 x 4096, 8 359 / 350 / 336; MXFP4 256 x 1024 x 4096, 4 138 / 128 / 120, 8 205 / 186 / 194; block FP8 288 x 512 x
+  // 4096, 4 131 / 120 / 115, 8 190 / 181 / 189; 256 x 1024 x 6144, 2 187 / 173 / 177, 8 429 / 420 / 442. The second stream stays where it was
+  // taken launched and is no slower: a wide shared expert (40 x 2048 x 7168, 4 tokens 321 / 331), sixteen tokens unless both passes
+  // merge (NVFP4 288 x 512 x 4096 223 / 231 / 206, block FP8 285 / 300 / 296).
+  const bool fp8 = w_.format == GlmExpertFormat::Fp8, nvfp4 = !fp8 && fp4_group_ == 16;
+  const double down_mb = tokens * (K + 1.0) * H * I * (fp8 ? 1.0 : 0.53) / 1e6;
+  const bool down_with_shared = tokens * K * 2 <= cfg_.n_experts && (nvfp4 || down_mb <= 100.0);
+  const bool up_with_shared = tokens < 3 || (3ll * H * w_.shared_inter <= (32 << 20) && (tokens < 16 || (nvfp4 && down_with_shared)));
+  bool up_done = false;
+  if (sh_args && order == nullptr && out_bf16 != nullptr && up_with_shared && dgpp_tune_get(9) == 0) {
+    const int group = fp8 ? 0 : fp4_group_;
+    const DgppMoeConfig c = cfg_.c_config();
+    const dgpp_amd::RouterScores select = {sel_scores, sel_biased, d_ids_, d_weights_, &c};
+    const dgpp_amd::SharedExpert shared = {{w_.sh_payload[0], w_.sh_payload[1], w_.sh_payload[2]},
+                                           {w_.sh_scales[0], w_.sh_scales[1], w_.sh_scales[2]}, w_.shared_inter, w_.sh_rs, w_.sh_cs};
+    detail::check(dgpp_amd::gate_up_with_shared(group, fused ? &select : nullptr, x, x_stride, ids, d_views_, I, H, shared, d_slot_act_,
+                                                max_inter_, tokens, K, cfg_.swiglu_limit, stream, up_done));
+    bool done = false;
+    if (up_done && down_with_shared)
+      detail::check(dgpp_amd::down_accum_with_shared(group, d_slot_act_, static_cast<size_t>(max_inter_), ids, d_views_, H, I, shared, tokens,
+                                                     K, weights, out_bf16, stream, done));
+    if (done) return;
+  }
   StreamFork fork{stream, side_, fork_, join_};
   if (split) fork.begin();
   // One launcher call per pass and stream: the routed pass on the caller's stream, the shared pass beside it.
@@ -420,7 +447,8 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
                             out_bf16, out_f32, d_chain_ready_, d_chain_status_, stream);
       return;
     }
-    if (fused) {
+    if (up_done) {
+    } else if (fused) {
       launch_moe_select_gate_up_swiglu(sel_scores, sel_biased, d_ids_, d_weights_, cfg_, tokens, x, x_stride, d_views_, I, H,
                                        d_slot_act_, max_inter_, cfg_.swiglu_limit, stream);
       if (slot_shared)   // the shared slot's pass: the routed pass already ran above
@@ -456,7 +484,8 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
                                 weights, out_bf16, out_f32, d_chain_ready_, d_chain_status_, stream, fp4_group_);
       return;
     }
-    if (fused) {
+    if (up_done) {
+    } else if (fused) {
       launch_moe_select_gate_up_swiglu_fp4(sel_scores, sel_biased, d_ids_, d_weights_, cfg_, tokens, x, x_stride, d_views_, I,
                                            H, d_slot_act_, max_inter_, cfg_.swiglu_limit, stream, fp4_group_);
       if (slot_shared)

@@ -44,7 +44,8 @@ extern "C" {
  * 2048 blocks); key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row
  * form, 2 = tiles of 128 activation rows wherever the rows are 16-byte aligned, 3 = grouped passes of 32 there (0 =
  * automatic: dgpp_bench_dense_takes_tiles, dgpp_bench_grouped_takes_narrow, dgpp_bench_grouped_takes_tiles). The MXFP8
- * GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows; 0 = automatic);
+ * GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows) through registers,
+ * 5 - 9 = of 32 x 64, 64 x 64, 64 x 128, 128 x 64 or 128 x 128 through a ring of LDS stages (0 = automatic);
  * key 16: blocks that share the passes of a segment and a row tile in the grouped tiles (0 = automatic); key 17: the
  * MXFP8 shared expert's projections of more than 64 rows on the layer driver's second stream: 1 = the form that is
  * faster alone, 2 = the tiles (0 = automatic). Outputs do not depend on keys 1 - 4 and 6 - 17; keys 0 and 5 change the
@@ -59,7 +60,7 @@ int dgpp_tune_enabled(void);
 /* How many launches took a form of key 15's tiles so far, counted in a process that enabled the switches. */
 int dgpp_bench_tiled_launches(void);
 /* Likewise by form: 0 those, 1 the grouped passes of 32 rows, 2 streamed dense products, 3 dense products whose parts of K were
- * split over a workspace. */
+ * split over a workspace, 4 passes of the layer driver that took the routed and the shared expert in one launch. */
 int dgpp_bench_form_launches(int form);
 
 /* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):

@@ -191,6 +191,43 @@ def test_shared_expert_streams_by_batch_and_capture_give_the_same_bits(gpu, T, H
     layer.close()
 
 
+@pytest.mark.parametrize("E,H,I,K,kind,sI,tokens,passes", [
+    (64, 512, 128, 4, "nvfp4", 128, (1, 2, 3, 8), 2),      # down and accumulation too
+    (64, 512, 128, 4, "nvfp4", 384, (1, 3, 9, 15), None),  # a shared expert of its own width; from nine tokens on gate and up alone
+    (32, 512, 256, 8, "fp8", 256, (1, 2), 2),
+    (33, 1024, 576, 2, "mxfp4", 256, (1, 5), 1),           # widths whose rows do not walk alike: down apart
+    (36, 512, 1152, 3, "mxfp4", 1152, (1, 2, 6), 2),       # rows past the fast set-up of down
+    (40, 5120, 512, 4, "nvfp4", 512, (1, 2, 5), 2),        # and of gate and up, the selection apart
+    (20, 320, 160, 2, "fp8", 272, (1, 3), None),
+])
+def test_routed_and_shared_expert_in_one_launch_give_the_same_bits(gpu, E, H, I, K, kind, sI, tokens, passes):
+    """A small batch's routed experts and its block-FP8 shared expert share a launch per pass; same bits as with a launch for
+    each (bench switch 9), launched and as a captured graph."""
+    from dgpp_amd import _lib
+    for T in tokens:
+        p = moe_data.make_problem(E, H, I, K, T, kind, 1100 + E + T + sI, shared_kind="fp8", shared_I=sI, limit=10.0, std=0.05)
+        d = DeviceMoe(p)
+        layer = make_layer(p, d, 0, 2.5, T)
+        want = dev_empty((T, H), np.uint16)
+        before = _lib.load().dgpp_bench_form_launches(4)
+        _lib.load().dgpp_tune_set(9, 3)
+        try:
+            layer.enqueue_decode(d.x, H, want, T)
+            sync()
+        finally:
+            _lib.load().dgpp_tune_set(9, 0)
+        assert _lib.load().dgpp_bench_form_launches(4) == before
+        got = dev_empty((T, H), np.uint16)
+        got.zero_()
+        layer.enqueue_decode(d.x, H, got, T)
+        sync()
+        assert np.array_equal(host(got, np.uint16), host(want, np.uint16)), T
+        ran = _lib.load().dgpp_bench_form_launches(4) - before
+        assert ran == passes if passes else ran >= 1, (T, ran)
+        _two_stream_runs(layer, d, got, host(want, np.uint16).copy(), T, H, torch.cuda.Stream())
+        layer.close()
+
+
 GOLDEN_CASES = sorted((__import__("pathlib").Path(__file__).resolve().parent / "golden").glob("moe_*.npz"))
 
 
