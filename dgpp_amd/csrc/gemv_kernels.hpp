@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <type_traits>
 
 #include "../../include/dgpp_amd.h"
@@ -1172,6 +1173,47 @@ inline bool grouped_fills_narrow(int fmt, bool a4, bool gate_up, int n_segs, int
          !grouped_fills_tiles(fmt, a4, gate_up, n_segs, k, max_rows, total_rows, long_segs);
 }
 
+// Which tile a dense product takes: its activation rows, 128, 64 or 32, or 0 where streaming (or what runs in its place) is faster. A block
+// walks all of k, so few blocks take as long as a round: 128-row tiles of 4096 x 4096 took 45 us from 65 to 600 rows. Narrow tiles decode a
+// weight more often, but there are more of them. Estimated from the blocks of the fullest XCD over its 32 CUs (a row of tiles stays on one XCD:
+// 22 rows of tiles by 11 passes are 33 blocks on six XCDs, 91 us, and by 6 passes 18, 68 us): us at k = 4096, past the start of 4.4, 5.5 and 6.5,
+// for up to one block per CU, up to two, and each of more, and of streaming per 1024 elements of k for each round of three blocks per CU, fitted
+// to 600 shapes drawn from 512 to 17408 weight rows, k = 1024 to 8192 and 33 to 1024 activation rows:
+//                  32 rows           64 rows             128 rows         streaming
+//   block FP8  20, 31,   15.3    25.3, 40, 22.2    39,   66, 39    6   + 12.8
+//   NVFP4      18, 29,   13.6    23.2, 38, 20.9    33,   61, 35.6  6.8 + 10.8
+//   MXFP4    11.5, 19,   10.6    17.9, 32, 17.7    28.5, 59, 27.8  4.6 +  9.6
+//   MXFP8    23.3, 42,   22      25.3, 47, 26.6    35.5, 71, 37.4  4.7 + 19.5
+// A last pass of up to 64 rows takes two thirds of a wide one's time. The estimates are 4 to 14 % off, so that streaming and the 128-row tiles are
+// left only for one that is 8 % lower: over 600 other shapes the mean was 11 % faster than with the two by the line above, none more than 6 % slower.
+// us before -> after, 4096 x 4096, block FP8 200 rows 30 -> 26, 400 45 -> 32, MXFP8 200 44 -> 25, NVFP4 400 40 -> 30, MXFP4
+// 200 23.8 -> 16.4; 12288 x 4096, block FP8 150 rows 45 -> 35, MXFP4 100 34 -> 23; 1024 x 2048, 1000 rows 21 -> 14.5.
+inline int dense_tile_cols(int fmt, int m, int n, int k) {
+  if (m <= kNarrowCols) return 0;
+  struct Cost { double start, one, two, each; };
+  struct Costs { Cost tile[3]; double stream_start, stream_round; };
+  static constexpr Costs kCosts[4] = {{{{4.4, 20, 31, 15.3}, {5.5, 25.3, 40, 22.2}, {6.5, 39, 66, 39}}, 6, 12.8},
+                                      {{{4.4, 18, 29, 13.6}, {5.5, 23.2, 38, 20.9}, {6.5, 33, 61, 35.6}}, 6.8, 10.8},
+                                      {{{4.4, 11.5, 19, 10.6}, {5.5, 17.9, 32, 17.7}, {6.5, 28.5, 59, 27.8}}, 4.6, 9.6},
+                                      {{{4.4, 23.3, 42, 22}, {5.5, 25.3, 47, 26.6}, {6.5, 35.5, 71, 37.4}}, 4.7, 19.5}};
+  const Costs& costs = kCosts[fmt == kFmtNvfp4 ? 1 : fmt == kFmtMxfp4 ? 2 : fmt == kFmtFp8E8M0 ? 3 : 0];
+  const bool fills = dense_fills_tiles(fmt, m, n, k);
+  const double kk = k / 4096.0, rows_per_xcd = ((n + kTiledRows - 1) / kTiledRows + kXcds - 1) / kXcds;
+  int best = 0;
+  double least = 1e30;
+  if (!fills) least = 0.92 * (costs.stream_start + costs.stream_round * ((n + 31) / 32) * ((m + 15) / 16) / 3072.0 * (k / 1024.0));
+  for (int c = 0; c < 3; ++c) {
+    const Cost& t = costs.tile[c];
+    const int cols = kNarrowCols << c, passes = (m + cols - 1) / cols;
+    const double blocks = rows_per_xcd * passes / 32.0;
+    double us = blocks <= 1 ? t.one : blocks <= 2 ? t.two : t.each * (0.7 * std::ceil(blocks) + 0.3 * blocks);
+    if (cols == kTiledCols && m - (passes - 1) * cols <= kHalfCols) us *= passes == 1 ? 0.66 : blocks <= 1 ? 1 : (passes - 0.34) / passes;
+    us = (t.start + us * kk) * (fills && cols == kTiledCols ? 0.92 : 1);
+    if (us < least) least = us, best = cols;
+  }
+  return best;
+}
+
 // Row groups per block of the dense matrix-core launch that runs the four parts of K side by side inside a block
 // (0: the row-tile form). Four up to one round of the chip's 256 CUs - one such block fills a CU, and 272 tiles, two
 // rounds with the second nearly empty, measured slower than the row-tile form; two (blocks half the size, two to a CU)
@@ -1210,13 +1252,15 @@ inline bool tiled_rows_aligned(const Args& a) {
   if (a.a4_scales == nullptr) return (a.act_stride & 7u) == 0;
   return (a.act_stride & 15u) == 0 && ((reinterpret_cast<uintptr_t>(a.a4_scales) | a.a4_scale_stride) & 1u) == 0;
 }
-// Bench / test switch 15: 1 never, 2 always (where it can); 16: passes of a segment side by side.
+// Bench / test switch 15: 1 never, 2 always (where it can), 5 and 6 dense tiles of 64 and of 32 rows; 16: passes of a segment side by side.
+// split: a workspace takes the parts of K.
 template <int FMT>
-inline bool dense_takes_tiled(const DenseArgs& a) {
+inline bool dense_takes_tiled(const DenseArgs& a, bool split) {
   const int knob = tune_get(kTuneTiled);
   if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return false;
-  if (knob == 2) return true;
-  return a.beside ? a.m > 64 : dense_fills_tiles(FMT, a.m, a.n, a.k);
+  if (knob == 2 || knob == 5 || knob == 6) return true;
+  if (a.beside || a.a4_scales != nullptr || split || tune_get(kTuneTeams) != 0) return a.beside ? a.m > 64 : dense_fills_tiles(FMT, a.m, a.n, a.k);
+  return dense_tile_cols(FMT, a.m, a.n, a.k) != 0;
 }
 template <int FMT>
 inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
@@ -1274,18 +1318,23 @@ template <int FMT>
 hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
   note_launch(kFormTiles);
   const MGeom g = mgeom<FMT>(a.k);
-  const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows, passes = (a.m + kTiledCols - 1) / kTiledCols;
-  const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
-  auto go = [&](auto kern) {
+  const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows;
+  auto go = [&](auto kern, int cols) {
+    const int passes = (a.m + cols - 1) / cols;
+    const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
     hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), 0, stream, a, g, row_tiles, passes);
   };
   if constexpr (FMT == kFmtNvfp4) {
     if (a.a4_scales != nullptr) {
-      go(tiled_dense_kernel<FMT, true>);
+      go(tiled_dense_kernel<FMT, true, kTiledCols>, kTiledCols);
       return hipGetLastError();
     }
   }
-  go(tiled_dense_kernel<FMT, false>);
+  const int knob = tune_get(kTuneTiled), rule = a.beside || knob == 2 ? kTiledCols : dense_tile_cols(FMT, a.m, a.n, a.k);
+  const int cols = knob == 5 ? kHalfCols : knob == 6 ? kNarrowCols : rule;
+  if (cols == kNarrowCols) go(tiled_dense_kernel<FMT, false, kNarrowCols>, kNarrowCols);
+  else if (cols == kHalfCols) go(tiled_dense_kernel<FMT, false, kHalfCols>, kHalfCols);
+  else go(tiled_dense_kernel<FMT, false, kTiledCols>, kTiledCols);
   return hipGetLastError();
 }
 
@@ -1317,10 +1366,10 @@ inline int64_t stream_blocks(const DenseArgs& a, const MGeom& g) {
 }
 template <int FMT>
 hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, size_t ws_bytes) {
-  if (dense_takes_tiled<FMT>(a)) return launch_dense_tiled<FMT>(a, stream);
   const MGeom g = mgeom<FMT>(a.k);
   const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
   const bool split = ws != nullptr && ws_bytes >= need && dense_mfma_would_split(g.parts, a.m, a.n) && a.a4_scales == nullptr;
+  if (dense_takes_tiled<FMT>(a, split)) return launch_dense_tiled<FMT>(a, stream);
   if (dense_takes_stream<FMT>(a, g, split)) {
     note_launch(kFormStreamed);
     const int col_tiles = (a.m + kTileCols - 1) / kTileCols;

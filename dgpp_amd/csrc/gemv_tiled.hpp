@@ -40,6 +40,7 @@
 namespace dgpp_amd {
 
 constexpr int kTiledCols = 128;                   // activation rows of the widest pass
+constexpr int kHalfCols = 64;
 constexpr int kNarrowCols = 32;                   // of the kernel for short segments
 constexpr int kTiledRows = 128;                   // weight rows of a block (gate + up: 64 of each)
 
@@ -631,8 +632,8 @@ __device__ __forceinline__ void tiled_rows(const TiledRows& rows, const float (&
                                            const TiledStages<FMT, A4, COLS>& st) {
   if constexpr (COLS == kNarrowCols)
     tiled_pass<FMT, GU, A4, 2>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
-  else if (mt > 64)
-    tiled_pass<FMT, GU, A4, 8>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
+  else if (COLS > 64 && mt > 64)
+    tiled_pass<FMT, GU, A4, COLS / kTileCols>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
   else if (mt > 32)
     tiled_pass<FMT, GU, A4, 4>(rows, divisor, n, k, act, act_stride_bytes, act_rows, act_row0, out_row0, mt, a4, g, o, st);
   else
@@ -840,11 +841,11 @@ __global__ __launch_bounds__(kBlockThreads, COLS == kNarrowCols ? 3 : 2) void ti
 }
 
 // grid.x = kXcds * ceil(row tiles / kXcds) * column passes.
-template <int FMT, bool A4>
-__global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs a, MGeom g, int row_tiles, int passes) {
-  DGPP_TILED_STAGES(st, FMT, A4, kTiledCols);
+template <int FMT, bool A4, int COLS>
+__global__ __launch_bounds__(kBlockThreads, COLS == kNarrowCols ? 3 : 2) void tiled_dense_kernel(DenseArgs a, MGeom g, int row_tiles, int passes) {
+  DGPP_TILED_STAGES(st, FMT, A4, COLS);
   const int lin = static_cast<int>(blockIdx.x), idx = lin / kXcds;
-  const int tile = idx / passes * kXcds + lin % kXcds, c0 = idx % passes * kTiledCols;
+  const int tile = idx / passes * kXcds + lin % kXcds, c0 = idx % passes * COLS;
   if (tile >= row_tiles) return;
   const int wave = threadIdx.x >> 6;
   TiledRows rows;
@@ -859,8 +860,8 @@ __global__ __launch_bounds__(kBlockThreads, 2) void tiled_dense_kernel(DenseArgs
   src.scales = a.a4_scales;
   src.scale_stride = a.a4_scale_stride;
   const TiledOut o = {a.out, nullptr, a.out_stride, a.out_f32, 0, 0.f, a.a4_gs};
-  tiled_rows<FMT, false, A4, kTiledCols>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
-                                    nullptr, c0, static_cast<size_t>(c0), min(kTiledCols, a.m - c0), src, g, o, st);
+  tiled_rows<FMT, false, A4, COLS>(rows, divisor, a.n, a.k, reinterpret_cast<const uint8_t*>(a.act), A4 ? a.act_stride : a.act_stride * 2,
+                                   nullptr, c0, static_cast<size_t>(c0), min(COLS, a.m - c0), src, g, o, st);
 }
 
 // A streamed launch's product that the block belongs to; `lin`: the block's number in it.

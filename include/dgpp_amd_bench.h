@@ -42,8 +42,8 @@ extern "C" {
  * automatic); key 14: the fused gate + up matrix-core grouped launch: 1 = every wavefront walks both matrices in turn,
  * 2 = the block's wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most
  * 2048 blocks); key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row
- * form, 2 = tiles of 128 activation rows wherever the rows are 16-byte aligned, 3 = grouped passes of 32 there (0 =
- * automatic: dgpp_bench_dense_takes_tiles, dgpp_bench_grouped_takes_narrow, dgpp_bench_grouped_takes_tiles). The MXFP8
+ * form, 2 = tiles of 128 activation rows wherever the rows are 16-byte aligned, 3 = grouped passes of 32 there, 5
+ * and 6 = dense tiles of 64 and of 32 (0 = automatic: dgpp_bench_dense_takes_tiles beside another product or with a workspace, dgpp_bench_grouped_takes_narrow, dgpp_bench_grouped_takes_tiles). The MXFP8
  * GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows) through registers,
  * 5 - 9 = of 32 x 64, 64 x 64, 64 x 128, 128 x 64 or 128 x 128 through a ring of LDS stages (0 = automatic);
  * key 16: blocks that share the passes of a segment and a row tile in the grouped tiles (0 = automatic); key 17: the

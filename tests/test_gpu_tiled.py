@@ -14,11 +14,14 @@ from test_gpu_moe_layer import make_layer
 pytestmark = pytest.mark.gpu
 
 
+TILES = 2   # bench switch 15: the tiled form that both() compares, 2 of 128 activation rows, of dense products 5 of 64 and 6 of 32
+
+
 def both(run, *outs, tiled=1):
     """The outputs of run() under the 16-row form and under the tiled one, in `tiled` launches of it (0: the rows are not
     aligned and the 16-row form stays)."""
     got = []
-    for form in (1, 2):
+    for form in (1, TILES):
         for o in outs:
             o.fill_(-1 if o.dtype.is_floating_point else 0x55)
         _lib.load().dgpp_tune_set(15, form)
@@ -28,7 +31,7 @@ def both(run, *outs, tiled=1):
         finally:
             _lib.load().dgpp_tune_set(15, 0)
         sync()
-        assert _lib.load().dgpp_bench_tiled_launches() - before == (tiled if form == 2 else 0)
+        assert _lib.load().dgpp_bench_tiled_launches() - before == (tiled if form == TILES else 0)
         got.append([host(o).copy() for o in outs])
     return got
 
@@ -69,6 +72,15 @@ def test_dense_tiled_is_bitwise_the_16_row_form(gpu, kind, m, n, k):
     scales = rng.uniform(0.5, 2.0, ((n + (1 << rs) - 1) >> rs, (k + (1 << cs) - 1) >> cs)).astype(np.float32) * 1e-3
     p_d, s_d = dev(payload), dev(scales)
     same(lambda: L.launch_mma_gemv_fp8_bf16(act_d, k, p_d, s_d, out, m, n, k, n + 4, rs, cs), kind, out, tiled=m > 1)   # a row keeps to the vector core
+
+
+@pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8", "fp8grid", "mxfp8"])
+@pytest.mark.parametrize("m,n,k", [(17, 40, 576), (33, 130, 1152), (64, 128, 2304), (97, 257, 4096), (129, 300, 640)])
+@pytest.mark.parametrize("form", [5, 6])
+def test_dense_tiles_of_fewer_rows_are_bitwise_the_16_row_form(gpu, kind, m, n, k, form, monkeypatch):
+    """Tiles of 64 and of 32 activation rows: their edges, one, two and four parts of k, k tiles whole and in part."""
+    monkeypatch.setitem(globals(), "TILES", form)
+    test_dense_tiled_is_bitwise_the_16_row_form(gpu, kind, m, n, k)
 
 
 @pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8"])
