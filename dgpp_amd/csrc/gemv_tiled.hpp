@@ -877,7 +877,7 @@ __device__ __forceinline__ const DenseArgs& stream_problem(const DenseMultiArgs&
 
 // ---- up to sixteen activation rows ------------------------------------------------------------------------------------
 // A dense product of one column tile reads every weight once and is bound by that read, if enough of it is on its way: a
-// wavefront takes two row groups and ONE part of K, three tiles ahead, and meets nobody until the parts are folded, in
+// wavefront takes two row groups and ONE part of K, two to three tiles ahead, and meets nobody until the parts are folded, in
 // the order of the forms above. The activation rows, the same few KB for all, come the way of the weights: asked for row by
 // row and turned in LDS of the wavefront's own (in the matrix core's order, sixteen rows side by side, their loads took
 // longer than the weights'). No barrier in the walk. 32 rows x 4 parts to a block of four wavefronts: a matrix of 17408
@@ -887,7 +887,9 @@ __device__ __forceinline__ const DenseArgs& stream_problem(const DenseMultiArgs&
 // What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and for larger FP4
 // matrices the decoding, a block at a time on each CU: NVFP4, K = 5120, 8 rows took 10.7 us for 256 blocks, 17.6 for 512 and 23 for 768, 3
 // to 4.6 of them the memory's (17408 x 5120, 544 blocks: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
-// slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half.
+// slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half. So two tiles are asked for one right after the
+// other: 17408 x 5120, 16 rows, NVFP4 21.2 -> 20.2 us, MXFP4 17.6 -> 16.5, MXFP8 39.3 -> 36.9; 12288 x 4096, 40 rows, MXFP8 35.9 -> 33, block
+// FP8 26.1 -> 23.2.
 // ROWS: activation rows that are loaded, 8 or 16 (those from m on repeat the last).
 // Args: DenseArgs, or DenseMultiArgs: up to four products of one k and one row count in one launch, their blocks one after the other
 // (whole rounds of the XCDs each), each output bitwise its single launch's.
@@ -960,10 +962,14 @@ __global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(Args arg
   Regs r0, r1, r2, r3;
   Acts b0, b1, b2, b3;
   typename Weights::ScaleWord sraw[2];
-  auto step = [&](int t, auto at, const Regs& now, Regs& coming, Regs& far, const Acts& coming_b, Acts& far_b) {
+  // Two tiles, the halves of a line, are asked for together, once the two before are multiplied: far0 and far1, at even steps.
+  auto step = [&](int t, auto at, const Regs& now, Regs& coming, Regs& far0, Regs& far1, const Acts& coming_b, Acts& far_b) {
     constexpr int kAt = decltype(at)::value;
     __builtin_amdgcn_sched_barrier(0);
-    w.load(t + 3, full, far);
+    if constexpr (kAt % 2 == 0) {
+      w.load(t + 2, full, far0);
+      w.load(t + 3, full, far1);
+    }
     load_acts(t + 3, far_b);
     if constexpr (kAt == 0) w.load_scales(t + 4, sraw);
     multiply(t, kAt & 1, now);
@@ -974,23 +980,22 @@ __global__ __launch_bounds__(kBlockThreads, 3) void stream_dense_kernel(Args arg
   if (lo < full) {
     w.load_scales(lo, sraw);
     w.load(lo, full, r0);
-    load_acts(lo, b0);
     w.load(lo + 1, full, r1);
+    load_acts(lo, b0);
     load_acts(lo + 1, b1);
-    w.load(lo + 2, full, r2);
     load_acts(lo + 2, b2);
     w.put_scales(x, sraw);
     w.template exchange<false>(x, 0, r0);
     put_acts(0, b0);
     int t = lo;
     auto turn = [&](int steps) {   // a constant where this is inlined, or the last turn's
-      step(t, std::integral_constant<int, 0>{}, r0, r1, r3, b1, b3);
+      step(t, std::integral_constant<int, 0>{}, r0, r1, r2, r3, b1, b3);
       if (steps == 1) return;
-      step(t + 1, std::integral_constant<int, 1>{}, r1, r2, r0, b2, b0);
+      step(t + 1, std::integral_constant<int, 1>{}, r1, r2, r2, r3, b2, b0);
       if (steps == 2) return;
-      step(t + 2, std::integral_constant<int, 2>{}, r2, r3, r1, b3, b1);
+      step(t + 2, std::integral_constant<int, 2>{}, r2, r3, r0, r1, b3, b1);
       if (steps == 3) return;
-      step(t + 3, std::integral_constant<int, 3>{}, r3, r0, r2, b0, b2);
+      step(t + 3, std::integral_constant<int, 3>{}, r3, r0, r0, r1, b0, b2);
     };
     for (; t + 4 <= full; t += 4) turn(4);
     if (t < full) turn(full - t);
