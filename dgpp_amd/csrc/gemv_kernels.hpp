@@ -1284,13 +1284,13 @@ inline bool grouped_takes_narrow(const GroupedArgs& a, int n_segs) {
 // 18.8, 64 rows 74 -> 51, 77 -> 45; 16000 x 1024, 32 rows 10.6 -> 8.3, 11.2 -> 6.4, 11.5 -> 8.9.
 // Not where another form fills the chip better. A streaming block is 32, 64 or 128 rows with four, two or one parts of K, and takes
 // about as long beside another one on its CU as alone, so that just over a block per CU is its worst size. Time of the other form over
-// streaming's, over 500 shapes of 512 to 17408 rows of weights, 9 to 200 of activations (NVFP4 from one), by 64 x 16 tiles:
-// * block FP8 and MXFP8, one column tile, four parts: up to 128 tiles 1.1 to 2.1 (over a workspace 0.86 to 1.3), 129 to 256 0.79 to 0.97
-//   (0.74 to 1.0; block FP8 at 272 0.92 to 0.99 and 0.78, MXFP8 1.26 and 0.95), more column tiles 0.95 to 1.5. Two parts, block FP8: up
-//   to 256 tiles 1.3 to 1.8 (0.92 to 1.3), 257 to 288 0.86 (0.80);
-// * both over a workspace, longer rows, two to four column tiles, 129 to 192 tiles 0.82 to 1.1, on average 0.95 and 0.92; one column tile
-//   of more than ten rows, 33 to 64 tiles 0.86 to 0.96;
-// * both with one part, more than 512 and up to 768 tiles 0.72 to 1.08, on average 0.85 and 0.90; one column tile of 97 to 256 tiles 0.91 to 0.98;
+// streaming's, by 64 x 16 tiles:
+// * block FP8 and MXFP8 with their parts in the block, 540 shapes of 512 to 46400 rows of weights, 5 to 64 of activations: 1.0 to 1.6 (8467 x 7296,
+//   8 rows, 25.0 us to 16.8; 17810 x 6816, 16 rows, 49.8 to 30.8), but of one part, two column tiles or more, 513 to 768 tiles and rows of weights
+//   that are no whole 64 bytes 0.81 to 1.1, on average 0.92 (whole ones 1.05 to 1.2);
+// * both over a workspace, one column tile, four parts: up to 128 tiles 0.86 to 1.3, 129 to 256 0.74 to 1.0, two parts, block FP8, up to 256
+//   tiles 0.92 to 1.3, 257 to 288 0.80; longer rows, two to four column tiles, 129 to 192 tiles 0.82 to 1.1, on average 0.95 and 0.92; one
+//   column tile of more than ten rows, 33 to 64 tiles 0.86 to 0.96;
 // * NVFP4 of one part, k up to 1024, up to 256 tiles 0.82 to 1.02, on average 0.93 (k = 1536 0.98 to 1.1); over a workspace, longer rows,
 //   one column tile of 129 to 160 tiles 0.85 to 1.0, of 272 0.94 to 0.98 (236 and 249 1.07 to 1.11).
 // With other work beside it (`beside`) it streams: no second launch, no partial sums. `act_up` and rows that are no whole 16-byte vectors
@@ -1307,7 +1307,8 @@ inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g, bool split) {
     if (g.parts == 1) return a.k > 1024 || tiles > 256;
     return !(longer && column && ((tiles > 128 && tiles <= 160) || (tiles > 256 && tiles <= 288)));
   }
-  if (g.parts == 1) return !(column && tiles > 96 && tiles <= 256) && !(tiles > 512 && tiles <= 768);
+  if (g.parts == 1) return column || tiles <= 512 || tiles > 768 || a.k % 64 == 0;
+  if (!split) return true;
   if (longer && a.m <= 4 * kTileCols && tiles > 128 && tiles <= 192) return false;
   if (longer && column && a.m > 10 && tiles > 32 && tiles <= 64) return false;
   if (!column) return true;
