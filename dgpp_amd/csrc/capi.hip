@@ -1554,7 +1554,7 @@ int dgpp_amd::gate_up_with_shared(int fp4_group, const RouterScores* select, con
 
 int dgpp_amd::down_accum_with_shared(int fp4_group, const uint16_t* act, size_t act_stride, const int32_t* ids,
                                      const DgppMoeExpertView* views, int hidden, int inter, const SharedExpert& shared, int tokens, int top_k,
-                                     const float* weights, uint16_t* out_bf16, void* stream, bool& taken) {
+                                     const float* weights, uint16_t* out_bf16, bool ask, void* stream, bool& taken) {
   taken = false;
   const int fmt = fp4_group == 0 ? kFmtFp8F32 : fp4_group == 16 ? kFmtNvfp4 : kFmtMxfp4;
   if (tokens <= 0 || tokens > 65535 || top_k <= 0 || !act || !ids || !views || !weights || !out_bf16 || hidden <= 0 || inter <= 0 ||
@@ -1575,8 +1575,8 @@ int dgpp_amd::down_accum_with_shared(int fp4_group, const uint16_t* act, size_t 
   a.tokens = tokens;
   a.top_k = top_k;
   hipError_t err = hipSuccess;
-  taken = launch_token_down_shared(fmt, a, fp8_mat(shared.payload[2], shared.scales[2], shared.rs, shared.cs), shared.inter, as_stream(stream), err);
-  return taken ? finish(err, "moe_down_accum_with_shared") : DGPP_OK;
+  taken = launch_token_down_shared(fmt, a, fp8_mat(shared.payload[2], shared.scales[2], shared.rs, shared.cs), shared.inter, ask, as_stream(stream), err);
+  return taken && !ask ? finish(err, "moe_down_accum_with_shared") : DGPP_OK;
 }
 
 int dgpp_amd::grouped_mma(int fp4_group, const uint16_t* act, size_t act_stride, const DgppMoeSegment* segs, int n_segs,

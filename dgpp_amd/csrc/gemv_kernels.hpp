@@ -988,8 +988,9 @@ inline int pick_steps(long long block_steps_total) {
 
 hipError_t launch_dense(int fmt, const DenseArgs& a, hipStream_t stream);
 // A pass of the routed and of a block-FP8 shared expert in one launch (gemv_shared.hpp); false, and nothing launched: not of this form.
+// ask: only whether it is.
 bool launch_gate_up_shared(int fmt, const SlotArgs& a, const SlotArgs& sh, const SelectArgs* sel, bool ask, hipStream_t stream, hipError_t& err);
-bool launch_token_down_shared(int fmt, const TokenDownArgs& a, const MatRef& shared, int k_shared, hipStream_t stream, hipError_t& err);
+bool launch_token_down_shared(int fmt, const TokenDownArgs& a, const MatRef& shared, int k_shared, bool ask, hipStream_t stream, hipError_t& err);
 // `count` problems (<= kMaxDenseProblems) of one k, one row count (<= the rows one stage holds) in one vector-core launch.
 hipError_t launch_dense_multi(int fmt, const DenseArgs* problems, int count, hipStream_t stream);
 template <int FMT> hipError_t launch_dense_multi_fmt(const DenseArgs* problems, int count, hipStream_t stream);

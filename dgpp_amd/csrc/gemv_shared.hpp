@@ -167,7 +167,7 @@ bool launch_gate_up_shared_fmt(const SlotArgs& a, const SlotArgs& sh, const Sele
 }
 
 template <int FMT>
-bool launch_token_down_shared_fmt(const TokenDownArgs& a, const MatRef& shared, int k_shared, hipStream_t stream, hipError_t& err) {
+bool launch_token_down_shared_fmt(const TokenDownArgs& a, const MatRef& shared, int k_shared, bool ask, hipStream_t stream, hipError_t& err) {
   constexpr int SHARED = FMT == kFmtFp8F32 ? 1 : 2;
   const RowGeom g = geom_for<FMT>(a.k);
   SharedDown s;
@@ -189,6 +189,7 @@ bool launch_token_down_shared_fmt(const TokenDownArgs& a, const MatRef& shared, 
   const size_t lds = static_cast<size_t>(a.top_k) * stage_bytes(1, a.k) + SHARED * stage_bytes(1, k_shared) +
                      static_cast<size_t>(a.top_k + 1) * rows_per_block * sizeof(float);
   if (lds > kMaxLdsBytes) return false;
+  if (ask) return true;
   const bool split = tune_get(kTuneSplitStage) != 1 && a.k <= 8 * kSplitStageVecs * kWave && k_shared <= 8 * kSplitStageVecs * kWave && (a.act_stride & 7u) == 0 &&
                      (reinterpret_cast<uintptr_t>(a.act) & 15u) == 0;
   const dim3 grid(static_cast<unsigned>(b.tiles) * static_cast<unsigned>(a.tokens));

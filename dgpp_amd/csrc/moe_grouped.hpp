@@ -29,7 +29,7 @@ int scale_gemm_mxfp8(const uint16_t* act, size_t act_stride, const uint8_t* payl
 
 // The routed experts and a block-FP8 shared expert of a small decode batch, a launch per pass: gate + up + SwiGLU (with scores, the
 // selection of a one-token step too), then down and the tokens' accumulation. Bit for bit the launches they stand for. DGPP_OK and
-// taken false: the call is not of that form or would be refused, and nothing was launched.
+// taken false: the call is not of that form or would be refused, and nothing was launched. ask: only whether it is of that form.
 struct SharedExpert {
   const uint8_t* payload[3];
   const float* scales[3];
@@ -47,6 +47,6 @@ int gate_up_with_shared(int fp4_group, const RouterScores* select, const uint16_
                         int tokens, int top_k, float limit, void* stream, bool& taken);
 int down_accum_with_shared(int fp4_group, const uint16_t* act, size_t act_stride, const int32_t* ids, const DgppMoeExpertView* views,
                            int hidden, int inter, const SharedExpert& shared, int tokens, int top_k, const float* weights,
-                           uint16_t* out_bf16, void* stream, bool& taken);
+                           uint16_t* out_bf16, bool ask, void* stream, bool& taken);
 
 }  // namespace dgpp_amd

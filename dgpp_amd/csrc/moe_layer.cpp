@@ -68,6 +68,29 @@ Layout layout_of(const GlmMoeConfig& c, int max_tokens, int shared_inter, size_t
   return l;
 }
 
+// How many passes of a decode step take the routed experts and a block-FP8 shared one in one launch: 2 both, 1 gate + up, 0 neither.
+// Down comes with the accumulation then, token by token: it reads an expert once per slot and the shared rows once per token, which
+// is felt once a pass has about 100 MB of routed rows; NVFP4, bound by its decoding, goes on where down's walks are long or a token has
+// a block of ten wavefronts. The second stream, which both replace, stays where it is no slower: a wide shared expert (40 x 2048
+// x 7168, 4 tokens 321 / 331), sixteen tokens unless both passes merge. Launched, us, two layers, a launch for each / gate + up in one / both:
+// NVFP4 288 x 512 x 4096, 2 tokens 93 / 82 / 65, 8 155 / 140 / 135, 16 223 / 231 / 206; 256 x 2048 x 4096, 8 359 / 350 / 336; 180 x 768 x 6144,
+// top 4, 5 133 / 118 / 119, 9 179 / 166 / 182, 15 246 / 229 / 267; MXFP4 256 x 1024 x 4096, 4 138 / 128 / 120, 8 205 / 186 / 194; block FP8
+// 288 x 512 x 4096, 4 131 / 120 / 115, 8 190 / 181 / 189; 256 x 1024 x 6144, 2 187 / 173 / 177, 8 429 / 420 / 442.
+// In a captured step a fork costs little, and the two streams hide the shared passes from three tokens on: gate + up alone never pays (220 layers of
+// each format, 3 to 16 tokens, 0.83 to 1.1 times as fast as two streams, on average 0.95, 0.98 and 0.96 for NVFP4, MXFP4 and block FP8), both do up to 64
+// MB of routed rows (0.98 to 1.4; 64 to 80 MB 0.92 to 1.2, past 100 MB 0.8 to 1.1): NVFP4 288 x 512 x 4096, 3 tokens 101 -> 80, 12 167 / 178.
+// Popular experts (8, 12 or 24 of 128 to 288 take all tokens) change no sign: 2 to 12 tokens 1.02 to 1.5 times as fast as a launch for each.
+int merged_passes(bool fp8, bool nvfp4, int tokens, int top_k, int n_experts, int hidden, int inter, int shared_inter, bool captured,
+                  bool down_fits) {
+  captured = captured && tokens >= 3;
+  const double down_mb = tokens * (top_k + 1.0) * hidden * inter * (fp8 ? 1.0 : 0.53) / 1e6;
+  const bool down = down_fits && tokens * top_k * 2 <= n_experts &&
+                    (captured ? down_mb <= 64.0 : down_mb <= 100.0 || (nvfp4 && (inter >= 1536 || (tokens >= 16 && top_k >= 8))));
+  const bool up = tokens < 3 || (3ll * hidden * shared_inter <= (32 << 20) && (tokens < 16 || nvfp4) &&
+                                 (down || (tokens < 16 && !captured)));
+  return up ? 1 + down : 0;
+}
+
 bool is_capturing(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &status) != hipSuccess) {   // the default stream while another one is captured
@@ -392,31 +415,33 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
   if (slot_shared && out_f32 != nullptr)
     throw std::invalid_argument("GlmMoeLayer: an unrounded output with a shared expert is not a decode form");
   if (out_bf16 == nullptr && out_f32 == nullptr) throw std::invalid_argument("GlmMoeLayer: no output buffer");
-  // A block-FP8 shared expert and the routed ones in one launch per pass, where the batch is small enough to need no slot order.
-  // Down comes with the accumulation then, token by token: it reads an expert once per slot and the shared rows once per token, which
-  // NVFP4, bound by its decoding, does not feel while few slots share an expert, the others from about 100 MB of routed rows on. Measured, us,
-  // two layers, a launch for each / gate + up in one / both in one: NVFP4 288 x 512 x 4096, 2 tokens 93 / 82 / 65, 8 155 / 140 / 135, 12 191 /
-  // 175 / 177; 256 x 2048 x 4096, 8 359 / 350 / 336; MXFP4 256 x 1024 x 4096, 4 138 / 128 / 120, 8 205 / 186 / 194; block FP8 288 x 512 x
-  // 4096, 4 131 / 120 / 115, 8 190 / 181 / 189; 256 x 1024 x 6144, 2 187 / 173 / 177, 8 429 / 420 / 442. The second stream stays where it was
-  // taken launched and is no slower: a wide shared expert (40 x 2048 x 7168, 4 tokens 321 / 331), sixteen tokens unless both passes
-  // merge (NVFP4 288 x 512 x 4096 223 / 231 / 206, block FP8 285 / 300 / 296).
-  const bool fp8 = w_.format == GlmExpertFormat::Fp8, nvfp4 = !fp8 && fp4_group_ == 16;
-  const double down_mb = tokens * (K + 1.0) * H * I * (fp8 ? 1.0 : 0.53) / 1e6;
-  const bool down_with_shared = tokens * K * 2 <= cfg_.n_experts && (nvfp4 || down_mb <= 100.0);
-  const bool up_with_shared = tokens < 3 || (3ll * H * w_.shared_inter <= (32 << 20) && (tokens < 16 || (nvfp4 && down_with_shared)));
+  // A block-FP8 shared expert and the routed ones in one launch per pass, where the batch needs no slot order and the rule says so.
+  // Bench / test switch 9: 5 gate + up, 6 both wherever they have that form, 1 to 4 neither.
+  const int merge = dgpp_tune_get(9);
   bool up_done = false;
-  if (sh_args && order == nullptr && out_bf16 != nullptr && up_with_shared && dgpp_tune_get(9) == 0) {
+  if (sh_args && order == nullptr && out_bf16 != nullptr && (merge == 0 || merge >= 5)) {
+    const bool fp8 = w_.format == GlmExpertFormat::Fp8, captured = merge == 0 && tokens >= 3 && is_capturing(stream);
     const int group = fp8 ? 0 : fp4_group_;
-    const DgppMoeConfig c = cfg_.c_config();
-    const dgpp_amd::RouterScores select = {sel_scores, sel_biased, d_ids_, d_weights_, &c};
     const dgpp_amd::SharedExpert shared = {{w_.sh_payload[0], w_.sh_payload[1], w_.sh_payload[2]},
                                            {w_.sh_scales[0], w_.sh_scales[1], w_.sh_scales[2]}, w_.shared_inter, w_.sh_rs, w_.sh_cs};
-    detail::check(dgpp_amd::gate_up_with_shared(group, fused ? &select : nullptr, x, x_stride, ids, d_views_, I, H, shared, d_slot_act_,
-                                                max_inter_, tokens, K, cfg_.swiglu_limit, stream, up_done));
-    bool done = false;
-    if (up_done && down_with_shared)
+    auto down = [&](bool ask, bool& taken) {
       detail::check(dgpp_amd::down_accum_with_shared(group, d_slot_act_, static_cast<size_t>(max_inter_), ids, d_views_, H, I, shared, tokens,
-                                                     K, weights, out_bf16, stream, done));
+                                                     K, weights, out_bf16, ask, stream, taken));
+    };
+    auto passes = [&](bool down_fits) {
+      return merge != 0 ? (merge >= 6 && down_fits ? 2 : 1)
+                        : merged_passes(fp8, group == 16, tokens, K, cfg_.n_experts, H, I, w_.shared_inter, captured, down_fits);
+    };
+    bool with_down = passes(true) == 2;
+    if (with_down) down(true, with_down);
+    if (passes(with_down) != 0) {
+      const DgppMoeConfig c = cfg_.c_config();
+      const dgpp_amd::RouterScores select = {sel_scores, sel_biased, d_ids_, d_weights_, &c};
+      detail::check(dgpp_amd::gate_up_with_shared(group, fused ? &select : nullptr, x, x_stride, ids, d_views_, I, H, shared, d_slot_act_,
+                                                  max_inter_, tokens, K, cfg_.swiglu_limit, stream, up_done));
+    }
+    bool done = false;
+    if (up_done && with_down) down(false, done);
     if (done) return;
   }
   StreamFork fork{stream, side_, fork_, join_};
@@ -781,6 +806,11 @@ struct DgppMoeLayer {
 };
 
 extern "C" {
+
+int dgpp_bench_merged_passes(int fmt, int tokens, int top_k, int n_experts, int hidden, int inter, int shared_inter, int captured,
+                             int down_fits) {
+  return dgpp::merged_passes(fmt == 0, fmt == 2, tokens, top_k, n_experts, hidden, inter, shared_inter, captured != 0, down_fits != 0);
+}
 
 const char* dgpp_moe_layer_last_error(void) { return g_layer_error.c_str(); }
 

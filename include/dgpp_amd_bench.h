@@ -26,10 +26,11 @@ extern "C" {
  * of a one-token step a launch of its own (default: repeated in the gate/up blocks,
  * dgpp_launch_moe_select_gate_up_swiglu); key 8: row tiles an XCD takes for one token before it turns to the next
  * token in the token-major down + accumulate launch (0 = automatic: 1 from 64 routed slots on, else plain token-major
- * order); key 9: 1 keeps the shared expert's passes of the layer driver on the caller's stream, 2 moves them to a
- * second stream beside the routed passes at every batch size (default: from three tokens on in a captured step or with
- * more than 32 M shared weights, else from sixteen on); 3 and 4 keep one stream and never / always fold the
- * accumulation into the shared down pass (default: at one token); key 10: 2 or 4 runs the router's token-tiled score
+ * order); key 9: a block-FP8 shared expert's passes of the layer driver. 0 = the routed experts' launches take them where
+ * dgpp_bench_merged_passes says so; elsewhere, and with any other value but 5 and 6, launches of their own: 1 on the caller's
+ * stream, 2 on a second stream beside the routed passes at every batch size (default: from three tokens on in a captured step
+ * or with more than 32 M shared weights, else from sixteen on); 3 and 4 keep one stream and never / always fold the
+ * accumulation into the shared down pass (default: at one token); 5 and 6 merge gate + up or both passes wherever they have that form; key 10: 2 or 4 runs the router's token-tiled score
  * kernel at every batch size with that many tokens per wavefront, 16 or 32 the one on the matrix core with tiles of
  * that many (0 = automatic: tiled from 32 rows on, 4 tokens from 128 rows on, the matrix core where its blocks' walk
  * is shorter than the sums in lanes); key 11: the form of the dense matrix-core launch below the tiles: 4 streamed
@@ -76,6 +77,11 @@ int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_se
 /* Whether that launch, of n weight rows, takes the passes of 32 rows: only if total_rows is known. */
 int dgpp_bench_grouped_takes_narrow(int fmt, int act_nvfp4, int gate_up, int n_segs, int n, int k, int max_rows, int total_rows,
                                     int long_segs);
+/* How many passes of a decode step of the layer driver take the routed and a block-FP8 shared expert in one launch: 2 gate + up and
+ * down with the accumulation, 1 gate + up, 0 neither. fmt: 0 block FP8, 2 NVFP4, 3 MXFP4; captured: on a stream that is being captured;
+ * down_fits: the row widths have that form of down. Host arithmetic only. */
+int dgpp_bench_merged_passes(int fmt, int tokens, int top_k, int n_experts, int hidden, int inter, int shared_inter, int captured,
+                             int down_fits);
 /* What a block of the grouped launch's 128-row form works on (the last long_segs of the table's segments are known to
  * have max_rows rows): place[0 .. 3] = segment (-1: nothing), row tile, first pass and step of its passes of 128 rows.
  * Returns the number of blocks; block b runs on XCD b % 8. Host arithmetic only. */

@@ -224,7 +224,21 @@ def test_routed_and_shared_expert_in_one_launch_give_the_same_bits(gpu, E, H, I,
         assert np.array_equal(host(got, np.uint16), host(want, np.uint16)), T
         ran = _lib.load().dgpp_bench_form_launches(4) - before
         assert ran == passes if passes else ran >= 1, (T, ran)
-        _two_stream_runs(layer, d, got, host(want, np.uint16).copy(), T, H, torch.cuda.Stream())
+        # in a captured step of three tokens and more the second stream is faster than gate and up alone
+        s, before = torch.cuda.Stream(), _lib.load().dgpp_bench_form_launches(4)
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=s):
+            layer.enqueue_decode(d.x, H, got, T, s)
+        assert _lib.load().dgpp_bench_form_launches(4) - before == (ran if T < 3 or ran == 2 else 0), T
+        for switch in (5, 6):   # past the rule
+            _lib.load().dgpp_tune_set(9, switch)
+            try:
+                got.zero_()
+                layer.enqueue_decode(d.x, H, got, T)
+                sync()
+            finally:
+                _lib.load().dgpp_tune_set(9, 0)
+            assert np.array_equal(host(got, np.uint16), host(want, np.uint16)), (T, switch)
+        _two_stream_runs(layer, d, got, host(want, np.uint16).copy(), T, H, s)
         layer.close()
 
 
