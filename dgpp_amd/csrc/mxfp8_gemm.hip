@@ -594,12 +594,13 @@ __global__ __launch_bounds__(512) void mxfp8_gemm_ring_kernel(
 #pragma unroll
     for (int t = 0; t < MT; ++t) av[t] = as_operand(unit[region_unit(wm + t * 16 + r, g)], unit[region_unit(wm + t * 16 + r, 4 + g)]);
     if (s == cut) {   // clears what came from behind k (asm: else every step selects)
+      // A matrix instruction may read what a vector one wrote two wait states later. The compiler does not see into asm: they are in it.
 #pragma unroll
       for (int e = 4; e < 8; ++e) {
 #pragma unroll
-        for (int t = 0; t < WT; ++t) asm volatile("v_mov_b32 %0, 0" : "=v"(wv[t][e]));
+        for (int t = 0; t < WT; ++t) asm volatile("v_mov_b32 %0, 0\n\ts_nop 1" : "=v"(wv[t][e]));
 #pragma unroll
-        for (int t = 0; t < MT; ++t) asm volatile("v_mov_b32 %0, 0" : "=v"(av[t][e]));
+        for (int t = 0; t < MT; ++t) asm volatile("v_mov_b32 %0, 0\n\ts_nop 1" : "=v"(av[t][e]));
       }
     }
     if (SIDE == 4 ? s < steps : left > 0) {
