@@ -78,7 +78,8 @@ Layout layout_of(const GlmMoeConfig& c, int max_tokens, int shared_inter, size_t
 // 288 x 512 x 4096, 4 131 / 120 / 115, 8 190 / 181 / 189; 256 x 1024 x 6144, 2 187 / 173 / 177, 8 429 / 420 / 442.
 // In a captured step a fork costs little, and the two streams hide the shared passes from three tokens on: gate + up alone never pays (220 layers of
 // each format, 3 to 16 tokens, 0.83 to 1.1 times as fast as two streams, on average 0.95, 0.98 and 0.96 for NVFP4, MXFP4 and block FP8), both do up to 64
-// MB of routed rows (0.98 to 1.4; 64 to 80 MB 0.92 to 1.2, past 100 MB 0.8 to 1.1): NVFP4 288 x 512 x 4096, 3 tokens 101 -> 80, 12 167 / 178.
+// MB of routed rows (0.98 to 1.4; 64 to 80 MB 0.92 to 1.2, past 100 MB 0.8 to 1.1): NVFP4 288 x 512 x 4096, 3 tokens 101 -> 80, 12 167 / 178; 180
+// x 768 x 6144, top 4, 15 tokens 215 / 270.
 // Popular experts (8, 12 or 24 of 128 to 288 take all tokens) change no sign: 2 to 12 tokens 1.02 to 1.5 times as fast as a launch for each.
 int merged_passes(bool fp8, bool nvfp4, int tokens, int top_k, int n_experts, int hidden, int inter, int shared_inter, bool captured,
                   bool down_fits) {
