@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "../../include/dgpp_amd.h"
+#include "../../include/dgpp_amd_bench.h"
 #include "capi_errors.hpp"
 #include "gemv_core.hpp"
 #include "numerics.hpp"
@@ -710,35 +711,43 @@ hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t*
 // The 16-row form stays where its blocks, 16 rows of W each, are one round of the CUs and up to 48 rows of A (us, 16-row form /
 // ring: n = 4096, k = 6144: 17 rows 10.1 / 15.2, 48 13.5 / 15.3, 64 16.6 / 15.8; n = 2048, k = 5184: 32 9.9 / 11.1, 48 12.0 / 11.2), two
 // rounds and up to 16 rows (n = 6144, k = 6144: 1 row 12.7 / 15.5, 16 14.9 / 15.5; three rounds, n = 12288, k = 4096: 16.2 / 13.3 and
-// 18.0 / 13.4), and where k is less than sixteen steps and its passes of 16 x 16 are few (n = 1024, k = 1088: 300 rows 5.5 / 6.0, 1024
-// 12.3 / 6.9). Past one round it loses from 17 rows on (n = 6144, k = 4096: 17 rows 12.4 / 11.5, 64 21.4 / 11.9; n = 12288: 20.2 / 13.6).
+// 18.0 / 13.4), up to three quarters of a round below k = 3072 (56 shapes 0.76 to 1.3 times the ring's time, on average 0.97:
+// 147 rows of n = 630, k = 2176 5.9 / 7.7; from 3072 on 0.79 to 1.6, 1.2), and where k is less than sixteen steps and its passes of 16 x 16 are few (n = 1024, k = 1088: 300 rows 5.5 /
+// 6.0, 1024 12.3 / 6.9). Past one round it loses from 17 rows on (n = 6144, k = 4096: 17 rows 12.4 / 11.5, 64 21.4 / 11.9; n = 12288: 20.2 / 13.6).
 //
-// Among the ring's tiles the one whose rounds of 256 blocks cost least. A round's cost by tile is what it took at k = 6144: 32 x 64
+// Among the ring's tiles the one whose rounds of 256 blocks cost least, counted on the fullest XCD (a row of tiles stays on one: 10688 rows of W in
+// tiles of 128 by three passes are 33 blocks on three XCDs, two rounds). A round's cost by tile is what it took at k = 6144: 32 x 64
 // 15 us, each further round 9 (two blocks fit a CU); 64 x 64 17; 64 x 128 23; 128 x 64 26; 128 x 128 35. n = 12288, k = 4096: 100
 // rows 64 x 128 18.5 (32 x 64 24, 128 x 128 26), 160 128 x 128 26 (64 x 128 31), 300 128 x 64 36 (128 x 128 50, 64 x 64 46).
 //
-// A panel holds the scales of 8192 of k, 6656 beside the largest tile; past that the tiles through registers: the smallest while
-// they are no more than the CUs, the largest once there are two for every CU.
+// The panel and the first stages of a block are paid by its walk, and the tiles through registers start sooner. 283 shapes of k = 128 to 1023, up to
+// 131072 rows of W: the ring on average 1.08 times as long, up to 1.9 (20 rows of n = 37178, k = 192 8.0 / 13.2; 163 of 28995, k = 576 20.6
+// / 28.8). From 1024 to 2047, 267 shapes: in one round 0.54 to 1.03, on average 0.83 (the largest tile from 1536 on; 1538 rows of n = 2164, k = 1024
+// 17.9 / 21.6), in more 0.69 to 1.29, 0.99, up to 32 rows of A (against the 16-row form) 0.78 to 1.5, 1.09. Past 2048, 450 shapes, on average 0.82.
+//
+// A panel holds the scales of 8192 of k, 6656 beside the largest tile. Without the ring, tiles through registers: the smallest while
+// they are no more than the CUs, the largest once there are two for every CU; the 16-row form up to 32 rows and where its passes are few.
 int tiles_for(int m, int n, int k) {
   if (k < 128) return 0;   // the tiles read whole words of scales
   const int knob = tune_get(kTuneTiled);   // bench / test switch: 1 never tiled, 2 - 9 the tiles
   if (knob >= 1 && knob <= (k <= 6656 ? 9 : k <= 8192 ? 8 : 4)) return knob - 1;
   constexpr int64_t kCus = 256;
   auto blocks = [&](int tn, int tm) { return static_cast<int64_t>((n + tn - 1) / tn) * ((m + tm - 1) / tm); };
-  if (k <= 8192) {
+  if (k >= 1024 && k <= 8192) {
     if (m <= 16 && blocks(16, 64) <= 2 * kCus) return 0;
     if (m <= 48 && blocks(16, 64) <= kCus) return 0;
-    if (k < 2048 && blocks(16, 16) <= 7 * kCus) return 0;
-    auto rounds = [&](int tn, int tm) { return (blocks(tn, tm) + kCus - 1) / kCus; };
-    const int64_t cost[5] = {6 + 9 * rounds(32, 64), 17 * rounds(64, 64), 23 * rounds(64, 128), 26 * rounds(128, 64),
-                             k <= 6656 ? 35 * rounds(128, 128) : int64_t{1} << 40};
+    if (k < 2048 && (m <= 32 || blocks(16, 16) <= 7 * kCus)) return 0;
+    if (k < 3072 && blocks(16, 64) <= kCus * 3 / 4) return 0;
+    auto rounds = [&](int tn, int tm) { return (static_cast<int64_t>((n + tn - 1) / tn + 7) / 8 * ((m + tm - 1) / tm) + 31) / 32; };
+    const int64_t of[5] = {rounds(32, 64), rounds(64, 64), rounds(64, 128), rounds(128, 64), rounds(128, 128)};
+    const int64_t cost[5] = {6 + 9 * of[0], 17 * of[1], 23 * of[2], 26 * of[3], k >= 1536 && k <= 6656 ? 35 * of[4] : int64_t{1} << 40};
     int best = 0;
     for (int i = 1; i < 5; ++i)
       if (cost[i] < cost[best]) best = i;
-    return 4 + best;
+    if (k >= 2048 || of[best] == 1) return 4 + best;
   }
   if (m <= 32 || (m <= 64 && blocks(64, 64) <= kCus)) return 0;
-  if (m > 64 && blocks(16, 16) <= 4 * kCus) return 0;
+  if (m > 64 && blocks(16, 16) <= (k < 2048 ? 7 : 4) * kCus) return 0;
   if (m > 512 && blocks(64, 128) >= 2 * kCus) return 3;
   return blocks(32, 64) <= kCus ? 1 : 2;
 }
@@ -804,6 +813,8 @@ int quantize(const uint16_t* x, const uint16_t* up, bool fused, size_t stride, i
 using namespace dgpp_amd;
 
 extern "C" {
+
+int dgpp_bench_mxfp8_form(int m, int n, int k) { return m <= 0 || n <= 0 || k <= 0 || k % 64 != 0 ? -1 : tiles_for(m, n, k); }
 
 int dgpp_launch_mxfp8_quantize_rows(const uint16_t* x, size_t x_stride, int rows, int k, uint8_t* codes, uint8_t* scales,
                                     void* stream) {

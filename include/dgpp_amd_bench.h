@@ -77,6 +77,8 @@ int dgpp_bench_grouped_takes_tiles(int fmt, int act_nvfp4, int gate_up, int n_se
 /* Whether that launch, of n weight rows, takes the passes of 32 rows: only if total_rows is known. */
 int dgpp_bench_grouped_takes_narrow(int fmt, int act_nvfp4, int gate_up, int n_segs, int n, int k, int max_rows, int total_rows,
                                     int long_segs);
+/* Which form the MXFP8 GEMM takes: 0 the 16-row one, 1 to 8 the tiles that key 15 numbers from 2 on; -1: k out of range. */
+int dgpp_bench_mxfp8_form(int m, int n, int k);
 /* How many passes of a decode step of the layer driver take the routed and a block-FP8 shared expert in one launch: 2 gate + up and
  * down with the accumulation, 1 gate + up, 0 neither. fmt: 0 block FP8, 2 NVFP4, 3 MXFP4; captured: on a stream that is being captured;
  * down_fits: the row widths have that form of down. Host arithmetic only. */
