@@ -253,6 +253,7 @@ BENCH_SIGNATURES = {
     "dgpp_bench_dense_takes_tiles": (_I, [_I, _I, _I, _I]),
     "dgpp_bench_grouped_takes_tiles": (_I, [_I, _I, _I, _I, _I, _I, _I, _I]),
     "dgpp_bench_grouped_takes_narrow": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I]),
+    "dgpp_bench_dense_tile_rows": (_I, [_I, _I, _I, _I, _I, _I, _I]),
     "dgpp_bench_mxfp8_form": (_I, [_I, _I, _I]),
     "dgpp_bench_merged_passes": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I]),
     "dgpp_bench_tiled_place": (_I, [_I, _I, _I, _I, _I, _P]),

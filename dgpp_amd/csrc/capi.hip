@@ -179,25 +179,27 @@ namespace {
 //   1024, 8 rows 8.7 -> 7.8 and 7.2 -> 8.0) and keep the bits that the vector core's fused launches share with it. With a
 //   split-K workspace the matrix core wins from five rows on at any size, from three for matrices of 48 M weights and more;
 //   block FP8, whose second vector pass starts at six rows, from six rows on for 8 M weights, from four for 64 M, while the
-//   parts of K side by side fit one round of the chip (dense_mfma_team_row_groups);
+//   parts of K side by side would fit one round of the chip (dense_mfma_team_row_groups; such calls stream now);
 // * up to four rows (three of a large matrix): the vector core.
 // Which form is a function of m, n, k, the format and the workspace, so that a row's bits do not depend on where it lies. Rows that
 // are no whole 16-byte vectors have no streaming form, but the vector core loses more by them than the matrix core's other
 // forms: vector -> matrix core, us, such rows, five of 4096 x 4096: block FP8 34.7 -> 14.3, MXFP8 33.6 -> 19.9, NVFP4 20.1 -> 14.9, MXFP4
 // 19.5 -> 14.2; eight of 12288 x 4096: 163 -> 18, 162 -> 24, 86 -> 17.
 constexpr int kVectorPassRows = kMaxActRows;
+int k_parts(int fmt, int k) {
+  switch (fmt) {
+    case kFmtFp8F32: return mgeom<kFmtFp8F32>(k).parts;
+    case kFmtFp8E8M0: return mgeom<kFmtFp8E8M0>(k).parts;
+    case kFmtNvfp4: return mgeom<kFmtNvfp4>(k).parts;
+    default: return mgeom<kFmtMxfp4>(k).parts;
+  }
+}
 bool dense_takes_matrix_core(int fmt, int m, int n, int k, size_t ws_bytes, bool have_ws, int from_rows) {
   if (m > kVectorPassRows || m > max_stage_rows(k)) return true;
   if (from_rows > 0 && m >= from_rows) return true;   // the caller's own boundary (the reference's mma_from_rows)
   const size_t weights = static_cast<size_t>(n) * static_cast<size_t>(k);
   if (m >= 5 && weights >= ((k >= 4096 ? 16u : 64u) << 20)) return true;
-  int parts = 1;
-  switch (fmt) {
-    case kFmtFp8F32: parts = mgeom<kFmtFp8F32>(k).parts; break;
-    case kFmtFp8E8M0: parts = mgeom<kFmtFp8E8M0>(k).parts; break;
-    case kFmtNvfp4: parts = mgeom<kFmtNvfp4>(k).parts; break;
-    default: parts = mgeom<kFmtMxfp4>(k).parts; break;
-  }
+  const int parts = k_parts(fmt, k);
   const bool split = have_ws && parts > 1 && (n + 63) / 64 < 1024 &&
                      ws_bytes >= static_cast<size_t>(parts) * m * static_cast<size_t>(n) * sizeof(float);
   if (split) return m >= 5 || (m >= 3 && weights >= (48u << 20));
@@ -480,6 +482,10 @@ int dgpp_bench_tiled_plan(int n_segs, int long_segs, int row_tiles, int max_rows
   return plan.items;
 }
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k) { return dense_fills_tiles(fmt, m, n, k) ? 1 : 0; }
+int dgpp_bench_dense_tile_rows(int fmt, int act_nvfp4, int m, int n, int k, int beside, int workspace) {
+  const bool split = workspace != 0 && act_nvfp4 == 0 && dense_mfma_would_split(k_parts(fmt, k), m, n);
+  return dense_cols(fmt, act_nvfp4 != 0, m, n, k, beside != 0, split);
+}
 
 int dgpp_moe_config_validate(const DgppMoeConfig* c) {
   // src/models/glm/moe.hpp:119-133

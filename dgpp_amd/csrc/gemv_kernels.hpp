@@ -1185,8 +1185,15 @@ inline bool grouped_fills_narrow(int fmt, bool a4, bool gate_up, int n_segs, int
 //   NVFP4      18, 29,   13.6    23.2, 38, 20.9    33,   61, 35.6  6.8 + 10.8
 //   MXFP4    11.5, 19,   10.6    17.9, 32, 17.7    28.5, 59, 27.8  4.6 +  9.6
 //   MXFP8    23.3, 42,   22      25.3, 47, 26.6    35.5, 71, 37.4  4.7 + 19.5
-// A last pass of up to 64 rows takes two thirds of a wide one's time. The estimates are 4 to 14 % off, so that streaming and the 128-row tiles are
-// left only for one that is 8 % lower: over 600 other shapes the mean was 11 % faster than with the two by the line above, none more than 6 % slower.
+// A last pass of up to 64 rows takes two thirds of a wide one's time. The estimates are 4 to 14 % off on average, and by half where there are few
+// weight rows: streaming's blocks are counted over all CUs, though a row's column tiles stay on one XCD, and the choice takes 1.2 to 1.75 times the best
+// form's time in 29 of 1020 shapes, most of less than 2300 weight rows (662 x 3776, block FP8, 850 rows 33.1 against 23.4 of the 32-row tiles). So
+// streaming is left only for an estimate 14 % lower, below k = 1024, which the fit does not hold (441 rows of 802 x 448, block FP8 5.9 against 7.1),
+// 30 %, and the 128-row tiles for one 8 % lower. Against the two by the line above: over 600 other shapes 10 % faster on average, none more than 6 %
+// slower; over 420 of up to 131072 weight and 3000 activation rows 5 %, one 7 % slower (129 rows of 6973 x 1536, NVFP4); over 300 of k = 256 to 992 3 %, two 3 and 5 % slower.
+// Up to 32 rows it streams, as before there were narrow tiles. That is right up to about 12288 weight rows (4096 x 4096, 17 rows 8.5
+// against 24); past that the 32-row tiles would be ahead: 17 to 32 rows, k = 4096, block FP8 32768 x 4096 31 / 27, 131072 151 / 122, NVFP4 31 / 24 and 122 /
+// 70, MXFP4 24.5 / 17 and 98 / 60, MXFP8 50 / 31 and 206 / 155.
 // us before -> after, 4096 x 4096, block FP8 200 rows 30 -> 26, 400 45 -> 32, MXFP8 200 44 -> 25, NVFP4 400 40 -> 30, MXFP4
 // 200 23.8 -> 16.4; 12288 x 4096, block FP8 150 rows 45 -> 35, MXFP4 100 34 -> 23; 1024 x 2048, 1000 rows 21 -> 14.5.
 inline int dense_tile_cols(int fmt, int m, int n, int k) {
@@ -1202,7 +1209,7 @@ inline int dense_tile_cols(int fmt, int m, int n, int k) {
   const double kk = k / 4096.0, rows_per_xcd = ((n + kTiledRows - 1) / kTiledRows + kXcds - 1) / kXcds;
   int best = 0;
   double least = 1e30;
-  if (!fills) least = 0.92 * (costs.stream_start + costs.stream_round * ((n + 31) / 32) * ((m + 15) / 16) / 3072.0 * (k / 1024.0));
+  if (!fills) least = (k < 1024 ? 0.7 : 0.86) * (costs.stream_start + costs.stream_round * ((n + 31) / 32) * ((m + 15) / 16) / 3072.0 * (k / 1024.0));
   for (int c = 0; c < 3; ++c) {
     const Cost& t = costs.tile[c];
     const int cols = kNarrowCols << c, passes = (m + cols - 1) / cols;
@@ -1215,8 +1222,19 @@ inline int dense_tile_cols(int fmt, int m, int n, int k) {
   return best;
 }
 
+// Activation rows to a tile of a dense launch of whole 16-byte rows, or 0 for a form of 16-row passes. Beside another product the wide tiles
+// from 65 rows on, which take less of the chip from it. A launch whose parts of K are split over a workspace (split) keeps that form: the estimates
+// above have not been measured against it, and at many rows it is behind (MXFP8 4096 x 4096, 200 rows 44 us over a workspace, 25 without).
+// Quantized activations have no narrow tiles.
+inline int dense_cols(int fmt, bool a4, int m, int n, int k, bool beside, bool split) {
+  if (beside) return m > 64 ? kTiledCols : 0;
+  if (split) return 0;
+  if (a4) return dense_fills_tiles(fmt, m, n, k) ? kTiledCols : 0;
+  return dense_tile_cols(fmt, m, n, k);
+}
+
 // Row groups per block of the dense matrix-core launch that runs the four parts of K side by side inside a block
-// (0: the row-tile form). Four up to one round of the chip's 256 CUs - one such block fills a CU, and 272 tiles, two
+// (0: the row-tile form). Without a workspace only rows that are no whole 16-byte vectors come here: all others stream. Four up to one round of the chip's 256 CUs - one such block fills a CU, and 272 tiles, two
 // rounds with the second nearly empty, measured slower than the row-tile form; two (blocks half the size, two to a CU)
 // for up to eight activation rows when the row tiles just exceed a round. Bench switch 11: 1 never, 2 four, 3 two.
 constexpr size_t kTeamsMaxTiles = 256;
@@ -1254,14 +1272,16 @@ inline bool tiled_rows_aligned(const Args& a) {
   return (a.act_stride & 15u) == 0 && ((reinterpret_cast<uintptr_t>(a.a4_scales) | a.a4_scale_stride) & 1u) == 0;
 }
 // Bench / test switch 15: 1 never, 2 always (where it can), 5 and 6 dense tiles of 64 and of 32 rows; 16: passes of a segment side by side.
-// split: a workspace takes the parts of K.
+// Activation rows to a tile, 0: not in tiles. split: a workspace takes the parts of K.
 template <int FMT>
-inline bool dense_takes_tiled(const DenseArgs& a, bool split) {
+inline int dense_takes_tiled(const DenseArgs& a, bool split) {
   const int knob = tune_get(kTuneTiled);
-  if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return false;
-  if (knob == 2 || knob == 5 || knob == 6) return true;
-  if (a.beside || a.a4_scales != nullptr || split || tune_get(kTuneTeams) != 0) return a.beside ? a.m > 64 : dense_fills_tiles(FMT, a.m, a.n, a.k);
-  return dense_tile_cols(FMT, a.m, a.n, a.k) != 0;
+  const bool a4 = a.a4_scales != nullptr;
+  if (knob == 1 || a.act_up != nullptr || !tiled_rows_aligned(a)) return 0;
+  if (knob == 5 || knob == 6) return a4 ? kTiledCols : knob == 5 ? kHalfCols : kNarrowCols;
+  if (knob == 2) return kTiledCols;
+  if (tune_get(kTuneTeams) != 0 && !a.beside && !dense_fills_tiles(FMT, a.m, a.n, a.k)) return 0;
+  return dense_cols(FMT, a4, a.m, a.n, a.k, a.beside, split);
 }
 template <int FMT>
 inline bool grouped_takes_tiled(const GroupedArgs& a, int n_segs) {
@@ -1317,26 +1337,24 @@ inline bool dense_takes_stream(const DenseArgs& a, const MGeom& g, bool split) {
   return blocks <= 256 || (FMT == kFmtFp8F32 ? blocks > 640 : g.parts == 2 || blocks > 512);
 }
 template <int FMT>
-hipError_t launch_dense_tiled(const DenseArgs& a, hipStream_t stream) {
+hipError_t launch_dense_tiled(const DenseArgs& a, int cols, hipStream_t stream) {
   note_launch(kFormTiles);
   const MGeom g = mgeom<FMT>(a.k);
   const int row_tiles = (a.n + kTiledRows - 1) / kTiledRows;
-  auto go = [&](auto kern, int cols) {
-    const int passes = (a.m + cols - 1) / cols;
-    const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
+  const int passes = (a.m + cols - 1) / cols;
+  const dim3 grid(static_cast<unsigned>((row_tiles + kXcds - 1) / kXcds * kXcds) * static_cast<unsigned>(passes));
+  auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(kBlockThreads), 0, stream, a, g, row_tiles, passes);
   };
   if constexpr (FMT == kFmtNvfp4) {
-    if (a.a4_scales != nullptr) {
-      go(tiled_dense_kernel<FMT, true, kTiledCols>, kTiledCols);
+    if (a.a4_scales != nullptr) {   // cols: always kTiledCols
+      go(tiled_dense_kernel<FMT, true, kTiledCols>);
       return hipGetLastError();
     }
   }
-  const int knob = tune_get(kTuneTiled), rule = a.beside || knob == 2 ? kTiledCols : dense_tile_cols(FMT, a.m, a.n, a.k);
-  const int cols = knob == 5 ? kHalfCols : knob == 6 ? kNarrowCols : rule;
-  if (cols == kNarrowCols) go(tiled_dense_kernel<FMT, false, kNarrowCols>, kNarrowCols);
-  else if (cols == kHalfCols) go(tiled_dense_kernel<FMT, false, kHalfCols>, kHalfCols);
-  else go(tiled_dense_kernel<FMT, false, kTiledCols>, kTiledCols);
+  if (cols == kNarrowCols) go(tiled_dense_kernel<FMT, false, kNarrowCols>);
+  else if (cols == kHalfCols) go(tiled_dense_kernel<FMT, false, kHalfCols>);
+  else go(tiled_dense_kernel<FMT, false, kTiledCols>);
   return hipGetLastError();
 }
 
@@ -1371,7 +1389,7 @@ hipError_t launch_dense_mfma(const DenseArgs& a, hipStream_t stream, float* ws, 
   const MGeom g = mgeom<FMT>(a.k);
   const size_t need = static_cast<size_t>(g.parts) * a.m * a.n * sizeof(float);
   const bool split = ws != nullptr && ws_bytes >= need && dense_mfma_would_split(g.parts, a.m, a.n) && a.a4_scales == nullptr;
-  if (dense_takes_tiled<FMT>(a, split)) return launch_dense_tiled<FMT>(a, stream);
+  if (const int cols = dense_takes_tiled<FMT>(a, split)) return launch_dense_tiled<FMT>(a, cols, stream);
   if (dense_takes_stream<FMT>(a, g, split)) {
     note_launch(kFormStreamed);
     const int col_tiles = (a.m + kTileCols - 1) / kTileCols;

@@ -44,9 +44,9 @@ extern "C" {
  * 2 = the block's wavefronts split into gate walkers and up walkers (0 = automatic: split while the grid is at most
  * 2048 blocks); key 15: the forms for many activation rows. The dense and grouped matrix-core launches: 1 = the 16-row
  * form, 2 = tiles of 128 activation rows wherever the rows are 16-byte aligned, 3 = grouped passes of 32 there, 5
- * and 6 = dense tiles of 64 and of 32 (0 = automatic: dgpp_bench_dense_takes_tiles beside another product or with a workspace, dgpp_bench_grouped_takes_narrow, dgpp_bench_grouped_takes_tiles). The MXFP8
- * GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows) through registers,
- * 5 - 9 = of 32 x 64, 64 x 64, 64 x 128, 128 x 64 or 128 x 128 through a ring of LDS stages (0 = automatic);
+ * and 6 = dense tiles of 64 and of 32 (0 = automatic: dgpp_bench_dense_tile_rows, dgpp_bench_grouped_takes_narrow,
+ * dgpp_bench_grouped_takes_tiles). The MXFP8 GEMM: 1 = the 16-row form, 2 - 4 = tiles of 32 x 64, 64 x 64 or 64 x 128 (weight x activation rows) through registers,
+ * 5 - 9 = of 32 x 64, 64 x 64, 64 x 128, 128 x 64 or 128 x 128 through a ring of LDS stages (0 = automatic: dgpp_bench_mxfp8_form);
  * key 16: blocks that share the passes of a segment and a row tile in the grouped tiles (0 = automatic); key 17: the
  * MXFP8 shared expert's projections of more than 64 rows on the layer driver's second stream: 1 = the form that is
  * faster alone, 2 = the tiles (0 = automatic). Outputs do not depend on keys 1 - 4 and 6 - 17; keys 0 and 5 change the
@@ -64,9 +64,13 @@ int dgpp_bench_tiled_launches(void);
  * split over a workspace, 4 passes of the layer driver that took the routed and the shared expert in one launch. */
 int dgpp_bench_form_launches(int form);
 
-/* Which form a dense matrix-core launch of m activation rows takes by its default rule (16-byte aligned rows):
- * 1 = tiles of 128 x 128, 0 = a form of 16-row passes (streamed; or with its K parts in one block, side by side in a block, or
- * split over a workspace). fmt: 0 block FP8, 1 MXFP8, 2 NVFP4 (BF16 or NVFP4 activations), 3 MXFP4. Host arithmetic only. */
+/* Activation rows to a tile, 128, 64 or 32, of the form that a dense matrix-core launch of m rows takes by its default rule (16-byte
+ * aligned rows), or 0: a form of 16-row passes (streamed; or with its K parts in one block or split over a workspace). fmt: 0 block
+ * FP8, 1 MXFP8, 2 NVFP4, 3 MXFP4; act_nvfp4: NVFP4 activations; beside: another product runs beside it; workspace: the caller's holds
+ * the parts of K. Host arithmetic only. */
+int dgpp_bench_dense_tile_rows(int fmt, int act_nvfp4, int m, int n, int k, int beside, int workspace);
+/* The line, 1 above it, from which on the 128-row tiles take a launch of NVFP4 activations, no launch splits its K parts over a workspace, and a
+ * plain launch does not stream. */
 int dgpp_bench_dense_takes_tiles(int fmt, int m, int n, int k);
 /* Likewise for a grouped matrix-core launch, where dgpp_bench_grouped_takes_narrow does not say 1: over n_segs
  * segments (act_nvfp4: NVFP4 activations; gate_up: gate and up in one launch) of max_rows rows at most and total_rows

@@ -83,6 +83,56 @@ def test_dense_tiles_of_fewer_rows_are_bitwise_the_16_row_form(gpu, kind, m, n, 
     test_dense_tiled_is_bitwise_the_16_row_form(gpu, kind, m, n, k)
 
 
+def fp8_bytes(n, k, seed):
+    rng = np.random.default_rng(seed)
+    return dev(rng.integers(0, 120, (n, k), dtype=np.uint8)), dev(rng.uniform(0.5, 2.0, ((n + 127) >> 7, (k + 127) >> 7)).astype(np.float32) * 1e-3)
+
+
+@pytest.mark.parametrize("m,n,k,rows", [(949, 995, 384, 32), (1123, 850, 1024, 64), (1171, 1103, 960, 128)])
+def test_the_rule_reaches_each_width_of_dense_tiles(gpu, m, n, k, rows):
+    lib = _lib.load()
+    assert lib.dgpp_bench_dense_tile_rows(0, 0, m, n, k, 0, 0) == rows
+    p_d, s_d = fp8_bytes(n, k, m)
+    act_d, got = dev(hg.normal_bf16(0xD00 + n, (m, k))), []
+    for form in (0, 1):
+        out = dev_empty((m, n), np.uint16)
+        out.fill_(0x55)
+        before = lib.dgpp_bench_tiled_launches()
+        lib.dgpp_tune_set(15, form)
+        try:
+            L.launch_mma_gemv_fp8_bf16(act_d, k, p_d, s_d, out, m, n, k, n, 7, 7)
+        finally:
+            lib.dgpp_tune_set(15, 0)
+        sync()
+        assert lib.dgpp_bench_tiled_launches() - before == (form == 0)
+        got.append(host(out).copy())
+    assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("m,n", [(5, 1000), (16, 4096), (8, 16390), (9, 16390)])
+def test_rows_of_no_whole_vectors_take_the_other_forms_by_the_rule(gpu, m, n):
+    """The parts of k side by side, in blocks of four and of two row groups, and row tiles: what the rule leaves to rows that do not
+    stream. Same bits as the rows streamed."""
+    lib, k = _lib.load(), 4096
+    p_d, s_d = fp8_bytes(n, k, n)
+    act, got = hg.normal_bf16(0xD10 + n, (m, k)), []
+    wide = np.zeros((m, k + 1), np.uint16)
+    wide[:, :k] = act
+    lib.dgpp_tune_set(5, 2)
+    try:
+        for rows, stride in ((act, k), (wide, k + 1)):
+            rows_d, out = dev(rows), dev_empty((m, n), np.float32)
+            out.fill_(-7.0)
+            before = lib.dgpp_bench_form_launches(2)
+            L.launch_mma_gemv_fp8_f32(rows_d, stride, p_d, s_d, out, m, n, k, n, 7, 7)
+            sync()
+            assert lib.dgpp_bench_form_launches(2) - before == (stride == k)
+            got.append(host(out).view(np.uint32).copy())
+    finally:
+        lib.dgpp_tune_set(5, 0)
+    assert np.array_equal(*got)
+
+
 @pytest.mark.parametrize("kind", ["nvfp4", "mxfp4", "fp8"])
 @pytest.mark.parametrize("H,I", [(1152, 576), (2048, 640)])
 def test_grouped_tiled_is_bitwise_the_16_row_form(gpu, kind, H, I):

@@ -11,16 +11,41 @@ def takes_tiles(fmt, m, n, k):
     return _lib.load().dgpp_bench_dense_takes_tiles(fmt, m, n, k)
 
 
+def tile_rows(fmt, m, n, k, a4=0, beside=0, ws=0):
+    return _lib.load().dgpp_bench_dense_tile_rows(fmt, a4, m, n, k, beside, ws)
+
+
 @pytest.mark.parametrize("fmt", [FP8, MXFP8, NVFP4, MXFP4])
 def test_dense_tiles_only_where_the_16_row_form_needs_more_than_a_round(fmt):
+    """The line of the wide tiles alone: what a launch of NVFP4 activations follows, and from where on a plain one does not stream."""
     # few blocks of 128 x 128 leave the chip idle: measured 1.1 to 5 times slower than the 16-row form
     for m, n, k in [(65, 512, 6144), (100, 512, 4096), (100, 4096, 4096), (129, 1536, 2048), (256, 4096, 4096), (1000, 512, 8192),
                     (65, 12288, 4096), (300, 2048, 1024), (64, 131072, 4096), (1, 4096, 4096)]:
         assert not takes_tiles(fmt, m, n, k), (m, n, k)
+        assert tile_rows(NVFP4, m, n, k, a4=1) == 0
     # measured 1.05 to 3.3 times faster
     for m, n, k in [(1000, 12288, 6144), (300, 6144, 4096), (1000, 2048, 2048), (128, 12288, 8192), (512, 4096, 1024), (4096, 512, 512),
                     (65, 17408, 4096)]:
         assert takes_tiles(fmt, m, n, k), (m, n, k)
+        assert tile_rows(NVFP4, m, n, k, a4=1) == 128 and tile_rows(fmt, m, n, k) > 0
+
+
+@pytest.mark.parametrize("fmt,m,n,k,rows", [
+    # measured: 45 us in 128-row tiles from 65 to 600 rows; the narrow ones 26, 32; 25; 30; 16.4
+    (FP8, 200, 4096, 4096, 32), (FP8, 400, 4096, 4096, 64), (MXFP8, 200, 4096, 4096, 32), (NVFP4, 400, 4096, 4096, 64),
+    (MXFP4, 200, 4096, 4096, 32), (FP8, 150, 12288, 4096, 32), (MXFP4, 100, 12288, 4096, 32), (FP8, 1000, 1024, 2048, 32),
+    (FP8, 1000, 12288, 6144, 128), (MXFP8, 64, 131072, 4096, 128),
+    # streamed: few blocks, short walks past the fit (5.9 us against 7.1, 5.7 against 7.1), and up to 32 rows at any size
+    (FP8, 100, 4096, 4096, 0), (FP8, 441, 802, 448, 0), (NVFP4, 256, 493, 512, 0), (FP8, 85, 4460, 416, 0), (MXFP8, 33, 512, 1024, 0),
+    (FP8, 32, 131072, 4096, 0), (FP8, 33, 131072, 4096, 64), (NVFP4, 1, 131072, 4096, 0)])
+def test_dense_tiles_of_a_plain_launch(fmt, m, n, k, rows):
+    assert tile_rows(fmt, m, n, k) == rows
+    # beside another product only the wide ones, and over a workspace that takes the parts of k none
+    assert tile_rows(fmt, m, n, k, beside=1) == (128 if m > 64 else 0)
+    if k >= 2048 and -(-n // 64) * -(-m // 16) < 1024:
+        assert tile_rows(fmt, m, n, k, ws=1) == 0
+    else:
+        assert tile_rows(fmt, m, n, k, ws=1) == rows
 
 
 @pytest.mark.parametrize("fmt", [FP8, MXFP8, NVFP4, MXFP4])
@@ -31,6 +56,7 @@ def test_dense_tiles_never_take_a_launch_that_splits_over_a_workspace(fmt):
         for m in (17, 64, 65, 80, 129, 256, 257, 1024, 2000):
             if -(-n // 64) * -(-m // 16) < 1024:
                 assert not any(takes_tiles(fmt, m, n, k) for k in (512, 2048, 4096, 17408)), (m, n)
+                assert not any(tile_rows(fmt, m, n, k, ws=1) for k in (2048, 4096, 17408)), (m, n)
 
 
 @pytest.mark.parametrize("fmt,a4,gate_up,k,below,above", [
