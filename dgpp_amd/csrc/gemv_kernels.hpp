@@ -651,6 +651,25 @@ __device__ __forceinline__ void stage_issue_agent(const uint16_t* __restrict__ x
   }
 }
 
+// Block -> (row tile, token). Consecutive blocks go to the chip's eight XCDs in turn (block b runs on XCD b % 8 as
+// the b / 8-th block there) and each XCD has an L2 of its own. An XCD therefore takes `xcd_group` of its row tiles
+// for one token, then the SAME tiles for the next token, and so on through the batch before it moves on: tokens that
+// routed to the same expert find its rows in that L2 instead of fetching them again over the fabric. A large group
+// (all of an XCD's tiles) is plain token-major order: the longest sequential walk through each expert's rows, the
+// better order while few tokens share experts.
+__device__ __forceinline__ void token_tile(const TokenDownArgs& a, int b, int& t, int& tile) {
+  const int G = a.xcd_group;
+  if (G > 0) {     // tiles is a multiple of 8 * G
+    const int seq = b >> 3;
+    const int gi = seq % G, rest = seq / G;
+    t = rest % a.tokens;
+    tile = ((rest / a.tokens) * G + gi) * 8 + (b & 7);
+  } else {
+    t = b / a.tiles;
+    tile = b - t * a.tiles;
+  }
+}
+
 // The body of token_down_accum_kernel for block `b` of its grid. CHAIN: the act rows come from gate/up blocks of the
 // same launch (`aw`); wavefronts beyond top_k (a block sized for the gate/up part) only join the barrier.
 template <int FMT, int NB, bool SPLIT, bool CHAIN>
@@ -658,25 +677,8 @@ __device__ __forceinline__ void token_down_body(const TokenDownArgs& a, const Ro
                                                 int b, const SlotAwait* aw = nullptr) {
   constexpr int kPieces = FmtTraits<FMT>::kPieces;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
-  // Block -> (row tile, token). Consecutive blocks go to the chip's eight XCDs in turn (block b runs on XCD b % 8 as
-  // the b / 8-th block there) and each XCD has an L2 of its own. An XCD therefore takes `xcd_group` of its row tiles
-  // for one token, then the SAME tiles for the next token, and so on through the batch before it moves on: tokens that
-  // routed to the same expert find its rows in that L2 instead of fetching them again over the fabric. A large group
-  // (all of an XCD's tiles) is plain token-major order: the longest sequential walk through each expert's rows, the
-  // better order while few tokens share experts.
   int t, tile;
-  {
-    const int G = a.xcd_group;
-    if (G > 0) {     // tiles is a multiple of 8 * G
-      const int seq = b >> 3;
-      const int gi = seq % G, rest = seq / G;
-      t = rest % a.tokens;
-      tile = ((rest / a.tokens) * G + gi) * 8 + (b & 7);
-    } else {
-      t = b / a.tiles;
-      tile = b - t * a.tiles;
-    }
-  }
+  token_tile(a, b, t, tile);
   const int chunks = a.k / FmtTraits<FMT>::kElemsPerChunk;
   const int row_vecs = kPieces * chunks;
   const int rpw = kWave >> g.l2;
@@ -774,18 +776,7 @@ __device__ __forceinline__ void token_down_pair_body(const TokenDownArgs& a, con
   constexpr int XV = kSplitStageVecs;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
   int t, tile;
-  {
-    const int G = a.xcd_group;
-    if (G > 0) {     // tiles is a multiple of 8 * G (see token_down_body)
-      const int seq = b >> 3;
-      const int gi = seq % G, rest = seq / G;
-      t = rest % a.tokens;
-      tile = ((rest / a.tokens) * G + gi) * 8 + (b & 7);
-    } else {
-      t = b / a.tiles;
-      tile = b - t * a.tiles;
-    }
-  }
+  token_tile(a, b, t, tile);
   const int chunks = a.k / FmtTraits<FMT>::kElemsPerChunk;
   const int row_vecs = kPieces * chunks;
   const int rpw = kWave >> g.l2;

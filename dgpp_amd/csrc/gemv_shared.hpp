@@ -54,18 +54,7 @@ __global__ __launch_bounds__(1024) void token_down_shared_kernel(TokenDownArgs a
   constexpr int kPieces = FmtTraits<FMT>::kPieces, kSharedPieces = FmtTraits<kFmtFp8F32>::kPieces;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
   int t, tile;
-  {
-    const int G = a.xcd_group, b = static_cast<int>(blockIdx.x);
-    if (G > 0) {     // tiles is a multiple of 8 * G (see token_down_body)
-      const int seq = b >> 3;
-      const int gi = seq % G, rest = seq / G;
-      t = rest % a.tokens;
-      tile = ((rest / a.tokens) * G + gi) * 8 + (b & 7);
-    } else {
-      t = b / a.tiles;
-      tile = b - t * a.tiles;
-    }
-  }
+  token_tile(a, static_cast<int>(blockIdx.x), t, tile);
   const int rows_per_block = (kWave >> g.l2) * steps, tile_row0 = tile * rows_per_block;
   const int row_vecs = kPieces * (a.k / FmtTraits<FMT>::kElemsPerChunk);
   const int shared_vecs = kSharedPieces * (s.k / FmtTraits<kFmtFp8F32>::kElemsPerChunk);
