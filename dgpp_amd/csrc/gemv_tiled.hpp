@@ -884,10 +884,12 @@ __device__ __forceinline__ const DenseArgs& stream_problem(const DenseMultiArgs&
 // rows has 544 blocks, all resident at once (three to a CU), where the blocks of sixteen wavefronts of the form with
 // the parts side by side made just over one round. More rows go in column tiles, the weights out of the XCD's L2.
 //
-// What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and for larger FP4
-// matrices the decoding, a block at a time on each CU: NVFP4, K = 5120, 8 rows took 10.7 us for 256 blocks, 17.6 for 512 and 23 for 768, 3
-// to 4.6 of them the memory's (17408 x 5120, 544 blocks: NVFP4 27.4 -> 21.7 us, MXFP4 30 -> 19.3). Nontemporal loads were
-// slower (23.2, 20.6): a tile takes half of a line, and the line did not stay for the other half. So two tiles are asked for one right after the
+// What bounds it: the walk's latency where a wavefront has few tiles (4096 x 4096: 8 a part, 7.5 us in all), and otherwise the chain of a tile -
+// loads, LDS, decoding, products, one behind the other - on CUs with one to three blocks. K = 5120, 8 rows, NVFP4 10.4 us for 256 blocks, 15.6 for 512,
+// 18.9 for 544 (17408 rows: three blocks on 32 CUs) and 20.3 for 768; MXFP4 7.8, 11.5, 14.2, 15.5. With one thing left out, 544 blocks, NVFP4
+// 18.9 / MXFP4 14.2: the decoding 15.4 / 14.2, the weights' loads 18.3 / 11.5, the rows and their way through LDS 17.7 / 12.6, the weights'
+// way through LDS 18.2 / 13.6, the scales 18.7 / 13.8, the products 18.2 / 13.8. Nontemporal loads were slower (23.2 against 21.7, 20.6 against
+// 19.3 when that was all): a tile takes half of a line, and the line did not stay for the other half. So two tiles are asked for one right after the
 // other: 17408 x 5120, 16 rows, NVFP4 21.2 -> 20.2 us, MXFP4 17.6 -> 16.5, MXFP8 39.3 -> 36.9; 12288 x 4096, 40 rows, MXFP8 35.9 -> 33, block
 // FP8 26.1 -> 23.2.
 // ROWS: activation rows that are loaded, 8 or 16 (those from m on repeat the last).

@@ -76,19 +76,20 @@ Layout layout_of(const GlmMoeConfig& c, int max_tokens, int shared_inter, size_t
 // NVFP4 288 x 512 x 4096, 2 tokens 93 / 82 / 65, 8 155 / 140 / 135, 16 223 / 231 / 206; 256 x 2048 x 4096, 8 359 / 350 / 336; 180 x 768 x 6144,
 // top 4, 5 133 / 118 / 119, 9 179 / 166 / 182, 15 246 / 229 / 267; MXFP4 256 x 1024 x 4096, 4 138 / 128 / 120, 8 205 / 186 / 194; block FP8
 // 288 x 512 x 4096, 4 131 / 120 / 115, 8 190 / 181 / 189; 256 x 1024 x 6144, 2 187 / 173 / 177, 8 429 / 420 / 442.
-// In a captured step a fork costs little, and the two streams hide the shared passes from three tokens on: gate + up alone never pays (220 layers of
-// each format, 3 to 16 tokens, 0.83 to 1.1 times as fast as two streams, on average 0.95, 0.98 and 0.96 for NVFP4, MXFP4 and block FP8), both do up to 64
-// MB of routed rows (0.98 to 1.4; 64 to 80 MB 0.92 to 1.2, past 100 MB 0.8 to 1.1): NVFP4 288 x 512 x 4096, 3 tokens 101 -> 80, 12 167 / 178; 180
-// x 768 x 6144, top 4, 15 tokens 215 / 270.
-// Popular experts (8, 12 or 24 of 128 to 288 take all tokens) change no sign: 2 to 12 tokens 1.02 to 1.5 times as fast as a launch for each.
+// In a captured step a fork costs little, and two streams hide the shared passes from three tokens on. Over them, 1120 layers of 3 to 16 tokens: gate +
+// up alone 0.83 to 1.1 times as fast, on average 0.95, 0.98 and 0.96 (NVFP4, MXFP4, block FP8), and ahead only where an FP4 batch of eight tokens and
+// more has a large shared expert to hide (256 x 1024 x 4096 MXFP4, 15 tokens 303 -> 282; 128 x 1024 x 4096 NVFP4 and 2048, 12 311 -> 296); both while
+// the routed rows are few (up to 40 MB 0.9 to 1.4, to 80 0.9 to 1.2, past 100 0.8 to 1.1: NVFP4 288 x 512 x 4096, 3 tokens 101 -> 80, 12 167 / 178; 180 x 768 x
+// 6144, top 4, 15 tokens 215 / 270). The rule is 3 % ahead of two streams; thirteen of the layers are more than 3 % behind, to a tenth.
+// Popular experts (8, 12 or 24 of 128 to 288 take all tokens) change no sign: launched, 2 to 12 tokens 1.02 to 1.5 times as fast as a launch for each.
 int merged_passes(bool fp8, bool nvfp4, int tokens, int top_k, int n_experts, int hidden, int inter, int shared_inter, bool captured,
                   bool down_fits) {
   captured = captured && tokens >= 3;
-  const double down_mb = tokens * (top_k + 1.0) * hidden * inter * (fp8 ? 1.0 : 0.53) / 1e6;
-  const bool down = down_fits && tokens * top_k * 2 <= n_experts &&
-                    (captured ? down_mb <= 64.0 : down_mb <= 100.0 || (nvfp4 && (inter >= 1536 || (tokens >= 16 && top_k >= 8))));
-  const bool up = tokens < 3 || (3ll * hidden * shared_inter <= (32 << 20) && (tokens < 16 || nvfp4) &&
-                                 (down || (tokens < 16 && !captured)));
+  const double down_mb = tokens * (top_k + 1.0) * hidden * inter * (fp8 ? 1.0 : 0.53) / 1e6, shared_m = 3.0 * hidden * shared_inter / 1e6;
+  const bool goes_on = nvfp4 && !captured && (inter >= 1536 || (tokens >= 16 && top_k >= 8));
+  const bool down = down_fits && tokens * top_k * 2 <= n_experts && (down_mb <= (nvfp4 && captured ? 84.0 : 100.0) || goes_on);
+  const bool alone = tokens < 16 && (!captured || (!fp8 && tokens >= 8 && shared_m >= (nvfp4 ? 24.0 : 12.0)));
+  const bool up = tokens < 3 || (3ll * hidden * shared_inter <= (32 << 20) && (tokens < 16 || nvfp4) && (down || alone));
   return up ? 1 + down : 0;
 }
 
@@ -325,8 +326,8 @@ void GlmMoeLayer::enqueue_decode_routed(const uint16_t* x, size_t x_stride, cons
 }
 
 // The dense shared expert: gate and up projections of every token row, SwiGLU, the down projection (unrounded).
-// Above 64 rows the projections have two forms: row tiles of 16, which end sooner where they are few, and tiles of 128, which
-// decode a weight once. Beside the routed chain the second takes less of the chip from it, and is hidden as long as it ends
+// Above 64 rows the projections have two forms: what a launch takes alone (dense_cols: passes of 16 rows, mostly with the parts of K split over
+// the workspace), which ends sooner where they are few, and tiles of 128, which decode a weight once. Beside the routed chain the second takes less of the chip from it, and is hidden as long as it ends
 // first: where the prompt is long (the 16-row form's work grows with it), or where the routed chain - its weights, once more
 // for every 16 rows that an expert has - is long against the walks of hidden, hidden and the shared width. Measured over 184
 // layers of 65 to 591 tokens and 32 to 288 NVFP4 experts, time with the tiles over the time with the form that is faster

@@ -711,7 +711,7 @@ hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t*
 // The 16-row form stays where its blocks, 16 rows of W each, are one round of the CUs and up to 48 rows of A (us, 16-row form /
 // ring: n = 4096, k = 6144: 17 rows 10.1 / 15.2, 48 13.5 / 15.3, 64 16.6 / 15.8; n = 2048, k = 5184: 32 9.9 / 11.1, 48 12.0 / 11.2), two
 // rounds and up to 16 rows (n = 6144, k = 6144: 1 row 12.7 / 15.5, 16 14.9 / 15.5; three rounds, n = 12288, k = 4096: 16.2 / 13.3 and
-// 18.0 / 13.4), up to three quarters of a round below k = 3072 (56 shapes 0.76 to 1.3 times the ring's time, on average 0.97:
+// 18.0 / 13.4; one row of n = 32768, k = 4096 35 / 24, of 65536 68 / 56), up to three quarters of a round below k = 3072 (56 shapes 0.76 to 1.3 times the ring's time, on average 0.97:
 // 147 rows of n = 630, k = 2176 5.9 / 7.7; from 3072 on 0.79 to 1.6, 1.2), and where k is less than sixteen steps and its passes of 16 x 16 are few (n = 1024, k = 1088: 300 rows 5.5 /
 // 6.0, 1024 12.3 / 6.9). Past one round it loses from 17 rows on (n = 6144, k = 4096: 17 rows 12.4 / 11.5, 64 21.4 / 11.9; n = 12288: 20.2 / 13.6).
 //
