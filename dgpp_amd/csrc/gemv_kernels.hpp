@@ -1179,9 +1179,10 @@ inline bool grouped_fills_narrow(int fmt, bool a4, bool gate_up, int n_segs, int
 // A last pass of up to 64 rows takes two thirds of a wide one's time. The estimates are 4 to 14 % off on average, and by half where there are few
 // weight rows: streaming's blocks are counted over all CUs, though a row's column tiles stay on one XCD, and the choice takes 1.2 to 1.75 times the best
 // form's time in 29 of 1020 shapes, most of less than 2300 weight rows (662 x 3776, block FP8, 850 rows 33.1 against 23.4 of the 32-row tiles). So
-// streaming is left only for an estimate 14 % lower, below k = 1024, which the fit does not hold (441 rows of 802 x 448, block FP8 5.9 against 7.1),
-// 30 %, and the 128-row tiles for one 8 % lower. Against the two by the line above: over 600 other shapes 10 % faster on average, none more than 6 %
-// slower; over 420 of up to 131072 weight and 3000 activation rows 5 %, one 7 % slower (129 rows of 6973 x 1536, NVFP4); over 300 of k = 256 to 992 3 %, two 3 and 5 % slower.
+// streaming and the 128-row tiles are left only for an estimate 8 % lower, and streaming below k = 1024, past the fit, for one 13 % lower (320 rows
+// of 587 x 512, NVFP4 6.0 against 7.2, 441 of 802 x 448, block FP8 5.9 against 7.1; with 30 % as many shapes lose as much). Against the two by
+// the line above: over 600 other shapes 11 % faster on average, none more than 6 % slower; over 420 of up to 131072 weight and 3000 activation rows
+// 5 %, three 7 to 14 % slower (74 rows of 12175 x 1024, MXFP4 9.0 -> 10.5); over 300 of k = 256 to 992 5 %, six 6 to 12 % slower.
 // Up to 32 rows it streams, as before there were narrow tiles. That is right up to about 12288 weight rows (4096 x 4096, 17 rows 8.5
 // against 24); past that the 32-row tiles would be ahead: 17 to 32 rows, k = 4096, block FP8 32768 x 4096 31 / 27, 131072 151 / 122, NVFP4 31 / 24 and 122 /
 // 70, MXFP4 24.5 / 17 and 98 / 60, MXFP8 50 / 31 and 206 / 155.
@@ -1200,7 +1201,7 @@ inline int dense_tile_cols(int fmt, int m, int n, int k) {
   const double kk = k / 4096.0, rows_per_xcd = ((n + kTiledRows - 1) / kTiledRows + kXcds - 1) / kXcds;
   int best = 0;
   double least = 1e30;
-  if (!fills) least = (k < 1024 ? 0.7 : 0.86) * (costs.stream_start + costs.stream_round * ((n + 31) / 32) * ((m + 15) / 16) / 3072.0 * (k / 1024.0));
+  if (!fills) least = (k < 1024 ? 0.87 : 0.92) * (costs.stream_start + costs.stream_round * ((n + 31) / 32) * ((m + 15) / 16) / 3072.0 * (k / 1024.0));
   for (int c = 0; c < 3; ++c) {
     const Cost& t = costs.tile[c];
     const int cols = kNarrowCols << c, passes = (m + cols - 1) / cols;
