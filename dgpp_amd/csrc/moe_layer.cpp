@@ -326,9 +326,9 @@ void GlmMoeLayer::enqueue_decode_routed(const uint16_t* x, size_t x_stride, cons
 }
 
 // The dense shared expert: gate and up projections of every token row, SwiGLU, the down projection (unrounded).
-// Above 64 rows the projections have two forms: what a launch takes alone (dense_cols: passes of 16 rows, mostly with the parts of K split over
-// the workspace), which ends sooner where they are few, and tiles of 128, which decode a weight once. Beside the routed chain the second takes less of the chip from it, and is hidden as long as it ends
-// first: where the prompt is long (the 16-row form's work grows with it), or where the routed chain - its weights, once more
+// Above 64 rows the projections have two forms: what a launch takes alone (dense_cols: passes of 16 rows, mostly with the parts
+// of K split over the workspace), which ends sooner where they are few, and tiles of 128, which decode a weight once. Beside the
+// routed chain the second takes less of the chip from it, and is hidden as long as it ends first: where the prompt is long (the 16-row form's work grows with it), or where the routed chain - its weights, once more
 // for every 16 rows that an expert has - is long against the walks of hidden, hidden and the shared width. Measured over 184
 // layers of 65 to 591 tokens and 32 to 288 NVFP4 experts, time with the tiles over the time with the form that is faster
 // alone: 0.87 to 1.08 where this rule takes the tiles (672 -> 582 us with 74 experts, 7168 x 1024, 279 tokens; 906 -> 826
