@@ -723,7 +723,8 @@ hipError_t launch_gemm_tiled(const uint8_t* a, const uint8_t* as, const uint8_t*
 // The panel and the first stages of a block are paid by its walk, and the tiles through registers start sooner. 283 shapes of k = 128 to 1023, up to
 // 131072 rows of W: the ring on average 1.08 times as long, up to 1.9 (20 rows of n = 37178, k = 192 8.0 / 13.2; 163 of 28995, k = 576 20.6
 // / 28.8). From 1024 to 2047, 267 shapes: in one round 0.54 to 1.03, on average 0.83 (the largest tile from 1536 on; 1538 rows of n = 2164, k = 1024
-// 17.9 / 21.6), in more 0.69 to 1.29, 0.99, up to 32 rows of A (against the 16-row form) 0.78 to 1.5, 1.09. Past 2048, 450 shapes, on average 0.82.
+// 17.9 / 21.6), in more 0.69 to 1.29, 0.99; against the 16-row form
+// up to 16 rows of A 0.95 to 1.5, from 17 to 32 0.78 to 0.93 (32 rows of n = 22515, k = 1152 13.0 / 10.5). Past 2048, 450 shapes, on average 0.82.
 //
 // A panel holds the scales of 8192 of k, 6656 beside the largest tile. Without the ring, tiles through registers: the smallest while
 // they are no more than the CUs, the largest once there are two for every CU; the 16-row form up to 32 rows and where its passes are few.
@@ -736,7 +737,7 @@ int tiles_for(int m, int n, int k) {
   if (k >= 1024 && k <= 8192) {
     if (m <= 16 && blocks(16, 64) <= 2 * kCus) return 0;
     if (m <= 48 && blocks(16, 64) <= kCus) return 0;
-    if (k < 2048 && (m <= 32 || blocks(16, 16) <= 7 * kCus)) return 0;
+    if (k < 2048 && (m <= 16 || blocks(16, 16) <= 7 * kCus)) return 0;
     if (k < 3072 && blocks(16, 64) <= kCus * 3 / 4) return 0;
     auto rounds = [&](int tn, int tm) { return (static_cast<int64_t>((n + tn - 1) / tn + 7) / 8 * ((m + tm - 1) / tm) + 31) / 32; };
     const int64_t of[5] = {rounds(32, 64), rounds(64, 64), rounds(64, 128), rounds(128, 64), rounds(128, 128)};
@@ -744,7 +745,7 @@ int tiles_for(int m, int n, int k) {
     int best = 0;
     for (int i = 1; i < 5; ++i)
       if (cost[i] < cost[best]) best = i;
-    if (k >= 2048 || of[best] == 1) return 4 + best;
+    if (k >= 2048 || m <= 32 || of[best] == 1) return 4 + best;
   }
   if (m <= 32 || (m <= 64 && blocks(64, 64) <= kCus)) return 0;
   if (m > 64 && blocks(16, 16) <= (k < 2048 ? 7 : 4) * kCus) return 0;

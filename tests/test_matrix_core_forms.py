@@ -202,10 +202,10 @@ def test_merged_passes_of_a_decode_step(fmt, tokens, top_k, experts, hidden, int
 
 @pytest.mark.parametrize("m,n,k,form", [
     # through registers or 16 rows, measured faster than the ring: short walks, few rows of them, several rounds
-    (20, 37178, 192, 0), (1, 131072, 1984, 0), (32, 65536, 1088, 0), (64, 40000, 128, 2), (163, 28995, 576, 2), (1113, 7514, 576, 3),
+    (20, 37178, 192, 0), (1, 131072, 1984, 0), (16, 65536, 1088, 0), (64, 40000, 128, 2), (163, 28995, 576, 2), (1113, 7514, 576, 3),
     (300, 4096, 960, 2), (1734, 4355, 1472, 3), (1538, 2164, 1024, 2), (160, 10571, 1088, 2), (147, 630, 2176, 0),
     # the ring: one round below sixteen steps, the chip's fullest XCD counted; any from there on
-    (300, 4096, 1024, 6), (54, 8160, 1728, 4), (399, 7013, 1856, 8), (1, 16384, 4096, 5), (300, 4096, 6144, 6), (300, 6144, 4096, 7),
+    (300, 4096, 1024, 6), (32, 22515, 1152, 7), (17, 65536, 1088, 7), (54, 8160, 1728, 4), (399, 7013, 1856, 8), (1, 16384, 4096, 5), (300, 4096, 6144, 6), (300, 6144, 4096, 7),
     (1000, 6144, 4096, 6), (267, 10658, 2688, 6), (33, 8192, 8192, 4),
     # and what no panel holds
     (1000, 6144, 6720, 6), (64, 8192, 8256, 0), (300, 8192, 8256, 2), (16, 4096, 6144, 0), (48, 4096, 6144, 0), (49, 4096, 6144, 4), (1, 1, 64, 0)])
