@@ -406,7 +406,8 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
   // layers of 288 x 512 x 4096 NVFP4 experts with an FP8 one of 512: launched 3 tokens 103 / 118, 8 151 / 158, 14 203 / 203, 18 338 / 278,
   // captured 3 tokens 107 / 101, 8 155 / 139; 64 x 1024 x 4096 and 2048: launched 141 / 150, 248 / 255, 364 / 362, 557 / 408, captured 146 /
   // 132, 252 / 233; 128 x 2048 x 6144 and 2048 (38 M shared weights): launched 255 / 252, 516 / 512, captured 260 / 233.
-  const bool beside_pays = tokens >= 3 && (tokens >= 16 || 3ll * H * w_.shared_inter > (32 << 20) || is_capturing(stream));
+  const bool captured = slot_shared && tokens >= 3 && is_capturing(stream);
+  const bool beside_pays = tokens >= 3 && (tokens >= 16 || 3ll * H * w_.shared_inter > (32 << 20) || captured);
   const bool split = slot_shared && side_ != nullptr && dgpp_tune_get(9) != 1 && (beside_pays || dgpp_tune_get(9) == 2);
   // On one stream the shared down pass ends with the token's accumulation (no launch of its own).
   // (One token, where a launch is a fifth of the step; measured level at two tokens. Bench switch 9 = 4 folds at any
@@ -422,7 +423,7 @@ void GlmMoeLayer::expert_chain_slots(const uint16_t* x, size_t x_stride, const i
   const int merge = dgpp_tune_get(9);
   bool up_done = false;
   if (sh_args && order == nullptr && out_bf16 != nullptr && (merge == 0 || merge >= 5)) {
-    const bool fp8 = w_.format == GlmExpertFormat::Fp8, captured = merge == 0 && tokens >= 3 && is_capturing(stream);
+    const bool fp8 = w_.format == GlmExpertFormat::Fp8;
     const int group = fp8 ? 0 : fp4_group_;
     const dgpp_amd::SharedExpert shared = {{w_.sh_payload[0], w_.sh_payload[1], w_.sh_payload[2]},
                                            {w_.sh_scales[0], w_.sh_scales[1], w_.sh_scales[2]}, w_.shared_inter, w_.sh_rs, w_.sh_cs};
